@@ -583,3 +583,16 @@ def test_prefill_random_shapes(seed, monkeypatch):
         assert np.isfinite(got).all(), case
         assert np.abs(got - want).max() <= ATOL * max(1.0, np.abs(want).max()), case
         assert np.abs(to_np(lse[0]) - wlse).max() <= 5e-2, case
+
+
+@pytest.mark.parametrize("tm, tn", [(128, 64), (7, 5), (130, 200)])
+@pytest.mark.parametrize("case", [
+    # (Sq, C, S, W, P): the runs of candidate tiles touch or overlap (old summaries behind the prefix's end,
+    # windows that reach the prefix), one chunk per m-tile and many, one row, no old summaries at all
+    (1, 128, 8, 4, 0), (137, 128, 8, 0, 8), (700, 3, 9, 1, 20), (701, 2, 1, 0, 233), (640, 5, 4, 2, 0),
+    (900, 136, 8, 1 << 20, 48), (513, 60, 4, 1, 119),
+])
+def test_index_candidate_runs(case, tm, tn):
+    Sq, C, S, W, P = case
+    for skip_old in (False, True):
+        _index_case(Sq, C, S, W, P, skip_old, tm, tn)
