@@ -2,6 +2,7 @@
 or does not load, every operator of this package raises."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 
@@ -93,10 +94,35 @@ def check(code: int, what: str):
         raise KsaError(f"{what}: {msg} (code {code})")
 
 
+_I64x3 = ctypes.c_int64 * 3
+
+
 def strides3(t, dims):
     """int64[3] of element strides of tensor `t` along the three named dims."""
-    return (ctypes.c_int64 * 3)(*[t.stride(d) for d in dims])
+    s = t.stride()
+    return _I64x3(s[dims[0]], s[dims[1]], s[dims[2]])
 
 
 def stream_ptr(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """Handle of the current stream of a GPU (asked for at every call: 0.1 us where a Stream object takes 1.5)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if device.index is None else device.index)
+
+
+_HERE_ALREADY = contextlib.nullcontext()
+
+
+def on_device(device):
+    """Context in which `device` is the current GPU; nothing to enter (and 2 us of host time less) where it
+    is that already."""
+    return _HERE_ALREADY if device.index in (None, torch._C._cuda_getDevice()) else torch.cuda.device(device)
+
+
+def direct(*tensors) -> bool:
+    """Whether an operator's kernels may be called without the dispatcher (10 us of host time per call, as much
+    as a small launch takes on the GPU): plain tensors, and nobody compiles, traces, records or transforms."""
+    if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._get_tracing_state() is not None:
+        return False
+    for t in tensors:
+        if t is not None and (type(t) is not torch.Tensor or (t.requires_grad and torch.is_grad_enabled())):
+            return False
+    return True

@@ -38,7 +38,7 @@ def _move_rows(src: torch.Tensor, dst: torch.Tensor, nrows: int, src_start: int 
         src = src.contiguous()
     if src.shape[0] != bsz or src.shape[1] != heads:
         src = src.expand(bsz, heads, src.shape[2], D)
-    with torch.cuda.device(dst.device):
+    with _lib.on_device(dst.device):
         rc = _lib.lib().ksa_copy_rows(
             src.data_ptr(), dst.data_ptr(),
             src_index.data_ptr() if src_index is not None else None,
@@ -82,7 +82,7 @@ def _move_rows_multi(moves) -> None:
         for j, dim in enumerate((0, 1, 2)):
             sst[3 * i + j], dst_[3 * i + j] = src.stride(dim), dst.stride(dim)
     dev = moves[0][1].device
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib().ksa_copy_rows_multi(n, srcs, dsts, seqs, s0, d0, nr, bsz, heads, D, sst, dst_,
                                             _lib.stream_ptr(dev))
     _lib.check(rc, "ksa_copy_rows_multi")

@@ -17,41 +17,54 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
+from .prefill import kernel_head_dim, pad_head_dim
 
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
+
+
+def _launch_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
+    b, Hq, Q, D = q.shape
+    Hkv = kcache.shape[1]
+    dev = q.device
+    lib = _lib.lib()
+    out = torch.empty((b, Q, Hq, D), dtype=q.dtype, device=dev)
+    ws = None
+    ws_bytes = 0
+    if nsplit > 1:
+        ws_bytes = lib.ksa_decode_workspace_bytes(b, Hq, Hkv, Q, D, nsplit)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    dims = (0, 1, 2)
+    with _lib.on_device(dev):
+        rc = lib.ksa_decode_fwd(
+            q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(),
+            start.data_ptr() if start is not None else None,
+            end.data_ptr() if end is not None else None, start0, end0,
+            b, Hq, Hkv, Q, D, _DTYPES[q.dtype],
+            _lib.strides3(q, dims), _lib.strides3(kcache, dims), _lib.strides3(vcache, dims), _lib.strides3(out, dims),
+            scale, nsplit, ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_ptr(dev))
+    if rc:
+        _lib.check(rc, "ksa_decode_fwd")
+    return out
 
 
 @torch.library.custom_op("ksa_amd::decode_fwd", mutates_args=())
 def _decode_fwd(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
                 start: Optional[torch.Tensor], end: Optional[torch.Tensor], start0: int, end0: int,
                 scale: float, nsplit: int) -> torch.Tensor:
-    b, Hq, Q, D = q.shape
-    Hkv = kcache.shape[1]
-    lib = _lib.lib()
-    out = torch.empty((b, Q, Hq, D), dtype=q.dtype, device=q.device)
-    ws = None
-    ws_bytes = 0
-    if nsplit > 1:
-        ws_bytes = lib.ksa_decode_workspace_bytes(b, Hq, Hkv, Q, D, nsplit)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
-        rc = lib.ksa_decode_fwd(
-            q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(),
-            start.data_ptr() if start is not None else None,
-            end.data_ptr() if end is not None else None, start0, end0,
-            b, Hq, Hkv, Q, D, _DTYPES[q.dtype],
-            _lib.strides3(q, (0, 1, 2)), _lib.strides3(kcache, (0, 1, 2)),
-            _lib.strides3(vcache, (0, 1, 2)), _lib.strides3(out, (0, 1, 2)),
-            float(scale), nsplit, ws.data_ptr() if ws is not None else None, ws_bytes,
-            _lib.stream_ptr(q.device))
-    _lib.check(rc, "ksa_decode_fwd")
-    return out
+    return _launch_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit)
 
 
 @_decode_fwd.register_fake
 def _(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
     b, Hq, Q, D = q.shape
     return q.new_empty((b, Q, Hq, D))
+
+
+def _bound(v, default: int, b: int, device) -> torch.Tensor:
+    """A row bound as the int32 [b] device tensor that the kernels read."""
+    if isinstance(v, torch.Tensor) and v.dtype == torch.int32 and v.device == device and v.shape == (b,) and v.stride(0) == 1:
+        return v
+    return torch.as_tensor(default if v is None else v, device=device).to(torch.int32).expand(b).contiguous()
 
 
 def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
@@ -72,8 +85,7 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     t_start = t_end = None
     s0, e0 = 0, rows
     if isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor):
-        t_start = torch.as_tensor(start if start is not None else 0, device=q.device).to(torch.int32).expand(b).contiguous()
-        t_end = torch.as_tensor(end if end is not None else rows, device=q.device).to(torch.int32).expand(b).contiguous()
+        t_start, t_end = _bound(start, 0, b, q.device), _bound(end, rows, b, q.device)
         max_rows = rows
     else:
         s0 = 0 if start is None else int(start)
@@ -84,7 +96,6 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
         scale = float(D) ** -0.5
     if nsplit is None:
         nsplit = _lib.lib().ksa_decode_auto_splits(b, kcache.shape[1], max_rows)
-    from .prefill import kernel_head_dim, pad_head_dim
     Dk = kernel_head_dim(D)
     if Dk != D:
         # A head dimension without a kernel of its own (the kernels are built for 64 / 128 / 256): the
@@ -100,7 +111,8 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
         out = torch.ops.ksa_amd.decode_fwd(pad_head_dim(q, Dk), kcache, vcache, t_start, t_end, s0, e0,
                                            float(scale), int(nsplit))
         return out[..., :D].contiguous()
-    return torch.ops.ksa_amd.decode_fwd(q, kcache, vcache, t_start, t_end, s0, e0, float(scale), int(nsplit))
+    forward = _launch_decode if _lib.direct(q, kcache, vcache) else torch.ops.ksa_amd.decode_fwd
+    return forward(q, kcache, vcache, t_start, t_end, s0, e0, float(scale), int(nsplit))
 
 
 def ksa_decode_boundary(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, text_start, text_end,
@@ -139,7 +151,7 @@ def ksa_decode_boundary(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
         ws_bytes = lib.ksa_decode_boundary_workspace_bytes(b, Hq, Hkv, Q, D, nsplit)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     ptr = lambda t: t.data_ptr() if t is not None else None
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         rc = lib.ksa_decode_boundary_fwd(
             q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), ptr(ts), ptr(te), ts0, te0,
             ptr(ss), ptr(se), ss0, se0, b, Hq, Hkv, Q, D, _DTYPES[q.dtype], _lib.strides3(q, (0, 1, 2)),
@@ -176,7 +188,6 @@ def ksa_decode_weights(q: torch.Tensor, kcache: torch.Tensor, start=None, end=No
         assert 0 <= s0 < e0 <= rows, "row range out of bounds"
         L = e0 - s0
     assert L > 0
-    from .prefill import kernel_head_dim, pad_head_dim
     Dk = kernel_head_dim(D)
     if scale is None:
         scale = float(D) ** -0.5
@@ -197,7 +208,7 @@ def ksa_decode_weights(q: torch.Tensor, kcache: torch.Tensor, start=None, end=No
     out = torch.empty((b, Hq, Q, L), dtype=q.dtype, device=q.device)
     ws_bytes = lib.ksa_decode_weights_workspace_bytes(b, Hq, Q, L)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         rc = lib.ksa_decode_weights(
             q.data_ptr(), kcache.data_ptr(), out.data_ptr(), mask.data_ptr() if mask is not None else None,
             t_start.data_ptr() if t_start is not None else None, t_end.data_ptr() if t_end is not None else None,

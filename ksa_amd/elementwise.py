@@ -37,7 +37,7 @@ def _add_rmsnorm_partials(x: SplitKPartials, residual: torch.Tensor, weight: tor
     assert w.shape == (H,)
     out = torch.empty(r2.shape, dtype=x.dtype, device=x.device)
     s = torch.empty(r2.shape, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.lib().ksa_add_rmsnorm_partials(x.workspace.data_ptr(), x.ksplit, r2.data_ptr(), w.data_ptr(),
                                                  out.data_ptr(), s.data_ptr(), x.rows, H, r2.stride(0),
                                                  out.stride(0), s.stride(0), _DT[x.dtype], float(eps),
@@ -69,7 +69,7 @@ def add_rmsnorm(x: torch.Tensor, residual: Optional[torch.Tensor], weight: torch
     else:
         s = x2
         args = (None, w.data_ptr(), out.data_ptr(), None, x2.shape[0], H, x2.stride(0), 0, out.stride(0), 0)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = L.ksa_add_rmsnorm(x2.data_ptr(), *args, _DT[x.dtype], float(eps), _lib.stream_ptr(x.device))
     _lib.check(rc, "ksa_add_rmsnorm")
     return s.view(x.shape), out.view(x.shape)
@@ -84,7 +84,7 @@ def silu_mul(gate, up: Optional[torch.Tensor] = None) -> torch.Tensor:
         x = gate
         I = x.shape[-1] // 2
         out = torch.empty(x.rows, I, dtype=x.dtype, device=x.device)
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             rc = _lib.lib().ksa_silu_mul_partials(x.workspace.data_ptr(), x.ksplit, out.data_ptr(), x.rows, I,
                                                   out.stride(0), _DT[x.dtype], _lib.stream_ptr(x.device))
         _lib.check(rc, "ksa_silu_mul_partials")
@@ -96,7 +96,7 @@ def silu_mul(gate, up: Optional[torch.Tensor] = None) -> torch.Tensor:
     I = gate.shape[-1]
     g2, u2 = _rows2d(gate), _rows2d(up)
     out = torch.empty(g2.shape, dtype=gate.dtype, device=gate.device)
-    with torch.cuda.device(gate.device):
+    with _lib.on_device(gate.device):
         rc = _lib.lib().ksa_silu_mul(g2.data_ptr(), u2.data_ptr(), out.data_ptr(), g2.shape[0], I, g2.stride(0),
                                      u2.stride(0), out.stride(0), _DT[gate.dtype], _lib.stream_ptr(gate.device))
     _lib.check(rc, "ksa_silu_mul")
@@ -109,7 +109,7 @@ def argmax_rows(x: torch.Tensor) -> torch.Tensor:
     assert x.is_cuda and x.dtype in _DT
     x2 = _rows2d(x)
     out = torch.empty(x2.shape[0], dtype=torch.long, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.lib().ksa_argmax_rows(x2.data_ptr(), out.data_ptr(), x2.shape[0], x2.shape[1], x2.stride(0),
                                         _DT[x.dtype], _lib.stream_ptr(x.device))
     _lib.check(rc, "ksa_argmax_rows")

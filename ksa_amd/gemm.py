@@ -33,7 +33,7 @@ class TiledWeight:
         L = _lib.lib()
         self.shape, self.dtype, self.device = (N, K), weight.dtype, weight.device
         self.data = torch.empty(L.ksa_tile_weights_bytes(N, K) // 2, dtype=weight.dtype, device=weight.device)
-        with torch.cuda.device(weight.device):
+        with _lib.on_device(weight.device):
             rc = L.ksa_tile_weights(weight.data_ptr(), self.data.data_ptr(), N, K, weight.stride(0),
                                     _lib.stream_ptr(weight.device))
         _lib.check(rc, "ksa_tile_weights")
@@ -76,7 +76,7 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, defer: bool = False):
     M = x2.shape[0]
     assert 1 <= M <= MAX_ROWS, "linear_rows is for at most 128 rows"
     L = _lib.lib()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         ks = L.ksa_gemm_rows_splits(M, N, K)
     defer = defer and ks > 1
     out = None if defer else torch.empty(M, N, dtype=x.dtype, device=x.device)
@@ -85,7 +85,7 @@ def linear_rows(x: torch.Tensor, weight: torch.Tensor, defer: bool = False):
     if ks > 1:
         ws_bytes = L.ksa_gemm_rows_partials_bytes(M, N, ks)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = L.ksa_gemm_rows(x2.data_ptr(), weight.data_ptr(), None if defer else out.data_ptr(), M, N, K,
                              x2.stride(0), weight.stride(0), N, _DT[x.dtype], ks,
                              ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_ptr(x.device))
@@ -109,7 +109,7 @@ def gate_up_silu_rows(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     M = x2.shape[0]
     assert 1 <= M <= MAX_ROWS, "gate_up_silu_rows is for at most 128 rows"
     out = torch.empty(M, I, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.lib().ksa_gemm_rows_gate_up_silu(x2.data_ptr(), weight.data_ptr(), out.data_ptr(), M, I, K,
                                                    x2.stride(0), weight.stride(0), I, _DT[x.dtype],
                                                    _lib.stream_ptr(x.device))
@@ -164,7 +164,7 @@ def mlp_rows(x: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor, ws:
         x2 = x2.contiguous()
     M = x2.shape[0]
     L = _lib.lib()
-    with torch.cuda.device(x2.device):
+    with _lib.on_device(x2.device):
         ks = L.ksa_mlp_rows_down_splits(H, I)
         part = torch.empty(ks * 16 * H, dtype=torch.float32, device=x2.device)
         rc = L.ksa_mlp_rows(x2.data_ptr(), w_gate_up.data_ptr(), w_down.data_ptr(), part.data_ptr(), M, H, I,
@@ -190,7 +190,7 @@ def add_rmsnorm_mlp_rows(o_partials: SplitKPartials, residual: torch.Tensor, nor
     assert r2.shape[0] == M and r2.dtype == dt
     w = norm_weight.to(dt).contiguous()
     L = _lib.lib()
-    with torch.cuda.device(r2.device):
+    with _lib.on_device(r2.device):
         ks = L.ksa_mlp_rows_down_splits(H, I)
         out_sum = torch.empty(M, H, dtype=dt, device=r2.device)
         part = torch.empty(ks * 16 * H, dtype=torch.float32, device=r2.device)

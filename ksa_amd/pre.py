@@ -67,7 +67,7 @@ def pre_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_weig
     per_token = int(kv_out_row is not None and kv_out_row.dim() == 2)
     cstr = (ctypes.c_int64 * 3)(cos.stride(0) if cos.shape[0] > 1 else 0, cos.stride(1), 0)
     L = _lib.lib()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         rc = L.ksa_pre_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), qw.data_ptr(), kw.data_ptr(),
                                  cos.data_ptr(), sin.data_ptr(), qo.data_ptr(), ko.data_ptr(), vo.data_ptr(),
                                  b, S, Hq, Hkv, D, _DT[q.dtype], _bsh(q), _bsh(k), _bsh(v), _bsh(qo),
@@ -111,7 +111,7 @@ def pre_attention_partials(qkv, Hq: int, Hkv: int, D: int, q_norm_weight: torch.
     per_token = int(kv_out_row is not None and kv_out_row.dim() == 2)
     cstr = (ctypes.c_int64 * 3)(cos.stride(0) if cos.shape[0] > 1 else 0, cos.stride(1), 0)
     L = _lib.lib()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = L.ksa_pre_attention_partials(qkv.workspace.data_ptr(), qkv.ksplit, qw.data_ptr(), kw.data_ptr(),
                                           cos.data_ptr(), sin.data_ptr(), qo.data_ptr(), ko.data_ptr(),
                                           vo.data_ptr(), b, S, Hq, Hkv, D, _DT[dtype], _bsh(qo), _bsh(ko),

@@ -52,7 +52,9 @@ def compute_block_sparsity(seqlen_q: int, seqlen_k: int, chunk_size: int, summar
         raise AssertionError("compute_block_sparsity runs on the GPU only")
     M = -(-seqlen_q // tile_m)
     N = -(-seqlen_k // tile_n)
-    with torch.cuda.device(device):
+    if device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    with _lib.on_device(device):
         mc = torch.empty((1, 1, M), dtype=torch.int32, device=device)
         fc = torch.empty((1, 1, M), dtype=torch.int32, device=device)
         mi = torch.empty((1, 1, M, N), dtype=torch.int32, device=device)
@@ -102,7 +104,7 @@ def _analyse_summary_pos(summary_pos: torch.Tensor, Sq: int, C: int, S: int):
     under torch.inference_mode() and later rewritten in place must be followed by
     `clear_summary_pos_cache()`."""
     global _POS_ANALYSES
-    key = (summary_pos.data_ptr(), summary_pos.numel(), str(summary_pos.device), Sq, C, S)
+    key = (summary_pos.data_ptr(), summary_pos.numel(), summary_pos.device, Sq, C, S)
     ver = _pos_version(summary_pos)
     hit = _POS_CACHE.get(key)
     if hit is not None and hit[1] == ver:
@@ -134,16 +136,18 @@ def clear_summary_pos_cache() -> None:
 
 def _check_inputs(q, k, v):
     assert q.is_cuda and k.is_cuda and v.is_cuda, "inputs must be on a GPU"
-    assert q.dtype in _DTYPES, "inputs must be float16 or bfloat16"
-    assert q.dtype == k.dtype == v.dtype, "inputs must have the same dtype"
-    assert q.dim() == 4 and k.dim() == 4 and v.dim() == 4, "q/k/v must be [batch, seq, heads, head_dim]"
-    assert k.shape == v.shape, "k and v must have the same shape"
-    assert q.shape[0] == k.shape[0], "batch mismatch"
-    D = q.shape[-1]
-    assert k.shape[-1] == D, "head_dim mismatch"
+    dt = q.dtype
+    assert dt in _DTYPES, "inputs must be float16 or bfloat16"
+    assert dt == k.dtype == v.dtype, "inputs must have the same dtype"
+    qs, ks = q.shape, k.shape
+    assert len(qs) == 4 and len(ks) == 4 and v.dim() == 4, "q/k/v must be [batch, seq, heads, head_dim]"
+    assert ks == v.shape, "k and v must have the same shape"
+    assert qs[0] == ks[0], "batch mismatch"
+    D = qs[3]
+    assert ks[3] == D, "head_dim mismatch"
     assert D <= 256, "head dimension must be at most 256"
     assert D % 8 == 0, "head dimension must be a multiple of 8"
-    assert q.shape[2] % k.shape[2] == 0, "num_heads must be divisible by num_heads_kv"
+    assert qs[2] % ks[2] == 0, "num_heads must be divisible by num_heads_kv"
 
 
 def _lastdim_contig(t):
@@ -168,29 +172,39 @@ def pad_head_dim(t: torch.Tensor, Dk: int) -> torch.Tensor:
     return t if t.shape[-1] == Dk else torch.nn.functional.pad(t, (0, Dk - t.shape[-1]))
 
 
+def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P, skip_old, phys_prefix, scale, want_lse,
+                    shape):
+    b, Sq, Hq, D = q.shape
+    dev = q.device
+    out = torch.empty_like(q)
+    lse = torch.empty((b, Hq, Sq), dtype=torch.float32, device=dev) if want_lse else None
+    # work queues of this call alone, for a launch long enough to use them (the library's own bound is 32
+    # workgroups per CU; a workgroup takes 128 rows of one or two heads)
+    sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= 1 << 19 else None
+    dims = (0, 1, 2)
+    with _lib.on_device(dev):
+        rc = _lib.lib().ksa_prefill_fwd(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+            lse.data_ptr() if want_lse else None,
+            b, Sq, Hq, k.shape[2], D, _DTYPES[q.dtype],
+            _lib.strides3(q, dims), _lib.strides3(k, dims), _lib.strides3(out, dims),
+            C, S, W, P, int(skip_old), int(phys_prefix),
+            mask_cnt.data_ptr(), mask_idx.data_ptr(), full_cnt.data_ptr(), full_idx.data_ptr(),
+            mask_idx.shape[-1], scale, shape, sched.data_ptr() if sched is not None else None, _lib.stream_ptr(dev))
+    if rc:
+        _lib.check(rc, "ksa_prefill_fwd")
+    return out, lse
+
+
 @torch.library.custom_op("ksa_amd::summary_attn_fwd", mutates_args=())
 def _summary_attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                       mask_cnt: torch.Tensor, mask_idx: torch.Tensor, full_cnt: torch.Tensor,
                       full_idx: torch.Tensor, C: int, S: int, W: int, P: int, skip_old: bool,
                       phys_prefix: bool, scale: float, want_lse: bool,
                       shape: int) -> Tuple[torch.Tensor, torch.Tensor]:
-    b, Sq, Hq, D = q.shape
-    Hkv = k.shape[2]
-    out = torch.empty_like(q)
-    lse = torch.empty((b, Hq, Sq) if want_lse else (0,), dtype=torch.float32, device=q.device)
-    sched = torch.empty(8, dtype=torch.int32, device=q.device)   # work queues of this call alone
-    dims = (0, 1, 2)
-    with torch.cuda.device(q.device):
-        rc = _lib.lib().ksa_prefill_fwd(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-            lse.data_ptr() if want_lse else None,
-            b, Sq, Hq, Hkv, D, _DTYPES[q.dtype],
-            _lib.strides3(q, dims), _lib.strides3(k, dims), _lib.strides3(out, dims),
-            C, S, W, P, int(skip_old), int(phys_prefix),
-            mask_cnt.data_ptr(), mask_idx.data_ptr(), full_cnt.data_ptr(), full_idx.data_ptr(),
-            mask_idx.shape[-1], float(scale), int(shape), sched.data_ptr(), _lib.stream_ptr(q.device))
-    _lib.check(rc, "ksa_prefill_fwd")
-    return out, lse
+    out, lse = _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P, skip_old, phys_prefix, scale,
+                               want_lse, shape)
+    return out, torch.empty(0, dtype=torch.float32, device=q.device) if lse is None else lse
 
 
 @_summary_attn_fwd.register_fake
@@ -206,7 +220,7 @@ def _gathered_prefix(t: torch.Tensor, rows: torch.Tensor, P: int) -> torch.Tenso
     b, Sq, H, D = t.shape
     full = torch.empty((b, P + Sq, H, D), dtype=t.dtype, device=t.device)
     lib = _lib.lib()
-    with torch.cuda.device(t.device):
+    with _lib.on_device(t.device):
         st = _lib.stream_ptr(t.device)
         rc = lib.ksa_copy_rows(t.data_ptr(), full.data_ptr(), rows.data_ptr(), None, 0, 0, P, b, H, D,
                                _lib.strides3(t, (0, 2, 1)), _lib.strides3(full, (0, 2, 1)), st)
@@ -260,7 +274,8 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     Dk = kernel_head_dim(D)
     if Dk != D:   # a head dimension without a kernel of its own: zero-padded copies (see kernel_head_dim)
         q, k, v = pad_head_dim(q, Dk), pad_head_dim(k, Dk), pad_head_dim(v, Dk)
-    out, lse = torch.ops.ksa_amd.summary_attn_fwd(
+    forward = _launch_prefill if _lib.direct(q, k, v) else torch.ops.ksa_amd.summary_attn_fwd
+    out, lse = forward(
         q, k, v, idx[0], idx[1], idx[2], idx[3], C, S, W, P,
         bool(skip_old_summary), phys, scale, bool(return_lse),
         PREFILL_SHAPE if workgroup_shape is None else int(workgroup_shape))

@@ -157,3 +157,35 @@ def test_gpu_operators_equal_direct_calls_and_opcheck():
     # the workspace argument is declared as written to
     torch.library.opcheck(ns.mlp_rows, (x, W["gate_up"], W["down"], ws), test_utils=("test_schema", "test_faketensor"))
     assert int(ws[ksa_amd._lib.lib().ksa_mlp_rows_status_offset():][:8].view(torch.int64).item()) == 0
+
+
+@pytest.mark.gpu
+def test_direct_calls_step_aside_for_modes_and_subclasses():
+    """`_lib.direct` decides whether an attention call goes past the dispatcher: not under a dispatch mode,
+    not for tensor subclasses, not while gradients are asked for."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    import ksa_amd
+    from ksa_amd import _lib
+
+    class Seen(TorchDispatchMode):
+        def __init__(self):
+            super().__init__()
+            self.names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    q = torch.randn(1, 40, 4, 64, device="cuda", dtype=torch.bfloat16)
+    k, v = q[:, :, :2].contiguous(), q[:, :, 2:].contiguous()
+    plain, _ = ksa_amd.summary_attn_func(q, k, v, 32, 4, 1)
+    with Seen() as mode:
+        assert not _lib.direct(q)
+        moded, _ = ksa_amd.summary_attn_func(q, k, v, 32, 4, 1)
+    assert any("summary_attn_fwd" in n for n in mode.names)
+    assert torch.equal(plain, moded)
+    assert _lib.direct(q, None) and not _lib.direct(torch.nn.Parameter(q))
+    with torch.no_grad():
+        assert _lib.direct(q.detach().requires_grad_())
+    assert not _lib.direct(q.detach().requires_grad_())
