@@ -48,20 +48,20 @@
 #include "ksa_mask.h"
 #include "ksa_tile.h"
 
-// This source is compiled as five translation units, so that the instantiations of the kernel
-// compile side by side: unit 0 holds head_dim 64 and 128 and the entry point; units 1 to 4 (files
-// that include this one with KSA_PREFILL_UNIT set) hold one kernel of head_dim 256 each - bf16 /
-// fp16, regular / general tile addressing - because each of those takes over a minute to compile.
+// This source is compiled as seven translation units, so that the instantiations of the kernel
+// compile side by side: unit 0 holds head_dim 64 and 128 and the entry point; units 1 to 6 (files
+// that include this one with KSA_PREFILL_UNIT set) hold one kernel of head_dim 256 each - bf16
+// (1 to 3) / fp16 (4 to 6), general / regular / marked tile addressing - because each of those takes
+// over a minute to compile.
 #ifndef KSA_PREFILL_UNIT
 #define KSA_PREFILL_UNIT 0
 #endif
-// which of the two addressing variants a unit instantiates in launch_shape: 0 both, 1 regular, 2 general
-#if KSA_PREFILL_UNIT == 1 || KSA_PREFILL_UNIT == 3
-#define KSA_PREFILL_VARIANTS 1
-#elif KSA_PREFILL_UNIT == 2 || KSA_PREFILL_UNIT == 4
-#define KSA_PREFILL_VARIANTS 2
+// which of the three addressing variants a unit instantiates in launch_shape: -1 all, else that one
+// (kAddrGeneral, kAddrRegular, kAddrMarked)
+#if KSA_PREFILL_UNIT == 0
+#define KSA_PREFILL_VARIANT -1
 #else
-#define KSA_PREFILL_VARIANTS 0
+#define KSA_PREFILL_VARIANT ((KSA_PREFILL_UNIT - 1) % 3)
 #endif
 
 namespace {
@@ -136,10 +136,24 @@ __device__ __forceinline__ RowVis ksa_row_vis(const KsaMask& mk, int q) {
     return r;
 }
 
-// kRegular: every listed key tile lies entirely in the summary prefix or entirely in the
-// in-line region and inside the key axis (P and Sk multiples of 64), and in-place prefix
-// rows of one thread differ by a uniform step; then tile addressing is branch-free.
-//
+// kAddr: how the rows of K/V that a thread fills of a tile are found.
+//   kAddrRegular: they differ by a uniform step, in the prefix as in the in-line region, and every tile
+//     lies in one of the two and inside the key axis (the prefix and the key axis are multiples of 64
+//     rows): branch-free.
+//   kAddrMarked: the same step, any lengths (the usual prompt).  The two tiles that do not follow the
+//     rule - the one that holds the end of the prefix, the one that the end of the key axis cuts - are
+//     marked in their word: the loop's fills then take any 64 rows that exist, and the rows that belong
+//     there are fetched over them behind the score product (`fill_special`).  Marked tiles come last in
+//     the walk, so that only masked steps carry the branch: in every step it costs 4.5 % at 128k rows
+//     (it takes the row sums out of the place the compiler gives them at the end of the step), in the
+//     masked ones 4 % at 4k rows - which is why lengths that need no marks keep a variant of their own.
+//   kAddrGeneral: a division per lane and fill (700 to 1200 cycles a tile); left to a summary count that
+//     does not divide the step with a prefix read in place, and to fewer than 64 rows.
+// Lengths that are no multiple of 64 with the marked variant against the general one (32 query heads):
+// 1000 tokens 26.3 -> 23.5 us, 4000 78 -> 71 us, 2 x 3000 109 -> 96 us, 32800 1009 -> 980 us, three
+// prompts of 9001 tokens with an unbounded window in fp16 2267 -> 2169 us.
+enum { kAddrGeneral = 0, kAddrRegular = 1, kAddrMarked = 2 };
+
 // RB: 32-row query blocks per wave.  RB = 1: one query head per workgroup, wave w owns rows
 // 32w..32w+31, two workgroups per CU.  RB = 2: two query heads of one kv group per workgroup,
 // waves {0,1} / {2,3} own rows 0..63 / 64..127 of the first / second head, one workgroup per
@@ -156,7 +170,7 @@ struct PrefillShape {
     static constexpr int kThreads = 64 * kWaves;
 };
 
-template <typename T, int D, bool kRegular, int RB, int HW>
+template <typename T, int D, int kAddr, int RB, int HW>
 __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 128 ? 2 : 1)) void ksa_prefill_kernel(
     const PrefillParams p) {
     constexpr int kThreads = PrefillShape<RB, HW>::kThreads;
@@ -167,6 +181,8 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     constexpr int ROWB = 2 * D;      // LDS row of K / V in bytes (unpadded, XOR-swizzled chunks)
     constexpr int KLD = (kTileN * CPR) / kThreads;  // K (and V) loads per thread
     constexpr int RSTEP = kThreads / CPR;           // row distance between a thread's loads
+    constexpr bool kRegular = kAddr != kAddrGeneral;
+    constexpr bool kMarks = kAddr == kAddrMarked;
     constexpr float kTau = 8.f;      // lazy rescale: exponents stay below 2^kTau
 
     // K and V tiles travel global -> LDS directly (global_load_lds), 1 KB per wave
@@ -287,24 +303,18 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
 
     // Regular tiles: uniform offset word = byte offset of the tile's first row | 1 if the
     // tile lies in the in-line region (computed per lane when the walk order is fetched).
+    // 3: a tile that is not regular (see kRegular); its loop fills take the first 64 rows.
+    constexpr uint32_t kSpecialBit = 2u;
     auto tile_word = [&](int n) -> uint32_t {
         const int n0 = n * kTileN;
         const bool in_main = phys || n0 >= mk.P;
+        if (kMarks && n0 + kTileN > (in_main ? mk.Sk : mk.P)) return kSpecialBit | 1u;
         return in_main ? ((uint32_t)(phys ? n0 : n0 - mk.P) * rb) | 1u
                        : (uint32_t)(n0 / mk.S) * Bblk * rb;
     };
-    // one 1 KB piece (load i of KLD) of tile n into an LDS tile; `col` = kcol or vcol
+    // one 1 KB piece into an LDS tile, at the place of load i of KLD
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    auto fill1 = [&](const char* base, uint16_t* tile, uint32_t col, int n, uint32_t word, int i, uint32_t odd_xor) {
-        uint32_t ub, us, vo;
-        if constexpr (kRegular) {
-            const bool in_main = word & 1u;
-            ub = word & ~1u;
-            us = in_main ? step_main : step_pre;
-            vo = in_main ? thr_main : thr_pre;
-        } else {
-            tile_src(n * kTileN, i, ub, us, vo);
-        }
+    auto fill_from = [&](const char* src, uint32_t loff, uint16_t* tile, int i) {
         typedef __attribute__((address_space(3))) char* lptr;
         char* dst = reinterpret_cast<char*>(tile) + (RSTEP * i + wave_u * (64 / CPR)) * ROWB;
         // Uniform 64-bit base + one 32-bit lane offset (the scalar-base addressing form); M0
@@ -312,8 +322,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         // assembly so that the compiler does not track the fill: it would otherwise make LDS
         // reads wait for fills it cannot tell apart; which fills must have landed before a
         // barrier is decided by fills_done.
-        uint64_t ubase = reinterpret_cast<uint64_t>(base + (ub + us * i));
-        const uint32_t loff = vo + (col ^ ((i & 1) ? odd_xor : 0u));
+        uint64_t ubase = reinterpret_cast<uint64_t>(src);
         uint32_t lds_addr = (uint32_t)(uintptr_t)(lptr)dst;
         if constexpr (D > 128) {
             // (both are the same in every lane; at this size the compiler no longer proves it and
@@ -329,6 +338,35 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
                      : "s"(lds_addr), "v"(loff), "s"(ubase)
                      : "memory", "m0");
 #pragma clang diagnostic pop
+    };
+    // load i of KLD of tile n; `col` = kcol or vcol
+    auto fill1 = [&](const char* base, uint16_t* tile, uint32_t col, int n, uint32_t word, int i, uint32_t odd_xor) {
+        uint32_t ub, us, vo;
+        if constexpr (kRegular) {
+            const bool in_main = word & 1u;
+            ub = word & (kMarks ? ~3u : ~1u);
+            us = in_main ? step_main : step_pre;
+            vo = in_main ? thr_main : thr_pre;
+        } else {
+            tile_src(n * kTileN, i, ub, us, vo);
+        }
+        fill_from(base + (ub + us * i), vo + (col ^ ((i & 1) ? odd_xor : 0u)), tile, i);
+    };
+    // the rows of a tile that is not regular, over what the loop's fills put there (which have to have landed):
+    // a row of the prefix by the regular rule, a row of the in-line region or the last one where it is cut
+    auto fill_special = [&](const char* base, uint16_t* tile, uint32_t col, int n, uint32_t odd_xor) {
+        const uint32_t pre = (uint32_t)(n * kTileN / mk.S) * Bblk * rb;  // (unused where n is no tile of the prefix)
+        const int last = phys ? mk.Sk - 1 : mk.Sq - 1;
+        // (this thread's row from an opaque lane number: nothing of this rare path lives in a register of the loop)
+        int zero = 0;
+        asm volatile("" : "+v"(zero));
+        const int lane2 = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+        int row = (phys ? n * kTileN : n * kTileN - mk.P) + (wave_u * 64 + lane2) / CPR;  // negative in the prefix
+#pragma unroll 1
+        for (int i = 0; i < KLD; ++i, row += RSTEP) {
+            const uint32_t off = row < 0 ? pre + step_pre * i + thr_pre : (uint32_t)min(row, last) * rb;
+            fill_from(base, off + (col ^ ((i & 1) ? odd_xor : 0u)), tile, i);
+        }
     };
     auto fill = [&](const char* base, uint16_t* tile, uint32_t col, int n, uint32_t word, uint32_t odd_xor) {
 #pragma unroll
@@ -374,6 +412,10 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     const int32_t* plist = p.mask_idx + (int64_t)mt * p.idx_stride;
     const int32_t* flist = p.full_idx + (int64_t)mt * p.idx_stride;
     int nquick = 0;
+    // the marked tile at the end of the prefix, if the row tile lists it: its position in the list
+    const int n_mark = kMarks && !phys && mk.P % kTileN != 0 ? mk.P / kTileN : -1;
+    int mark_pos = 0;
+    bool has_mark = false;
     int c0 = 0, c1 = 0;  // entries [c0, c1) of the list of partial tiles: the uniform in-line tiles described below
     {
         const int c_first = (mt * kTileM) / Bblk;
@@ -411,7 +453,8 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         // below n_c1: counted by the whole wave, 128 entries per round of independent loads, instead
         // of binary searches whose dependent loads would cost several microseconds at the start of
         // every workgroup
-        const int lim = min(npart, max(nlim, n_c1));
+        int lim = min(npart, max(nlim, n_c1));
+        if constexpr (kMarks) lim = min(npart, max(lim, n_mark + 1));
         int cnt = 0, cnt0 = 0, cnt1 = 0;
         for (int base = 0; base < lim; base += 128) {
             const int i0 = base + lane, i1 = base + 64 + lane;
@@ -420,6 +463,10 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             cnt += __popcll(__ballot(e0 < nlim)) + __popcll(__ballot(e1 < nlim));
             cnt0 += __popcll(__ballot(e0 < n_c0)) + __popcll(__ballot(e1 < n_c0));
             cnt1 += __popcll(__ballot(e0 < n_c1)) + __popcll(__ballot(e1 < n_c1));
+            if constexpr (kMarks) {
+                mark_pos += __popcll(__ballot(e0 < n_mark)) + __popcll(__ballot(e1 < n_mark));
+                has_mark = has_mark || (__ballot(e0 == n_mark) | __ballot(e1 == n_mark)) != 0ull;
+            }
         }
         nquick = cnt;
         c0 = max(cnt0, nquick);
@@ -428,14 +475,26 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     const bool last_full_cut = nfull > 0 && (flist[nfull - 1] + 1) * kTileN > mk.Sk;
     const int nfull_a = nfull - (last_full_cut ? 1 : 0);
     // Walk order.  Phase A: the leading prefix tiles, the uniform in-line tiles, the full tiles; phase B:
-    // the other partial tiles (those in front of the uniform run, those behind it, a cut full tile).
+    // the other partial tiles (those in front of the uniform run, those behind it, a cut full tile; the
+    // tile at the end of the prefix last).
     const int ncheap = c1 - c0;
     const int n_a = nquick + ncheap + nfull_a;
+    // (the marked tile's place among phase B's entries: it is never one of phase A)
+    const int mark_j = mark_pos - nquick - (mark_pos >= c1 ? ncheap : 0);
+    // Steps of phase A that may run as such: a step requests the tiles of the next two, and the marked ones - the
+    // tile at the end of the prefix, the last two in front of it where the key axis cuts a tile - need masked steps.
+    int n_run = n_a;
+    if constexpr (kMarks) {
+        const bool cut = mk.Sk % kTileN != 0 && mk.P + min((mt + 1) * kTileM, mk.Sq) > mk.Sk / kTileN * kTileN;
+        if (has_mark || cut) n_run = min(n_a, max(ntiles - (has_mark ? 1 : 0) - (cut ? 2 : 0) - 2, 0));
+    }
     auto tile_at = [&](int i) {
         if (i < nquick) return plist[i];
         if (i < nquick + ncheap) return plist[c0 + (i - nquick)];
         if (i < n_a) return flist[i - nquick - ncheap];
-        int j = i - n_a + nquick;            // entries [nquick, c0), then [c1, npart)
+        int j = i - n_a;
+        if (kMarks && has_mark) j = i == ntiles - 1 ? mark_j : j + (j >= mark_j ? 1 : 0);
+        j += nquick;                         // entries [nquick, c0), then [c1, npart)
         if (j >= c0) j += ncheap;
         return j < npart ? plist[j] : flist[nfull - 1];
     };
@@ -736,6 +795,13 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if constexpr (kMarks && kGeneral) {
+            if ((wk | wv) & kSpecialBit) {
+                fills_done();
+                if (wk & kSpecialBit) fill_special(kbase, kdst, kcol, nk, kKOdd);
+                if (wv & kSpecialBit) fill_special(vbase, vdst, vcol, nv, 0u);
+            }
+        }
         if constexpr (!kSafe) {
             // 2^24: some exponent exceeded the reference by more than ~19
 #pragma unroll
@@ -816,6 +882,16 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             fill(vbase, Vs0, vcol, seq(0, 0), seq_word(0, 0), 0u);
             fill(kbase, Ks1, kcol, seq(i1, 0), seq_word(i1, 0), kKOdd);
             fills_done();
+            if constexpr (kMarks) {
+                if ((seq_word(0, 0) | seq_word(i1, 0)) & kSpecialBit) {
+                    if (seq_word(0, 0) & kSpecialBit) {
+                        fill_special(kbase, Ks0, kcol, seq(0, 0), kKOdd);
+                        fill_special(vbase, Vs0, vcol, seq(0, 0), 0u);
+                    }
+                    if (seq_word(i1, 0) & kSpecialBit) fill_special(kbase, Ks1, kcol, seq(i1, 0), kKOdd);
+                    fills_done();
+                }
+            }
             __syncthreads();
             scores(s0, Ks0);
 #pragma unroll
@@ -833,11 +909,11 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             }
         }
         int it = 0;
-        for (; it + 2 <= n_a; it += 2) {
+        for (; it + 2 <= n_run; it += 2) {
             step(safe_tag, A{}, Even{}, it, s0, s1, it < nquick + ncheap);
             step(safe_tag, A{}, Odd{}, it + 1, s1, s0, it + 1 < nquick + ncheap);
         }
-        if (it < n_a) {
+        if (it < n_run) {
             step(safe_tag, A{}, Even{}, it, s0, s1, it < nquick + ncheap);
             copy_scores();
             ++it;
@@ -924,20 +1000,22 @@ __global__ void ksa_prefill_zero_queues_kernel(int32_t* sched) {
     if (threadIdx.x < 8) sched[threadIdx.x] = 0;
 }
 
-// whether a launch can use the kernel variant with regular tile addressing (see kRegular)
+// the addressing variant of a launch (see kAddr; the 64-row shape has no registers for marks)
 template <int D, int RB, int HW>
-bool prefill_regular(const PrefillParams& p) {
+int prefill_addr(const PrefillParams& p) {
     constexpr int RSTEP = PrefillShape<RB, HW>::kThreads / (D / 8);
     const KsaMask& mk = p.mk;
-    const bool prefix_ok = mk.P == 0 || p.phys_prefix || (RSTEP % mk.S == 0 && mk.P % kTileN == 0);
-    return prefix_ok && mk.Sk % kTileN == 0;
+    const bool in_place = mk.P > 0 && !p.phys_prefix;
+    if (in_place && RSTEP % mk.S != 0) return kAddrGeneral;
+    if (mk.Sk % kTileN == 0 && (!in_place || mk.P % kTileN == 0)) return kAddrRegular;
+    return RB == 1 && (p.phys_prefix ? mk.Sk : mk.Sq) >= kTileN ? kAddrMarked : kAddrGeneral;
 }
 
 template <typename T, int D, int RB, int HW>
 int launch_shape(const PrefillParams& p, int batch, hipStream_t stream) {
     constexpr int kThreads = PrefillShape<RB, HW>::kThreads;
-    const bool regular = prefill_regular<D, RB, HW>(p);
-    if ((KSA_PREFILL_VARIANTS == 1 && !regular) || (KSA_PREFILL_VARIANTS == 2 && regular)) return KSA_ERR_INVALID;
+    const int addr = prefill_addr<D, RB, HW>(p);
+    if (KSA_PREFILL_VARIANT >= 0 && addr != KSA_PREFILL_VARIANT) return KSA_ERR_INVALID;
     PrefillParams pp = p;
     pp.n_items = p.M * (p.Hq / HW);
     pp.total = pp.n_items * batch;
@@ -955,12 +1033,15 @@ int launch_shape(const PrefillParams& p, int batch, hipStream_t stream) {
         pp.sched = nullptr;
     }
     dim3 grid(pp.total + spare);
-#if KSA_PREFILL_VARIANTS != 2
-    if (regular) hipLaunchKernelGGL((ksa_prefill_kernel<T, D, true, RB, HW>), grid, dim3(kThreads), 0, stream, pp);
-#endif
-#if KSA_PREFILL_VARIANTS != 1
-    if (!regular) hipLaunchKernelGGL((ksa_prefill_kernel<T, D, false, RB, HW>), grid, dim3(kThreads), 0, stream, pp);
-#endif
+    auto go = [&](auto tag) {
+        constexpr int kAddr = decltype(tag)::value;
+        if constexpr ((KSA_PREFILL_VARIANT < 0 || KSA_PREFILL_VARIANT == kAddr) && !(kAddr == kAddrMarked && RB != 1))
+            if (addr == kAddr)
+                hipLaunchKernelGGL((ksa_prefill_kernel<T, D, kAddr, RB, HW>), grid, dim3(kThreads), 0, stream, pp);
+    };
+    go(std::integral_constant<int, kAddrGeneral>{});
+    go(std::integral_constant<int, kAddrRegular>{});
+    go(std::integral_constant<int, kAddrMarked>{});
     return ksa_check_launch();
 }
 
@@ -984,25 +1065,30 @@ bool stride_ok(int64_t s) { return (s % 8) == 0; }
 }  // namespace
 
 // head_dim 256: one launcher per translation unit (they all see the same PrefillParams)
-int ksa_prefill_launch_d256_bf16_regular(const void* params, int batch, void* stream);
-int ksa_prefill_launch_d256_bf16_general(const void* params, int batch, void* stream);
-int ksa_prefill_launch_d256_f16_regular(const void* params, int batch, void* stream);
-int ksa_prefill_launch_d256_f16_general(const void* params, int batch, void* stream);
+#define KSA_PREFILL_D256(type, addr) ksa_prefill_launch_d256_##type##_##addr(const void* params, int batch, void* stream)
+int KSA_PREFILL_D256(bf16, general);
+int KSA_PREFILL_D256(bf16, regular);
+int KSA_PREFILL_D256(bf16, marked);
+int KSA_PREFILL_D256(f16, general);
+int KSA_PREFILL_D256(f16, regular);
+int KSA_PREFILL_D256(f16, marked);
 #if KSA_PREFILL_UNIT == 1
-int ksa_prefill_launch_d256_bf16_regular(const void* params, int batch, void* stream) {
-    return launch<KsaBf16, 256>(*static_cast<const PrefillParams*>(params), batch, (hipStream_t)stream);
-}
+int KSA_PREFILL_D256(bf16, general)
 #elif KSA_PREFILL_UNIT == 2
-int ksa_prefill_launch_d256_bf16_general(const void* params, int batch, void* stream) {
-    return launch<KsaBf16, 256>(*static_cast<const PrefillParams*>(params), batch, (hipStream_t)stream);
-}
+int KSA_PREFILL_D256(bf16, regular)
 #elif KSA_PREFILL_UNIT == 3
-int ksa_prefill_launch_d256_f16_regular(const void* params, int batch, void* stream) {
-    return launch<KsaF16, 256>(*static_cast<const PrefillParams*>(params), batch, (hipStream_t)stream);
-}
+int KSA_PREFILL_D256(bf16, marked)
 #elif KSA_PREFILL_UNIT == 4
-int ksa_prefill_launch_d256_f16_general(const void* params, int batch, void* stream) {
-    return launch<KsaF16, 256>(*static_cast<const PrefillParams*>(params), batch, (hipStream_t)stream);
+int KSA_PREFILL_D256(f16, general)
+#elif KSA_PREFILL_UNIT == 5
+int KSA_PREFILL_D256(f16, regular)
+#elif KSA_PREFILL_UNIT == 6
+int KSA_PREFILL_D256(f16, marked)
+#endif
+#if KSA_PREFILL_UNIT >= 1
+{
+    return launch<std::conditional_t<(KSA_PREFILL_UNIT <= 3), KsaBf16, KsaF16>, 256>(
+        *static_cast<const PrefillParams*>(params), batch, (hipStream_t)stream);
 }
 #else
 
@@ -1074,15 +1160,21 @@ extern "C" int ksa_prefill_fwd(const void* q, const void* k, const void* v, void
     if (dtype == KSA_DTYPE_BF16) {
         if (D == 128) return launch<KsaBf16, 128>(p, batch, st);
         if (D == 64) return launch<KsaBf16, 64>(p, batch, st);
-        if (D == 256)
-            return prefill_regular<256, 1, 1>(p) ? ksa_prefill_launch_d256_bf16_regular(&p, batch, stream)
-                                                 : ksa_prefill_launch_d256_bf16_general(&p, batch, stream);
+        if (D == 256) {
+            const int addr = prefill_addr<256, 1, 1>(p);
+            return addr == kAddrRegular  ? ksa_prefill_launch_d256_bf16_regular(&p, batch, stream)
+                   : addr == kAddrMarked ? ksa_prefill_launch_d256_bf16_marked(&p, batch, stream)
+                                         : ksa_prefill_launch_d256_bf16_general(&p, batch, stream);
+        }
     } else {
         if (D == 128) return launch<KsaF16, 128>(p, batch, st);
         if (D == 64) return launch<KsaF16, 64>(p, batch, st);
-        if (D == 256)
-            return prefill_regular<256, 1, 1>(p) ? ksa_prefill_launch_d256_f16_regular(&p, batch, stream)
-                                                 : ksa_prefill_launch_d256_f16_general(&p, batch, stream);
+        if (D == 256) {
+            const int addr = prefill_addr<256, 1, 1>(p);
+            return addr == kAddrRegular  ? ksa_prefill_launch_d256_f16_regular(&p, batch, stream)
+                   : addr == kAddrMarked ? ksa_prefill_launch_d256_f16_marked(&p, batch, stream)
+                                         : ksa_prefill_launch_d256_f16_general(&p, batch, stream);
+        }
     }
     return KSA_ERR_UNSUPPORTED;  // other head dimensions: the caller pads to 64 / 128 / 256
 }

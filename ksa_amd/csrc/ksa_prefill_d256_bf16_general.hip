@@ -1,4 +1,4 @@
-// Translation unit of ksa_prefill.hip that holds the bf16 kernel of head_dim 256 with general tile addressing
-// (compiled next to the main unit instead of inside it: each of these instantiations takes over a minute).
-#define KSA_PREFILL_UNIT 2
+// Prefill kernel, head_dim 256, bf16, general tile addressing: a translation unit of its own
+// (see the head of ksa_prefill.hip).
+#define KSA_PREFILL_UNIT 1
 #include "ksa_prefill.hip"

@@ -1,4 +1,4 @@
-// Translation unit of ksa_prefill.hip that holds the fp16 kernel of head_dim 256 with regular tile addressing
-// (compiled next to the main unit instead of inside it: each of these instantiations takes over a minute).
-#define KSA_PREFILL_UNIT 3
+// Prefill kernel, head_dim 256, fp16, regular tile addressing: a translation unit of its own
+// (see the head of ksa_prefill.hip).
+#define KSA_PREFILL_UNIT 5
 #include "ksa_prefill.hip"

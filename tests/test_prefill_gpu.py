@@ -596,3 +596,26 @@ def test_index_candidate_runs(case, tm, tn):
     Sq, C, S, W, P = case
     for skip_old in (False, True):
         _index_case(Sq, C, S, W, P, skip_old, tm, tn)
+
+
+@pytest.mark.parametrize("D, shape", [(128, 32), (128, 2), (64, 0), (256, 0)])
+@pytest.mark.parametrize("Sq", [64, 65, 136, 191, 1088 + 8, 1089, 1216 - 1])
+def test_prefill_marked_tiles(Sq, D, shape):
+    """Lengths whose prefix ends inside a key tile and whose key axis cuts one (and, at 64 rows and 1088 + 8,
+    only one of the two): the tiles that the regular addressing leaves to `fill_special`, for windows
+    that see them from everywhere, from the first chunks only and not at all."""
+    import ksa_amd
+    dev = torch.device("cuda")
+    C, S = 128, 8
+    q, k, v = (t.bfloat16() for t in make_qkv(Sq, 4, 2, D, seed=Sq + D, scaled=False))
+    sp = O.summary_positions(Sq, C, S)
+    for W in (0, 2, 1000):
+        for spt in (torch.as_tensor(sp, device=dev), None):
+            out, lse = ksa_amd.summary_attn_func(q[None].to(dev), k[None].to(dev), v[None].to(dev), C, S, W,
+                                                 summary_pos=spt, return_lse=True, workgroup_shape=shape)
+            want, wlse = c_oracle.attention_rows(to_np(q), to_np(k), to_np(v), C, S, W,
+                                                 summary_pos=None if spt is None else sp)
+            got = to_np(out[0])
+            assert np.isfinite(got).all(), (Sq, D, W)
+            assert np.abs(got - want).max() <= ATOL * max(1.0, np.abs(want).max()), (Sq, D, W)
+            assert np.abs(to_np(lse[0]) - wlse).max() <= 5e-2, (Sq, D, W)
