@@ -66,6 +66,21 @@
 
 namespace {
 
+// n / d for 0 <= n < 2^31 with d fixed per launch: one multiplication, where the compiler's division by
+// a number it does not know is some 35 instructions - a workgroup has about twenty of them in front of
+// its first tile.  With p = 31 + ceil(log2 d) and m = ceil(2^p / d), m d - 2^p < d <= 2^(p - 31), hence
+// floor(n m / 2^p) = floor(n / d); m < 2^32 and 2 n < 2^32, so n m / 2^p is (2 n m / 2^32) / 2^ceil(log2 d).
+struct FastDiv {
+    uint32_t d, m, s;
+    FastDiv() = default;
+    explicit FastDiv(uint32_t n) : d(n), s(0) {
+        while ((1ull << s) < d) ++s;
+        m = (uint32_t)(((1ull << (31 + s)) + d - 1) / d);
+    }
+    __device__ __forceinline__ int div(int n) const { return (int)(__umulhi(2u * (uint32_t)n, m) >> s); }
+    __device__ __forceinline__ int mod(int n) const { return n - div(n) * (int)d; }
+};
+
 struct PrefillParams {
     const uint16_t* q;
     const uint16_t* k;
@@ -99,6 +114,9 @@ struct PrefillParams {
     int n_items;      // items per batch element
     int total;        // items in all
     int n_static;     // multiple of 8
+    FastDiv by_items, by_hkv, by_gper;  // n_items, Hkv, query heads (pairs) per kv head
+    FastDiv by_block, by_S;             // C + S, S
+    int phase_shift;                    // the least multiple of C + S that is not below P
 };
 
 constexpr int kTileM = 128;
@@ -112,9 +130,9 @@ struct RowVis {
     bool b_text;
 };
 
-__device__ __forceinline__ RowVis ksa_row_vis(const KsaMask& mk, int q) {
+__device__ __forceinline__ RowVis ksa_row_vis(const KsaMask& mk, const FastDiv& by_block, int q) {
     const int B = mk.C + mk.S;
-    const int c = q / B, o = q % B;
+    const int c = by_block.div(q), o = q - c * B;
     RowVis r;
     if (o >= mk.C) {  // summary row: own chunk, causal, every column kind
         r.xa = 0;
@@ -223,15 +241,25 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         item = s_item;
         if (item < 0) return;  // every queue is empty: a spare workgroup
     }
-    const int bz = item / p.n_items;
+    const int bz = p.by_items.div(item);
     const int id = item - bz * p.n_items;
-    const int kvh = id % p.Hkv;
-    const int rest = id / p.Hkv;
+    const int rest = p.by_hkv.div(id);
+    const int kvh = id - rest * p.Hkv;
     constexpr int kWavesPerHead = 4 / RB;
 
-    const int gper = p.g / HW;
-    const int gi = rest % gper;
-    const int mt = p.M - 1 - rest / gper;
+    const int up = p.by_gper.div(rest);
+    const int gi = rest - up * (p.g / HW);
+    const int mt = p.M - 1 - up;
+    // The counts and the first entries of the two lists of tiles are requested before anything else (rows of the
+    // index are N entries, zeroed behind the counts): they head the chain of trips to memory in front of the first
+    // tile, and with the counts awaited before the entries it was one trip longer.
+    const int32_t* plist = p.mask_idx + (int64_t)mt * p.idx_stride;
+    const int32_t* flist = p.full_idx + (int64_t)mt * p.idx_stride;
+    const int npart = p.mask_cnt[mt];
+    const int nfull = p.full_cnt[mt];
+    const int list_p0 = plist[min(lane, p.idx_stride - 1)];
+    const int list_p1 = plist[min(64 + lane, p.idx_stride - 1)];
+    const int list_f0 = flist[min(lane, p.idx_stride - 1)];
     const int head = kvh * p.g + HW * gi + wave / kWavesPerHead;
     const int row0 = mt * kTileM + (wave % kWavesPerHead) * 32 * RB;
     const KsaMask mk = p.mk;
@@ -247,7 +275,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     for (int r = 0; r < RB; ++r) {
         qrow[r] = row0 + 32 * r + lq;
         const int qrow_c = min(qrow[r], mk.Sq - 1);
-        rv[r] = ksa_row_vis(mk, qrow_c);
+        rv[r] = ksa_row_vis(mk, p.by_block, qrow_c);
         const uint16_t* qp = p.q + bz * p.q_bs + (int64_t)qrow_c * p.q_rs + head * p.q_hs + 8 * lh;
 #pragma unroll
         for (int s = 0; s < KS; ++s) qf[r][s] = *reinterpret_cast<const u32x4*>(qp + 16 * s);
@@ -271,16 +299,16 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     const uint32_t thr_main = (uint32_t)ld_row * rb;
     // in-place prefix: prefix row j lives at in-line row (j / S) * B + C + j % S; when S
     // divides the per-thread row step the rows of one thread differ by a uniform amount
-    const bool s_fast = !phys && (RSTEP % mk.S == 0);
+    const bool s_fast = !phys && p.by_S.mod(RSTEP) == 0;
     const uint32_t thr_pre =
-        s_fast ? (uint32_t)((ld_row / mk.S) * Bblk + mk.C + ld_row % mk.S) * rb : 0u;
+        s_fast ? (uint32_t)(p.by_S.div(ld_row) * Bblk + mk.C + p.by_S.mod(ld_row)) * rb : 0u;
     const uint32_t step_main = RSTEP * rb;
-    const uint32_t step_pre = s_fast ? (uint32_t)(RSTEP / mk.S) * Bblk * rb : 0u;
+    const uint32_t step_pre = s_fast ? (uint32_t)p.by_S.div(RSTEP) * Bblk * rb : 0u;
 
     auto src_row = [&](int kv) -> uint32_t {  // generic key column -> K/V row
         kv = min(kv, mk.Sk - 1);
         if (phys || kv >= mk.P) return (uint32_t)(phys ? kv : kv - mk.P);
-        return (uint32_t)((kv / mk.S) * Bblk + mk.C + kv % mk.S);
+        return (uint32_t)(p.by_S.div(kv) * Bblk + mk.C + p.by_S.mod(kv));
     };
 
     // tile, load i -> (uniform byte offset, uniform per-load step, this thread's byte offset for load i)
@@ -291,7 +319,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             ustep = step_main;
             voff = thr_main;
         } else if (s_fast && n0 + kTileN <= mk.P) {
-            ubase = (uint32_t)(n0 / mk.S) * Bblk * rb;
+            ubase = (uint32_t)p.by_S.div(n0) * Bblk * rb;
             ustep = step_pre;
             voff = thr_pre;
         } else {
@@ -310,7 +338,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         const bool in_main = phys || n0 >= mk.P;
         if (kMarks && n0 + kTileN > (in_main ? mk.Sk : mk.P)) return kSpecialBit | 1u;
         return in_main ? ((uint32_t)(phys ? n0 : n0 - mk.P) * rb) | 1u
-                       : (uint32_t)(n0 / mk.S) * Bblk * rb;
+                       : (uint32_t)p.by_S.div(n0) * Bblk * rb;
     };
     // one 1 KB piece into an LDS tile, at the place of load i of KLD
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
@@ -355,7 +383,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     // the rows of a tile that is not regular, over what the loop's fills put there (which have to have landed):
     // a row of the prefix by the regular rule, a row of the in-line region or the last one where it is cut
     auto fill_special = [&](const char* base, uint16_t* tile, uint32_t col, int n, uint32_t odd_xor) {
-        const uint32_t pre = (uint32_t)(n * kTileN / mk.S) * Bblk * rb;  // (unused where n is no tile of the prefix)
+        const uint32_t pre = (uint32_t)p.by_S.div(n * kTileN) * Bblk * rb;  // (unused where n is no tile of the prefix)
         const int last = phys ? mk.Sk - 1 : mk.Sq - 1;
         // (this thread's row from an opaque lane number: nothing of this rare path lives in a register of the loop)
         int zero = 0;
@@ -406,11 +434,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     };
 
     // ---- walk order ----
-    const int npart = p.mask_cnt[mt];
-    const int nfull = p.full_cnt[mt];
     const int ntiles = npart + nfull;
-    const int32_t* plist = p.mask_idx + (int64_t)mt * p.idx_stride;
-    const int32_t* flist = p.full_idx + (int64_t)mt * p.idx_stride;
     int nquick = 0;
     // the marked tile at the end of the prefix, if the row tile lists it: its position in the list
     const int n_mark = kMarks && !phys && mk.P % kTileN != 0 ? mk.P / kTileN : -1;
@@ -418,7 +442,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     bool has_mark = false;
     int c0 = 0, c1 = 0;  // entries [c0, c1) of the list of partial tiles: the uniform in-line tiles described below
     {
-        const int c_first = (mt * kTileM) / Bblk;
+        const int c_first = p.by_block.div(mt * kTileM);
         const int w_first = c_first > mk.W ? c_first - mk.W : 0;
         // every text row of the tile has xa >= w_first * S and blo >= P >= thr
         const int thr = (prefix_mode && !mk.skip_old) ? min(w_first * mk.S, mk.P) : 0;
@@ -436,14 +460,15 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
 #ifndef KSA_PREFILL_NO_UNIFORM_TILES
         if (mk.S == 8 && mk.C % 8 == 0 && mk.P % 8 == 0 && Bblk >= kTileN + 8) {
             const int R0 = mt * kTileM, R1 = min(R0 + kTileM, mk.Sq) - 1;
-            const int q_ft = (R0 % Bblk) < mk.C ? R0 : (R0 / Bblk + 1) * Bblk;            // first text row
-            const int q_lt = (R1 % Bblk) < mk.C ? R1 : (R1 / Bblk) * Bblk + mk.C - 1;      // last text row
-            const int q_fs = (R0 % Bblk) >= mk.C ? R0 : (R0 / Bblk) * Bblk + mk.C;          // first summary row
+            const int s0 = c_first * Bblk, s1 = p.by_block.div(R1) * Bblk;      // starts of the first and the last chunk
+            const int q_ft = R0 - s0 < mk.C ? R0 : s0 + Bblk;                  // first text row
+            const int q_lt = R1 - s1 < mk.C ? R1 : s1 + mk.C - 1;              // last text row
+            const int q_fs = R0 - s0 >= mk.C ? R0 : s0 + mk.C;                 // first summary row
             if (q_ft <= R1 && q_lt >= q_ft) {
-                const int c_lt = q_lt / Bblk;
+                const int c_lt = p.by_block.div(q_lt);
                 const int lo = mk.P + (c_lt > mk.W ? c_lt - mk.W : 0) * Bblk;
                 int hi = mk.P + q_ft + 1;
-                if (q_fs <= R1) hi = min(hi, mk.P + (q_fs / Bblk) * Bblk);
+                if (q_fs <= R1) hi = min(hi, mk.P + s0);
                 n_c0 = (lo + kTileN - 1) / kTileN;
                 n_c1 = max(hi / kTileN, n_c0);
             }
@@ -458,8 +483,8 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         int cnt = 0, cnt0 = 0, cnt1 = 0;
         for (int base = 0; base < lim; base += 128) {
             const int i0 = base + lane, i1 = base + 64 + lane;
-            const int e0 = i0 < lim ? plist[i0] : 0x7fffffff;
-            const int e1 = i1 < lim ? plist[i1] : 0x7fffffff;
+            const int e0 = i0 < lim ? (base == 0 ? list_p0 : plist[i0]) : 0x7fffffff;
+            const int e1 = i1 < lim ? (base == 0 ? list_p1 : plist[i1]) : 0x7fffffff;
             cnt += __popcll(__ballot(e0 < nlim)) + __popcll(__ballot(e1 < nlim));
             cnt0 += __popcll(__ballot(e0 < n_c0)) + __popcll(__ballot(e1 < n_c0));
             cnt1 += __popcll(__ballot(e0 < n_c1)) + __popcll(__ballot(e1 < n_c1));
@@ -472,7 +497,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         c0 = max(cnt0, nquick);
         c1 = max(cnt1, c0);
     }
-    const bool last_full_cut = nfull > 0 && (flist[nfull - 1] + 1) * kTileN > mk.Sk;
+    const bool last_full_cut = mk.Sk % kTileN != 0 && nfull > 0 && (flist[nfull - 1] + 1) * kTileN > mk.Sk;
     const int nfull_a = nfull - (last_full_cut ? 1 : 0);
     // Walk order.  Phase A: the leading prefix tiles, the uniform in-line tiles, the full tiles; phase B:
     // the other partial tiles (those in front of the uniform run, those behind it, a cut full tile; the
@@ -488,29 +513,41 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         const bool cut = mk.Sk % kTileN != 0 && mk.P + min((mt + 1) * kTileM, mk.Sq) > mk.Sk / kTileN * kTileN;
         if (has_mark || cut) n_run = min(n_a, max(ntiles - (has_mark ? 1 : 0) - (cut ? 2 : 0) - 2, 0));
     }
-    auto tile_at = [&](int i) {
-        if (i < nquick) return plist[i];
-        if (i < nquick + ncheap) return plist[c0 + (i - nquick)];
-        if (i < n_a) return flist[i - nquick - ncheap];
+    // entry i of the order: index >= 0 into the list of partial tiles, ~index into the list of full ones
+    auto order_at = [&](int i) {
+        if (i < nquick) return i;
+        if (i < nquick + ncheap) return c0 + (i - nquick);
+        if (i < n_a) return ~(i - nquick - ncheap);
         int j = i - n_a;
         if (kMarks && has_mark) j = i == ntiles - 1 ? mark_j : j + (j >= mark_j ? 1 : 0);
         j += nquick;                         // entries [nquick, c0), then [c1, npart)
         if (j >= c0) j += ncheap;
-        return j < npart ? plist[j] : flist[nfull - 1];
+        return j < npart ? j : ~(nfull - 1);
     };
-    // The order is kept in registers, 64 entries at a time (lane i holds entry base + i),
-    // so the loop never waits on a dependent index load.
-    auto seq_chunk = [&](int base) { return base + lane < ntiles ? tile_at(base + lane) : 0; };
-    int seq_cur = seq_chunk(0);
-    int seq_nxt = seq_chunk(64);
+    // The order is kept in registers, 64 entries at a time (lane i holds entry base + i), so the loop never waits
+    // on a dependent index load.
+    auto seq_chunk = [&](int base) {
+        const int k = order_at(base + lane);
+        return base + lane < ntiles ? (k < 0 ? flist[~k] : plist[k]) : 0;
+    };
+    // ... and its first 128 entries come from the lanes that hold the first loads, where they have brought them
+    auto first_chunk = [&](int base) {
+        const int k = order_at(base + lane), a = k < 0 ? ~k : k;
+        const int e0 = __shfl(list_p0, a), e1 = __shfl(list_p1, a), f0 = __shfl(list_f0, a);
+        int n = k < 0 ? f0 : (a < 64 ? e0 : e1);
+        const bool live = base + lane < ntiles;
+        if (live && a >= (k < 0 ? 64 : 128)) n = k < 0 ? flist[a] : plist[a];
+        return live ? n : 0;
+    };
+    int seq_cur = first_chunk(0);
+    int seq_nxt = first_chunk(64);
     uint32_t word_cur = kRegular ? tile_word(seq_cur) : 0u;
     uint32_t word_nxt = kRegular ? tile_word(seq_nxt) : 0u;
     // Where a tile's first column stands in the period of C text + S summary columns of the
     // in-line region, (n0 - P) mod (C + S) in [0, C + S): computed with the walk order, one
     // division per lane and 64 tiles, so that the masked steps have none.
     auto tile_phase = [&](int n) {
-        const int r = (n * kTileN - mk.P) % Bblk;
-        return r < 0 ? r + Bblk : r;
+        return p.by_block.mod(n * kTileN - mk.P + p.phase_shift);
     };
     int phase_cur = tile_phase(seq_cur);
     int phase_nxt = tile_phase(seq_nxt);
@@ -861,12 +898,14 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         constexpr bool kSafe = decltype(safe_tag)::value;
         using A = std::false_type;
         using B = std::true_type;
-        seq_cur = seq_chunk(0);
-        seq_nxt = seq_chunk(64);
-        word_cur = kRegular ? tile_word(seq_cur) : 0u;
-        word_nxt = kRegular ? tile_word(seq_nxt) : 0u;
-        phase_cur = tile_phase(seq_cur);
-        phase_nxt = tile_phase(seq_nxt);
+        if constexpr (kSafe) {  // from the start again
+            seq_cur = seq_chunk(0);
+            seq_nxt = seq_chunk(64);
+            word_cur = kRegular ? tile_word(seq_cur) : 0u;
+            word_nxt = kRegular ? tile_word(seq_nxt) : 0u;
+            phase_cur = tile_phase(seq_cur);
+            phase_nxt = tile_phase(seq_nxt);
+        }
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
             m_ref[r] = -1e30f;  // finite: the first rescale multiplies the zero accumulators by 0
@@ -1020,6 +1059,9 @@ int launch_shape(const PrefillParams& p, int batch, hipStream_t stream) {
     pp.n_items = p.M * (p.Hq / HW);
     pp.total = pp.n_items * batch;
     pp.n_static = pp.total;
+    pp.by_items = FastDiv((uint32_t)pp.n_items);
+    pp.by_hkv = FastDiv((uint32_t)p.Hkv);
+    pp.by_gper = FastDiv((uint32_t)(p.g / HW));
     int spare = 0;
     // Queues only for long launches (32 workgroups per CU and more; measured at 128k rows: +2.2 %,
     // at 32k rows with 17 per CU: -0.8 %), where the tail they even out is worth the clearing kernel
@@ -1147,6 +1189,9 @@ extern "C" int ksa_prefill_fwd(const void* q, const void* k, const void* v, void
     p.mk = KsaMask{C, S, W, P, skip_old ? 1 : 0, Sq, Sk};
     p.scale = scale;
     p.scale_log2 = scale * 1.4426950408889634f;
+    p.by_block = FastDiv((uint32_t)(C + S));
+    p.by_S = FastDiv((uint32_t)S);
+    p.phase_shift = (P + C + S - 1) / (C + S) * (C + S);
     p.sched = sched;
     // Workgroup shape (D = 128, even group size; anything else uses one head per workgroup):
     // 2 = two heads on 8 waves; 32 = one head on 4 waves; 64 = two heads on 4 waves with 64 query
