@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
         const int nst = min(kChunkSteps, s_end - c0);
         u32x4 a[kChunkSteps];
 #pragma unroll
-        for (int u = 0; u < kChunkSteps; ++u) a[u] = *reinterpret_cast<const u32x4*>(wl.p + wl.step * min(c0 + u, s_end - 1));
+        for (int u = 0; u < kChunkSteps; ++u) a[u] = ksa_load_weights(wl.p + wl.step * min(c0 + u, s_end - 1));
         // x[0:M][32 c0 .. 32 (c0 + nst)) -> LDS, 16 bytes per thread and pass
         for (int e = threadIdx.x; e < p.M * (kChunkK / 8); e += 256) {
             const int m = e / (kChunkK / 8), j = e % (kChunkK / 8);
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(con
     };
     u32x4 a[kChunkSteps];
     auto w_request = [&](int c, int u) {
-        a[u] = *reinterpret_cast<const u32x4*>(wl.p + wl.step * min(c * kChunkSteps + u, steps - 1));
+        a[u] = ksa_load_weights(wl.p + wl.step * min(c * kChunkSteps + u, steps - 1));
     };
     // the products of one chunk; kMore: there is a next chunk, whose x and weights are requested on the way
     // (two copies of the loop body rather than a condition inside it: with branches between the MFMAs the
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     u32x4 a[kB];
     auto load_steps = [&](int s0) {
 #pragma unroll
-        for (int u = 0; u < kB; ++u) a[u] = *reinterpret_cast<const u32x4*>(wl.p + wl.step * min(s0 + u, steps - 1));
+        for (int u = 0; u < kB; ++u) a[u] = ksa_load_weights(wl.p + wl.step * min(s0 + u, steps - 1));
     };
     load_steps(slice * kChunkSteps);  // in flight while x is staged (every slice has a first chunk: S <= chunks)
     const int per_row = p.K / 8;

@@ -191,7 +191,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
             if (r < kTileCols) {
 #pragma unroll
                 for (int k = 0; k < kB; ++k)
-                    a[k] = *reinterpret_cast<const u32x4*>(wl.p + wl.step * min(s0 + k, sl_steps - 1));
+                    a[k] = ksa_load_weights(wl.p + wl.step * min(s0 + k, sl_steps - 1));
             }
         };
         load_steps(0);  // in flight while x is waited for and staged
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
     u32x4 ad[kChunkSteps];
     if (live) {  // on their way while the activation is waited for
 #pragma unroll
-        for (int k = 0; k < kChunkSteps; ++k) ad[k] = *reinterpret_cast<const u32x4*>(wl.p + wl.step * min(k, nst - 1));
+        for (int k = 0; k < kChunkSteps; ++k) ad[k] = ksa_load_weights(wl.p + wl.step * min(k, nst - 1));
     }
     unsigned long long launch = 0;  // (thread 0 only) launches before this one
     if (tid == 0) {

@@ -252,7 +252,9 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     const int mt = p.M - 1 - up;
     // The counts and the first entries of the two lists of tiles are requested before anything else (rows of the
     // index are N entries, zeroed behind the counts): they head the chain of trips to memory in front of the first
-    // tile, and with the counts awaited before the entries it was one trip longer.
+    // tile, and with the counts awaited before the entries it was one trip longer (with the divisions gone too, a
+    // workgroup starts its walk 3.2 instead of 4.5 us behind its own start at 300 tokens, 4.8 instead of 6.0 at 4k:
+    // 38.2 against 39.6 us a launch there, 933 against 955 us at 32k, +1.1 % at 128k).
     const int32_t* plist = p.mask_idx + (int64_t)mt * p.idx_stride;
     const int32_t* flist = p.full_idx + (int64_t)mt * p.idx_stride;
     const int npart = p.mask_cnt[mt];
