@@ -28,65 +28,119 @@ struct GemmParams {
     float* part;         // [ksplit, ksa_partial_rows(M), N] when ksplit > 1
     int64_t xs, ws, os;
     int M, N, K, ksplit;
+    int tiles, steps, chunks, chunks_per_split;  // tiles of 16 columns; steps of 32 and chunks of 512 elements of K
 };
 
-// grid: (tiles of 64 output columns, K splits); block: 4 waves, each 16 columns over the whole K
-// slice.  Per chunk of 512 K elements a wave first requests its 16 weight fragments (16 x 16
-// bytes per lane in flight), the workgroup copies the chunk of x into LDS once, and the MFMAs
-// then take their B operands from there: x is fetched once per 64 columns instead of once per
-// wave and step, which is what held a first version of this kernel at 60 % of the rate below.
-template <typename T>
+// grid: (tiles of 64 output columns, K splits); block: 4 waves, each 16 columns over the K slice of the
+// workgroup, in chunks of 512 elements.  x is fetched once per workgroup and chunk, through LDS (fetched by
+// every wave for itself it held a first version of this kernel at 60 % of the rate).
+//
+// A launch streams 20 to 50 MB in 5 to 12 us, so what counts besides the rate is how soon a wave has its
+// requests out and how little is left to do behind the last one:
+//   * all that a wave's addresses need comes from the host or from scalar registers (streaming layout: a
+//     fragment is a scalar base plus one 32-bit lane offset), nothing is divided, rows past M and steps
+//     past K repeat the last one instead of being branched around;
+//   * x is requested in front of the weights: it is in LDS while most of the weights are on their way, and a
+//     fragment meets it as it arrives.  (Requested behind them it came last, and all products waited for it.)
+//   * with more than one chunk a fragment's registers are refilled behind its MFMA.
+// Per call in a graph of calls on distinct weights, 1 / 8 / 16 rows: 6144 x 2560 7.7 / 8.4 / 9.3 ->
+// 6.6 / 7.2 / 7.7 us, 2560 x 4096 7.2 / 7.9 / 8.8 -> 6.1 / 6.7 / 7.2, 2560 x 9728 12.0 / 12.9 / 14.5 -> 9.4 / 10.0 / 10.5 (31,
+// 21 and 50 MB are read in 6.1, 4.6 and 8.5 us by a kernel that does nothing else).
+template <typename T, bool kTiled, int XT>
 __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) {
     using C = KsaCvt<T>;
-    __shared__ __attribute__((aligned(16))) unsigned char xs[2][16 * kRowB];
+    __shared__ __attribute__((aligned(16))) unsigned char xs[2][4 * XT * kRowB];
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15;   // row of W inside the tile (A operand) / row of x (B operand)
     const int kq = lane >> 4;  // which 8 of the 32 K elements of a step
-    const int n0 = (blockIdx.x * 4 + wave) * 16;
-    const int steps = p.K / 32;
-    const int per_split = (steps + p.ksplit - 1) / p.ksplit;
-    const int s_begin = blockIdx.y * per_split;
-    const int s_end = min(steps, s_begin + per_split);
+    const int tile = blockIdx.x * 4 + wave;
+    const int n0 = tile * 16;
+    const int c_begin = blockIdx.y * p.chunks_per_split;
+    const int c_end = min(p.chunks, c_begin + p.chunks_per_split);
 
-    const KsaWeightLane wl = ksa_weight_lane(p.w, p.ws, p.K, n0, r, kq, p.N);
-    // rows of x beyond M repeat the last one: their columns of the product are never stored
-    const int xrow = min(r, p.M - 1);
+    // streaming layout: [ceil(N / 16)][steps][1 KB], lane offset 64 r + 16 kq; a wave past the matrix reads its last
+    // tile (nothing of it is stored).  Row-major: lane r reads row n0 + r (or the last one).
+    const char* wtile = reinterpret_cast<const char*>(p.w);
+    uint32_t wlane;
+    if constexpr (kTiled) {
+        wtile += (int64_t)min(tile, p.tiles - 1) * p.steps * 1024;
+        wlane = (uint32_t)(64 * r + 16 * kq);
+    } else {
+        wtile += (int64_t)min(n0 + r, p.N - 1) * p.ws * 2;
+        wlane = (uint32_t)(16 * kq);
+    }
+    u32x4 a[kChunkSteps];
+    auto w_request = [&](int c, int u) {
+        const int64_t s = min(c * kChunkSteps + u, p.steps - 1);
+        a[u] = ksa_load_weights(reinterpret_cast<const uint16_t*>(wtile + s * (kTiled ? 1024 : 64) + wlane));
+    };
+    // staging of a chunk of x: thread = (row wave + 4 i, 16-byte piece lane); pieces past a short last chunk become
+    // zeros, so that its missing steps add nothing
+    const uint16_t* xrow[XT];
+#pragma unroll
+    for (int i = 0; i < XT; ++i) xrow[i] = p.x + (int64_t)min(wave + 4 * i, p.M - 1) * p.xs;
+    u32x4 xt[XT];
+    auto x_request = [&](int c) {
+        const int piece = min(c * (4 * kChunkSteps) + lane, 4 * p.steps - 1);
+#pragma unroll
+        for (int i = 0; i < XT; ++i) xt[i] = *reinterpret_cast<const u32x4*>(xrow[i] + 8 * piece);
+    };
+    auto x_store = [&](int c, int buf) {
+        const bool live = c * (4 * kChunkSteps) + lane < 4 * p.steps;
+#pragma unroll
+        for (int i = 0; i < XT; ++i) {
+            u32x4 v = xt[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = live ? v[e] : 0u;
+            *reinterpret_cast<u32x4*>(xs[buf] + (wave + 4 * i) * kRowB + 16 * lane) = v;
+        }
+    };
+    const int xoff = min(r, 4 * XT - 1) * kRowB + 16 * kq;
 
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    int buf = 0;
-    for (int c0 = s_begin; c0 < s_end; c0 += kChunkSteps) {
-        const int nst = min(kChunkSteps, s_end - c0);
-        u32x4 a[kChunkSteps];
-#pragma unroll
-        for (int u = 0; u < kChunkSteps; ++u) a[u] = ksa_load_weights(wl.p + wl.step * min(c0 + u, s_end - 1));
-        // x[0:M][32 c0 .. 32 (c0 + nst)) -> LDS, 16 bytes per thread and pass
-        for (int e = threadIdx.x; e < p.M * (kChunkK / 8); e += 256) {
-            const int m = e / (kChunkK / 8), j = e % (kChunkK / 8);
-            if (j < nst * 4)
-                *reinterpret_cast<u32x4*>(xs[buf] + m * kRowB + 16 * j) =
-                    *reinterpret_cast<const u32x4*>(p.x + (int64_t)m * p.xs + 32 * c0 + 8 * j);
-        }
-        // (one barrier per chunk is enough with two buffers: nobody passes the next chunk's
-        // barrier before everybody has finished reading this one)
-        __syncthreads();
+    auto chunk = [&](auto more_tag, int cn, int buf) __attribute__((always_inline)) {  // cn: the next chunk (kMore)
+        constexpr bool kMore = decltype(more_tag)::value;
+        if constexpr (kMore) x_request(cn);
 #pragma unroll
         for (int u = 0; u < kChunkSteps; ++u) {
-            if (u < nst) {
-                const u32x4 b = *reinterpret_cast<const u32x4*>(xs[buf] + xrow * kRowB + 64 * u + 16 * kq);
-                acc = mfma16<T>(a[u], b, acc);
-            }
+            acc = mfma16<T>(a[u], *reinterpret_cast<const u32x4*>(xs[buf] + xoff + 64 * u), acc);
+            if constexpr (kMore) w_request(cn, u);
         }
-        buf ^= 1;
-    }
-    // C layout of the 16x16 tile: lane holds column (row of x) lane % 16, rows (of W) 4 * (lane / 16) + i
-    if (r < p.M) {
+    };
+    if (c_begin < c_end) {  // (a split count beyond the chunks leaves slices without any: zeros)
+        x_request(c_begin);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int n = n0 + 4 * kq + i;
-            if (n < p.N) {
-                if (p.ksplit == 1) p.out[(int64_t)r * p.os + n] = C::down(acc[i]);
-                else p.part[((int64_t)blockIdx.y * 16 + r) * p.N + n] = acc[i];
+        for (int u = 0; u < kChunkSteps; ++u) w_request(c_begin, u);
+        x_store(c_begin, 0);
+        __syncthreads();
+        int buf = 0;
+        for (int c = c_begin; c + 1 < c_end; ++c) {
+            chunk(std::true_type{}, c + 1, buf);
+            // (one barrier per chunk is enough with two buffers: nobody passes the next chunk's
+            // barrier before everybody has finished reading this one)
+            buf ^= 1;
+            x_store(c + 1, buf);
+            __syncthreads();
+        }
+        chunk(std::false_type{}, c_end, buf);
+    }
+
+    // C layout of the 16x16 tile: lane holds column (row of x) lane % 16, rows (of W) 4 * (lane / 16) + i
+    const int n = n0 + 4 * kq;
+    if (r < p.M && n < p.N) {
+        if (p.ksplit == 1) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n + i < p.N) p.out[(int64_t)r * p.os + n + i] = C::down(acc[i]);
+        } else {
+            float* dst = p.part + ((int64_t)blockIdx.y * 16 + r) * p.N + n;
+            if (p.N % 4 == 0) {
+                *reinterpret_cast<f32x4*>(dst) = acc;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < p.N) dst[i] = acc[i];
             }
         }
     }
@@ -334,9 +388,20 @@ int launch_wide(const WideParams& p, hipStream_t st) {
 }
 
 template <typename T>
-int launch_gemm(const GemmParams& p, hipStream_t st) {
-    dim3 grid((p.N + 63) / 64, p.ksplit);
-    hipLaunchKernelGGL(ksa_gemm_rows_kernel<T>, grid, dim3(256), 0, st, p);
+int launch_gemm(GemmParams p, hipStream_t st) {
+    p.tiles = (p.N + 15) / 16;
+    p.steps = p.K / 32;
+    p.chunks = (p.steps + kChunkSteps - 1) / kChunkSteps;
+    p.chunks_per_split = (p.chunks + p.ksplit - 1) / p.ksplit;
+    const dim3 grid((p.N + 63) / 64, p.ksplit), block(256);
+    auto go = [&](auto tiled) {
+        constexpr bool kT = decltype(tiled)::value;
+        if (p.M <= 4) hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 1>), grid, block, 0, st, p);
+        else if (p.M <= 8) hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 2>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 4>), grid, block, 0, st, p);
+    };
+    if (p.ws == kWTiled) go(std::true_type{});
+    else go(std::false_type{});
     if (p.ksplit > 1 && p.out) {
         const int64_t n = (int64_t)p.M * p.N;
         hipLaunchKernelGGL(ksa_gemm_rows_reduce_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);
@@ -439,22 +504,19 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
 
 }  // namespace
 
-// K splits that give about two workgroups per CU of the current device (256 CUs assumed when no
-// device can be asked) without slices shorter than one chunk
-// of 512; when one chunk per workgroup is at least that many splits and still a moderate grid,
-// that is taken instead: a workgroup then stages x once and has no loop (measured 11 % faster at
-// N = 19456, K = 2560).
+// K splits for at most 16 rows: slices are whole chunks of 512, none empty.  One chunk per workgroup where
+// that is not more than 2048 workgroups (a workgroup then has no loop: 11 % faster at N = 19456, K = 2560; the
+// sums of up to 32 slices are added by the consumer), otherwise about two workgroups per CU of the current
+// device (256 CUs assumed when no device can be asked).
 extern "C" int ksa_gemm_rows_auto_splits(int N, int K) {
     if (N <= 0 || K <= 0) return 1;
     const int tiles = (N + 63) / 64;
+    const int chunks = (K / 32 + kChunkSteps - 1) / kChunkSteps;
     const int want = 2 * ksa_cu_count_or(256);
     int sp = (want + tiles - 1) / tiles;
-    const int chunks = K / 32 / 16 > 1 ? K / 32 / 16 : 1;
-    if (sp > chunks) sp = chunks;
-    if (sp > 16) sp = 16;
-    if (sp < 1) sp = 1;
-    if (sp > 1 && chunks >= sp && chunks <= 16 && (long long)tiles * chunks <= 2048 && K % (32 * 16) == 0) sp = chunks;
-    return sp;
+    if (sp > 1 && chunks <= 32 && (long long)tiles * chunks <= 2048) sp = chunks;
+    if (sp > 32) sp = 32;
+    return wide_plan(K, sp).ksplit;
 }
 
 extern "C" size_t ksa_gemm_rows_workspace_bytes(int N, int ksplit) {
