@@ -189,3 +189,44 @@ def test_direct_calls_step_aside_for_modes_and_subclasses():
     with torch.no_grad():
         assert _lib.direct(q.detach().requires_grad_())
     assert not _lib.direct(q.detach().requires_grad_())
+
+
+def test_direct_calls_step_aside_for_transforms_and_negative_views():
+    """... nor inside `torch.func` transforms and function modes, nor for views whose negative bit is set."""
+    from torch.overrides import TorchFunctionMode
+
+    from ksa_amd import _lib
+
+    seen = []
+
+    def ask(a):
+        seen.append(_lib.direct(a))
+        return a * 1
+
+    x = torch.randn(2, 3)
+    torch.func.vmap(ask)(x)
+    torch.func.jvp(ask, (x,), (x,))
+    torch.func.functionalize(ask)(x)
+    torch.func.grad(lambda a: ask(a).sum())(x)
+    assert seen == [False] * 4
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert not _lib.direct(x)
+    assert _lib.direct(x)
+    neg = torch.complex(x, x).conj().imag
+    assert neg.is_neg() and not _lib.direct(neg)
+
+
+@pytest.mark.gpu
+def test_prefill_under_vmap():
+    """Attention calls inside `torch.func.vmap` equal one call per slice."""
+    import ksa_amd
+    q = torch.randn(2, 1, 40, 4, 64, device="cuda", dtype=torch.bfloat16)
+    k, v = q[:, :, :, :2].contiguous(), q[:, :, :, 2:].contiguous()
+    f = lambda a, b, c: ksa_amd.summary_attn_func(a, b, c, 32, 4, 1)[0]
+    got = torch.func.vmap(f)(q, k, v)
+    assert torch.equal(got, torch.stack([f(q[i], k[i], v[i]) for i in range(2)]))
