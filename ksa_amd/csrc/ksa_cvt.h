@@ -44,6 +44,7 @@ struct KsaCvt<KsaBf16> {
             : "v"(a0), "v"(b0), "v"(a1), "v"(b1), "v"(a2), "v"(b2), "v"(a3), "v"(b3));
     }
     static constexpr uint32_t kOnes = 0x3f803f80u;  // (1.0, 1.0)
+    static constexpr uint32_t kInfBits = 0x7f80u;
 };
 template <>
 struct KsaCvt<KsaF16> {
@@ -79,6 +80,7 @@ struct KsaCvt<KsaF16> {
         r0 = dot2(a0, b0, 0.f), r1 = dot2(a1, b1, 0.f), r2 = dot2(a2, b2, 0.f), r3 = dot2(a3, b3, 0.f);
     }
     static constexpr uint32_t kOnes = 0x3c003c00u;
+    static constexpr uint32_t kInfBits = 0x7c00u;
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));

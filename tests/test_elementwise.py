@@ -130,3 +130,29 @@ def test_gpu_argmax_rows(dtype, rows, N):
     if rows > 3 and N > 20:
         x[3, 17] = float("nan")                               # a NaN counts as the largest value
         assert int(argmax_rows(dev(x))[3]) == 17 == int(x.float().argmax(-1)[3])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N", [9, 8192, 81920, 81928, 163851])
+def test_gpu_argmax_rows_ties_and_special_values(dtype, N):
+    """Equal maxima in every place of the scan (batches of 81920 values, items of 8, the values behind the
+    last item), rows of one value, -inf, zeros of both signs, and NaNs of both signs: first index, as torch."""
+    from ksa_amd.elementwise import argmax_rows
+    g = torch.Generator().manual_seed(N)
+    Np = (N + 7) // 8 * 8
+    x = torch.randn(8, Np, generator=g).to(dtype)
+    places = sorted({0, 7, 8, N // 2, N - 2, N - 1, min(N, 81919), min(N - 1, 81920), min(N - 1, 1024 * 8)} & set(range(N)))
+    for i, first in enumerate((0, 1, len(places) // 2)):
+        x[i, places[first:]] = 40.0
+    x[3] = float("-inf")
+    x[4] = -1.5
+    x[5] = -torch.rand(Np, generator=g).to(dtype) - 1
+    x[5, places[1]] = -0.0
+    x[5, places[-1]] = 0.0
+    x[6, places[-1]] = float("nan")
+    x[6, places[1]] = -float("nan")
+    x[6, 0] = float("inf")
+    x[7, N - 1] = float("inf")
+    got = argmax_rows(x.cuda()[:, :N]).cpu()
+    assert torch.equal(got, x[:, :N].float().argmax(-1))
