@@ -276,8 +276,8 @@ int ksa_silu_mul_partials(const float* partials, int ksplit, void* out, int rows
  *   K a multiple of 32; fp32 accumulation, one rounding at the end.
  * ksplit > 1 splits K over workgroups and needs a device workspace for the partial sums:
  * ksa_gemm_rows_splits(M, N, K) gives the split count to use and ksa_gemm_rows_partials_bytes(M, N,
- * ksplit) the bytes (ksa_gemm_rows_auto_splits(N, K) and ksa_gemm_rows_workspace_bytes(N, ksplit) are
- * the same answers for M <= 16).  For M > 16 (a kernel of its own: every weight fragment meets each
+ * ksplit) the bytes (for M <= 16 also ksa_gemm_rows_auto_splits(N, K), at most 16 splits, and
+ * ksa_gemm_rows_workspace_bytes(N, ksplit)).  For M > 16 (a kernel of its own: every weight fragment meets each
  * 16-row block of x, staged through LDS in chunks of 512 elements of K) only split counts that
  * ksa_gemm_rows_splits can return are taken - slices are whole chunks, none empty - anything else is
  * KSA_ERR_INVALID.  With ksplit > 1 out may be NULL: the partial sums (fp32 [ksplit][R][N], R = M

@@ -504,34 +504,43 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
 
 }  // namespace
 
-// K splits for at most 16 rows: slices are whole chunks of 512, none empty.  One chunk per workgroup where
-// that is not more than 2048 workgroups (a workgroup then has no loop: 11 % faster at N = 19456, K = 2560; the
-// sums of up to 32 slices are added by the consumer), otherwise about two workgroups per CU of the current
-// device (256 CUs assumed when no device can be asked).
+// K splits for at most 16 rows by the matrix alone, at most 16: about two workgroups per CU of the current device
+// (256 CUs assumed when no device can be asked) without slices shorter than one chunk of 512; one chunk per
+// workgroup where that is a moderate grid.  `ksa_gemm_rows_splits` below gives the faster count, of up to 32.
 extern "C" int ksa_gemm_rows_auto_splits(int N, int K) {
     if (N <= 0 || K <= 0) return 1;
     const int tiles = (N + 63) / 64;
-    const int chunks = (K / 32 + kChunkSteps - 1) / kChunkSteps;
     const int want = 2 * ksa_cu_count_or(256);
     int sp = (want + tiles - 1) / tiles;
-    if (sp > 1 && chunks <= 32 && (long long)tiles * chunks <= 2048) sp = chunks;
-    if (sp > 32) sp = 32;
-    return wide_plan(K, sp).ksplit;
+    const int chunks = K / 32 / 16 > 1 ? K / 32 / 16 : 1;
+    if (sp > chunks) sp = chunks;
+    if (sp > 16) sp = 16;
+    if (sp < 1) sp = 1;
+    if (sp > 1 && chunks >= sp && chunks <= 16 && (long long)tiles * chunks <= 2048 && K % (32 * 16) == 0) sp = chunks;
+    return sp;
 }
 
 extern "C" size_t ksa_gemm_rows_workspace_bytes(int N, int ksplit) {
     return ksplit > 1 ? (size_t)ksplit * 16 * (size_t)N * sizeof(float) : 0;
 }
 
-// The same two questions for a product of M rows (M <= 16: the answers above).  For more rows a slice
+// The same two questions for a product of M rows.  At most 16 rows: slices are whole chunks of 512, none empty; one
+// chunk per workgroup where that is not more than 2048 workgroups (a workgroup then has no loop: 11 % faster at
+// N = 19456, K = 2560; the sums of up to 32 slices are added by the consumer), otherwise about two
+// workgroups per CU.  For more rows a slice
 // of the partial sums has ksa_partial_rows(M) rows, and K is split as far as the grid (tiles of 128
 // columns x splits) stays within about one workgroup per CU - one resident workgroup is all a CU holds
 // of this kernel, and a second round costs more than longer slices do (measured at 72 rows on the
 // projections of the 4B shape: 6144 x 2560 best at 5 splits, 2560 x 4096 at 8, 2560 x 9728 at 10,
 // 19456 x 2560 at 2).
 extern "C" int ksa_gemm_rows_splits(int M, int N, int K) {
-    if (M <= 16) return ksa_gemm_rows_auto_splits(N, K);
     if (N <= 0 || K <= 0) return 1;
+    if (M <= 16) {
+        const int tiles = (N + 63) / 64, chunks = (K / 32 + kChunkSteps - 1) / kChunkSteps;
+        int sp = (2 * ksa_cu_count_or(256) + tiles - 1) / tiles;
+        if (sp > 1 && chunks <= 32 && (long long)tiles * chunks <= 2048) sp = chunks;
+        return wide_plan(K, sp < 32 ? sp : 32).ksplit;
+    }
     const int tiles = (N + 127) / 128;
     const int want = (ksa_cu_count_or(256) * 5 / 4) / tiles;
     return wide_plan(K, want).ksplit;
