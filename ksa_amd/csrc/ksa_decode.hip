@@ -73,6 +73,9 @@ __device__ __forceinline__ int ksa_decode_slot(const DecodeParams& p, int qi, in
     return qi == 0 ? gi : 32 + (qi - 1) * p.g + gi;
 }
 
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+
 constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kRows = 32;  // key rows per wave tile
@@ -301,49 +304,74 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
     }  // column blocks of this workgroup
 }
 
-// second stage: merge the splits of one (sequence, kv head, column)
+// Second stage: merge the splits of one (sequence, kv head, column).  A chain of memory trips, nothing else, so
+// there is one: D / 4 threads take four elements each, the G such groups of a workgroup every G-th split, and a
+// group requests up to eight splits (64 in all at head_dim 128) with their maxima and sums at once; the groups
+// meet in LDS.  (A thread per element that walked the splits eight at a time, maxima first, took 2 to 16 trips:
+// decode + merge of one sequence of 16384 rows in
+// 64 splits 29.8 -> 19.4 us, 4096 rows in 16 13.4 -> 12.0.)
+constexpr int kMergeThreads = 256;
 template <typename T, int D>
-__global__ __launch_bounds__(D) void ksa_decode_merge_kernel(const DecodeParams p) {
+__global__ __launch_bounds__(kMergeThreads) void ksa_decode_merge_kernel(const DecodeParams p) {
     using Ops = KsaOps<T>;
+    constexpr int TPG = D / 4;                 // threads of a group
+    constexpr int G = kMergeThreads / TPG;
+    constexpr int kBatch = 8;
+    __shared__ float s_m[G], s_l[G];
+    __shared__ __attribute__((aligned(16))) float s_o[G][D];
     const int oq = blockIdx.x / p.g, og = blockIdx.x % p.g;  // logical column: query token, head in the group
     const int cg = ksa_decode_slot(p, oq, og);
     const int kvh = blockIdx.y;
     const int bz = blockIdx.z;
-    const int d = threadIdx.x;
+    const int grp = threadIdx.x / TPG, d4 = 4 * (threadIdx.x % TPG);
     const int64_t base = (((int64_t)bz * p.Hkv + kvh) * p.nsplit) * p.ncols_pad + cg;
-    // the loads of eight splits are requested together (two passes: maximum, then weighted sums)
-    float mx = -INFINITY;
-    for (int s0 = 0; s0 < p.nsplit; s0 += 8) {
-        float m[8];
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    float mx = -INFINITY, l = 0.f;
+    for (int s0 = grp; s0 < p.nsplit; s0 += kBatch * G) {
+        floatx4 o[kBatch];
+        floatx2 ml[kBatch];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) m[u] = p.ws_ml[(base + (int64_t)min(s0 + u, p.nsplit - 1) * p.ncols_pad) * 2];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) mx = fmaxf(mx, m[u]);
-    }
-    float acc = 0.f, l = 0.f;
-    for (int s0 = 0; s0 < p.nsplit; s0 += 8) {
-        float m[8], ls[8], o[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int64_t slot = base + (int64_t)min(s0 + u, p.nsplit - 1) * p.ncols_pad;
-            m[u] = p.ws_ml[slot * 2];
-            ls[u] = p.ws_ml[slot * 2 + 1];
-            o[u] = p.ws_o[slot * D + d];
+        for (int u = 0; u < kBatch; ++u) {
+            const int64_t slot = base + (int64_t)min(s0 + u * G, p.nsplit - 1) * p.ncols_pad;
+            ml[u] = *reinterpret_cast<const floatx2*>(p.ws_ml + slot * 2);
+            o[u] = *reinterpret_cast<const floatx4*>(p.ws_o + slot * D + d4);
         }
+        float m_new = mx;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            if (s0 + u < p.nsplit) {
-                // (an empty slice leaves its sums unwritten: nothing of it may enter, not even times zero)
-                const bool some = m[u] != -INFINITY;
-                const float f = some ? ksa_exp2(m[u] - mx) : 0.f;
-                acc = some ? fmaf(o[u], f, acc) : acc;
-                l = some ? fmaf(ls[u], f, l) : l;
+        for (int u = 0; u < kBatch; ++u) m_new = fmaxf(m_new, ml[u][0]);
+        const float f0 = mx == -INFINITY ? 0.f : ksa_exp2(mx - m_new);
+        l *= f0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] *= f0;
+        mx = m_new;
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            // (an empty slice leaves its sums unwritten: nothing of it may enter, not even times zero)
+            if (s0 + u * G < p.nsplit && ml[u][0] != -INFINITY) {
+                const float f = ksa_exp2(ml[u][0] - mx);
+                l = fmaf(ml[u][1], f, l);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = fmaf(o[u][i], f, acc[i]);
             }
         }
     }
-    const float val = l > 0.f ? acc / l : 0.f;
-    uint16_t* op = p.out + bz * p.o_bs + oq * p.o_qs + (kvh * p.g + og) * p.o_hs + d;
-    *op = (uint16_t)(Ops::pack2(val, 0.f) & 0xffffu);
+    *reinterpret_cast<floatx4*>(&s_o[grp][d4]) = acc;
+    if (d4 == 0) s_m[grp] = mx, s_l[grp] = l;
+    __syncthreads();
+    const int d = threadIdx.x;
+    if (d < D) {
+        const int ng = min(G, p.nsplit);
+        float top = -INFINITY, sum = 0.f, val = 0.f;
+        for (int w = 0; w < ng; ++w) top = fmaxf(top, s_m[w]);
+        for (int w = 0; w < ng; ++w) {
+            const float f = s_m[w] == -INFINITY ? 0.f : ksa_exp2(s_m[w] - top);
+            sum = fmaf(s_l[w], f, sum);
+            val = fmaf(s_o[w][d], f, val);
+        }
+        val = sum > 0.f ? val / sum : 0.f;
+        uint16_t* op = p.out + bz * p.o_bs + oq * p.o_qs + (kvh * p.g + og) * p.o_hs + d;
+        *op = (uint16_t)(Ops::pack2(val, 0.f) & 0xffffu);
+    }
 }
 
 template <typename T, int D>
@@ -353,7 +381,7 @@ int launch(const DecodeParams& p, int batch, hipStream_t stream) {
     hipLaunchKernelGGL((ksa_decode_kernel<T, D>), grid, dim3(kThreads), 0, stream, p);
     if (p.nsplit > 1) {
         dim3 g2(p.ncols, p.Hkv, batch);
-        hipLaunchKernelGGL((ksa_decode_merge_kernel<T, D>), g2, dim3(D), 0, stream, p);
+        hipLaunchKernelGGL((ksa_decode_merge_kernel<T, D>), g2, dim3(kMergeThreads), 0, stream, p);
     }
     return ksa_check_launch();
 }
@@ -370,8 +398,9 @@ extern "C" size_t ksa_decode_workspace_bytes(int batch, int Hq, int Hkv, int Q, 
     return (size_t)batch * Hkv * nsplit * cols * (D + 2) * sizeof(float);
 }
 
-// Heuristic number of splits: at least two workgroups per CU of the current device (256 CUs
-// assumed when no device can be asked), but never splits shorter than 256 rows.
+// Number of splits by sequences, kv heads and rows alone: at least two workgroups per CU of the current device
+// (256 CUs assumed when no device can be asked), but never splits shorter than 256 rows.  Kept for callers of
+// ksa_decode_fwd_noalloc, whose scratch is of a fixed size; ksa_decode_splits below is faster on few rows.
 extern "C" int ksa_decode_auto_splits(int batch, int Hkv, int max_rows) {
     if (batch <= 0 || Hkv <= 0 || max_rows <= 0) return 1;
     const int units = batch * Hkv;
@@ -381,6 +410,25 @@ extern "C" int ksa_decode_auto_splits(int batch, int Hkv, int max_rows) {
     if (n > cap) n = cap;
     if (n > 64) n = 64;
     return n < 1 ? 1 : n;
+}
+
+// Number of splits for Q query tokens of Hq heads: two workgroups per CU, but splits of no fewer rows than a
+// workgroup's waves cover in one round (128) - a launch over few rows is a chain of memory trips per
+// round, 2.1 us each, and a split more costs the merge next to nothing.  From half a workgroup per CU on
+// (128 of them) a split must save two rounds (256 rows) to be worth the partial sums.  Decode + merge at
+// head_dim 128, 8 kv heads, former count -> this one: 1 sequence of 760 / 1500 / 4096 / 16384 rows
+// 13.2 / 13.4 / 13.4 / 29.8 -> 9.0 / 9.2 / 10.4 / 19.4 us (the last by the merge kernel alone), 8 sequences of
+// 760 / 1500 rows 14.5 / 19.9 -> 12.8 / 18.6; 16 and 32 sequences the same counts as before.
+extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int max_rows) {
+    if (batch <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || Q <= 0 || max_rows <= 0) return 1;
+    const int64_t units = (int64_t)batch * Hkv * ((Q * (int64_t)(Hq / Hkv) + 31) / 32);
+    const int cus = ksa_cu_count_or(256);
+    int64_t n = (2 * (int64_t)cus + units - 1) / units;
+    int64_t cap = max_rows / 256;
+    if (2 * units < cus) cap = max_rows <= 192 ? 1 : ((int64_t)max_rows + 127) / 128;
+    if (n > cap) n = cap;
+    if (n > 64) n = 64;
+    return n < 1 ? 1 : (int)n;
 }
 
 namespace {

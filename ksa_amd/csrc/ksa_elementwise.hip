@@ -235,7 +235,7 @@ __device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
 // keeps each thread's largest value and the request batch it came from (about 2.5 instructions an element);
 // the threads that hold the row's maximum look into that one batch again for its place.  A row with a NaN
 // (its magnitudes exceed infinity's) is searched once more for the first one.  1 / 8 / 64 rows
-// 24.4 / 24.6 / 25.5 -> 8.8 / 9.4 / 10.3 us.
+// 25.1 / 25.5 / 26.7 -> 9.0 / 9.3 / 10.3 us.
 template <typename T>
 __global__ __launch_bounds__(1024) void ksa_argmax_rows_kernel(const ArgmaxParams p) {
     using C = KsaCvt<T>;

@@ -95,7 +95,7 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     if scale is None:
         scale = float(D) ** -0.5
     if nsplit is None:
-        nsplit = _lib.lib().ksa_decode_auto_splits(b, kcache.shape[1], max_rows)
+        nsplit = _lib.lib().ksa_decode_splits(b, q.shape[1], kcache.shape[1], q.shape[2], max_rows)
     Dk = kernel_head_dim(D)
     if Dk != D:
         # A head dimension without a kernel of its own (the kernels are built for 64 / 128 / 256): the
