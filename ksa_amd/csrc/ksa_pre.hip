@@ -158,8 +158,9 @@ __global__ __launch_bounds__(256) void ksa_pre_attention_kernel(const PreParams 
         g.col0 = ((g.which == 0 ? 0 : (g.which == 1 ? p.Hq : p.Hq + p.Hkv)) + g.h0) * D;
         g.sbase = p.src[g.which] + nb * p.s_bs[g.which] + (int64_t)ns * p.s_rs[g.which] + (int64_t)g.h0 * p.s_hs[g.which];
         // (k and v may go to a row of their sequence that the host does not know: a cache cursor)
+        // (asked for live groups only: behind the last token there is no entry)
         int64_t drow = ns;
-        if (g.which != 0 && p.kv_row) drow = p.kv_row_per_token ? p.kv_row[g.tok] : ns + p.kv_row[nb];
+        if (g.live && g.which != 0 && p.kv_row) drow = p.kv_row_per_token ? p.kv_row[g.tok] : ns + p.kv_row[nb];
         g.dbase = p.dst[g.which] + nb * p.d_bs[g.which] + drow * p.d_rs[g.which] + (int64_t)g.h0 * p.d_hs[g.which];
         gi += gstep;
         return g;

@@ -292,3 +292,22 @@ def test_pre_attention_gpu_row_per_token(from_partials, b, S, Hq, Hkv, D):
             assert torch.equal(kc[i, :, r], k0[i, t]) and torch.equal(vc[i, :, r], v0[i, t])
     untouched = ~touched.to(dev)
     assert (kc.transpose(1, 2)[untouched] == 7.0).all() and (vc.transpose(1, 2)[untouched] == -3.0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,S", [(64, 2), (128, 1), (5, 3)])
+def test_pre_attention_gpu_row_table_at_the_end_of_its_allocation(b, S):
+    """Only the entries of the table are read: it is the end of a 20 MiB buffer, which the allocator takes from the
+    device as it is (a wave once looked up the row of the token behind the last one)."""
+    import ksa_amd
+    Hq, Hkv, D = 4, 2, 64
+    q, k, v, qw, kw = _inputs(b, S, Hq, Hkv, D, 3, torch.bfloat16)
+    cos, sin, _ = _rope_tables(S, D, dtype=torch.bfloat16)
+    buf = torch.zeros(20 << 18, dtype=torch.int32, device="cuda")
+    table = buf[-b * S:].view(b, S)
+    table.copy_(torch.arange(S, dtype=torch.int32).flip(0).expand(b, S))
+    kc, vc = (torch.zeros(b, Hkv, S, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    args = [t.cuda() for t in (q, k, v, qw, kw, cos, sin)]
+    want = ksa_amd.pre_attention(*args, eps=1e-6)
+    ksa_amd.pre_attention(*args, eps=1e-6, k_out=kc.transpose(1, 2), v_out=vc.transpose(1, 2), kv_out_row=table)
+    assert torch.equal(kc.transpose(1, 2).flip(1), want[1]) and torch.equal(vc.transpose(1, 2).flip(1), want[2])
