@@ -129,6 +129,23 @@ int ksa_decode_boundary_fwd(const void* q, const void* kcache, const void* vcach
                             const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
                             float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The attention of a one-token decode step from the K-split partial sums of its fused q | k | v projection
+ * (ksa_gemm_rows with out = NULL: fp32 [qkv_ksplit][batch rounded up to 16][(Hq + 2 Hkv) D]): the pre-attention step
+ * (HF:660-666) and the decode attention (HF:591-612) in one launch, with the results of
+ * ksa_pre_attention_partials followed by ksa_decode_fwd.
+ *   q_weight, k_weight [D]; cos, sin rows [D] of the token, cos_batch_stride elements apart (0: shared)
+ *   kcache, vcache [batch, Hkv, rows, D]: the new key and value row is written at row[b] (device int32[batch]) or
+ *   row0, which has to lie in the attended range [start[b], end[b]) / [start0, end0)
+ *   out [batch, 1, Hq, D]; workspace (nsplit > 1): ksa_decode_workspace_bytes(batch, Hq, Hkv, 1, D, nsplit) bytes,
+ *   16-byte aligned
+ * batch <= 128, head_dim 64 or 128, Hq / Hkv <= 32, nsplit <= 64. */
+int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                       const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                       void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                       const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                       const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                       float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ksa_decode_fwd for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
  * Same arguments and results as ksa_decode_fwd without the workspace: the split-K partials go to

@@ -30,6 +30,8 @@ _SIGNATURES = {
     "ksa_decode_splits": (_int, [_int] * 5),
     "ksa_decode_fwd": (_int, [_vp] * 6 + [_int] * 8 + [_i64p] * 4
                        + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
+    "ksa_decode_qkv_fwd": (_int, [_vp, _int] + [_vp] * 4 + [ctypes.c_longlong, ctypes.c_float] + [_vp] * 4 + [_int]
+                           + [_vp] * 2 + [_int] * 7 + [_i64p] * 3 + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
     "ksa_decode_noalloc_max_workspace_bytes": (ctypes.c_size_t, []),
     "ksa_decode_fwd_noalloc": (_int, [_vp] * 6 + [_int] * 8 + [_i64p] * 4 + [ctypes.c_float, _int, _vp]),
     "ksa_decode_weights_workspace_bytes": (ctypes.c_size_t, [_int] * 4),

@@ -14,12 +14,18 @@
 // private (max, sum, O^T) state that is merged across the waves through LDS at the
 // end; with more than one split the un-normalised partials go to a workspace and a
 // second kernel merges them.
+//
+// A one-token step of the decoder can hand over the K-split partial sums of its fused q | k | v projection instead
+// of q (kPre): the kernel then does the pre-attention step itself - sums, norm and rotary embedding of the query
+// rows of its group in every workgroup, of the new key and value rows in the one workgroup whose
+// slice holds their cache row - one launch, and one round trip of the rows through memory, less.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
 #include <mutex>
 
 #include "ksa_api_internal.h"
+#include "ksa_pre_row.h"
 #include "ksa_tile.h"
 
 namespace {
@@ -50,6 +56,19 @@ struct DecodeParams {
     const int32_t* start2;
     const int32_t* end2;
     int start20, end20;
+    // kPre: one new token per sequence, from the projection's partial sums (q and q_bs .. are then unused)
+    const float* qkv;           // [qkv_ksplit][qkv_prows][(Hq + 2 Hkv) D]
+    int qkv_ksplit, qkv_prows;
+    const uint16_t* wq;         // norm weights [D]
+    const uint16_t* wk;
+    const uint16_t* cos;        // rotary row of the token [D], batch stride c_bs
+    const uint16_t* sin;
+    int64_t c_bs;
+    float eps;
+    uint16_t* kw;               // the caches, to be written at the new row
+    uint16_t* vw;
+    const int32_t* row_seq;     // cache row of the new token per sequence, or null: row0
+    int row0;
 };
 
 // column lq of column block colblk -> (query token, head in the group); false: no such column
@@ -80,7 +99,12 @@ constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kRows = 32;  // key rows per wave tile
 
-template <typename T, int D>
+// kPre against the pre-attention launch in front, a decode step of 8 layers of the 4B shape: batch 1 665 -> 652 us,
+// batch 8 772 -> 759.  The chain of trips that it puts in front of the first scores (row and range, partial sums, LDS)
+// runs next to the loads of the first K / V tile; what it costs is that every split repeats it, and a
+// workgroup that is not among the first on its CU runs it behind full memory queues (who calls it keeps to launches whose
+// workgroups all fit at once).
+template <typename T, int D, bool kPre>
 __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kernel(const DecodeParams p) {
     using Ops = KsaOps<T>;
     constexpr int KS = D / 16;
@@ -94,6 +118,8 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
     constexpr int kSmemBytes = (kWaves * kStage * 2 > kMergeFloats * 4) ? kWaves * kStage * 2
                                                                         : kMergeFloats * 4;
     __shared__ __attribute__((aligned(16))) unsigned char smem[kSmemBytes];
+    // (kPre) the query rows of the group, then the new key and value row
+    __shared__ __attribute__((aligned(16))) uint16_t s_new[kPre ? (32 + 2) * D : 8];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -147,16 +173,6 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
     if (!col_ok) qi = 0, gi = 0;
     const int head = kvh * p.g + gi;
 
-    u32x4 qf[KS];
-    {
-        const uint16_t* qp = p.q + bz * p.q_bs + head * p.q_hs + qi * p.q_qs + 8 * lh;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            u32x4 z = {0u, 0u, 0u, 0u};
-            qf[s] = col_ok ? *reinterpret_cast<const u32x4*>(qp + 16 * s) : z;
-        }
-    }
-
     const uint16_t* kbase = p.k + bz * p.k_bs + kvh * p.k_hs;
     const uint16_t* vbase = p.v + bz * p.v_bs + kvh * p.v_hs;
     const int last_row = max(r_end - 1, r_begin);
@@ -188,7 +204,88 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
     const float c2 = p.scale_log2;
 
     int row0 = s0 + wave * kRows;
-    if (row0 < s1) load_tile(row0);
+    u32x4 qf[KS];
+    int new_row = -1;  // (kPre) the new token's cache row, if it lies in this workgroup's slice
+    if constexpr (!kPre) {
+        const uint16_t* qp = p.q + bz * p.q_bs + head * p.q_hs + qi * p.q_qs + 8 * lh;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            u32x4 z = {0u, 0u, 0u, 0u};
+            qf[s] = col_ok ? *reinterpret_cast<const u32x4*>(qp + 16 * s) : z;
+        }
+        if (row0 < s1) load_tile(row0);
+    } else {
+        using C = KsaCvt<T>;
+        constexpr int LPR = D / 8;      // lanes per head row
+        constexpr int RPW = 64 / LPR;   // head rows per wave
+        const int t = lane % LPR;
+        new_row = p.row_seq ? p.row_seq[bz] : p.row0;
+        if (new_row < s0 || new_row >= s1) new_row = -1;
+        const int rows_here = p.g + (new_row >= 0 ? 2 : 0);  // query rows, then the key and the value row
+        const int width = (p.Hq + 2 * p.Hkv) * D;
+        bool loaded = false;
+        for (int i0 = wave * RPW; i0 < rows_here; i0 += kWaves * RPW) {  // (at most once for up to 14 query rows of 128)
+            const int it = min(i0 + lane / LPR, rows_here - 1);          // (lanes past the last row repeat it)
+            const int hrow = it < p.g ? kvh * p.g + it : p.Hq + (it - p.g) * p.Hkv + kvh;
+            // requested in this order: the partial sums (first eight slices), the rotary row and the weight, the
+            // first K / V tile - the sums are then worked on while the tile is on its way
+            const float* src = p.qkv + (int64_t)bz * width + (int64_t)hrow * D + 8 * t;
+            const int64_t pitch = (int64_t)p.qkv_prows * width;
+            f32x4 lo[8], hi[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float* sp = src + pitch * min(u, p.qkv_ksplit - 1);
+                lo[u] = *reinterpret_cast<const f32x4*>(sp);
+                hi[u] = *reinterpret_cast<const f32x4*>(sp + 4);
+            }
+            const u32x4 w = *reinterpret_cast<const u32x4*>((it < p.g ? p.wq : p.wk) + 8 * t);
+            const u32x4 cr = *reinterpret_cast<const u32x4*>(p.cos + bz * p.c_bs + 8 * t);
+            const u32x4 sr = *reinterpret_cast<const u32x4*>(p.sin + bz * p.c_bs + 8 * t);
+            if (!loaded && row0 < s1) load_tile(row0);
+            loaded = true;
+            float ac[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // summed and rounded as ksa_sum_partials8
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (u < p.qkv_ksplit) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) ac[i] += lo[u][i], ac[4 + i] += hi[u][i];
+                }
+            }
+            for (int u = 8; u < p.qkv_ksplit; ++u) {
+                const f32x4 l4 = *reinterpret_cast<const f32x4*>(src + pitch * u);
+                const f32x4 h4 = *reinterpret_cast<const f32x4*>(src + pitch * u + 4);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ac[i] += l4[i], ac[4 + i] += h4[i];
+            }
+            u32x4 raw;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) raw[i] = C::down2(ac[2 * i], ac[2 * i + 1]);
+            const uint32_t sgn = t < LPR / 2 ? 0x80008000u : 0u;
+            uint32_t wl[4], wh[4], cl[4], ch[4], sl[4], sh[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                wl[i] = w[i] & 0xffffu, wh[i] = w[i] & 0xffff0000u;
+                cl[i] = cr[i] & 0xffffu, ch[i] = cr[i] & 0xffff0000u;
+                sl[i] = (sr[i] ^ sgn) & 0xffffu, sh[i] = (sr[i] ^ sgn) & 0xffff0000u;
+            }
+            const u32x4 z = ksa_row_scale<T>(raw, ksa_row_inv_rms<T, LPR>(raw, p.eps), wl, wh);
+            const u32x4 rot = ksa_row_rope<T, LPR>(z, cl, ch, sl, sh);
+            const u32x4 val = it == p.g + 1 ? raw : rot;  // (the value row changes its place only)
+            *reinterpret_cast<u32x4*>(s_new + (it < p.g ? it : 32 + it - p.g) * D + 8 * t) = val;
+            if (it >= p.g) {
+                uint16_t* dst = it == p.g ? p.kw + bz * p.k_bs + kvh * p.k_hs + (int64_t)new_row * p.k_rs
+                                          : p.vw + bz * p.v_bs + kvh * p.v_hs + (int64_t)new_row * p.v_rs;
+                __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst + 8 * t));
+            }
+        }
+        if (!loaded && row0 < s1) load_tile(row0);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            u32x4 z = {0u, 0u, 0u, 0u};
+            qf[s] = col_ok ? *reinterpret_cast<const u32x4*>(s_new + gi * D + 16 * s + 8 * lh) : z;
+        }
+    }
 
     for (; row0 < s1; row0 += kWaves * kRows) {
         ksa_wave_lds_fence();
@@ -202,6 +299,18 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
             *reinterpret_cast<u32x4*>(Kw + (u / CPR) * KROW + 8 * (u % CPR)) = kreg[i];
             *reinterpret_cast<u32x4*>(Vw + (u / CPR) * VROW + 8 * (u % CPR)) = vreg[i];
             if (has_next) load_piece(next, i);
+        }
+        if constexpr (kPre) {
+            // the new row, over what the cache held in its place - and, where it is the last one, over its
+            // repetitions in the rows past the end (their probabilities are 0, so they have to be finite)
+            if (new_row >= row0 && new_row < row0 + kRows) {
+                const bool is_v = lane >= CPR;
+                const u32x4 v = *reinterpret_cast<const u32x4*>(s_new + (is_v ? 33 : 32) * D + 8 * (lane % CPR));
+                const int first = new_row - row0, last = new_row == last_row ? kRows - 1 : first;
+                for (int j = first; j <= last; ++j)
+                    if (lane < 2 * CPR)
+                        *reinterpret_cast<u32x4*>((is_v ? Vw + j * VROW : Kw + j * KROW) + 8 * (lane % CPR)) = v;
+            }
         }
         ksa_wave_lds_fence();
 
@@ -378,7 +487,14 @@ template <typename T, int D>
 int launch(const DecodeParams& p, int batch, hipStream_t stream) {
     const int colblks = p.split_q ? 1 : p.ncols_pad / 32;  // (boundary form: a workgroup walks its column blocks)
     dim3 grid(p.nsplit, p.Hkv * colblks, batch);
-    hipLaunchKernelGGL((ksa_decode_kernel<T, D>), grid, dim3(kThreads), 0, stream, p);
+    if (p.qkv) {
+        if constexpr (D <= 128)
+            hipLaunchKernelGGL((ksa_decode_kernel<T, D, true>), grid, dim3(kThreads), 0, stream, p);
+        else
+            return KSA_ERR_UNSUPPORTED;
+    } else {
+        hipLaunchKernelGGL((ksa_decode_kernel<T, D, false>), grid, dim3(kThreads), 0, stream, p);
+    }
     if (p.nsplit > 1) {
         dim3 g2(p.ncols, p.Hkv, batch);
         hipLaunchKernelGGL((ksa_decode_merge_kernel<T, D>), g2, dim3(kMergeThreads), 0, stream, p);
@@ -432,6 +548,14 @@ extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int max_rows
 }
 
 namespace {
+
+template <typename T>
+int launch_head_dim(const DecodeParams& p, int D, int batch, hipStream_t st) {
+    if (D == 128) return launch<T, 128>(p, batch, st);
+    if (D == 64) return launch<T, 64>(p, batch, st);
+    if (D == 256) return launch<T, 256>(p, batch, st);
+    return KSA_ERR_UNSUPPORTED;
+}
 
 int decode_fwd_impl(const void* q, const void* kcache, const void* vcache, void* out,
                     const int32_t* start, const int32_t* end, int start0, int end0, int batch, int Hq,
@@ -487,16 +611,7 @@ int decode_fwd_impl(const void* q, const void* kcache, const void* vcache, void*
         p.ws_ml = p.ws_o + (size_t)batch * Hkv * nsplit * p.ncols_pad * D;
     }
     hipStream_t st = (hipStream_t)stream;
-    if (dtype == KSA_DTYPE_BF16) {
-        if (D == 128) return launch<KsaBf16, 128>(p, batch, st);
-        if (D == 64) return launch<KsaBf16, 64>(p, batch, st);
-        if (D == 256) return launch<KsaBf16, 256>(p, batch, st);
-    } else {
-        if (D == 128) return launch<KsaF16, 128>(p, batch, st);
-        if (D == 64) return launch<KsaF16, 64>(p, batch, st);
-        if (D == 256) return launch<KsaF16, 256>(p, batch, st);
-    }
-    return KSA_ERR_UNSUPPORTED;
+    return dtype == KSA_DTYPE_BF16 ? launch_head_dim<KsaBf16>(p, D, batch, st) : launch_head_dim<KsaF16>(p, D, batch, st);
 }
 
 // ---- scratch of the entry point that allocates nothing ----
@@ -559,6 +674,58 @@ extern "C" int ksa_decode_boundary_fwd(const void* q, const void* kcache, const 
     return decode_fwd_impl(q, kcache, vcache, out, text_start, text_end, text_start0, text_end0, batch, Hq, Hkv, Q, D,
                            dtype, q_strides, k_strides, v_strides, out_strides, scale, nsplit, workspace,
                            workspace_bytes, stream, true, sum_start, sum_end, sum_start0, sum_end0);
+}
+
+// A decode step's attention from the K-split partial sums of its fused q | k | v projection: the pre-attention step
+// (HF:660-666) and the attention over the cache (HF:591-612) in one launch.  Arithmetic and results are those of
+// ksa_pre_attention_partials followed by ksa_decode_fwd.
+extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                                  const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                  void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                                  const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                  const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                                  float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!qkv_partials || !q_weight || !k_weight || !cos || !sin || !kcache || !vcache || !k_strides || !v_strides)
+        return KSA_ERR_NULL;
+    if (!out || !out_strides || (start == nullptr) != (end == nullptr)) return KSA_ERR_NULL;
+    if (batch <= 0 || batch > kMaxPartialRows || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Hq / Hkv > 32 || qkv_ksplit < 1 ||
+        qkv_ksplit > 64 || nsplit < 1 || nsplit > 64 || !(eps >= 0.f))
+        return KSA_ERR_INVALID;
+    if (!start && (start0 < 0 || end0 <= start0)) return KSA_ERR_INVALID;
+    if (!row && (row0 < 0 || (!start && (row0 < start0 || row0 >= end0)))) return KSA_ERR_INVALID;
+    if (dtype != KSA_DTYPE_BF16 && dtype != KSA_DTYPE_F16) return KSA_ERR_UNSUPPORTED;
+    if (D != 64 && D != 128) return KSA_ERR_UNSUPPORTED;
+    for (const void* ptr : {(const void*)qkv_partials, q_weight, k_weight, cos, sin, (const void*)kcache, (const void*)vcache,
+                            (const void*)workspace})
+        if (reinterpret_cast<uintptr_t>(ptr) & 15) return KSA_ERR_ALIGN;
+    for (int i = 0; i < 3; ++i)
+        if ((k_strides[i] % 8) || (v_strides[i] % 8)) return KSA_ERR_ALIGN;
+    if (cos_batch_stride % 8) return KSA_ERR_ALIGN;
+    DecodeParams p{};
+    p.qkv = qkv_partials, p.qkv_ksplit = qkv_ksplit, p.qkv_prows = ksa_partial_rows(batch);
+    p.wq = (const uint16_t*)q_weight, p.wk = (const uint16_t*)k_weight;
+    p.cos = (const uint16_t*)cos, p.sin = (const uint16_t*)sin, p.c_bs = cos_batch_stride;
+    p.eps = eps;
+    p.k = p.kw = (uint16_t*)kcache;
+    p.v = p.vw = (uint16_t*)vcache;
+    p.row_seq = row, p.row0 = row0;
+    p.out = (uint16_t*)out;
+    p.start = start, p.end = end, p.start0 = start0, p.end0 = end0;
+    p.Hq = Hq, p.Hkv = Hkv, p.g = Hq / Hkv, p.Q = 1;
+    p.ncols = p.g;
+    p.ncols_pad = pad_cols(p.ncols);
+    p.nsplit = nsplit;
+    p.k_bs = k_strides[0], p.k_hs = k_strides[1], p.k_rs = k_strides[2];
+    p.v_bs = v_strides[0], p.v_hs = v_strides[1], p.v_rs = v_strides[2];
+    p.o_bs = out_strides[0], p.o_qs = out_strides[1], p.o_hs = out_strides[2];
+    p.scale_log2 = scale * 1.4426950408889634f;
+    if (nsplit > 1) {
+        if (!workspace || workspace_bytes < ksa_decode_workspace_bytes(batch, Hq, Hkv, 1, D, nsplit)) return KSA_ERR_WORKSPACE;
+        p.ws_o = (float*)workspace;
+        p.ws_ml = p.ws_o + (size_t)batch * Hkv * nsplit * p.ncols_pad * D;
+    }
+    hipStream_t st = (hipStream_t)stream;
+    return dtype == KSA_DTYPE_BF16 ? launch_head_dim<KsaBf16>(p, D, batch, st) : launch_head_dim<KsaF16>(p, D, batch, st);
 }
 
 extern "C" size_t ksa_decode_noalloc_max_workspace_bytes(void) { return kNoAllocScratchBytes; }

@@ -21,6 +21,7 @@
 #include "ksa_api_internal.h"
 #include "ksa_tile.h"
 #include "ksa_cvt.h"
+#include "ksa_pre_row.h"
 
 namespace {
 
@@ -45,27 +46,6 @@ struct PreParams {
 
 template <typename T>
 using PreCvt = KsaCvt<T>;
-
-// value of the lane `n` places further inside the same row of 16 lanes (cyclic)
-template <int N>
-__device__ __forceinline__ uint32_t pre_row_ror(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x120 + N, 0xf, 0xf, false);
-}
-
-// sum over the LPR lanes that hold one head row; every lane of the row gets the total
-template <int LPR>
-__device__ __forceinline__ float pre_row_sum(float ss) {
-    if constexpr (LPR == 16) {  // rotations inside a DPP row (16 lanes)
-        ss += __builtin_bit_cast(float, pre_row_ror<8>(__builtin_bit_cast(uint32_t, ss)));
-        ss += __builtin_bit_cast(float, pre_row_ror<4>(__builtin_bit_cast(uint32_t, ss)));
-        ss += __builtin_bit_cast(float, pre_row_ror<2>(__builtin_bit_cast(uint32_t, ss)));
-        ss += __builtin_bit_cast(float, pre_row_ror<1>(__builtin_bit_cast(uint32_t, ss)));
-    } else {
-#pragma unroll
-        for (int m = 1; m < LPR; m <<= 1) ss += __shfl_xor(ss, m);
-    }
-    return ss;
-}
 
 // One workgroup takes a few consecutive tokens; its four waves share
 // their head rows, RPW rows of one of q / k / v per wave instruction, the same number for every

@@ -115,6 +115,78 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     return forward(q, kcache, vcache, t_start, t_end, s0, e0, float(scale), int(nsplit))
 
 
+def decode_qkv_supported(Hq: int, Hkv: int, D: int) -> bool:
+    return D in (64, 128) and Hq % Hkv == 0 and Hq // Hkv <= 32
+
+
+def decode_qkv_pays(kcache: torch.Tensor, Hq: int, start, end) -> bool:
+    """Whether `ksa_decode_qkv` takes the place of `pre_attention_partials` and `ksa_decode`: where all its workgroups
+    run at once (two per CU).  A workgroup that starts later pays for its query rows behind the others' loads:
+    a decode step of 4 layers, 8 kv heads, separate -> one launch: 1 / 16 / 32 / 64 sequences
+    402 -> 393 / 563 -> 552 / 597 -> 589 / 800 -> 774 us, but 24 (576 workgroups) 577 -> 582 and 48 (768) 684 -> 702."""
+    b, Hkv, rows, D = kcache.shape
+    if not decode_qkv_supported(Hq, Hkv, D):
+        return False
+    L = _lib.lib()
+    device = isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor)
+    with _lib.on_device(kcache.device):
+        n = L.ksa_decode_splits(b, Hq, Hkv, 1, rows if device else max(1, int(end) - int(start)))
+        return b * Hkv * n <= 2 * max(1, L.ksa_device_cu_count())
+
+
+def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                   eps: float, kcache: torch.Tensor, vcache: torch.Tensor, Hq: int, row, start, end,
+                   scale: Optional[float] = None, nsplit: Optional[int] = None) -> torch.Tensor:
+    """`pre_attention_partials` + `ksa_decode` of one new token per sequence in one launch (`ksa_decode_qkv_fwd`).
+
+    qkv: the deferred q | k | v projection (`SplitKPartials` [b, 1, (Hq + 2 Hkv) D]); cos / sin [1 or b, 1, D].  The
+    token's key and value go to `row` of the caches and are attended with the rest of [start, end), which has
+    to hold that row (each an int, or an int32 GPU tensor [b]).  Returns [b, 1, Hq D]."""
+    from .gemm import SplitKPartials
+    assert isinstance(qkv, SplitKPartials) and qkv.dtype in _DTYPES and qkv.dtype == kcache.dtype == vcache.dtype
+    b, Hkv, rows, D = kcache.shape
+    dev = qkv.device
+    assert qkv.shape == (b, 1, (Hq + 2 * Hkv) * D) and vcache.shape == kcache.shape and decode_qkv_supported(Hq, Hkv, D)
+    assert kcache.stride(-1) == 1 and vcache.stride(-1) == 1, "cache rows must be contiguous"
+    dt = qkv.dtype
+    cos, sin = (t.to(dt).reshape(-1, D).contiguous() for t in (cos, sin))
+    qw, kw = q_norm_weight.to(dt).contiguous(), k_norm_weight.to(dt).contiguous()
+    assert cos.shape == sin.shape and cos.shape[0] in (1, b) and qw.shape == (D,) and kw.shape == (D,)
+    t_row = t_start = t_end = None
+    s0, e0, r0 = 0, 1, 0
+    if isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor):
+        t_start, t_end = _bound(start, 0, b, dev), _bound(end, rows, b, dev)
+        max_rows = rows
+    else:
+        s0, e0 = int(start), int(end)
+        assert 0 <= s0 < e0 <= rows, "row range out of bounds"
+        max_rows = e0 - s0
+    if isinstance(row, torch.Tensor):
+        t_row = _bound(row, 0, b, dev)
+    else:
+        r0 = int(row)
+        assert 0 <= r0 < rows and (t_start is not None or s0 <= r0 < e0), "the new row must lie in the attended range"
+    L = _lib.lib()
+    ptr = lambda t: None if t is None else t.data_ptr()
+    with _lib.on_device(dev):
+        if nsplit is None:
+            nsplit = L.ksa_decode_splits(b, Hq, Hkv, 1, max_rows)
+        ws = None
+        ws_bytes = L.ksa_decode_workspace_bytes(b, Hq, Hkv, 1, D, nsplit)
+        if nsplit > 1:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        out = torch.empty((b, 1, Hq, D), dtype=dt, device=dev)
+        dims = (0, 1, 2)
+        rc = L.ksa_decode_qkv_fwd(
+            qkv.workspace.data_ptr(), qkv.ksplit, qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+            D if cos.shape[0] > 1 else 0, float(eps), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), ptr(t_row), r0,
+            ptr(t_start), ptr(t_end), s0, e0, b, Hq, Hkv, D, _DTYPES[dt], _lib.strides3(kcache, dims),
+            _lib.strides3(vcache, dims), _lib.strides3(out, dims),
+            float(D) ** -0.5 if scale is None else float(scale), nsplit, ptr(ws), ws_bytes, _lib.stream_ptr(dev))
+    _lib.check(rc, "ksa_decode_qkv_fwd")
+    return out.view(b, 1, Hq * D)
+
+
 def ksa_decode_boundary(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, text_start, text_end,
                         sum_start, sum_end, scale: Optional[float] = None,
                         nsplit: Optional[int] = None) -> torch.Tensor:

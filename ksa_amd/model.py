@@ -140,6 +140,7 @@ class HipOps:
         self.add_rmsnorm = elementwise.add_rmsnorm
         self.silu_mul = elementwise.silu_mul
         self._decode = decode.ksa_decode
+        self._decode_mod = decode
         self.decode_boundary = decode.ksa_decode_boundary   # text token + summary tokens of a boundary step, one launch
         self.move_rows_multi = cache._move_rows_multi        # the step's row moves, one launch for up to eight
         self._linear_rows = gemm.linear_rows
@@ -171,6 +172,14 @@ class HipOps:
 
     def decode(self, q, kbuf, vbuf, start, end, scale):
         return self._decode(q, kbuf, vbuf, start, end, scale=scale)
+
+    def decode_qkv(self, qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end, scale):
+        """The attention of a one-token step from its deferred q | k | v projection, the new row written to
+        the caches: [b, 1, Hq D]; None where `pre_attention` and `decode` have to do it."""
+        if not isinstance(qkv, self._gemm.SplitKPartials) or not self._decode_mod.decode_qkv_pays(kbuf, Hq, start, end):
+            return None
+        return self._decode_mod.ksa_decode_qkv(qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end,
+                                               scale=scale)
 
     def argmax(self, logits):
         """Greedy token choice over the last dimension (lowest index among equal values)."""
@@ -430,6 +439,27 @@ class KsaQwen3ForCausalLM:
                              (vc if in_cache else vs, vc, S, 0, rows["append"])])
         return attn
 
+    def _text_attention(self, lw, h, cos, sin, kc, vc, row, start, end, slots):
+        """Projection, q / k norm, rotary embedding and attention of one text token per sequence, its key and
+        value written to `row` of the caches (`slots`: the same as arguments of `pre_attention`):
+        [b, 1, Hq D]."""
+        cfg, ops = self.config, self.ops
+        Hq, Hkv, D = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+        qkv = ops.linear(h, lw["qkv_proj"], defer=True)
+        if hasattr(ops, "decode_qkv"):
+            attn = ops.decode_qkv(qkv, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps, kc, vc, Hq, row, start, end,
+                                  self.scaling)
+            if attn is not None:
+                return attn
+        if torch.is_tensor(qkv):
+            q, k, v = self._split_qkv(qkv)
+            q, _, _ = ops.pre_attention(q, k, v, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps, **slots)
+        else:  # still the K-split partial sums of the projection: added inside the kernel
+            q, _, _ = ops.pre_attention_partials(qkv, Hq, Hkv, D, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps,
+                                                 **slots)
+        attn = ops.decode(q.transpose(1, 2), kc, vc, start, end, self.scaling)
+        return attn.reshape(h.shape[0], 1, -1)
+
     def _post_attention(self, lw, attn, x):
         """The second half of a layer at a decode step, from the attention output: (x', delta) with
         x' = x + o_proj(attn) and delta = mlp(post_attention_layernorm(x')) (deferred sums)."""
@@ -591,18 +621,11 @@ class KsaQwen3ForCausalLM:
             x, h = self._add_norm(delta, x, lw["input_layernorm"])
             if not boundary:
                 k_slot, v_slot = cache.text_slots(li, b, Hkv, D, self.dtype, self.device)
-                qkv = ops.linear(h, lw["qkv_proj"], defer=True)
-                if torch.is_tensor(qkv):
-                    q, k, v = self._split_qkv(qkv)
-                    q, _, _ = ops.pre_attention(q, k, v, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps,
-                                                k_out=k_slot, v_out=v_slot)
-                else:  # still the K-split partial sums of the projection: added inside the kernel
-                    q, _, _ = ops.pre_attention_partials(qkv, cfg.num_attention_heads, Hkv, D, lw["q_norm"],
-                                                         lw["k_norm"], cos, sin, cfg.rms_norm_eps,
-                                                         k_out=k_slot, v_out=v_slot)
                 a, e = cache.attention_range(li)
-                attn = ops.decode(q.transpose(1, 2), cache.key_cache[li], cache.value_cache[li], a, e,
-                                  self.scaling)
+                # (a text token's row: the last one of a large window, the first one of a small one)
+                attn = self._text_attention(lw, h, cos, sin, cache.key_cache[li], cache.value_cache[li],
+                                            e - 1 if cache.is_large_window[li] else a, a, e,
+                                            dict(k_out=k_slot, v_out=v_slot))
             else:
                 fused = hasattr(ops, "decode_boundary") and cache.boundary_fits_one_piece(li)
                 if fused:
@@ -640,7 +663,7 @@ class KsaQwen3ForCausalLM:
                                       lw["post_attention_layernorm"])
                 delta = self._mlp(lw, h, defer=True)
             else:
-                x, delta = self._post_attention(lw, attn.reshape(b, ids.shape[1], -1), x)
+                x, delta = self._post_attention(lw, attn, x)
         cache.reset_chunk_counter()
         if not boundary:
             return self._logits(x, delta)
@@ -663,17 +686,9 @@ class KsaQwen3ForCausalLM:
             # k and v go straight to the cache row the device-side cursor names
             slots = dict(k_out=cache.key_cache[li][:, :, :1].transpose(1, 2),
                          v_out=cache.value_cache[li][:, :, :1].transpose(1, 2), kv_out_row=st["cur"][kind, 0])
-            qkv = ops.linear(h, lw["qkv_proj"], defer=True)
-            if torch.is_tensor(qkv):
-                q, k, v = self._split_qkv(qkv)
-                q, _, _ = ops.pre_attention(q, k, v, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps, **slots)
-            else:  # still the K-split partial sums of the projection: added inside the kernel
-                q, _, _ = ops.pre_attention_partials(qkv, cfg.num_attention_heads, cfg.num_key_value_heads,
-                                                     cfg.head_dim, lw["q_norm"], lw["k_norm"], cos, sin,
-                                                     cfg.rms_norm_eps, **slots)
-            attn = ops.decode(q.transpose(1, 2), cache.key_cache[li], cache.value_cache[li],
-                              st["cur"][kind, 1], st["cur"][kind, 2], self.scaling)
-            x, delta = self._post_attention(lw, attn.reshape(b, 1, -1), x)
+            attn = self._text_attention(lw, h, cos, sin, cache.key_cache[li], cache.value_cache[li], *st["cur"][kind],
+                                        slots)
+            x, delta = self._post_attention(lw, attn, x)
         return self._logits(x, delta)
 
     def _boundary_step_body(self, st, cache):

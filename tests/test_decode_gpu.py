@@ -286,3 +286,50 @@ def test_decode_boundary_equals_two_decodes(D, dtype, g, nsplit):
             two = torch.cat([ksa_amd.ksa_decode(qd[:, :, :1], kd, vd, ta, tb, nsplit=nsplit),
                              ksa_amd.ksa_decode(qd[:, :, 1:], kd, vd, sa, sb, nsplit=nsplit)], dim=1)
             assert torch.equal(got, two)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,Hq,Hkv,D,rows,start,end,row,nsplit", [
+    (1, 32, 8, 128, 700, 3, 690, 3, None),        # first row of the range (a small window)
+    (1, 32, 8, 128, 700, 0, 700, 699, 12),        # last row (a large window), splits without rows
+    (1, 32, 8, 128, 5000, 0, 4999, 2500, 64),     # more splits than are requested at once
+    (2, 8, 8, 128, 300, 10, 299, 138, 2),         # one query head per kv head; last row of a workgroup's round
+    (3, 15, 3, 128, 300, 0, 129, 128, 2),         # group of 5; a slice of one row, the new one
+    (4, 32, 1, 128, 260, 1, 258, 33, 3),          # group of 32: several passes over the query rows
+    (8, 32, 4, 64, 500, 5, 400, 6, 4),
+    (2, 16, 8, 64, 90, 0, 64, 63, 1),             # no split
+    (16, 32, 8, 128, 400, 0, 300, 200, 3),
+])
+def test_decode_qkv_equals_separate_launches(dtype, b, Hq, Hkv, D, rows, start, end, row, nsplit):
+    """The attention of a step from the projection's partial sums against the pre-attention step and the decode
+    call it stands for: output and caches bit for bit."""
+    import ksa_amd
+    from ksa_amd import decode, gemm, pre
+    g = torch.Generator(device="cuda").manual_seed(b * 1000 + end)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    H = 1536 if D == 128 else 5120                 # 3 or 10 slices of the projection's K
+    width = (Hq + 2 * Hkv) * D
+    h, w = rnd(b, 1, H).to(dtype), (rnd(width, H) * H ** -0.5).to(dtype)
+    qw, kw = (1 + 0.1 * rnd(D)).to(dtype), (1 + 0.1 * rnd(D)).to(dtype)
+    ang = rnd(1, 1, D // 2)
+    ang = torch.cat((ang, ang), -1)
+    cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+    qkv = gemm.linear_rows(h, w, defer=True)
+    assert isinstance(qkv, gemm.SplitKPartials)
+    caches = [rnd(b, Hkv, rows, D).to(dtype) for _ in range(2)]
+    caches[0][:, :, row] = float("nan")            # what the new row overwrites must not be read
+    caches[1][:, :, row] = float("nan")
+    for device_bounds in (False, True):
+        kc, vc = (c.clone() for c in caches)
+        kr, vr = (c.clone() for c in caches)
+        at = torch.full((b,), row, dtype=torch.int32, device="cuda")
+        q, _, _ = pre.pre_attention_partials(qkv, Hq, Hkv, D, qw, kw, cos, sin, 1e-6, k_out=kr[:, :, :1].transpose(1, 2),
+                                             v_out=vr[:, :, :1].transpose(1, 2), kv_out_row=at)
+        lo, hi, r = start, end, row
+        if device_bounds:
+            lo, hi, r = (torch.full((b,), x, dtype=torch.int32, device="cuda") for x in (start, end, row))
+        want = ksa_amd.ksa_decode(q.transpose(1, 2), kr, vr, lo, hi, nsplit=nsplit)
+        got = decode.ksa_decode_qkv(qkv, qw, kw, cos, sin, 1e-6, kc, vc, Hq, r, lo, hi, nsplit=nsplit)
+        assert torch.equal(got, want.reshape(b, 1, Hq * D)) and torch.isfinite(got.float()).all()
+        assert torch.equal(kc, kr) and torch.equal(vc, vr)

@@ -326,3 +326,18 @@ def test_decode_splits_rule(b, hq, hkv, q):
             assert n == 1
         last = max(n, 1)
     assert L.ksa_decode_splits(1, 32, 7, 1, 1000) == 1 and L.ksa_decode_splits(0, 32, 8, 1, 1000) == 1
+
+
+def test_decode_qkv_argument_checks():
+    """Shapes the fused decode call does not take are refused on the host."""
+    from ksa_amd import _lib, decode
+    L = _lib.lib()
+    assert decode.decode_qkv_supported(32, 8, 128) and not decode.decode_qkv_supported(32, 8, 256)
+    assert not decode.decode_qkv_supported(33, 1, 64)
+    st = (ctypes.c_int64 * 3)(8, 8, 8)
+    base = dict(qkv=16, ks=2, qw=16, kw=16, cos=16, sin=16, cbs=0, eps=1e-6, kc=16, vc=16, out=16, row=None, row0=3,
+                start=None, end=None, s0=0, e0=10, b=1, hq=4, hkv=2, d=64, dt=0, kst=st, vst=st, ost=st, scale=0.1, ns=1,
+                ws=None, wb=0, stream=None)
+    call = lambda **kw: L.ksa_decode_qkv_fwd(*{**base, **kw}.values())
+    assert call(qkv=None) != 0 and call(d=256) != 0 and call(row0=10) != 0 and call(row0=-1) != 0 and call(e0=0) != 0
+    assert call(hq=5) != 0 and call(ns=2) != 0 and call(out=None) != 0 and call(kc=8) != 0 and call(b=129) != 0
