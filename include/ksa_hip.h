@@ -254,6 +254,17 @@ int ksa_add_rmsnorm(const void* x, const void* residual, const void* weight, voi
                     long long residual_row_stride, long long norm_row_stride,
                     long long sum_row_stride, int dtype, float eps, void* stream);
 
+/* The head of a decode step in one launch: out[r] = table[ids[r]] (the embedding rows), out_norm[r] = weight *
+ * rmsnorm(out[r]) as ksa_add_rmsnorm without a residual gives it, rope_out = rope_table[*rope_row].
+ *   table [table_rows, H], row stride in elements, a multiple of 8; ids device int64[rows]: a negative id counts from
+ *   the end, one outside the table gives a row of NaN; out, out_norm [rows, H] contiguous
+ *   rope_table [rope_rows, rope_width] contiguous, rope_row device int32 (kept inside the table)
+ * H (at most 8192) and rope_width multiples of 8; all but ids and rope_row 16-byte aligned. */
+int ksa_embed_rmsnorm(const void* table, long long table_rows, long long table_row_stride, const long long* ids,
+                      const void* weight, void* out, void* out_norm, int rows, int H, const void* rope_table,
+                      int rope_rows, int rope_width, const int32_t* rope_row, void* rope_out, int dtype, float eps,
+                      void* stream);
+
 /* ksa_add_rmsnorm whose x is not a tensor yet but the K-split partial sums that ksa_gemm_rows
  * leaves in its workspace when called with out == NULL (fp32 [ksplit][R][H], R = rows rounded up to a
  * multiple of 16): x = the sum over

@@ -46,6 +46,8 @@ _SIGNATURES = {
                                    + [_vp, _int, ctypes.c_float, _vp]),
     "ksa_add_rmsnorm": (_int, [_vp] * 5 + [ctypes.c_longlong, _int] + [ctypes.c_longlong] * 4
                         + [_int, ctypes.c_float, _vp]),
+    "ksa_embed_rmsnorm": (_int, [_vp, ctypes.c_longlong, ctypes.c_longlong] + [_vp] * 4 + [_int, _int, _vp, _int, _int]
+                          + [_vp, _vp, _int, ctypes.c_float, _vp]),
     "ksa_add_rmsnorm_partials": (_int, [_vp, _int] + [_vp] * 4 + [_int, _int] + [ctypes.c_longlong] * 3
                                  + [_int, ctypes.c_float, _vp]),
     "ksa_silu_mul": (_int, [_vp] * 3 + [ctypes.c_longlong, _int] + [ctypes.c_longlong] * 3 + [_int, _vp]),

@@ -75,6 +75,33 @@ def add_rmsnorm(x: torch.Tensor, residual: Optional[torch.Tensor], weight: torch
     return s.view(x.shape), out.view(x.shape)
 
 
+def embed_rmsnorm_supported(table: torch.Tensor, weight: torch.Tensor) -> bool:
+    return (table.is_cuda and table.dtype in _DT and table.dim() == 2 and table.stride(1) == 1 and table.stride(0) % 8 == 0
+            and table.data_ptr() % 16 == 0 and table.shape[1] % 8 == 0 and table.shape[1] <= 8192
+            and weight.dtype == table.dtype and weight.shape == table.shape[1:] and weight.is_contiguous()
+            and weight.data_ptr() % 16 == 0)
+
+
+def embed_rmsnorm(table: torch.Tensor, ids: torch.Tensor, weight: torch.Tensor, eps: float, rope_table: torch.Tensor,
+                  rope_row: torch.Tensor, out: torch.Tensor, out_norm: torch.Tensor, rope_out: torch.Tensor) -> None:
+    """The head of a decode step (`ksa_embed_rmsnorm`) into the caller's buffers: out = table[ids], out_norm = weight *
+    rmsnorm(out), rope_out = rope_table[rope_row].  ids: int64, contiguous; rope_row: int32 [1]."""
+    rows, H = ids.numel(), table.shape[1]
+    assert embed_rmsnorm_supported(table, weight) and ids.dtype == torch.long and ids.is_contiguous()
+    assert rope_row.dtype == torch.int32 and rope_row.numel() == 1 and rope_table.is_contiguous() and rope_out.is_contiguous()
+    assert out.numel() == out_norm.numel() == rows * H and out.is_contiguous() and out_norm.is_contiguous()
+    width = rope_out.numel()
+    assert rope_table.numel() % width == 0
+    for t in (ids, weight, rope_row, rope_table, out, out_norm, rope_out):
+        assert t.device == table.device and (t.dtype == table.dtype or t is ids or t is rope_row)
+    with _lib.on_device(table.device):
+        rc = _lib.lib().ksa_embed_rmsnorm(table.data_ptr(), table.shape[0], table.stride(0), ids.data_ptr(), weight.data_ptr(),
+                                          out.data_ptr(), out_norm.data_ptr(), rows, H, rope_table.data_ptr(),
+                                          rope_table.numel() // width, width, rope_row.data_ptr(), rope_out.data_ptr(),
+                                          _DT[table.dtype], float(eps), _lib.stream_ptr(table.device))
+    _lib.check(rc, "ksa_embed_rmsnorm")
+
+
 def silu_mul(gate, up: Optional[torch.Tensor] = None) -> torch.Tensor:
     """round(silu(gate)) * up; gate and up may be strided views (halves of one GEMM output).
     With `up` left out, `gate` is the whole gate | up projection [..., 2 I]: a tensor, or the

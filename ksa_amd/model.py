@@ -139,6 +139,8 @@ class HipOps:
         self.summary_attn_func = prefill.summary_attn_func
         self.add_rmsnorm = elementwise.add_rmsnorm
         self.silu_mul = elementwise.silu_mul
+        self.embed_rmsnorm = elementwise.embed_rmsnorm       # the head of a recorded step in one launch
+        self.embed_rmsnorm_supported = elementwise.embed_rmsnorm_supported
         self._decode = decode.ksa_decode
         self._decode_mod = decode
         self.decode_boundary = decode.ksa_decode_boundary   # text token + summary tokens of a boundary step, one launch
@@ -675,14 +677,17 @@ class KsaQwen3ForCausalLM:
         per-step quantity (token ids, position, the cache row the new K/V go to, the attended row
         range) is read from device tensors of `st`, never baked into a launch."""
         cfg, ops = self.config, self.ops
-        rope = st["rope_tab"].index_select(0, st["rope_rel"])   # [1, 2, D]: this step's cos and sin rows
+        if st["head"] is not None:     # filled in front of the replay, see `decode_step_graph`
+            x, h, rope = st["head"]
+        else:
+            rope = st["rope_tab"].index_select(0, st["rope_rel"])   # [1, 2, D]: this step's cos and sin rows
+            x, h = self.w["embed_tokens"][st["tok"]], None
         cos, sin = rope[:, 0][None], rope[:, 1][None]
-        x = self.w["embed_tokens"][st["tok"]]
-        b = x.shape[0]
         delta = None
         for li, lw in enumerate(self.w["layers"]):
             kind = 1 if cache.is_large_window[li] else 0
-            x, h = self._add_norm(delta, x, lw["input_layernorm"])
+            if li or h is None:
+                x, h = self._add_norm(delta, x, lw["input_layernorm"])
             # k and v go straight to the cache row the device-side cursor names
             slots = dict(k_out=cache.key_cache[li][:, :, :1].transpose(1, 2),
                          v_out=cache.value_cache[li][:, :, :1].transpose(1, 2), kv_out_row=st["cur"][kind, 0])
@@ -817,14 +822,22 @@ class KsaQwen3ForCausalLM:
             sids = torch.arange(S, device=self.device, dtype=torch.long) + cfg.summary_token_begin
             st = {"batch": b, "owner": self, "graphs": {}, "rings": {},
                   "tok": torch.zeros(b, 1, dtype=torch.long, device=self.device),
-                  # [kind: small / large window][destination row, range start, range end][sequence]
-                  "cur": torch.zeros(2, 3, b, dtype=torch.int32, device=self.device),
+                  # a step inside a chunk: [kind: small / large window][destination row, range start, range end]
+                  # [sequence], and behind it the step's row of the rotary table
+                  "step": torch.zeros(6 * b + 1, dtype=torch.int32, device=self.device),
                   # the same for a boundary step (see `_boundary_step_body`), its ids and positions
                   "bcur": torch.zeros(2, 6, b, dtype=torch.int32, device=self.device),
                   "btok": torch.cat([torch.zeros(b, 1, dtype=torch.long, device=self.device),
                                      sids[None].expand(b, -1)], dim=1).contiguous(),
                   "bpos": torch.zeros(1, 1 + S, dtype=torch.int32, device=self.device),
-                  "bsum_rows": torch.arange(1, 1 + S, device=self.device)}
+                  "bsum_rows": torch.arange(1, 1 + S, device=self.device),
+                  "head": None}
+            st["cur"], st["rope_rel"] = st["step"][:6 * b].view(2, 3, b), st["step"][6 * b:]
+            emb, norm = self.w["embed_tokens"], self.w["layers"][0]["input_layernorm"]
+            if getattr(self.ops, "embed_rmsnorm_supported", lambda *a: False)(emb, norm):
+                # the first layer's residual row and norm, and the rotary row of the step
+                st["head"] = (*(torch.zeros(b, 1, cfg.hidden_size, dtype=emb.dtype, device=self.device) for _ in range(2)),
+                              torch.zeros(1, 2, D, dtype=emb.dtype, device=self.device))
             cache._ksa_graph_state = st
         kinds = [1 if cache.is_large_window[li] else 0 for li in range(nl)]
         if cache.get_cur_chunk_size() == C - 1:
@@ -876,8 +889,6 @@ class KsaQwen3ForCausalLM:
                 a, e = cache.attention_range(li)
                 vals[kinds[li]] = [rows[kinds[li]], a, e]
                 rows[kinds[li]] = None
-        self._stage_ints(st, "cur", [v for kind in vals for x in kind for v in [x] * b])
-        st["tok"].copy_(token_ids.to(self.device))
         # rotary rows of a window of positions, made with the prefill's own tensor ops (so a step's
         # cos / sin are the values `_rope_tables` gives) and refilled in place when p leaves it; the
         # recorded step only picks a row
@@ -889,9 +900,16 @@ class KsaQwen3ForCausalLM:
                 st["rope_tab"].copy_(tab)
             else:
                 st["rope_tab"] = tab.contiguous()
-                st["rope_rel"] = torch.zeros(1, dtype=torch.long, device=self.device)
             st["rope_p0"] = p
-        st["rope_rel"].fill_(p - st["rope_p0"])
+        self._stage_ints(st, "step", [v for kind in vals for x in kind for v in [x] * b] + [p - st["rope_p0"]])
+        ids = token_ids
+        if st["head"] is None or ids.device != self.device or ids.dtype != torch.long or ids.shape != (b, 1) \
+                or not ids.is_contiguous():
+            ids = st["tok"].copy_(token_ids.to(self.device))
+        if st["head"] is not None:
+            x, h, rope = st["head"]
+            self.ops.embed_rmsnorm(self.w["embed_tokens"], ids, self.w["layers"][0]["input_layernorm"], cfg.rms_norm_eps,
+                                   st["rope_tab"], st["rope_rel"], x, h, rope)
         self._warm_up(st, "text", self._text_step_body, cache)   # a step inside a chunk is idempotent
         logits = self._replay(st, "text", self._text_step_body, cache)
         cache.reset_chunk_counter()

@@ -156,3 +156,33 @@ def test_gpu_argmax_rows_ties_and_special_values(dtype, N):
     x[7, N - 1] = float("inf")
     got = argmax_rows(x.cuda()[:, :N]).cpu()
     assert torch.equal(got, x[:, :N].float().argmax(-1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,H,vocab,D", [(1, 64, 9, 64), (3, 2560, 1000, 128), (4, 520, 50, 256), (8, 8192, 40, 8),
+                                            (129, 4096, 300, 128)])
+def test_gpu_embed_rmsnorm_equals_separate_launches(dtype, rows, H, vocab, D):
+    """The head of a step against embedding lookup, norm and row choice, bit for bit; a table with padded rows."""
+    from ksa_amd.elementwise import add_rmsnorm, embed_rmsnorm
+    g = torch.Generator(device="cuda").manual_seed(rows + H)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
+    table, w, rope = rnd(vocab, H + 8)[:, :H], rnd(H), rnd(70, 2, D)
+    ids = torch.randint(-vocab, vocab, (rows, 1), generator=g, device="cuda")
+    ids[0], ids[-1] = vocab - 1, -vocab
+    for at in (0, 69):
+        x, h, r = (torch.full(s, 7.0, dtype=dtype, device="cuda") for s in ((rows, 1, H), (rows, 1, H), (1, 2, D)))
+        embed_rmsnorm(table, ids, w, 1e-6, rope, torch.tensor([at], dtype=torch.int32, device="cuda"), x, h, r)
+        s, n = add_rmsnorm(table[ids], None, w, 1e-6)
+        assert torch.equal(x, s) and torch.equal(h, n) and torch.equal(r[0], rope[at])
+
+
+def test_embed_rmsnorm_argument_checks():
+    """What the head-of-step kernel does not take is refused on the host."""
+    from ksa_amd import _lib
+    base = dict(table=16, vocab=10, stride=64, ids=8, w=16, out=16, norm=16, rows=2, H=64, rope=16, rr=4, rw=16, row=4, ro=16,
+                dt=0, eps=1e-6, st=None)
+    call = lambda **kw: _lib.lib().ksa_embed_rmsnorm(*{**base, **kw}.values())
+    for bad in (dict(table=None), dict(ids=None), dict(row=None), dict(rows=0), dict(H=60), dict(H=8200), dict(vocab=0),
+                dict(rr=0), dict(rw=12), dict(table=24), dict(stride=60), dict(ro=8), dict(dt=5), dict(eps=-1.0)):
+        assert call(**bad) != 0
