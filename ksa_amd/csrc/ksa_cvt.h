@@ -91,21 +91,21 @@ __host__ __device__ __forceinline__ int ksa_partial_rows(int rows) { return (row
 // eight consecutive columns of a row of x = the rounded sum of fp32 slices [ksplit][prows][width]
 // (the K-split partial sums of ksa_gemm_rows, prows = ksa_partial_rows(rows of x)), added in split
 // order like its own reduction
-template <typename T>
+template <typename T, int kBatch = 8>
 __device__ __forceinline__ u32x4 ksa_sum_partials8(const float* part, int ksplit, int prows, int width, int row, int col) {
     using C = KsaCvt<T>;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int sp0 = 0; sp0 < ksplit; sp0 += 8) {  // eight slices requested together
-        f32x4 lo[8], hi[8];
+    for (int sp0 = 0; sp0 < ksplit; sp0 += kBatch) {  // so many slices requested together
+        f32x4 lo[kBatch], hi[kBatch];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < kBatch; ++u) {
             const int sp = min(sp0 + u, ksplit - 1);
             const float* src = part + ((int64_t)sp * prows + row) * width + col;
             lo[u] = *reinterpret_cast<const f32x4*>(src);
             hi[u] = *reinterpret_cast<const f32x4*>(src + 4);
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < kBatch; ++u) {
             if (sp0 + u < ksplit) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[i] += lo[u][i], acc[4 + i] += hi[u][i];

@@ -113,7 +113,11 @@ __global__ __launch_bounds__(256) void ksa_add_rmsnorm_kernel(const NormParams p
 // per row, as many threads as the row has 16-byte items (up to 512, then NJ = 2 items per thread),
 // adds the slices in split order, rounds (which is what the GEMM's own reduction does), adds the
 // residual and normalises.  Everything that does not depend on the sums is requested first.
-template <typename T, int NJ>
+// kBatch: slices requested together; every further batch is another trip to memory, which is what this kernel's time
+// is.  Twenty take the 19 slices of the 4B shape's down projection in one trip (184 registers, no matter with
+// one workgroup per row) where eight take three: decode step of 8 layers 643.1 -> 640.0 us (batch 1), 752.6 -> 750.1
+// (batch 8).  Up to eight slices, and rows of two items per thread, keep the batch of eight.
+template <typename T, int NJ, int kBatch>
 __global__ __launch_bounds__(512) void ksa_add_rmsnorm_partials_kernel(const NormParams p) {
     using C = KsaCvt<T>;
     __shared__ float s_ss[8];
@@ -134,7 +138,7 @@ __global__ __launch_bounds__(512) void ksa_add_rmsnorm_partials_kernel(const Nor
     for (int j = 0; j < NJ; ++j) {
         const int idx = tid + nthr * j;
         if (idx < items) {
-            const u32x4 x = ksa_sum_partials8<T>(p.part, p.ksplit, ksa_partial_rows(p.rows), p.H, row, 8 * idx);
+            const u32x4 x = ksa_sum_partials8<T, kBatch>(p.part, p.ksplit, ksa_partial_rows(p.rows), p.H, row, 8 * idx);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 r[j][i] = C::down2(C::lo(x[i]) + C::lo(q[j][i]), C::hi(x[i]) + C::hi(q[j][i]));
@@ -173,8 +177,9 @@ int dispatch_norm_partials(const NormParams& p, hipStream_t st) {
     const int threads = items >= 512 ? 512 : (items + 63) / 64 * 64;
     const int need = (items + threads - 1) / threads;
     const dim3 grid((unsigned)p.rows), block(threads);
-    if (need <= 1) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 1>), grid, block, 0, st, p);
-    else if (need <= 2) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 2>), grid, block, 0, st, p);
+    if (need <= 1 && p.ksplit > 8) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 1, 20>), grid, block, 0, st, p);
+    else if (need <= 1) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 1, 8>), grid, block, 0, st, p);
+    else if (need <= 2) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 2, 8>), grid, block, 0, st, p);
     else return KSA_ERR_UNSUPPORTED;
     return ksa_check_launch();
 }

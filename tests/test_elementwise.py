@@ -186,3 +186,26 @@ def test_embed_rmsnorm_argument_checks():
     for bad in (dict(table=None), dict(ids=None), dict(row=None), dict(rows=0), dict(H=60), dict(H=8200), dict(vocab=0),
                 dict(rr=0), dict(rw=12), dict(table=24), dict(stride=60), dict(ro=8), dict(dt=5), dict(eps=-1.0)):
         assert call(**bad) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ksplit", [1, 8, 9, 19, 20, 21, 40, 41, 64])
+@pytest.mark.parametrize("rows,H", [(1, 2560), (17, 4096), (3, 4104)])
+def test_gpu_add_rmsnorm_partials_slice_counts(dtype, ksplit, rows, H):
+    """Slice counts around the batches in which they are requested: the residual sum is bit for bit that of the
+    slices added in order, the norm within one rounding."""
+    from ksa_amd.elementwise import add_rmsnorm
+    from ksa_amd.gemm import SplitKPartials
+    g = torch.Generator().manual_seed(ksplit * 100 + rows)
+    part = torch.randn(ksplit, (rows + 15) // 16 * 16, H, generator=g) * ksplit ** -0.5
+    acc = torch.zeros(rows, H)
+    for s in part:
+        acc = acc + s[:rows]
+    r = torch.randn(rows, H, generator=g).to(dtype)
+    w = (1 + 0.1 * torch.randn(H, generator=g)).to(dtype)
+    x = SplitKPartials(part.cuda().view(-1).view(torch.uint8), ksplit, rows, (rows, H), dtype)
+    s, y = add_rmsnorm(x, r.cuda(), w.cuda(), 1e-6)
+    s_exp, y_exp = cpu_path.add_rmsnorm(acc.to(dtype), r, w, 1e-6)
+    assert torch.equal(s.cpu(), s_exp)
+    _ulp_check(y, y_exp, 5e-3)
