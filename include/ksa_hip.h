@@ -105,9 +105,9 @@ int ksa_prefill_fwd(const void* q, const void* k, const void* v, void* out, floa
  *   ksa_decode_workspace_bytes(...) bytes (fp32 partials). */
 size_t ksa_decode_workspace_bytes(int batch, int Hq, int Hkv, int Q, int D, int nsplit);
 int ksa_decode_auto_splits(int batch, int Hkv, int max_rows);
-/* The split count for Q query tokens of Hq heads (faster than ksa_decode_auto_splits on few rows, with a larger
+/* The split count for Q query tokens of Hq heads of head_dim D (faster than ksa_decode_auto_splits on few rows, with a larger
  * workspace: ksa_decode_auto_splits remains the count to use with ksa_decode_fwd_noalloc). */
-int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int max_rows);
+int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int max_rows);
 int ksa_decode_fwd(const void* q, const void* kcache, const void* vcache, void* out,
                    const int32_t* start, const int32_t* end, int start0, int end0, int batch,
                    int Hq, int Hkv, int Q, int D, int dtype, const int64_t* q_strides,

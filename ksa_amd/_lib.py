@@ -27,7 +27,7 @@ _SIGNATURES = {
                         + [_int, ctypes.c_float, _int, _vp, _vp]),
     "ksa_decode_workspace_bytes": (ctypes.c_size_t, [_int] * 6),
     "ksa_decode_auto_splits": (_int, [_int] * 3),
-    "ksa_decode_splits": (_int, [_int] * 5),
+    "ksa_decode_splits": (_int, [_int] * 6),
     "ksa_decode_fwd": (_int, [_vp] * 6 + [_int] * 8 + [_i64p] * 4
                        + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
     "ksa_decode_qkv_fwd": (_int, [_vp, _int] + [_vp] * 4 + [ctypes.c_longlong, ctypes.c_float] + [_vp] * 4 + [_int]

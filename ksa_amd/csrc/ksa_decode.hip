@@ -535,10 +535,26 @@ extern "C" int ksa_decode_auto_splits(int batch, int Hkv, int max_rows) {
 // head_dim 128, 8 kv heads, former count -> this one: 1 sequence of 760 / 1500 / 4096 / 16384 rows
 // 13.2 / 13.4 / 13.4 / 29.8 -> 9.0 / 9.2 / 10.4 / 19.4 us (the last by the merge kernel alone), 8 sequences of
 // 760 / 1500 rows 14.5 / 19.9 -> 12.8 / 18.6; 16 and 32 sequences the same counts as before.
-extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int max_rows) {
-    if (batch <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || Q <= 0 || max_rows <= 0) return 1;
+// At head_dim 256 a CU holds one workgroup, so two per CU run one behind the other, with a second start: there the
+// count is the one with the least rounds x (steps of 128 rows + 2 for the start) + 1.5 for the merge, in units of a
+// step.  8 kv heads, count by the rule above -> this one: 1 sequence of 4430 / 16384 rows 24.3 / 39.3 -> 18.8 / 33.6 us,
+// 2 of 4430 32.3 -> 25.5 (before either rule 24.9), 4 of 3000 35.1 -> 27.9, 8 of 1500 37.4 -> 28.1, 16 of 3000 80.3 -> 74.8,
+// 20 of 6000 191 -> 173; few rows the same counts.
+extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int max_rows) {
+    if (batch <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || Q <= 0 || D <= 0 || max_rows <= 0) return 1;
     const int64_t units = (int64_t)batch * Hkv * ((Q * (int64_t)(Hq / Hkv) + 31) / 32);
     const int cus = ksa_cu_count_or(256);
+    if (D > 128) {
+        const int64_t steps = ((int64_t)max_rows + 127) / 128;
+        int best = 1;
+        int64_t least = INT64_MAX;  // (in half steps)
+        for (int i = 1; i <= 64 && i <= steps; ++i) {
+            const int64_t per = (steps + i - 1) / i, used = (steps + per - 1) / per;  // splits that have rows
+            const int64_t cost = (units * used + cus - 1) / cus * (2 * per + 4) + (used > 1 ? 3 : 0);
+            if (cost < least) least = cost, best = (int)used;
+        }
+        return best;
+    }
     int64_t n = (2 * (int64_t)cus + units - 1) / units;
     int64_t cap = max_rows / 256;
     if (2 * units < cus) cap = max_rows <= 192 ? 1 : ((int64_t)max_rows + 127) / 128;

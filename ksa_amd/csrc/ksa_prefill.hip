@@ -333,7 +333,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
 
     // Regular tiles: uniform offset word = byte offset of the tile's first row | 1 if the
     // tile lies in the in-line region (computed per lane when the walk order is fetched).
-    // 3: a tile that is not regular (see kRegular); its loop fills take the first 64 rows.
+    // 3: a tile that is not regular (see kAddr); its loop fills take the first 64 rows.
     constexpr uint32_t kSpecialBit = 2u;
     auto tile_word = [&](int n) -> uint32_t {
         const int n0 = n * kTileN;

@@ -95,7 +95,7 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     if scale is None:
         scale = float(D) ** -0.5
     if nsplit is None:
-        nsplit = _lib.lib().ksa_decode_splits(b, q.shape[1], kcache.shape[1], q.shape[2], max_rows)
+        nsplit = _lib.lib().ksa_decode_splits(b, q.shape[1], kcache.shape[1], q.shape[2], D, max_rows)
     Dk = kernel_head_dim(D)
     if Dk != D:
         # A head dimension without a kernel of its own (the kernels are built for 64 / 128 / 256): the
@@ -130,7 +130,7 @@ def decode_qkv_pays(kcache: torch.Tensor, Hq: int, start, end) -> bool:
     L = _lib.lib()
     device = isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor)
     with _lib.on_device(kcache.device):
-        n = L.ksa_decode_splits(b, Hq, Hkv, 1, rows if device else max(1, int(end) - int(start)))
+        n = L.ksa_decode_splits(b, Hq, Hkv, 1, D, rows if device else max(1, int(end) - int(start)))
         return b * Hkv * n <= 2 * max(1, L.ksa_device_cu_count())
 
 
@@ -170,7 +170,7 @@ def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor
     ptr = lambda t: None if t is None else t.data_ptr()
     with _lib.on_device(dev):
         if nsplit is None:
-            nsplit = L.ksa_decode_splits(b, Hq, Hkv, 1, max_rows)
+            nsplit = L.ksa_decode_splits(b, Hq, Hkv, 1, D, max_rows)
         ws = None
         ws_bytes = L.ksa_decode_workspace_bytes(b, Hq, Hkv, 1, D, nsplit)
         if nsplit > 1:

@@ -320,12 +320,14 @@ def test_decode_splits_rule(b, hq, hkv, q):
     units = b * hkv * -(-q * (hq // hkv) // 32)
     last = 0
     for rows in (1, 128, 192, 193, 256, 300, 513, 1000, 4096, 16384, 131072, 2**31 - 1):
-        n = L.ksa_decode_splits(b, hq, hkv, q, rows)
+        n = L.ksa_decode_splits(b, hq, hkv, q, 128, rows)
         assert last <= n <= 64 and (n == 1 or (n - 1) * units < 2 * 256 and (n - 1) * 128 < rows)
         if rows <= 192:
             assert n == 1
         last = max(n, 1)
-    assert L.ksa_decode_splits(1, 32, 7, 1, 1000) == 1 and L.ksa_decode_splits(0, 32, 8, 1, 1000) == 1
+        wide = L.ksa_decode_splits(b, hq, hkv, q, 256, rows)   # one workgroup per CU: no split without rows
+        assert 1 <= wide <= 64 and (wide == 1 or (wide - 1) * -(-rows // 128 // wide) * 128 < rows)
+    assert L.ksa_decode_splits(1, 32, 7, 1, 128, 1000) == 1 and L.ksa_decode_splits(0, 32, 8, 1, 128, 1000) == 1
 
 
 def test_decode_qkv_argument_checks():
