@@ -547,3 +547,31 @@ def test_gpu_config4_full_depth_decode_equals_prefill():
     print(f"full depth: max logit difference {err / scale:.3e} of the logit scale, rms {rms / scale:.3e}, "
           f"arg-max agreement {agree:.2f}")
     assert err <= 5e-2 * scale and rms <= 1e-2 * scale, (err / scale, rms / scale)
+
+
+@pytest.mark.gpu
+def test_gpu_graph_decode_forms_of_token_ids():
+    """A recorded step reads int64 ids where they are and takes every other form through a copy: the same
+    logits bit for bit, and those of the separate launches that other operators' recordings hold."""
+    from ksa_amd.model import HipOps
+    cfg = tiny_config(summary_chunk_size=128, summary_token_num=8, head_dim=128, num_attention_heads=8,
+                      num_key_value_heads=2, hidden_size=256, intermediate_size=512, num_hidden_layers=2,
+                      summary_sliding_chunk_num=[1, 1 << 20], vocab_size=1000, summary_token_begin=1000)
+    w = init_weights(cfg, "cuda", torch.bfloat16, 8)
+    ids = torch.randint(0, cfg.vocab_size, (3, 140), generator=torch.Generator().manual_seed(10))
+    tok = torch.tensor([[5], [999], [0]], device="cuda")
+
+    class SeparateHead(HipOps):
+        def __init__(self):
+            super().__init__()
+            self.embed_rmsnorm_supported = lambda table, weight: False
+
+    forms = (tok, tok.int(), tok.cpu(), torch.cat((tok, tok), 1)[:, :1], tok - cfg.embedding_rows())
+    got = []
+    for ops, form in [(HipOps(), f) for f in forms] + [(SeparateHead(), tok)]:
+        model = KsaQwen3ForCausalLM(cfg, w, ops)
+        _, cache = model.prefill(ids)
+        steps = [model.decode_step_graph(form, cache).clone() for _ in range(3)]
+        got.append(torch.stack(steps))
+    for g in got[1:]:
+        assert torch.equal(g, got[0])
