@@ -535,6 +535,9 @@ extern "C" int ksa_decode_auto_splits(int batch, int Hkv, int max_rows) {
 // head_dim 128, 8 kv heads, former count -> this one: 1 sequence of 760 / 1500 / 4096 / 16384 rows
 // 13.2 / 13.4 / 13.4 / 29.8 -> 9.0 / 9.2 / 10.4 / 19.4 us (the last by the merge kernel alone), 8 sequences of
 // 760 / 1500 rows 14.5 / 19.9 -> 12.8 / 18.6; 16 and 32 sequences the same counts as before.
+// Up to three rounds (four of half the bytes at head_dim 64) one workgroup walks them faster than the merge's launch:
+// 1 split against several, 1 sequence of 200 / 300 / 500 rows 6.2 / 7.5 / 10.2 against 7.5 / 7.7 / 8.2 us, at head_dim
+// 64 4.9 / 5.7 / 6.5 against 6.8 / 6.9 / 6.9; there 120 units of 1000 rows also want the 3 splits (12.7 us) and not 5 (13.3).
 // At head_dim 256 a CU holds one workgroup, so two per CU run one behind the other, with a second start: there the
 // count is the one with the least rounds x (steps of 128 rows + 2 for the start) + 1.5 for the merge, in units of a
 // step.  8 kv heads, count by the rule above -> this one: 1 sequence of 4430 / 16384 rows 24.3 / 39.3 -> 18.8 / 33.6 us,
@@ -557,7 +560,8 @@ extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int m
     }
     int64_t n = (2 * (int64_t)cus + units - 1) / units;
     int64_t cap = max_rows / 256;
-    if (2 * units < cus) cap = max_rows <= 192 ? 1 : ((int64_t)max_rows + 127) / 128;
+    const bool few = D <= 64 ? 3 * units < cus : 2 * units < cus;
+    if (few) cap = max_rows <= (D <= 64 ? 512 : 384) ? 1 : ((int64_t)max_rows + 127) / 128;
     if (n > cap) n = cap;
     if (n > 64) n = 64;
     return n < 1 ? 1 : (int)n;
