@@ -46,7 +46,8 @@ struct GemmParams {
 // Per call in a graph of calls on distinct weights, 1 / 8 / 16 rows: 6144 x 2560 7.7 / 8.4 / 9.3 ->
 // 6.6 / 7.2 / 7.7 us, 2560 x 4096 7.2 / 7.9 / 8.8 -> 6.1 / 6.7 / 7.2, 2560 x 9728 12.0 / 12.9 / 14.5 -> 9.4 / 10.0 / 10.5 (31,
 // 21 and 50 MB are read in 6.1, 4.6 and 8.5 us by a kernel that does nothing else).
-template <typename T, bool kTiled, int XT>
+// kShortEnd: K is no multiple of 512 (a kernel of its own: the branch around the clearing cost the others 0.2 us).
+template <typename T, bool kTiled, int XT, bool kShortEnd>
 __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) {
     using C = KsaCvt<T>;
     __shared__ __attribute__((aligned(16))) unsigned char xs[2][4 * XT * kRowB];
@@ -76,7 +77,7 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
         a[u] = ksa_load_weights(reinterpret_cast<const uint16_t*>(wtile + s * (kTiled ? 1024 : 64) + wlane));
     };
     // staging of a chunk of x: thread = (row wave + 4 i, 16-byte piece lane); pieces past a short last chunk become
-    // zeros, so that its missing steps add nothing
+    // zeros, and so do the weights of its missing steps, so that these add nothing
     const uint16_t* xrow[XT];
 #pragma unroll
     for (int i = 0; i < XT; ++i) xrow[i] = p.x + (int64_t)min(wave + 4 * i, p.M - 1) * p.xs;
@@ -123,6 +124,7 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
             x_store(c + 1, buf);
             __syncthreads();
         }
+        if constexpr (kShortEnd) ksa_clear_missing_steps(a, p.steps - (c_end - 1) * kChunkSteps);
         chunk(std::false_type{}, c_end, buf);
     }
 
@@ -228,8 +230,8 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(con
 #pragma unroll
         for (int i = 0; i < XT; ++i) xt[i] = *reinterpret_cast<const u32x4*>(src + xrow_off[i]);
     };
-    // (a short last chunk is filled up with zeros: its missing steps then add nothing, whatever weights
-    // the clamped requests fetch for them)
+    // (a short last chunk is filled up with zeros, like the weights that the clamped requests fetch for its
+    // missing steps: these then add nothing)
     auto x_store = [&](int c) {
         const bool live = tj < 4 * min(kChunkSteps, steps - c * kChunkSteps);
 #pragma unroll
@@ -280,6 +282,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(con
             x_store(c + 1);
             __syncthreads();
         }
+        ksa_clear_missing_steps(a, steps - (c_end - 1) * kChunkSteps);
         chunk(std::false_type{}, c_end);
     }
     // C layout of a 16x16 tile: lane holds row (of x) lane % 16 of the block, columns n0 + 4 * (lane / 16) + i
@@ -394,14 +397,18 @@ int launch_gemm(GemmParams p, hipStream_t st) {
     p.chunks = (p.steps + kChunkSteps - 1) / kChunkSteps;
     p.chunks_per_split = (p.chunks + p.ksplit - 1) / p.ksplit;
     const dim3 grid((p.N + 63) / 64, p.ksplit), block(256);
-    auto go = [&](auto tiled) {
-        constexpr bool kT = decltype(tiled)::value;
-        if (p.M <= 4) hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 1>), grid, block, 0, st, p);
-        else if (p.M <= 8) hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 2>), grid, block, 0, st, p);
-        else hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 4>), grid, block, 0, st, p);
+    auto go = [&](auto tiled, auto short_end) {
+        constexpr bool kT = decltype(tiled)::value, kE = decltype(short_end)::value;
+        if (p.M <= 4) hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 1, kE>), grid, block, 0, st, p);
+        else if (p.M <= 8) hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 2, kE>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((ksa_gemm_rows_kernel<T, kT, 4, kE>), grid, block, 0, st, p);
     };
-    if (p.ws == kWTiled) go(std::true_type{});
-    else go(std::false_type{});
+    auto go_layout = [&](auto short_end) {
+        if (p.ws == kWTiled) go(std::true_type{}, short_end);
+        else go(std::false_type{}, short_end);
+    };
+    if (p.steps % kChunkSteps) go_layout(std::true_type{});
+    else go_layout(std::false_type{});
     if (p.ksplit > 1 && p.out) {
         const int64_t n = (int64_t)p.M * p.N;
         hipLaunchKernelGGL(ksa_gemm_rows_reduce_kernel<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p);

@@ -354,3 +354,23 @@ def test_gpu_streaming_weight_layout(dtype):
             s0, d0 = add_rmsnorm_mlp_rows(o, res, nw, 1e-6, w_gu, w_dn, ws)
             assert torch.equal(s0, s1) and torch.equal(sums(d0), sums(d1)), M
     assert not ws.failed()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 5, 16, 17, 72])
+@pytest.mark.parametrize("K", [32, 544, 1504, 2048])
+def test_gpu_linear_rows_infinite_weight_in_the_last_step(dtype, M, K):
+    """An infinite weight in the last elements of K (a short last chunk, or a whole one): its output column is
+    infinite with the sign of x there, as in torch, and no other column changes."""
+    from ksa_amd.gemm import TiledWeight, linear_rows
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randn(M, K, generator=g).to(dtype).cuda()
+    x[:, K - 3] = torch.where(x[:, K - 3] < 0, -1.0, 1.0).to(dtype)
+    w = (torch.randn(80, K, generator=g) * 0.05).to(dtype).cuda()
+    bad = w.clone()
+    bad[5, K - 3] = float("inf")
+    for wrap in (lambda t: t, TiledWeight):
+        want = linear_rows(x, wrap(w))
+        want[:, 5] = x[:, K - 3] * float("inf")
+        assert torch.equal(linear_rows(x, wrap(bad)), want)
