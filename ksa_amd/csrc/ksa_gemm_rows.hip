@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
     u32x4 a[kChunkSteps];
     auto w_request = [&](int c, int u) {
         const int64_t s = min(c * kChunkSteps + u, p.steps - 1);
-        a[u] = ksa_load_weights(reinterpret_cast<const uint16_t*>(wtile + s * (kTiled ? 1024 : 64) + wlane));
+        a[u] = ksa_load_weights<kTiled>(reinterpret_cast<const uint16_t*>(wtile + s * (kTiled ? 1024 : 64) + wlane));
     };
     // staging of a chunk of x: thread = (row wave + 4 i, 16-byte piece lane); pieces past a short last chunk become
     // zeros, and so do the weights of its missing steps, so that these add nothing
@@ -182,7 +182,7 @@ struct WideParams {
 };
 constexpr int kWideWaves = 8;
 
-template <typename T, int MB, bool kPair>
+template <typename T, int MB, bool kPair, bool kTiled>
 __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(const WideParams p) {
     using C = KsaCvt<T>;
     extern __shared__ __attribute__((aligned(16))) unsigned char wide_lds[];
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(con
     };
     u32x4 a[kChunkSteps];
     auto w_request = [&](int c, int u) {
-        a[u] = ksa_load_weights(wl.p + wl.step * min(c * kChunkSteps + u, steps - 1));
+        a[u] = ksa_load_weights<kTiled>(wl.p + wl.step * min(c * kChunkSteps + u, steps - 1));
     };
     // the products of one chunk; kMore: there is a next chunk, whose x and weights are requested on the way
     // (two copies of the loop body rather than a condition inside it: with branches between the MFMAs the
@@ -364,8 +364,8 @@ static WidePlan wide_plan(int K, int want_splits) {
     return pl;
 }
 
-template <typename T, bool kPair>
-int launch_wide(const WideParams& p, hipStream_t st) {
+template <typename T, bool kPair, bool kTiled>
+int launch_wide_layout(const WideParams& p, hipStream_t st) {
     const int mb = (p.M + 15) / 16;
     constexpr int cols = kPair ? 16 * (kWideWaves / 2) : 16 * kWideWaves;
     const dim3 grid((p.N + cols - 1) / cols, p.ksplit), block(64 * kWideWaves);
@@ -381,13 +381,18 @@ int launch_wide(const WideParams& p, hipStream_t st) {
         return ksa_check_launch();
     };
     switch (mb) {
-        case 2: return go(ksa_gemm_rows_wide_kernel<T, 2, kPair>);
-        case 3: return go(ksa_gemm_rows_wide_kernel<T, 3, kPair>);
-        case 4: return go(ksa_gemm_rows_wide_kernel<T, 4, kPair>);
-        case 5: return go(ksa_gemm_rows_wide_kernel<T, 5, kPair>);
-        case 6: return go(ksa_gemm_rows_wide_kernel<T, 6, kPair>);
-        default: return go(ksa_gemm_rows_wide_kernel<T, 8, kPair>);
+        case 2: return go(ksa_gemm_rows_wide_kernel<T, 2, kPair, kTiled>);
+        case 3: return go(ksa_gemm_rows_wide_kernel<T, 3, kPair, kTiled>);
+        case 4: return go(ksa_gemm_rows_wide_kernel<T, 4, kPair, kTiled>);
+        case 5: return go(ksa_gemm_rows_wide_kernel<T, 5, kPair, kTiled>);
+        case 6: return go(ksa_gemm_rows_wide_kernel<T, 6, kPair, kTiled>);
+        default: return go(ksa_gemm_rows_wide_kernel<T, 8, kPair, kTiled>);
     }
+}
+
+template <typename T, bool kPair>
+int launch_wide(const WideParams& p, hipStream_t st) {
+    return p.ws == kWTiled ? launch_wide_layout<T, kPair, true>(p, st) : launch_wide_layout<T, kPair, false>(p, st);
 }
 
 template <typename T>
@@ -441,7 +446,7 @@ static inline size_t gate_up_lds_bytes(int M, int K, int S) {
     return xb > rb ? xb : rb;
 }
 
-template <typename T>
+template <typename T, bool kTiled>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) void ksa_gemm_gate_up_silu_kernel(const GateUpParams p) {
     using C = KsaCvt<T>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -465,7 +470,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
     u32x4 a[kB];
     auto load_steps = [&](int s0) {
 #pragma unroll
-        for (int u = 0; u < kB; ++u) a[u] = ksa_load_weights(wl.p + wl.step * min(s0 + u, steps - 1));
+        for (int u = 0; u < kB; ++u) a[u] = ksa_load_weights<kTiled>(wl.p + wl.step * min(s0 + u, steps - 1));
     };
     load_steps(slice * kChunkSteps);  // in flight while x is staged (every slice has a first chunk: S <= chunks)
     const int per_row = p.K / 8;
@@ -637,7 +642,10 @@ extern "C" int ksa_gemm_rows_gate_up_silu(const void* x, const void* w, void* ou
     const size_t lds = gate_up_lds_bytes(M, K, p.S);
     if (lds > 160 * 1024) return KSA_ERR_UNSUPPORTED;  // x does not fit LDS whole: M (K + 8) 2 bytes
     const dim3 grid((I + 15) / 16), block(128 * p.S);
-    auto kern = dtype == KSA_DTYPE_BF16 ? ksa_gemm_gate_up_silu_kernel<KsaBf16> : ksa_gemm_gate_up_silu_kernel<KsaF16>;
+    const bool tiled = w_row_stride == kWTiled;
+    auto kern = dtype == KSA_DTYPE_BF16
+                    ? (tiled ? ksa_gemm_gate_up_silu_kernel<KsaBf16, true> : ksa_gemm_gate_up_silu_kernel<KsaBf16, false>)
+                    : (tiled ? ksa_gemm_gate_up_silu_kernel<KsaF16, true> : ksa_gemm_gate_up_silu_kernel<KsaF16, false>);
     if (lds > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

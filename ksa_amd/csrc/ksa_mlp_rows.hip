@@ -95,7 +95,8 @@ __device__ __forceinline__ u32x4 ld_agent_x4_wait(const void* p) {
     return v;
 }
 
-template <typename T>
+// kTiled: both matrices in the streaming layout (what decides how they are loaded)
+template <typename T, bool kTiled>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) void ksa_mlp_rows_kernel(const MlpParams p) {
     using C = KsaCvt<T>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -191,7 +192,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
             if (r < kTileCols) {
 #pragma unroll
                 for (int k = 0; k < kB; ++k)
-                    a[k] = ksa_load_weights(wl.p + wl.step * min(s0 + k, sl_steps - 1));
+                    a[k] = ksa_load_weights<kTiled>(wl.p + wl.step * min(s0 + k, sl_steps - 1));
             }
         };
         load_steps(0);  // in flight while x is waited for and staged
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
     u32x4 ad[kChunkSteps];
     if (live) {  // on their way while the activation is waited for
 #pragma unroll
-        for (int k = 0; k < kChunkSteps; ++k) ad[k] = ksa_load_weights(wl.p + wl.step * min(k, nst - 1));
+        for (int k = 0; k < kChunkSteps; ++k) ad[k] = ksa_load_weights<kTiled>(wl.p + wl.step * min(k, nst - 1));
     }
     unsigned long long launch = 0;  // (thread 0 only) launches before this one
     if (tid == 0) {
@@ -405,7 +406,9 @@ int mlp_rows_launch(const void* x, long long x_row_stride, const float* o_partia
         return KSA_ERR_ALIGN;
     const size_t lds = mlp_lds_bytes(M, H);
     if (lds > 160 * 1024) return KSA_ERR_UNSUPPORTED;
-    auto kern = dtype == KSA_DTYPE_BF16 ? ksa_mlp_rows_kernel<KsaBf16> : ksa_mlp_rows_kernel<KsaF16>;
+    const bool tiled = w_gate_up_row_stride == kWTiled && w_down_row_stride == kWTiled;
+    auto kern = dtype == KSA_DTYPE_BF16 ? (tiled ? ksa_mlp_rows_kernel<KsaBf16, true> : ksa_mlp_rows_kernel<KsaBf16, false>)
+                                        : (tiled ? ksa_mlp_rows_kernel<KsaF16, true> : ksa_mlp_rows_kernel<KsaF16, false>);
     if (lds > 64 * 1024 &&
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)

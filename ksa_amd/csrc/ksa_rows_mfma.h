@@ -51,11 +51,19 @@ __device__ __forceinline__ KsaWeightLane ksa_weight_lane(const uint16_t* w, int6
     return l;
 }
 
-// 16 bytes of a weight matrix, which a step reads once: a non-temporal load (reading 32 / 96 / 144 MiB of
-// memory that is in no cache with 8 such loads per lane in flight takes 6.1 / 15.7 / 22.8 us, 6.7 / 16.4 /
-// 24.0 with plain ones)
+// 16 bytes of a weight matrix.  Streaming layout: a non-temporal load (reading 32 / 96 / 144 MiB of memory that is
+// in no cache with 8 such loads per lane in flight takes 6.1 / 15.7 / 22.8 us, 6.7 / 16.4 / 24.0 with plain ones).
+// Row-major: a plain one, since a fragment takes 64 bytes of a row and the next step's fragment the other half of
+// the 128-byte line, which a non-temporal load does not keep for it: 19456 x 2560 in no cache, 1 / 32 / 72 rows
+// 20.3 / 31.4 / 33.3 us plain, 26.8 / 38.2 / 39.7 non-temporal; the same matrix again and again 15.5 / 24.5 / 27.4 and 22.5 / 36.1 / 37.8.
+// (A streaming copy read again and again, 17 rows and more, is up to 9 % slower than with plain loads - 19456 x 2560, 32
+// rows 21.3 against 19.6 us - and 2 to 8 % faster where it comes from memory, as in a pass through a model's
+// layers: 24.6 against 25.9.)
+template <bool kTiled>
 __device__ __forceinline__ u32x4 ksa_load_weights(const uint16_t* p) {
-    return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    const u32x4* q = reinterpret_cast<const u32x4*>(p);
+    if constexpr (kTiled) return __builtin_nontemporal_load(q);
+    else return *q;
 }
 
 // Zeros in place of the weights of a last chunk's steps from `live` on (they repeat its last step's: with zeros of x
