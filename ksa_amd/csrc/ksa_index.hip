@@ -132,7 +132,7 @@ extern "C" int ksa_block_index(int Sq, int Sk, int C, int S, int W, int P, int s
     if (!mask_cnt || !mask_idx || !full_cnt || !full_idx) return KSA_ERR_NULL;
     const int M = (Sq + tile_m - 1) / tile_m;
     const int N = (Sk + tile_n - 1) / tile_n;
-    KsaMask mk{C, S, W, P, skip_old ? 1 : 0, Sq, Sk};
+    const KsaMask mk = ksa_make_mask(C, S, W, P, skip_old, Sq, Sk);
     hipLaunchKernelGGL(ksa_block_index_kernel, dim3(M), dim3(kIdxThreads), 0, (hipStream_t)stream,
                        mk, tile_m, tile_n, N, mask_cnt, mask_idx, full_cnt, full_idx);
     return ksa_check_launch();

@@ -31,6 +31,14 @@ struct KsaMask {
 KSA_HD int32_t ksa_imax(int32_t a, int32_t b) { return a > b ? a : b; }
 KSA_HD int32_t ksa_imin(int32_t a, int32_t b) { return a < b ? a : b; }
 
+// The mask of a launch.  A chunk (or a run of summary rows) that no row reaches the end of means the same at any
+// length: kept just above the key axis, so that C + S and all positions computed with it stay int32 ("one chunk" is
+// asked for as 2^31 - 1 too).  The bound is a multiple of 8, as the lengths that it may replace often are.
+static inline KsaMask ksa_make_mask(int C, int S, int W, int P, int skip_old, int Sq, int Sk) {
+    const int longest = (Sk + 7) / 8 * 8 + 64;
+    return KsaMask{ksa_imin(C, longest), ksa_imin(S, longest), W, P, skip_old ? 1 : 0, Sq, Sk};
+}
+
 // number of text rows (offset < C) among in-line rows [0, x), x >= 0
 KSA_HD int32_t ksa_text_below(int32_t x, int C, int B) {
     const int32_t r = x % B;

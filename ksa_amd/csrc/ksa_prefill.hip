@@ -1188,12 +1188,13 @@ extern "C" int ksa_prefill_fwd(const void* q, const void* k, const void* v, void
     p.o_bs = out_strides[0], p.o_rs = out_strides[1], p.o_hs = out_strides[2];
     p.lse_bs = (int64_t)Hq * Sq;
     p.lse_hs = Sq;
-    p.mk = KsaMask{C, S, W, P, skip_old ? 1 : 0, Sq, Sk};
+    p.mk = ksa_make_mask(C, S, W, P, skip_old, Sq, Sk);
     p.scale = scale;
     p.scale_log2 = scale * 1.4426950408889634f;
-    p.by_block = FastDiv((uint32_t)(C + S));
-    p.by_S = FastDiv((uint32_t)S);
-    p.phase_shift = (P + C + S - 1) / (C + S) * (C + S);
+    const int block = p.mk.C + p.mk.S;
+    p.by_block = FastDiv((uint32_t)block);
+    p.by_S = FastDiv((uint32_t)p.mk.S);
+    p.phase_shift = (P + block - 1) / block * block;
     p.sched = sched;
     // Workgroup shape (D = 128, even group size; anything else uses one head per workgroup):
     // 2 = two heads on 8 waves; 32 = one head on 4 waves; 64 = two heads on 4 waves with 64 query

@@ -619,3 +619,22 @@ def test_prefill_marked_tiles(Sq, D, shape):
             assert np.isfinite(got).all(), (Sq, D, W)
             assert np.abs(got - want).max() <= ATOL * max(1.0, np.abs(want).max()), (Sq, D, W)
             assert np.abs(to_np(lse[0]) - wlse).max() <= 5e-2, (Sq, D, W)
+
+
+@pytest.mark.parametrize("C", [1 << 30, 2**31 - 9, 2**31 - 1])
+def test_chunk_longer_than_any_sequence(C):
+    """"One chunk" asked for by a huge chunk size, up to where C + S no longer fits 32 bits: index and attention of
+    the shortest chunk that holds every row."""
+    import ksa_amd
+    S, D = 8, 64
+    for Sq, P in ((200, 0), (333, 40), (1000, 130)):
+        for skip_old in (False, True):
+            one = ksa_amd.compute_block_sparsity(Sq, Sq + P, Sq, S, 1, skip_old)
+            huge = ksa_amd.compute_block_sparsity(Sq, Sq + P, C, S, 1, skip_old)
+            assert int(one[0].sum()) > 0 and all(torch.equal(a, b) for a, b in zip(huge, one))
+        q, k, v = (t.bfloat16() for t in make_qkv(Sq + P, 2, 1, D, seed=Sq, scaled=False))
+        q = q[P:]
+        out, lse = ksa_amd.summary_attn_func(q[None].cuda(), k[None].cuda(), v[None].cuda(), C, S, 1, return_lse=True)
+        want, wlse = ksa_amd.summary_attn_func(q[None].cuda(), k[None].cuda(), v[None].cuda(), Sq, S, 1, return_lse=True)
+        assert torch.allclose(out.float(), want.float(), rtol=0, atol=ATOL)
+        assert torch.allclose(lse, wlse, rtol=0, atol=5e-2)
