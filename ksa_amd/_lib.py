@@ -124,12 +124,14 @@ def on_device(device):
 
 def direct(*tensors) -> bool:
     """Whether an operator's kernels may be called without the dispatcher (10 us of host time per call, as much
-    as a small launch takes on the GPU): plain tensors, and nobody compiles, traces, records or transforms.
+    as a small launch takes on the GPU): plain tensors, and nobody compiles, traces, records, profiles (the operator's
+    name belongs into the trace) or transforms.
     (Inside `torch.func` transforms a tensor may be a wrapper of the plain type that has no storage, and a view
     with its negative bit set holds other values than its memory: the dispatcher unwraps the first, slice by
     slice, and writes out the second.)"""
     if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None):
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
+            or torch.autograd._profiler_enabled()):
         return False
     for t in tensors:
         if t is not None and (type(t) is not torch.Tensor or (t.requires_grad and torch.is_grad_enabled())

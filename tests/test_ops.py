@@ -221,6 +221,17 @@ def test_direct_calls_step_aside_for_transforms_and_negative_views():
     assert neg.is_neg() and not _lib.direct(neg)
 
 
+def test_direct_calls_step_aside_for_profilers():
+    """Operators are seen by name in a profiler's trace."""
+    from ksa_amd import _lib
+    x = torch.randn(2, 3)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        assert not _lib.direct(x)
+    with torch.autograd.profiler.profile():
+        assert not _lib.direct(x)
+    assert _lib.direct(x)
+
+
 @pytest.mark.gpu
 def test_prefill_under_vmap():
     """Attention calls inside `torch.func.vmap` equal one call per slice."""
