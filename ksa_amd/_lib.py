@@ -128,13 +128,14 @@ def direct(*tensors) -> bool:
     name belongs into the trace) or transforms.
     (Inside `torch.func` transforms a tensor may be a wrapper of the plain type that has no storage, and a view
     with its negative bit set holds other values than its memory: the dispatcher unwraps the first, slice by
-    slice, and writes out the second.)"""
+    slice, and writes out the second.  It does the same for wrappers and all-zero tensors without memory that are met
+    outside of a transform.)"""
     if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
             or torch.autograd._profiler_enabled()):
         return False
     for t in tensors:
         if t is not None and (type(t) is not torch.Tensor or (t.requires_grad and torch.is_grad_enabled())
-                              or t.is_neg()):
+                              or t.is_neg() or t._is_zerotensor() or torch._is_functional_tensor(t)):
             return False
     return True

@@ -232,6 +232,15 @@ def test_direct_calls_step_aside_for_profilers():
     assert _lib.direct(x)
 
 
+def test_direct_calls_step_aside_for_tensors_without_memory():
+    """Wrappers and zero tensors have the plain type and no memory that a kernel could be given."""
+    from ksa_amd import _lib
+    x = torch.randn(2, 3)
+    assert not _lib.direct(torch._to_functional_tensor(x))
+    assert not _lib.direct(x, torch._efficientzerotensor((2, 3)))
+    assert _lib.direct(x, x)
+
+
 @pytest.mark.gpu
 def test_prefill_under_vmap():
     """Attention calls inside `torch.func.vmap` equal one call per slice."""
