@@ -111,7 +111,7 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
         out = torch.ops.ksa_amd.decode_fwd(pad_head_dim(q, Dk), kcache, vcache, t_start, t_end, s0, e0,
                                            float(scale), int(nsplit))
         return out[..., :D].contiguous()
-    forward = _launch_decode if _lib.direct(q, kcache, vcache) else torch.ops.ksa_amd.decode_fwd
+    forward = _launch_decode if _lib.direct(q, kcache, vcache, t_start, t_end) else torch.ops.ksa_amd.decode_fwd
     return forward(q, kcache, vcache, t_start, t_end, s0, e0, float(scale), int(nsplit))
 
 

@@ -242,6 +242,27 @@ def test_direct_calls_step_aside_for_tensors_without_memory():
 
 
 @pytest.mark.gpu
+def test_decode_row_ranges_that_are_wrappers():
+    """A row range of a subclass reaches the operator like the other inputs."""
+    import ksa_amd
+
+    class Ranges(torch.Tensor):
+        names = []
+
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            Ranges.names.append(str(func))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    q = torch.randn(2, 4, 1, 64, device="cuda", dtype=torch.bfloat16)
+    k, v = (torch.randn(2, 2, 300, 64, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    lo, hi = (torch.full((2,), n, dtype=torch.int32, device="cuda") for n in (3, 290))
+    got = ksa_amd.ksa_decode(q, k, v, lo.as_subclass(Ranges), hi)
+    assert any("decode_fwd" in n for n in Ranges.names)
+    assert torch.equal(got.as_subclass(torch.Tensor), ksa_amd.ksa_decode(q, k, v, lo, hi))
+
+
+@pytest.mark.gpu
 def test_prefill_under_vmap():
     """Attention calls inside `torch.func.vmap` equal one call per slice."""
     import ksa_amd
