@@ -4,6 +4,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import os
 
 import torch  # noqa: F401  (must be imported first so that its HIP runtime is the one in the process)
@@ -108,9 +109,27 @@ def strides3(t, dims):
     return _I64x3(s[dims[0]], s[dims[1]], s[dims[2]])
 
 
+def _private(*names):
+    """These private functions of torch, or None where one of them is missing: its next release may have renamed it,
+    and a CPU-only build has no `_cuda_*`.  What uses them then takes the public way."""
+    try:
+        return [functools.reduce(getattr, n.split("."), torch) for n in names]
+    except AttributeError:
+        return None
+
+
+_GPU = _private("_C._cuda_getDevice", "_C._cuda_getCurrentRawStream")
+# each false or None where nobody records, traces or transforms
+_WATCHERS = _private("_C._len_torch_dispatch_stack", "_C._len_torch_function_stack",
+                     "_C._functorch.peek_interpreter_stack", "_C._get_tracing_state", "autograd._profiler_enabled")
+_MEMORYLESS = _private("Tensor._is_zerotensor", "_is_functional_tensor")
+
+
 def stream_ptr(device) -> int:
     """Handle of the current stream of a GPU (asked for at every call: 0.1 us where a Stream object takes 1.5)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if device.index is None else device.index)
+    if _GPU is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _GPU[1](_GPU[0]() if device.index is None else device.index)
 
 
 _HERE_ALREADY = contextlib.nullcontext()
@@ -119,7 +138,9 @@ _HERE_ALREADY = contextlib.nullcontext()
 def on_device(device):
     """Context in which `device` is the current GPU; nothing to enter (and 2 us of host time less) where it
     is that already."""
-    return _HERE_ALREADY if device.index in (None, torch._C._cuda_getDevice()) else torch.cuda.device(device)
+    if device.index is None or (_GPU is not None and device.index == _GPU[0]()):
+        return _HERE_ALREADY
+    return torch.cuda.device(device)
 
 
 def direct(*tensors) -> bool:
@@ -130,12 +151,14 @@ def direct(*tensors) -> bool:
     with its negative bit set holds other values than its memory: the dispatcher unwraps the first, slice by
     slice, and writes out the second.  It does the same for wrappers and all-zero tensors without memory that are met
     outside of a transform.)"""
-    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._get_tracing_state() is not None
-            or torch.autograd._profiler_enabled()):
+    if _WATCHERS is None or _MEMORYLESS is None or torch.compiler.is_compiling():
         return False
+    for watcher in _WATCHERS:
+        if watcher():        # (the interpreter of a transform is an object, true like any)
+            return False
+    zero, wrapper = _MEMORYLESS
     for t in tensors:
         if t is not None and (type(t) is not torch.Tensor or (t.requires_grad and torch.is_grad_enabled())
-                              or t.is_neg() or t._is_zerotensor() or torch._is_functional_tensor(t)):
+                              or t.is_neg() or zero(t) or wrapper(t)):
             return False
     return True

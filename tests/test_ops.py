@@ -241,6 +241,37 @@ def test_direct_calls_step_aside_for_tensors_without_memory():
     assert _lib.direct(x, x)
 
 
+def test_calls_without_torchs_private_functions(monkeypatch):
+    """Where torch lacks one of the private functions in use, every call takes the dispatcher."""
+    from ksa_amd import _lib
+    x = torch.randn(2, 3)
+    assert _lib.direct(x)
+    with monkeypatch.context() as m:
+        m.delattr(torch._C, "_len_torch_function_stack")
+        assert _lib._private("_C._len_torch_dispatch_stack", "_C._len_torch_function_stack") is None
+        m.setattr(_lib, "_WATCHERS", None)
+        assert not _lib.direct(x)
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "_MEMORYLESS", None)
+        assert not _lib.direct(x)
+    assert _lib.direct(x)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("known", [True, False])
+def test_stream_and_device_without_torchs_private_functions(monkeypatch, known):
+    """The handle of the current stream, and no device to change to, with and without the private functions."""
+    from ksa_amd import _lib
+    if not known:
+        monkeypatch.setattr(_lib, "_GPU", None)
+    for s in (torch.cuda.current_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(s):
+            for device in (torch.device("cuda"), torch.device("cuda", 0)):
+                assert _lib.stream_ptr(device) == s.cuda_stream
+                with _lib.on_device(device):
+                    assert torch.cuda.current_device() == 0
+
+
 @pytest.mark.gpu
 def test_decode_row_ranges_that_are_wrappers():
     """A row range of a subclass reaches the operator like the other inputs."""
