@@ -122,7 +122,6 @@ _GPU = _private("_C._cuda_getDevice", "_C._cuda_getCurrentRawStream")
 # each false or None where nobody records, traces or transforms
 _WATCHERS = _private("_C._len_torch_dispatch_stack", "_C._len_torch_function_stack",
                      "_C._functorch.peek_interpreter_stack", "_C._get_tracing_state", "autograd._profiler_enabled")
-_MEMORYLESS = _private("Tensor._is_zerotensor", "_is_functional_tensor")
 
 
 def stream_ptr(device) -> int:
@@ -151,14 +150,13 @@ def direct(*tensors) -> bool:
     with its negative bit set holds other values than its memory: the dispatcher unwraps the first, slice by
     slice, and writes out the second.  It does the same for wrappers and all-zero tensors without memory that are met
     outside of a transform.)"""
-    if _WATCHERS is None or _MEMORYLESS is None or torch.compiler.is_compiling():
+    if _WATCHERS is None or torch.compiler.is_compiling():
         return False
-    for watcher in _WATCHERS:
-        if watcher():        # (the interpreter of a transform is an object, true like any)
-            return False
-    zero, wrapper = _MEMORYLESS
+    modes, functions, transform, trace, profiler = _WATCHERS
+    if modes() or functions() or transform() is not None or trace() is not None or profiler():
+        return False
     for t in tensors:
         if t is not None and (type(t) is not torch.Tensor or (t.requires_grad and torch.is_grad_enabled())
-                              or t.is_neg() or zero(t) or wrapper(t)):
+                              or t.is_neg() or not t.data_ptr()):
             return False
     return True

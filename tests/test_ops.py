@@ -251,9 +251,6 @@ def test_calls_without_torchs_private_functions(monkeypatch):
         assert _lib._private("_C._len_torch_dispatch_stack", "_C._len_torch_function_stack") is None
         m.setattr(_lib, "_WATCHERS", None)
         assert not _lib.direct(x)
-    with monkeypatch.context() as m:
-        m.setattr(_lib, "_MEMORYLESS", None)
-        assert not _lib.direct(x)
     assert _lib.direct(x)
 
 
