@@ -102,7 +102,7 @@ int ksa_prefill_fwd(const void* q, const void* k, const void* v, void* out, floa
  *   rows attended for sequence b: [start[b], end[b]) if start/end (device int32[batch])
  *   are given, else [start0, end0) for every sequence.  No mask, no causality.
  *   nsplit >= 1 splits of the row range; nsplit > 1 needs a workspace of
- *   ksa_decode_workspace_bytes(...) bytes (fp32 partials). */
+ *   ksa_decode_workspace_bytes(...) bytes (fp32 partials), on any 4-byte border. */
 size_t ksa_decode_workspace_bytes(int batch, int Hq, int Hkv, int Q, int D, int nsplit);
 int ksa_decode_auto_splits(int batch, int Hkv, int max_rows);
 /* The split count for Q query tokens of Hq heads of head_dim D (faster than ksa_decode_auto_splits on few rows, with a larger

@@ -93,7 +93,9 @@ __device__ __forceinline__ int ksa_decode_slot(const DecodeParams& p, int qi, in
 }
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
+// the same as the caller's workspace holds them: on any 4-byte border (still one wide load each)
+typedef float floatx4_ws __attribute__((ext_vector_type(4), aligned(4)));
+typedef float floatx2_ws __attribute__((ext_vector_type(2), aligned(4)));
 
 constexpr int kThreads = 256;
 constexpr int kWaves = 4;
@@ -438,12 +440,12 @@ __global__ __launch_bounds__(kMergeThreads) void ksa_decode_merge_kernel(const D
     float mx = -INFINITY, l = 0.f;
     for (int s0 = grp; s0 < p.nsplit; s0 += kBatch * G) {
         floatx4 o[kBatch];
-        floatx2 ml[kBatch];
+        floatx2_ws ml[kBatch];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
             const int64_t slot = base + (int64_t)min(s0 + u * G, p.nsplit - 1) * p.ncols_pad;
-            ml[u] = *reinterpret_cast<const floatx2*>(p.ws_ml + slot * 2);
-            o[u] = *reinterpret_cast<const floatx4*>(p.ws_o + slot * D + d4);
+            ml[u] = *reinterpret_cast<const floatx2_ws*>(p.ws_ml + slot * 2);
+            o[u] = *reinterpret_cast<const floatx4_ws*>(p.ws_o + slot * D + d4);
         }
         float m_new = mx;
 #pragma unroll

@@ -333,3 +333,23 @@ def test_decode_qkv_equals_separate_launches(dtype, b, Hq, Hkv, D, rows, start, 
         got = decode.ksa_decode_qkv(qkv, qw, kw, cos, sin, 1e-6, kc, vc, Hq, r, lo, hi, nsplit=nsplit)
         assert torch.equal(got, want.reshape(b, 1, Hq * D)) and torch.isfinite(got.float()).all()
         assert torch.equal(kc, kr) and torch.equal(vc, vr)
+
+
+@pytest.mark.parametrize("D,nsplit", [(128, 5), (64, 3), (256, 4)])
+def test_decode_workspace_on_a_four_byte_border(D, nsplit):
+    """A caller of the C entry may put the fp32 workspace anywhere floats go."""
+    import ctypes
+    import ksa_amd
+    from ksa_amd import _lib
+    q, k, v = (t.cuda() for t in _mk(2, 8, 2, 1, D, 700, seed=D))
+    want = ksa_amd.ksa_decode(q, k, v, 3, 690, nsplit=nsplit)
+    L = _lib.lib()
+    need = L.ksa_decode_workspace_bytes(2, 8, 2, 1, D, nsplit)
+    for shift in (4, 8, 12):
+        ws = torch.full((need + 16,), 0xff, dtype=torch.uint8, device="cuda")
+        out = torch.empty_like(want)
+        strides = [(ctypes.c_int64 * 3)(*t.stride()[:3]) for t in (q, k, v, out)]
+        rc = L.ksa_decode_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), None, None, 3, 690, 2, 8, 2, 1, D, 0,
+                              *strides, D ** -0.5, nsplit, ws.data_ptr() + shift, need, _lib.stream_ptr(q.device))
+        assert rc == 0 and torch.equal(out, want)
+        assert (ws[:shift] == 0xff).all() and (ws[shift + need:] == 0xff).all()
