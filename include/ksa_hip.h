@@ -314,7 +314,8 @@ int ksa_silu_mul_partials(const float* partials, int ksplit, void* out, int rows
  * KSA_ERR_INVALID.  With ksplit > 1 out may be NULL: the partial sums (fp32 [ksplit][R][N], R = M
  * rounded up to a multiple of 16) are then left in the workspace for a consumer that adds them itself
  * (ksa_add_rmsnorm_partials, ksa_silu_mul_partials, ksa_pre_attention_partials).  x and w 16-byte
- * aligned, for M > 16 the workspace as well (KSA_ERR_ALIGN otherwise). */
+ * aligned, for M > 16 the workspace as well (KSA_ERR_ALIGN otherwise); for M <= 16 it may lie on any 4-byte border
+ * (but the calls that take partial sums over want them 16-byte aligned). */
 /* The streaming layout of a weight matrix.  The few-rows kernels read a weight fragment of 16 rows x 32
  * elements of K per wave instruction - in a row-major w [N, K] that is 64 bytes of each of 16 rows K elements
  * apart.  ksa_tile_weights writes the same matrix as [ceil(N / 16)][K / 32][16][32] (rows past N: zeros;

@@ -138,7 +138,8 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
         } else {
             float* dst = p.part + ((int64_t)blockIdx.y * 16 + r) * p.N + n;
             if (p.N % 4 == 0) {
-                *reinterpret_cast<f32x4*>(dst) = acc;
+                typedef float f32x4_ws __attribute__((ext_vector_type(4), aligned(4)));  // (workspace on any 4-byte border)
+                *reinterpret_cast<f32x4_ws*>(dst) = acc;
             } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)

@@ -374,3 +374,29 @@ def test_gpu_linear_rows_infinite_weight_in_the_last_step(dtype, M, K):
         want = linear_rows(x, wrap(w))
         want[:, 5] = x[:, K - 3] * float("inf")
         assert torch.equal(linear_rows(x, wrap(bad)), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [64, 100, 101])
+@pytest.mark.parametrize("M", [1, 7, 16])
+def test_gpu_gemm_rows_workspace_on_a_four_byte_border(M, N):
+    """Up to 16 rows a caller of the C entry may put the partial sums anywhere floats go."""
+    from ksa_amd import _lib
+    g = torch.Generator().manual_seed(M + N)
+    K, ks = 1536, 3
+    x, w = (torch.randn(n, K, generator=g).bfloat16().cuda() for n in (M, N))
+    L = _lib.lib()
+    need = L.ksa_gemm_rows_partials_bytes(M, N, ks)
+    outs = []
+    for shift in (0, 4, 8, 12):
+        ws = torch.full((need + 16,), 0xff, dtype=torch.uint8, device="cuda")
+        out = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+        rc = L.ksa_gemm_rows(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, K, K, N, 0, ks, ws.data_ptr() + shift, need,
+                             _lib.stream_ptr(x.device))
+        assert rc == 0
+        assert (ws[:shift] == 0xff).all() and (ws[shift + need:] == 0xff).all()
+        outs.append(out)
+    # sums of K products of size ~1 rounded to bf16: 2^-8 of the value, and fp32's own error far below it
+    want = x.double().cpu() @ w.double().cpu().t()
+    assert all(torch.equal(o, outs[0]) for o in outs)
+    assert ((outs[0].double().cpu() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all()
