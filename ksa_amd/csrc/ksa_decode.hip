@@ -416,9 +416,9 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
 }
 
 // Second stage: merge the splits of one (sequence, kv head, column).  A chain of memory trips, nothing else, so
-// there is one: D / 4 threads take four elements each, the G such groups of a workgroup every G-th split, and a
-// group requests up to eight splits (64 in all at head_dim 128) with their maxima and sums at once; the groups
-// meet in LDS.  (A thread per element that walked the splits eight at a time, maxima first, took 2 to 16 trips:
+// there are few: D / 4 threads take four elements each, the G such groups of a workgroup every G-th split, and a
+// group requests up to eight splits with their maxima and sums at once - one trip for 128 / 64 / 32 splits at
+// head_dim 64 / 128 / 256, another for as many more; the groups meet in LDS.  (A thread per element that walked the splits eight at a time, maxima first, took 2 to 16 trips:
 // decode + merge of one sequence of 16384 rows in
 // 64 splits 29.8 -> 19.4 us, 4096 rows in 16 13.4 -> 12.0.)
 constexpr int kMergeThreads = 256;

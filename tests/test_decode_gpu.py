@@ -293,7 +293,7 @@ def test_decode_boundary_equals_two_decodes(D, dtype, g, nsplit):
 @pytest.mark.parametrize("b,Hq,Hkv,D,rows,start,end,row,nsplit", [
     (1, 32, 8, 128, 700, 3, 690, 3, None),        # first row of the range (a small window)
     (1, 32, 8, 128, 700, 0, 700, 699, 12),        # last row (a large window), splits without rows
-    (1, 32, 8, 128, 5000, 0, 4999, 2500, 64),     # more splits than are requested at once
+    (1, 32, 8, 128, 5000, 0, 4999, 2500, 64),     # most splits; 40 of them have rows
     (2, 8, 8, 128, 300, 10, 299, 138, 2),         # one query head per kv head; last row of a workgroup's round
     (3, 15, 3, 128, 300, 0, 129, 128, 2),         # group of 5; a slice of one row, the new one
     (4, 32, 1, 128, 260, 1, 258, 33, 3),          # group of 32: several passes over the query rows
@@ -333,6 +333,59 @@ def test_decode_qkv_equals_separate_launches(dtype, b, Hq, Hkv, D, rows, start, 
         got = decode.ksa_decode_qkv(qkv, qw, kw, cos, sin, 1e-6, kc, vc, Hq, r, lo, hi, nsplit=nsplit)
         assert torch.equal(got, want.reshape(b, 1, Hq * D)) and torch.isfinite(got.float()).all()
         assert torch.equal(kc, kr) and torch.equal(vc, vr)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,Hq,Hkv,D", [(5, 32, 8, 128), (6, 8, 4, 64), (17, 4, 2, 128)])
+@pytest.mark.parametrize("nsplit", [1, 4, None])
+def test_decode_qkv_with_a_range_row_and_position_per_sequence(dtype, b, Hq, Hkv, D, nsplit):
+    """Every sequence with its own range, new row and rotary row: the new row first, last, in between and at the
+    borders of a workgroup's rounds, long sequences next to ones of few rows (whose later splits are empty).
+    Bit for bit the separate launches, and within the usual bound of the oracle."""
+    import ksa_amd
+    from ksa_amd import decode, gemm, pre
+    rows = 1100
+    g = torch.Generator(device="cuda").manual_seed(b * 10 + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    forms = [(0, 1100, 1099), (7, 1031, 7), (3, 40, 20), (128, 129, 128), (0, 300, 127), (5, 645, 133), (90, 1000, 511)]
+    lo, hi, row = (np.array([forms[i % len(forms)][j] for i in range(b)], np.int32) for j in range(3))
+    dev = lambda a: torch.as_tensor(a, device="cuda")
+    H, width = 1536, (Hq + 2 * Hkv) * D
+    h, w = rnd(b, 1, H).to(dtype), (rnd(width, H) * H ** -0.5).to(dtype)
+    qw, kw = (1 + 0.1 * rnd(D)).to(dtype), (1 + 0.1 * rnd(D)).to(dtype)
+    ang = rnd(b, 1, D // 2)
+    ang = torch.cat((ang, ang), -1)
+    cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+    qkv = gemm.linear_rows(h, w, defer=True)
+    kc, vc = (rnd(b, Hkv, rows, D).to(dtype) for _ in range(2))
+    for i in range(b):                             # what the new rows overwrite must not be read
+        kc[i, :, row[i]] = vc[i, :, row[i]] = float("nan")
+    kr, vr = kc.clone(), vc.clone()
+    q, _, _ = pre.pre_attention_partials(qkv, Hq, Hkv, D, qw, kw, cos, sin, 1e-6, k_out=kr[:, :, :1].transpose(1, 2),
+                                         v_out=vr[:, :, :1].transpose(1, 2), kv_out_row=dev(row))
+    want = ksa_amd.ksa_decode(q.transpose(1, 2), kr, vr, dev(lo), dev(hi), nsplit=nsplit)
+    got = decode.ksa_decode_qkv(qkv, qw, kw, cos, sin, 1e-6, kc, vc, Hq, dev(row), dev(lo), dev(hi), nsplit=nsplit)
+    assert torch.equal(got, want.reshape(b, 1, Hq * D))
+    assert torch.equal(kc, kr) and torch.equal(vc, vr)
+    ref = c_oracle.decode(to_np(q.transpose(1, 2)), to_np(kr), to_np(vr), lo, hi)
+    assert np.abs(to_np(got).reshape(ref.shape) - ref).max() <= ATOL * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("Hkv,D,nsplit", [(2, 256, None), (4, 256, 64), (2, 256, 33), (1, 128, 100), (1, 64, 150)])
+def test_decode_merge_of_more_splits_than_one_pass_takes(Hkv, D, nsplit):
+    """The merge walks more than 32 splits at head_dim 256 (64 at 128, 128 at 64) in several passes.  Scores that
+    grow along the rows move the maximum in each of them; falling ones leave it in the first; a sequence of few
+    rows leaves all but the first splits empty."""
+    from ksa_amd import _lib
+    b, rows = 3, 64 * 300
+    if nsplit is None:
+        assert _lib.lib().ksa_decode_splits(b, 2 * Hkv, Hkv, 1, D, rows) > 32
+    q, k, v = _mk(b, 2 * Hkv, Hkv, 1, D, rows, seed=D + Hkv)
+    ramp = torch.linspace(0.1, 4.0, rows)[:, None]
+    k[0], k[1] = (k[0].float() * ramp).bfloat16(), (k[1].float() * ramp.flip(0)).bfloat16()
+    _check(q, k, v, np.array([0, 0, 11], np.int32), np.array([rows, rows - 3, 300], np.int32), nsplit)
+    _check(q[:1], k[:1], v[:1], 0, rows, nsplit)
 
 
 @pytest.mark.parametrize("D,nsplit", [(128, 5), (64, 3), (256, 4)])

@@ -177,6 +177,28 @@ def test_gpu_embed_rmsnorm_equals_separate_launches(dtype, rows, H, vocab, D):
         assert torch.equal(x, s) and torch.equal(h, n) and torch.equal(r[0], rope[at])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gpu_embed_rmsnorm_ids_outside_the_table(dtype):
+    """An id outside the table gives a row of NaN, normalised or not, and leaves the other rows alone; a rotary row
+    outside of its table is the nearest one of it."""
+    from ksa_amd.elementwise import add_rmsnorm, embed_rmsnorm
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
+    vocab, H, D = 50, 2560, 128
+    table, w, rope = rnd(vocab, H), rnd(H), rnd(70, 2, D)
+    ids = torch.tensor([[3], [vocab], [-vocab - 1], [49], [2**40], [-2**62], [-50]], device="cuda")
+    bad = torch.tensor([False, True, True, False, True, True, False])
+    for at, row in ((70, 69), (2**31 - 1, 69), (-1, 0)):
+        x, h, r = (torch.full(s, 7.0, dtype=dtype, device="cuda") for s in ((7, 1, H), (7, 1, H), (1, 2, D)))
+        embed_rmsnorm(table, ids, w, 1e-6, rope, torch.tensor([at], dtype=torch.int32, device="cuda"), x, h, r)
+        assert torch.equal(r[0], rope[row])
+        for t in (x, h):
+            assert t[bad].isnan().all() and t[~bad].isfinite().all()
+        s, n = add_rmsnorm(table[ids[~bad]], None, w, 1e-6)
+        assert torch.equal(x[~bad], s) and torch.equal(h[~bad], n)
+
+
 def test_embed_rmsnorm_argument_checks():
     """What the head-of-step kernel does not take is refused on the host."""
     from ksa_amd import _lib

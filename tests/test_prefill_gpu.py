@@ -621,6 +621,45 @@ def test_prefill_marked_tiles(Sq, D, shape):
             assert np.abs(to_np(lse[0]) - wlse).max() <= 5e-2, (Sq, D, W)
 
 
+@pytest.mark.parametrize("C", [128, 1024])
+@pytest.mark.parametrize("mode", ["prefix", "inline", "physical"])
+@pytest.mark.parametrize("D, shape", [(128, 32), (128, 2), (64, 0), (256, 0)])
+def test_prefill_marked_tiles_of_long_lists(D, shape, mode, C):
+    """Marked tiles behind lists of more tiles than are held at once: windows over everything (up to 160 tiles
+    of either list) and over four chunks (in-line mode: over 128 partial ones), the prefix and the key axis cut
+    inside a tile.  Two rows of every row tile, so that the marked tiles come at every place of the walk, and
+    all of the last tile's.  The second input makes summary rows walk again with exact references."""
+    import ksa_amd
+    dev = torch.device("cuda")
+    S, Sq = 8, 9997 if mode == "prefix" else 9341
+    rng = np.random.default_rng(D + shape + C)
+    rows = np.concatenate([i + rng.choice(min(128, Sq - i), 2, replace=False) for i in range(0, Sq, 128)] + [np.arange(Sq - 60, Sq)])
+    sp = O.summary_positions(Sq, C, S)
+    rows = np.unique(np.concatenate([rows, np.nonzero(sp)[0][::37]])).astype(np.int32)
+    P = int(sp.sum())
+    assert (P % 64 != 0 or mode == "inline") and (Sq % 64 != 0) and (Sq + P) % 64 != 0
+    for peaked in (False, True):
+        q, k, v = make_qkv(Sq, 2, 1, D, seed=D + C, scaled=False)
+        if peaked:
+            boost = torch.ones(Sq)
+            boost[torch.as_tensor(sp)] = 40.0
+            k = (k.float() * boost[:, None, None]).bfloat16()
+        kk, vv, spt, osp = k, v, torch.as_tensor(sp, device=dev), sp
+        if mode == "inline":
+            spt, osp = None, None
+        elif mode == "physical":
+            st = torch.as_tensor(sp)
+            kk, vv, spt = torch.cat([k[st], k]), torch.cat([v[st], v]), None
+        for W in (4, 1 << 20):
+            out, lse = ksa_amd.summary_attn_func(q[None].to(dev), kk[None].to(dev), vv[None].to(dev), C, S, W, summary_pos=spt,
+                                                 return_lse=True, workgroup_shape=shape)
+            got, glse = to_np(out[0]), to_np(lse[0])
+            want, wlse = c_oracle.attention_rows(to_np(q), to_np(k), to_np(v), C, S, W, summary_pos=osp, rows=rows)
+            assert np.isfinite(got).all() and np.isfinite(glse).all(), (peaked, W)
+            assert np.abs(got[rows] - want).max() <= ATOL * max(1.0, np.abs(want).max()), (peaked, W)
+            assert np.abs(glse[:, rows] - wlse).max() <= 0.1 + 1e-3 * np.abs(wlse).max(), (peaked, W)
+
+
 @pytest.mark.parametrize("C", [1 << 30, 2**31 - 9, 2**31 - 1])
 def test_chunk_longer_than_any_sequence(C):
     """"One chunk" asked for by a huge chunk size, up to where C + S no longer fits 32 bits: index and attention of
