@@ -116,7 +116,10 @@ __global__ __launch_bounds__(256) void ksa_add_rmsnorm_kernel(const NormParams p
 // kBatch: slices requested together; every further batch is another trip to memory, which is what this kernel's time
 // is.  Twenty take the 19 slices of the 4B shape's down projection in one trip (184 registers, no matter with
 // one workgroup per row) where eight take three: decode step of 8 layers 643.1 -> 640.0 us (batch 1), 752.6 -> 750.1
-// (batch 8).  Up to eight slices, and rows of two items per thread, keep the batch of eight.
+// (batch 8).  That pays where three trips become one and a workgroup is small: 17 to 20 slices of up to 2560 elements
+// (1 row of 1024 / 2560, 19 slices 3.92 / 5.40 -> 3.77 / 5.30 us; 3584 6.08 -> 6.33, so not there).  Elsewhere the
+// requests past the last slice cost more than the trips (9 / 16 / 24 slices of 2560 4.0 / 4.3 / 5.7 -> 4.7 / 4.9 / 7.3
+// us, of 4096 4.3 / 5.2 / 6.3 -> 5.4 / 6.3 / 9.3): eight.
 template <typename T, int NJ, int kBatch>
 __global__ __launch_bounds__(512) void ksa_add_rmsnorm_partials_kernel(const NormParams p) {
     using C = KsaCvt<T>;
@@ -177,7 +180,7 @@ int dispatch_norm_partials(const NormParams& p, hipStream_t st) {
     const int threads = items >= 512 ? 512 : (items + 63) / 64 * 64;
     const int need = (items + threads - 1) / threads;
     const dim3 grid((unsigned)p.rows), block(threads);
-    if (need <= 1 && p.ksplit > 8) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 1, 20>), grid, block, 0, st, p);
+    if (items <= 320 && p.ksplit > 16 && p.ksplit <= 20) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 1, 20>), grid, block, 0, st, p);
     else if (need <= 1) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 1, 8>), grid, block, 0, st, p);
     else if (need <= 2) hipLaunchKernelGGL((ksa_add_rmsnorm_partials_kernel<T, 2, 8>), grid, block, 0, st, p);
     else return KSA_ERR_UNSUPPORTED;
