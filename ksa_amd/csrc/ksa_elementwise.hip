@@ -9,6 +9,8 @@
 // is bound by the number of launches.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "ksa_api_internal.h"
 #include "ksa_cvt.h"
 
@@ -26,8 +28,10 @@ struct NormParams {
     int64_t xs, rs, ns, ss;  // row strides (elements)
     int H;
     float eps;
-    // kEmbed: row r of x is row ids[r] of a table of x_rows rows; the row behind the last one copies row *rope_row
-    // of a second table
+};
+// kEmbed: row r of x is row ids[r] of a table of x_rows rows; the row behind the last one copies row *rope_row of a
+// second table.  (Parameters of their own: the other launches would carry them along, 1 % of a few-rows norm.)
+struct EmbedParams : NormParams {
     const long long* ids;
     int64_t x_rows;
     const uint16_t* rope;  // [rope_rows][rope_width]
@@ -43,7 +47,7 @@ struct NormParams {
 // cost is its launches (4.5 us each behind one another, for some 10 KB): as one, and with the ids read where the
 // caller has them, a decode step of 8 layers went from 649 to 643 us (batch 1) and from 759 to 754 (batch 8).
 template <typename T, int NI, bool kEmbed = false>
-__global__ __launch_bounds__(256) void ksa_add_rmsnorm_kernel(const NormParams p) {
+__global__ __launch_bounds__(256) void ksa_add_rmsnorm_kernel(const std::conditional_t<kEmbed, EmbedParams, NormParams> p) {
     using C = KsaCvt<T>;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -59,12 +63,13 @@ __global__ __launch_bounds__(256) void ksa_add_rmsnorm_kernel(const NormParams p
         u32x4 r[NI];
         float ss = 0.f;
         int64_t src = row;
+        bool inside = true;
         if constexpr (kEmbed) {  // (a negative id counts from the end; one outside the table gives a row of NaN)
             src = p.ids[row];
             if (src < 0) src += p.x_rows;
+            inside = src >= 0 && src < p.x_rows;
+            if (!inside) src = 0;
         }
-        const bool inside = !kEmbed || (src >= 0 && src < p.x_rows);
-        if (!inside) src = 0;
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
             const int idx = lane + 64 * j;
@@ -189,10 +194,6 @@ int dispatch_norm_partials(const NormParams& p, hipStream_t st) {
 
 template <typename T, int NI>
 int launch_norm(const NormParams& p, hipStream_t st) {
-    if (p.ids) {
-        hipLaunchKernelGGL((ksa_add_rmsnorm_kernel<T, NI, true>), dim3((unsigned)((p.rows + 1 + 3) / 4)), dim3(256), 0, st, p);
-        return ksa_check_launch();
-    }
     const int64_t blocks = (p.rows + 3) / 4;
     // one short-lived workgroup per four rows (measured 5 % faster than a capped grid with a
     // grid-stride loop); the loop only serves row counts beyond the grid limit
@@ -201,9 +202,14 @@ int launch_norm(const NormParams& p, hipStream_t st) {
                        st, p);
     return ksa_check_launch();
 }
+template <typename T, int NI>
+int launch_norm(const EmbedParams& p, hipStream_t st) {
+    hipLaunchKernelGGL((ksa_add_rmsnorm_kernel<T, NI, true>), dim3((unsigned)((p.rows + 1 + 3) / 4)), dim3(256), 0, st, p);
+    return ksa_check_launch();
+}
 
-template <typename T>
-int dispatch_norm(const NormParams& p, hipStream_t st) {
+template <typename T, typename P>
+int dispatch_norm(const P& p, hipStream_t st) {
     const int need = (p.H / 8 + 63) / 64;
     if (need <= 1) return launch_norm<T, 1>(p, st);
     if (need <= 2) return launch_norm<T, 2>(p, st);
@@ -389,7 +395,7 @@ extern "C" int ksa_embed_rmsnorm(const void* table, long long table_rows, long l
     if (!al16(table) || !al16(weight) || !al16(out) || !al16(out_norm) || !al16(rope_table) || !al16(rope_out) ||
         table_row_stride % 8)
         return KSA_ERR_ALIGN;
-    NormParams p{};
+    EmbedParams p{};
     p.x = (const uint16_t*)table, p.x_rows = table_rows, p.xs = table_row_stride;
     p.ids = ids;
     p.w = (const uint16_t*)weight;
