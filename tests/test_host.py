@@ -343,3 +343,34 @@ def test_decode_qkv_argument_checks():
     call = lambda **kw: L.ksa_decode_qkv_fwd(*{**base, **kw}.values())
     assert call(qkv=None) != 0 and call(d=256) != 0 and call(row0=10) != 0 and call(row0=-1) != 0 and call(e0=0) != 0
     assert call(hq=5) != 0 and call(ns=2) != 0 and call(out=None) != 0 and call(kc=8) != 0 and call(b=129) != 0
+
+
+def _kernel_metadata(path):
+    """name -> metadata of every kernel in the code objects that a library carries."""
+    import msgpack
+    import struct
+    blob, magic, kernels = open(path, "rb").read(), b"__CLANG_OFFLOAD_BUNDLE__", {}
+    at = blob.find(magic)
+    while at >= 0:
+        pos = at + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", blob, at + len(magic))[0]):
+            off, size, n = struct.unpack_from("<QQQ", blob, pos)
+            target, pos = blob[pos + 24: pos + 24 + n], pos + 24 + n
+            elf = blob[at + off: at + off + size]
+            note = elf.find(b"AMDGPU\0\0")        # name of the note: name size, description size, type, name, description
+            if b"amdgcn" in target and note >= 12:
+                desc = elf[note + 8: note + 8 + struct.unpack_from("<I", elf, note - 8)[0]]
+                kernels.update({k[".name"]: k for k in msgpack.unpackb(desc)["amdhsa.kernels"]})
+        at = blob.find(magic, at + 1)
+    return kernels
+
+
+def test_no_kernel_keeps_arrays_in_scratch_memory():
+    """Arrays and what lambdas share stay in registers: a function that the compiler does not inline takes them to
+    scratch memory (six times the time of a prefill at head_dim 256)."""
+    from ksa_amd import _lib
+    pytest.importorskip("msgpack")
+    kernels = _kernel_metadata(_lib.LIB_PATH)
+    assert any("ksa_prefill_kernel" in n and "Li256ELi0E" in n for n in kernels)   # (head_dim 256, general addressing)
+    # (a few spilled registers are no array)
+    assert {n: k[".private_segment_fixed_size"] for n, k in kernels.items() if k[".private_segment_fixed_size"] > 32} == {}
