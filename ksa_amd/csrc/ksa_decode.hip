@@ -417,16 +417,18 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
 
 // Second stage: merge the splits of one (sequence, kv head, column).  A chain of memory trips, nothing else, so
 // there are few: D / 4 threads take four elements each, the G such groups of a workgroup every G-th split, and a
-// group requests up to eight splits with their maxima and sums at once - one trip for 128 / 64 / 32 splits at
-// head_dim 64 / 128 / 256, another for as many more; the groups meet in LDS.  (A thread per element that walked the splits eight at a time, maxima first, took 2 to 16 trips:
+// group requests up to eight splits with their maxima and sums at once; the groups meet in LDS.  One trip takes 32
+// splits with a thread per element (G = 4), which is the workgroup up to there, and 128 / 64 / 32 at head_dim
+// 64 / 128 / 256 with 256 threads, which is the one above; another trip takes as many more.  (256 threads for few
+// splits too cost a launch of thousands of columns more than it saved: 9 query tokens of 32 heads, 8 x 1500 rows in 5
+// splits at head_dim 64 16.7 -> 19.0 us, with a thread per element 16.4; 3 x 4096 rows in 16 18.9 -> 18.5, and 16.8.)  (A thread per element that walked the splits eight at a time, maxima first, took 2 to 16 trips:
 // decode + merge of one sequence of 16384 rows in
 // 64 splits 29.8 -> 19.4 us, 4096 rows in 16 13.4 -> 12.0.)
-constexpr int kMergeThreads = 256;
-template <typename T, int D>
-__global__ __launch_bounds__(kMergeThreads) void ksa_decode_merge_kernel(const DecodeParams p) {
+template <typename T, int D, int kThreads>
+__global__ __launch_bounds__(kThreads) void ksa_decode_merge_kernel(const DecodeParams p) {
     using Ops = KsaOps<T>;
     constexpr int TPG = D / 4;                 // threads of a group
-    constexpr int G = kMergeThreads / TPG;
+    constexpr int G = kThreads / TPG;
     constexpr int kBatch = 8;
     __shared__ float s_m[G], s_l[G];
     __shared__ __attribute__((aligned(16))) float s_o[G][D];
@@ -499,7 +501,10 @@ int launch(const DecodeParams& p, int batch, hipStream_t stream) {
     }
     if (p.nsplit > 1) {
         dim3 g2(p.ncols, p.Hkv, batch);
-        hipLaunchKernelGGL((ksa_decode_merge_kernel<T, D>), g2, dim3(kMergeThreads), 0, stream, p);
+        if (p.nsplit <= 32)
+            hipLaunchKernelGGL((ksa_decode_merge_kernel<T, D, D>), g2, dim3(D), 0, stream, p);
+        else
+            hipLaunchKernelGGL((ksa_decode_merge_kernel<T, D, 256>), g2, dim3(256), 0, stream, p);
     }
     return ksa_check_launch();
 }

@@ -372,10 +372,11 @@ def test_decode_qkv_with_a_range_row_and_position_per_sequence(dtype, b, Hq, Hkv
     assert np.abs(to_np(got).reshape(ref.shape) - ref).max() <= ATOL * max(1.0, np.abs(ref).max())
 
 
-@pytest.mark.parametrize("Hkv,D,nsplit", [(2, 256, None), (4, 256, 64), (2, 256, 33), (1, 128, 100), (1, 64, 150)])
+@pytest.mark.parametrize("Hkv,D,nsplit", [(2, 256, None), (4, 256, 64), (2, 256, 33), (1, 128, 100), (1, 64, 150), (2, 256, 32),
+                                          (2, 128, 32), (2, 128, 33), (1, 64, 32), (1, 64, 33)])
 def test_decode_merge_of_more_splits_than_one_pass_takes(Hkv, D, nsplit):
-    """The merge walks more than 32 splits at head_dim 256 (64 at 128, 128 at 64) in several passes.  Scores that
-    grow along the rows move the maximum in each of them; falling ones leave it in the first; a sequence of few
+    """The merge walks more than 32 splits at head_dim 256 (64 at 128, 128 at 64) in several passes; up to 32 it has
+    a thread per element, one pass.  Scores that grow along the rows move the maximum in each of them; falling ones leave it in the first; a sequence of few
     rows leaves all but the first splits empty."""
     from ksa_amd import _lib
     b, rows = 3, 64 * 300
