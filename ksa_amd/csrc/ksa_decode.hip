@@ -535,6 +535,67 @@ extern "C" int ksa_decode_auto_splits(int batch, int Hkv, int max_rows) {
     return n < 1 ? 1 : n;
 }
 
+// Several blocks of 32 columns (query tokens x heads of a group) up to head_dim 128: each block is a workgroup of its
+// own that reads the slice's K / V again.  The blocks of a slice are nsplit x kv heads workgroups apart: a multiple of 8
+// puts them on one XCD, where the K / V of the first one is in the L2 for the others, worth more than the last
+// workgroups' round alone.  From half a workgroup per CU on the count goes up to such a multiple if the one by the
+// slices alone allows it (from one split on long ranges only; at head_dim 64 it is the one by the slices if not), below
+// that down to a multiple, or to the least count with as many rounds of 128 rows.  head_dim 128, 9 query tokens, count by
+// the slices / by the workgroups / this one: 64 sequences of 4096 rows, 1 kv head of 8 72 / 97 / 72 us, 2 of 4 82 / 97 / 82;
+// 20 of 4096, 4 of 8 103 / 98 / 82; 64 of 600 and 4096, 4 of 8 71 / 54 / 54 and 202 / 235 / 196; 40 of 1650, 8 of 8 139 /
+// 99 / 99; 8 of 760, 4 of 8 19.3 / 22.4 / 18.4; 8 of 4096, 1 of 8 21.6 / 22.8 / 19.7; 3 of 1500, 8 of 4 18.6 / 18.9 / 17.1;
+// 1 of 1500, 8 of 4 16.4 / 12.6 / 12.6.  At head_dim 64 100 of 4096, 2 of 4 84 / 100 / 84.
+static int splits_of_column_blocks(int64_t slices, int64_t blocks, int Hkv, int D, int64_t max_rows, int64_t cus) {
+    const int64_t units = slices * blocks, rounds = (max_rows + 127) / 128;
+    int64_t a = 8;  // 8 / gcd(8, kv heads)
+    for (int h = Hkv; a > 1 && h % 2 == 0; h /= 2) a /= 2;
+    int64_t cap = max_rows / 256;
+    if (2 * units > cus) {
+        int64_t n = (2 * cus + units - 1) / units;
+        const int64_t by_slices = (2 * cus + slices - 1) / slices, aligned = (n + a - 1) / a * a;
+        if (aligned <= by_slices && (n > 1 || max_rows >= 2048)) n = aligned;
+        else if (n > 1 && n % a && D <= 64) n = by_slices;
+        n = n < cap ? n : cap;
+        return (int)(n < 1 ? 1 : n < 64 ? n : 64);
+    }
+    if (3 * units <= cus && blocks <= 4) cap = max_rows <= (D <= 64 ? 512 : 384) ? 1 : rounds;
+    int64_t n = 2 * cus / units;
+    n = n < cap ? n : cap;
+    n = n < 64 ? n : 64;
+    if (n <= 1) return 1;
+    if (a > 1 && n >= a) return (int)(n - n % a);
+    const int64_t per = (rounds + n - 1) / n;
+    return (int)((rounds + per - 1) / per);
+}
+
+// One block of columns, less than half a workgroup per CU (a third at head_dim 64): a round of 128 rows per split where
+// that is at most two workgroups per CU (eight workgroups more do no harm at head_dim 128, sixteen at 64 with few
+// columns), otherwise two per CU; but where those would walk several rounds and splits of 256 rows put one workgroup
+// on a CU, these.  Rounded up past two per CU the last workgroups run alone: 9 / 11 sequences of 8 kv heads, 4096 rows,
+// 8 -> 7 / 6 -> 5 splits 38.1 -> 33.2 / 48.7 -> 39.0 us, 1100 rows of 9 in 4 / 8 / 7 18.8 / 20.8 / 16.3; 3 of 2700 rows in 10 /
+// 22 / 21 14.7 / 15.1 / 15.3, with 20 columns 17.6 / 20.8 / 19.1; at head_dim 64 40 slices of 4096 rows in 13 -> 12 17.1
+// -> 16.0, at 128 25.5 -> 26.1.  Above 32 splits of more than 16 columns, the least count with as many rounds: 6 slices of
+// 10000 rows, 32 columns, 39 / 64 / 40 splits 18.8 / 20.4 / 18.0.
+static int splits_of_few_slices(int64_t units, int64_t columns, int D, int64_t max_rows, int64_t cus) {
+    if (max_rows <= (D <= 64 ? 512 : 384)) return 1;
+    const int64_t rounds = (max_rows + 127) / 128;
+    int64_t n = 2 * cus / units;
+    if (D <= 64 && columns <= 16 && rounds == n + 1 && n * units < 2 * cus) n = rounds;
+    if (rounds <= n) {
+        n = rounds;
+    } else {
+        if (D > 64) n = (2 * cus + cus / 32) / units;
+        const int64_t long_ones = max_rows / 256;
+        if (long_ones < n && long_ones * units <= cus && n * units > cus) n = long_ones;
+    }
+    if (n > 64) n = 64;
+    if (n > 32 && columns > 16) {
+        const int64_t per = (rounds + n - 1) / n;
+        n = (rounds + per - 1) / per;
+    }
+    return (int)n;
+}
+
 // Number of splits for Q query tokens of Hq heads: two workgroups per CU, but splits of no fewer rows than a
 // workgroup's waves cover in one round (128) - a launch over few rows is a chain of memory trips per
 // round, 2.1 us each, and a split more costs the merge next to nothing.  From half a workgroup per CU on
@@ -552,7 +613,7 @@ extern "C" int ksa_decode_auto_splits(int batch, int Hkv, int max_rows) {
 // 20 of 6000 191 -> 173; few rows the same counts.
 extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int max_rows) {
     if (batch <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || Q <= 0 || D <= 0 || max_rows <= 0) return 1;
-    const int64_t units = (int64_t)batch * Hkv * ((Q * (int64_t)(Hq / Hkv) + 31) / 32);
+    const int64_t blocks = (Q * (int64_t)(Hq / Hkv) + 31) / 32, units = (int64_t)batch * Hkv * blocks;
     const int cus = ksa_cu_count_or(256);
     if (D > 128) {
         const int64_t steps = ((int64_t)max_rows + 127) / 128;
@@ -565,10 +626,10 @@ extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int m
         }
         return best;
     }
+    if (blocks > 1) return splits_of_column_blocks((int64_t)batch * Hkv, blocks, Hkv, D, max_rows, cus);
+    if ((D <= 64 ? 3 : 2) * units < cus) return splits_of_few_slices(units, (int64_t)Q * (Hq / Hkv), D, max_rows, cus);
     int64_t n = (2 * (int64_t)cus + units - 1) / units;
-    int64_t cap = max_rows / 256;
-    const bool few = D <= 64 ? 3 * units < cus : 2 * units < cus;
-    if (few) cap = max_rows <= (D <= 64 ? 512 : 384) ? 1 : ((int64_t)max_rows + 127) / 128;
+    const int64_t cap = max_rows / 256;
     if (n > cap) n = cap;
     if (n > 64) n = 64;
     return n < 1 ? 1 : (int)n;
