@@ -56,9 +56,7 @@ __device__ __forceinline__ KsaWeightLane ksa_weight_lane(const uint16_t* w, int6
 // Row-major: a plain one, since a fragment takes 64 bytes of a row and the next step's fragment the other half of
 // the 128-byte line, which a non-temporal load does not keep for it: 19456 x 2560 in no cache, 1 / 32 / 72 rows
 // 20.3 / 31.4 / 33.3 us plain, 26.8 / 38.2 / 39.7 non-temporal; the same matrix again and again 15.5 / 24.5 / 27.4 and 22.5 / 36.1 / 37.8.
-// (A streaming copy read again and again, 17 rows and more, is up to 9 % slower than with plain loads - 19456 x 2560, 32
-// rows 21.3 against 19.6 us - and 2 to 8 % faster where it comes from memory, as in a pass through a model's
-// layers: 24.6 against 25.9.)
+// (The K-split products of 17 rows and more take plain loads in either layout: see launch_wide.)
 template <bool kTiled>
 __device__ __forceinline__ u32x4 ksa_load_weights(const uint16_t* p) {
     const u32x4* q = reinterpret_cast<const u32x4*>(p);
