@@ -46,7 +46,8 @@ struct GemmParams {
 // Per call in a graph of calls on distinct weights, 1 / 8 / 16 rows: 6144 x 2560 7.7 / 8.4 / 9.3 ->
 // 6.6 / 7.2 / 7.7 us, 2560 x 4096 7.2 / 7.9 / 8.8 -> 6.1 / 6.7 / 7.2, 2560 x 9728 12.0 / 12.9 / 14.5 -> 9.4 / 10.0 / 10.5 (31,
 // 21 and 50 MB are read in 6.1, 4.6 and 8.5 us by a kernel that does nothing else).
-// kShortEnd: K is no multiple of 512 (a kernel of its own: the branch around the clearing cost the others 0.2 us).
+// kShortEnd: K is no multiple of 512, the missing steps of the last chunk are left out (a kernel of its own: such branches
+// cost the others 0.2 us).  Their weights are the last step's again, and an infinite one would give inf x 0.
 template <typename T, bool kTiled, int XT, bool kShortEnd>
 __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) {
     using C = KsaCvt<T>;
@@ -77,7 +78,7 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
         a[u] = ksa_load_weights<kTiled>(reinterpret_cast<const uint16_t*>(wtile + s * (kTiled ? 1024 : 64) + wlane));
     };
     // staging of a chunk of x: thread = (row wave + 4 i, 16-byte piece lane); pieces past a short last chunk become
-    // zeros, and so do the weights of its missing steps, so that these add nothing
+    // zeros
     const uint16_t* xrow[XT];
 #pragma unroll
     for (int i = 0; i < XT; ++i) xrow[i] = p.x + (int64_t)min(wave + 4 * i, p.M - 1) * p.xs;
@@ -99,13 +100,15 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
     };
     const int xoff = min(r, 4 * XT - 1) * kRowB + 16 * kq;
 
+    const int live_last = p.steps - (c_end - 1) * kChunkSteps;  // (kShortEnd) steps of the last chunk, 16 and more: all
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     auto chunk = [&](auto more_tag, int cn, int buf) __attribute__((always_inline)) {  // cn: the next chunk (kMore)
         constexpr bool kMore = decltype(more_tag)::value;
         if constexpr (kMore) x_request(cn);
 #pragma unroll
         for (int u = 0; u < kChunkSteps; ++u) {
-            acc = mfma16<T>(a[u], *reinterpret_cast<const u32x4*>(xs[buf] + xoff + 64 * u), acc);
+            if (kMore || !kShortEnd || u < live_last)
+                acc = mfma16<T>(a[u], *reinterpret_cast<const u32x4*>(xs[buf] + xoff + 64 * u), acc);
             if constexpr (kMore) w_request(cn, u);
         }
     };
@@ -124,7 +127,6 @@ __global__ __launch_bounds__(256) void ksa_gemm_rows_kernel(const GemmParams p) 
             x_store(c + 1, buf);
             __syncthreads();
         }
-        if constexpr (kShortEnd) ksa_clear_missing_steps(a, p.steps - (c_end - 1) * kChunkSteps);
         chunk(std::false_type{}, c_end, buf);
     }
 
@@ -183,7 +185,7 @@ struct WideParams {
 };
 constexpr int kWideWaves = 8;
 
-template <typename T, int MB, bool kPair, bool kStream>
+template <typename T, int MB, bool kPair, bool kStream, bool kShortEnd>
 __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(const WideParams p) {
     using C = KsaCvt<T>;
     extern __shared__ __attribute__((aligned(16))) unsigned char wide_lds[];
@@ -231,8 +233,7 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(con
 #pragma unroll
         for (int i = 0; i < XT; ++i) xt[i] = *reinterpret_cast<const u32x4*>(src + xrow_off[i]);
     };
-    // (a short last chunk is filled up with zeros, like the weights that the clamped requests fetch for its
-    // missing steps: these then add nothing)
+    // (a short last chunk is filled up with zeros)
     auto x_store = [&](int c) {
         const bool live = tj < 4 * min(kChunkSteps, steps - c * kChunkSteps);
 #pragma unroll
@@ -283,8 +284,20 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(con
             x_store(c + 1);
             __syncthreads();
         }
-        ksa_clear_missing_steps(a, steps - (c_end - 1) * kChunkSteps);
-        chunk(std::false_type{}, c_end);
+        const int live = steps - (c_end - 1) * kChunkSteps;
+        if (!kShortEnd || live >= kChunkSteps) {
+            chunk(std::false_type{}, c_end);
+        } else {  // (the weights of the missing steps are the last step's again: an infinite one would give inf x 0 there)
+#pragma unroll
+            for (int u = 0; u < kChunkSteps - 1; ++u) {
+                if (u < live) {
+#pragma unroll
+                    for (int b = 0; b < MB; ++b)
+                        acc[b] = mfma16<T>(a[u], *reinterpret_cast<const u32x4*>(wide_lds + xoff[b] + 64 * u), acc[b]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
     }
     // C layout of a 16x16 tile: lane holds row (of x) lane % 16 of the block, columns n0 + 4 * (lane / 16) + i
     const int n = n0 + 4 * kq;
@@ -365,8 +378,8 @@ static WidePlan wide_plan(int K, int want_splits) {
     return pl;
 }
 
-template <typename T, bool kPair, bool kStream>
-int launch_wide_loads(const WideParams& p, hipStream_t st) {
+template <typename T, bool kPair, bool kStream, bool kShortEnd>
+int launch_wide_end(const WideParams& p, hipStream_t st) {
     const int mb = (p.M + 15) / 16;
     constexpr int cols = kPair ? 16 * (kWideWaves / 2) : 16 * kWideWaves;
     const dim3 grid((p.N + cols - 1) / cols, p.ksplit), block(64 * kWideWaves);
@@ -382,13 +395,19 @@ int launch_wide_loads(const WideParams& p, hipStream_t st) {
         return ksa_check_launch();
     };
     switch (mb) {
-        case 2: return go(ksa_gemm_rows_wide_kernel<T, 2, kPair, kStream>);
-        case 3: return go(ksa_gemm_rows_wide_kernel<T, 3, kPair, kStream>);
-        case 4: return go(ksa_gemm_rows_wide_kernel<T, 4, kPair, kStream>);
-        case 5: return go(ksa_gemm_rows_wide_kernel<T, 5, kPair, kStream>);
-        case 6: return go(ksa_gemm_rows_wide_kernel<T, 6, kPair, kStream>);
-        default: return go(ksa_gemm_rows_wide_kernel<T, 8, kPair, kStream>);
+        case 2: return go(ksa_gemm_rows_wide_kernel<T, 2, kPair, kStream, kShortEnd>);
+        case 3: return go(ksa_gemm_rows_wide_kernel<T, 3, kPair, kStream, kShortEnd>);
+        case 4: return go(ksa_gemm_rows_wide_kernel<T, 4, kPair, kStream, kShortEnd>);
+        case 5: return go(ksa_gemm_rows_wide_kernel<T, 5, kPair, kStream, kShortEnd>);
+        case 6: return go(ksa_gemm_rows_wide_kernel<T, 6, kPair, kStream, kShortEnd>);
+        default: return go(ksa_gemm_rows_wide_kernel<T, 8, kPair, kStream, kShortEnd>);
     }
+}
+
+// (K no multiple of 512: a kernel of its own, 3 % of the others' time at 6144 x 2560, 32 rows)
+template <typename T, bool kPair, bool kStream>
+int launch_wide_loads(const WideParams& p, hipStream_t st) {
+    return p.K % kChunkK ? launch_wide_end<T, kPair, kStream, true>(p, st) : launch_wide_end<T, kPair, kStream, false>(p, st);
 }
 
 template <typename T, bool kPair>

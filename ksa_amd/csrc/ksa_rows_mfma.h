@@ -63,14 +63,3 @@ __device__ __forceinline__ u32x4 ksa_load_weights(const uint16_t* p) {
     if constexpr (kTiled) return __builtin_nontemporal_load(q);
     else return *q;
 }
-
-// Zeros in place of the weights of a last chunk's steps from `live` on (they repeat its last step's: with zeros of x
-// alone an infinite or NaN weight there would come back as NaN).  A chunk of full length passes by.
-__device__ __forceinline__ void ksa_clear_missing_steps(u32x4 (&a)[kChunkSteps], int live) {
-    if (live < kChunkSteps) {
-#pragma unroll
-        for (int u = 1; u < kChunkSteps; ++u)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a[u][e] = u < live ? a[u][e] : 0u;
-    }
-}
