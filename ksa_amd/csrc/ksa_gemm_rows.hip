@@ -185,7 +185,7 @@ struct WideParams {
 };
 constexpr int kWideWaves = 8;
 
-template <typename T, int MB, bool kPair, bool kStream, bool kShortEnd>
+template <typename T, int MB, bool kPair, bool kShortEnd>
 __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(const WideParams p) {
     using C = KsaCvt<T>;
     extern __shared__ __attribute__((aligned(16))) unsigned char wide_lds[];
@@ -246,7 +246,10 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_gemm_rows_wide_kernel(con
     };
     u32x4 a[kChunkSteps];
     auto w_request = [&](int c, int u) {
-        a[u] = ksa_load_weights<kStream>(wl.p + wl.step * min(c * kChunkSteps + u, steps - 1));
+        // Plain loads in either layout.  Non-temporal ones gain up to 8 % on 17 to 33 rows of large matrices and lose up to 16 %
+        // on most others (streaming layout, 6144 x 2560, 17 / 72 / 128 rows 11.3 / 15.3 / 20.8 -> 11.1 / 17.5 / 24.2 us), and where
+        // the weights are still in a cache up to 23 %; gate | up gains 3 % from memory and loses 15 % from the cache.
+        a[u] = ksa_load_weights<false>(wl.p + wl.step * min(c * kChunkSteps + u, steps - 1));
     };
     // the products of one chunk; kMore: there is a next chunk, whose x and weights are requested on the way
     // (two copies of the loop body rather than a condition inside it: with branches between the MFMAs the
@@ -378,7 +381,7 @@ static WidePlan wide_plan(int K, int want_splits) {
     return pl;
 }
 
-template <typename T, bool kPair, bool kStream, bool kShortEnd>
+template <typename T, bool kPair, bool kShortEnd>
 int launch_wide_end(const WideParams& p, hipStream_t st) {
     const int mb = (p.M + 15) / 16;
     constexpr int cols = kPair ? 16 * (kWideWaves / 2) : 16 * kWideWaves;
@@ -395,30 +398,19 @@ int launch_wide_end(const WideParams& p, hipStream_t st) {
         return ksa_check_launch();
     };
     switch (mb) {
-        case 2: return go(ksa_gemm_rows_wide_kernel<T, 2, kPair, kStream, kShortEnd>);
-        case 3: return go(ksa_gemm_rows_wide_kernel<T, 3, kPair, kStream, kShortEnd>);
-        case 4: return go(ksa_gemm_rows_wide_kernel<T, 4, kPair, kStream, kShortEnd>);
-        case 5: return go(ksa_gemm_rows_wide_kernel<T, 5, kPair, kStream, kShortEnd>);
-        case 6: return go(ksa_gemm_rows_wide_kernel<T, 6, kPair, kStream, kShortEnd>);
-        default: return go(ksa_gemm_rows_wide_kernel<T, 8, kPair, kStream, kShortEnd>);
+        case 2: return go(ksa_gemm_rows_wide_kernel<T, 2, kPair, kShortEnd>);
+        case 3: return go(ksa_gemm_rows_wide_kernel<T, 3, kPair, kShortEnd>);
+        case 4: return go(ksa_gemm_rows_wide_kernel<T, 4, kPair, kShortEnd>);
+        case 5: return go(ksa_gemm_rows_wide_kernel<T, 5, kPair, kShortEnd>);
+        case 6: return go(ksa_gemm_rows_wide_kernel<T, 6, kPair, kShortEnd>);
+        default: return go(ksa_gemm_rows_wide_kernel<T, 8, kPair, kShortEnd>);
     }
 }
 
 // (K no multiple of 512: a kernel of its own, 3 % of the others' time at 6144 x 2560, 32 rows)
-template <typename T, bool kPair, bool kStream>
-int launch_wide_loads(const WideParams& p, hipStream_t st) {
-    return p.K % kChunkK ? launch_wide_end<T, kPair, kStream, true>(p, st) : launch_wide_end<T, kPair, kStream, false>(p, st);
-}
-
 template <typename T, bool kPair>
 int launch_wide(const WideParams& p, hipStream_t st) {
-    // Non-temporal loads for the gate | up product of the streaming layout only (17 / 72 / 128 rows, 9728 x 2560: 21.2 / 29.0 /
-    // 37.8 -> 20.5 / 28.3 / 37.4 us).  The K-split products gain up to 8 % on 17 to 33 rows of large matrices and lose up to
-    // 16 % on more rows (6144 x 2560, 17 / 72 / 128 rows 11.3 / 15.3 / 20.8 -> 11.1 / 17.5 / 24.2; 4096 x 4096, 72 16.5 -> 18.1),
-    // and 23 % where the matrix is still in a cache.
-    if constexpr (kPair)
-        if (p.ws == kWTiled) return launch_wide_loads<T, kPair, true>(p, st);
-    return launch_wide_loads<T, kPair, false>(p, st);
+    return p.K % kChunkK ? launch_wide_end<T, kPair, true>(p, st) : launch_wide_end<T, kPair, false>(p, st);
 }
 
 template <typename T>

@@ -56,7 +56,9 @@ __device__ __forceinline__ KsaWeightLane ksa_weight_lane(const uint16_t* w, int6
 // Row-major: a plain one, since a fragment takes 64 bytes of a row and the next step's fragment the other half of
 // the 128-byte line, which a non-temporal load does not keep for it: 19456 x 2560 in no cache, 1 / 32 / 72 rows
 // 20.3 / 31.4 / 33.3 us plain, 26.8 / 38.2 / 39.7 non-temporal; the same matrix again and again 15.5 / 24.5 / 27.4 and 22.5 / 36.1 / 37.8.
-// (The K-split products of 17 rows and more take plain loads in either layout: see launch_wide.)
+// (17 rows and more take plain loads in either layout, see ksa_gemm_rows_wide_kernel.  Up to 16 rows a streaming copy that is
+// still in the memory-side cache, 30 to 220 MB of weights read in turn, is 5 to 10 % slower in the gate | up product than
+// with plain loads, and 6 to 9 % faster from memory, where a model's decode step finds it.)
 template <bool kTiled>
 __device__ __forceinline__ u32x4 ksa_load_weights(const uint16_t* p) {
     const u32x4* q = reinterpret_cast<const u32x4*>(p);
