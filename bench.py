@@ -336,7 +336,7 @@ def main():
         end = torch.full((Bz,), S + C + ws + n_sum - min(W * S, n_sum), dtype=torch.int32, device=dev)
         L = (end - start).to(torch.int64)
         bytes_step = int((2 * L * Hkv * D * 2 + 2 * Hq * D * 2).sum())
-        nsplit = args.decode_splits or _lib.lib().ksa_decode_auto_splits(Bz, Hkv, cap)
+        nsplit = args.decode_splits or _lib.lib().ksa_decode_splits(Bz, Hq, Hkv, 1, D, cap)
 
         def dstep():
             ksa_amd.ksa_decode(qd, kc, vc, start, end, nsplit=nsplit)
