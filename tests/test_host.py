@@ -374,3 +374,20 @@ def test_no_kernel_keeps_arrays_in_scratch_memory():
     assert any("ksa_prefill_kernel" in n and "Li256ELi0E" in n for n in kernels)   # (head_dim 256, general addressing)
     # (a few spilled registers are no array)
     assert {n: k[".private_segment_fixed_size"] for n, k in kernels.items() if k[".private_segment_fixed_size"] > 32} == {}
+
+
+@pytest.mark.parametrize("b,hq,hkv,q", [(64, 8, 1, 9), (20, 32, 4, 9), (64, 8, 2, 9), (8, 32, 4, 9), (3, 32, 8, 9), (40, 64, 8, 9), (4, 32, 2, 9)])
+@pytest.mark.parametrize("D", [64, 128])
+def test_decode_splits_of_column_blocks(b, hq, hkv, q, D):
+    """Several blocks of columns per slice: never past two workgroups per CU by more than the alignment of the blocks asks
+    for, splits of at least a round, and the blocks of a slice on one XCD wherever the count is large enough."""
+    import math
+    from ksa_amd import _lib
+    blocks = -(-q * (hq // hkv) // 32)
+    a, slices = 8 // math.gcd(8, hkv), b * hkv
+    assert blocks > 1
+    for rows in (1, 300, 513, 900, 1500, 4096, 20000, 131072, 2**31 - 1):
+        n = _lib.lib().ksa_decode_splits(b, hq, hkv, q, D, rows)
+        assert 1 <= n <= 64 and (n == 1 or (n - 1) * 128 < rows) and (n == 1 or (n - 1) * slices < 512)
+        if rows >= 4096 and a * slices <= 512:
+            assert n % a == 0 or n < a
