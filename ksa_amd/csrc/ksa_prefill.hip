@@ -1052,6 +1052,9 @@ int prefill_addr(const PrefillParams& p) {
     const bool in_place = mk.P > 0 && !p.phys_prefix;
     if (in_place && RSTEP % mk.S != 0) return kAddrGeneral;
     if (mk.Sk % kTileN == 0 && (!in_place || mk.P % kTileN == 0)) return kAddrRegular;
+    // (a walk of a few tiles has nothing to hide a marked tile's second fetch behind: head_dim 64, no prefix, 150 / 400 / 520
+    // rows 8.9 / 12.3 / 13.7 us marked, 8.0 / 11.3 / 12.8 general; 700 / 1000 15.4 / 17.8 and 15.9 / 18.5)
+    if (D <= 64 && mk.P == 0 && mk.Sk <= 600) return kAddrGeneral;
     return RB == 1 && (p.phys_prefix ? mk.Sk : mk.Sq) >= kTileN ? kAddrMarked : kAddrGeneral;
 }
 
