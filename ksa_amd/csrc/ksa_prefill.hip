@@ -165,9 +165,10 @@ __device__ __forceinline__ RowVis ksa_row_vis(const KsaMask& mk, const FastDiv& 
 //     the walk, so that only masked steps carry the branch: in every step it costs 4.5 % at 128k rows
 //     (it takes the row sums out of the place the compiler gives them at the end of the step), in the
 //     masked ones 4 % at 4k rows - which is why lengths that need no marks keep a variant of their own.
-//   kAddrGeneral: a division per lane and fill (700 to 1200 cycles a tile); left to a summary count that
-//     does not divide the step with a prefix read in place, and to fewer than 64 rows.
-// Lengths that are no multiple of 64 with the marked variant against the general one (32 query heads):
+//   kAddrGeneral: a row number and its address per lane and fill; left to a summary count that does not
+//     divide the step with a prefix read in place, to fewer than 64 rows, and to short walks (prefill_addr).
+// Lengths that are no multiple of 64 with the marked variant against the general one with divisions in its
+// fills, 700 to 1200 cycles a tile (32 query heads; without them, head_dim 64, it is 2 to 8 % behind from 700 rows on):
 // 1000 tokens 26.3 -> 23.5 us, 4000 78 -> 71 us, 2 x 3000 109 -> 96 us, 32800 1009 -> 980 us, three
 // prompts of 9001 tokens with an unbounded window in fp16 2267 -> 2169 us.
 enum { kAddrGeneral = 0, kAddrRegular = 1, kAddrMarked = 2 };
@@ -399,7 +400,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         }
     };
     // (always inline: at head_dim 256 the general form, left to itself, is called, and what the kernel's functions share
-    // then lives in scratch memory: 8 heads, 63 rows 14.7 -> 86 us)
+    // then lives in scratch memory: 8 heads, 63 rows 86 us instead of 14.1)
     auto fill = [&](const char* base, uint16_t* tile, uint32_t col, int n, uint32_t word,
                     uint32_t odd_xor) __attribute__((always_inline)) {
 #pragma unroll
