@@ -168,7 +168,7 @@ __device__ __forceinline__ RowVis ksa_row_vis(const KsaMask& mk, const FastDiv& 
 //   kAddrGeneral: a row number and its address per lane and fill; left to a summary count that does not
 //     divide the step with a prefix read in place, to fewer than 64 rows, and to short walks (prefill_addr).
 // Lengths that are no multiple of 64 with the marked variant against the general one with divisions in its
-// fills, 700 to 1200 cycles a tile (32 query heads; without them, head_dim 64, it is 2 to 8 % behind from 700 rows on):
+// fills, 700 to 1200 cycles a tile (32 query heads; without them, head_dim 64, it is up to 9 % behind from 700 rows on):
 // 1000 tokens 26.3 -> 23.5 us, 4000 78 -> 71 us, 2 x 3000 109 -> 96 us, 32800 1009 -> 980 us, three
 // prompts of 9001 tokens with an unbounded window in fp16 2267 -> 2169 us.
 enum { kAddrGeneral = 0, kAddrRegular = 1, kAddrMarked = 2 };
