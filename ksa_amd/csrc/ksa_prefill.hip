@@ -26,6 +26,9 @@
 // step stands in front of the last MFMAs of its second product, which then cover the reads of
 // the next step's first fragments.
 //
+// Prompts whose summary rows lie in line behind whole chunks of C = 128, 256, 384 or 512 rows need no block index: their
+// tiles are laid along the chunks (kAddrChunks below).  What follows is the general form.
+//
 // Masking.  The walk has two phases that are uniform for the workgroup.  Phase A holds
 // the tiles that need no per-element mask: the leading partial tiles below every text
 // row's old-summary bound (there a row is visible as a whole iff it is a text row), the
@@ -48,18 +51,21 @@
 #include "ksa_mask.h"
 #include "ksa_tile.h"
 
-// This source is compiled as seven translation units, so that the instantiations of the kernel
-// compile side by side: unit 0 holds head_dim 64 and 128 and the entry point; units 1 to 6 (files
+// This source is compiled as ten translation units, so that the instantiations of the kernel
+// compile side by side: unit 0 holds head_dim 64 and 128 and the entry point for a block index, unit 9
+// the same head dimensions and the entry point for chunk tiles; units 1 to 8 (files
 // that include this one with KSA_PREFILL_UNIT set) hold one kernel of head_dim 256 each - bf16
-// (1 to 3) / fp16 (4 to 6), general / regular / marked tile addressing - because each of those takes
-// over a minute to compile.
+// (1 to 3) / fp16 (4 to 6), general / regular / marked tile addressing, and the chunk tiles in bf16 (7)
+// and fp16 (8) - because each of those takes over a minute to compile.
 #ifndef KSA_PREFILL_UNIT
 #define KSA_PREFILL_UNIT 0
 #endif
-// which of the three addressing variants a unit instantiates in launch_shape: -1 all, else that one
-// (kAddrGeneral, kAddrRegular, kAddrMarked)
+// which of the four addressing variants a unit instantiates in launch_shape: -1 the three for a block index, else that
+// one (kAddrGeneral, kAddrRegular, kAddrMarked, kAddrChunks)
 #if KSA_PREFILL_UNIT == 0
 #define KSA_PREFILL_VARIANT -1
+#elif KSA_PREFILL_UNIT >= 7
+#define KSA_PREFILL_VARIANT 3
 #else
 #define KSA_PREFILL_VARIANT ((KSA_PREFILL_UNIT - 1) % 3)
 #endif
@@ -114,9 +120,16 @@ struct PrefillParams {
     int n_items;      // items per batch element
     int total;        // items in all
     int n_static;     // multiple of 8
-    FastDiv by_items, by_hkv, by_gper;  // n_items, Hkv, query heads (pairs) per kv head
+    FastDiv by_items, by_hkv, by_gper;  // n_items (chunk tiles: batch elements), Hkv, query heads (pairs) per kv head
     FastDiv by_block, by_S;             // C + S, S
     int phase_shift;                    // the least multiple of C + S that is not below P
+    // kAddrChunks only
+    int chunk_tiles;       // the launch is one of chunk tiles
+    int n_chunks;          // complete chunks of a sequence (those with summary rows)
+    int rest_units;        // items per kv head of the incomplete chunk behind them
+    int sum_blocks;        // 32-column blocks of the g S summary queries of a kv head
+    FastDiv by_mt, by_nt;  // row tiles and key tiles per chunk
+    FastDiv by_group;      // items per kv head and group of chunks (as many as a workgroup has waves)
 };
 
 constexpr int kTileM = 128;
@@ -171,7 +184,23 @@ __device__ __forceinline__ RowVis ksa_row_vis(const KsaMask& mk, const FastDiv& 
 // fills, 700 to 1200 cycles a tile (32 query heads; without them, head_dim 64, it is up to 9 % behind from 700 rows on):
 // 1000 tokens 26.3 -> 23.5 us, 4000 78 -> 71 us, 2 x 3000 109 -> 96 us, 32800 1009 -> 980 us, three
 // prompts of 9001 tokens with an unbounded window in fp16 2267 -> 2169 us.
-enum { kAddrGeneral = 0, kAddrRegular = 1, kAddrMarked = 2 };
+//   kAddrChunks: tiles laid along the chunks instead of the 128 x 64 grid of the block index (ksa_prefill_chunks_fwd).  On
+//     the grid every row tile carries a few summary rows (6 % of the rows at C = 128, S = 8) that see nothing of most
+//     of its key tiles, every key tile of the window as many hidden summary columns, and window and diagonal begin inside
+//     tiles.  Here a row tile is 128 text rows of one chunk and a key tile 64 text rows of one chunk or 64 prefix rows, so
+//     all rows see the same tiles, all but the two on the diagonal and the rest of the prefix without a mask; the list
+//     is a closed form, no trip to memory.  The last tile with too few rows ends with the last row instead of beginning
+//     behind its predecessor, and the columns that repeat are masked.  The summary rows' queries - 1 / (C + S) of the work -
+//     go to workgroups of their own (ksa_summary_rows), placed in front of their chunks' text rows, which then find K/V in
+//     the L2: behind all text rows instead they read K/V from memory again, 8 x 10234 tokens, 8 heads, W = 1 335
+//     against 291 us, 3 x 844 tokens at head_dim 256 47 against 38 us (in front of them a launch of one round is up to 13 %
+//     slower, 2 x 438 tokens 9.4 against 10.9 us; still 14.7 on the grid).
+//     Tiles per row tile at C = 128, S = 8, W = 4: 73.9 instead of 75.7 at 128k tokens, 25.8 instead of 27.7 at 32k, and 6 % fewer row tiles.
+//     Measured, grid / chunks, us: 32 / 8 heads in bf16, W = 4, 300 tokens 15.0 / 12.7, 32k 896 / 795, 128k 8903 / 8123; 16 / 8
+//     heads, 4k 36.6 / 33.1; unbounded window, 3 x 9001 tokens in fp16 2119 / 1765; head_dim 64, 2 x 11013 tokens 309 / 232; head_dim
+//     256, 8 x 2608 tokens 787 / 625.  Of 140 shapes drawn over batch, heads, window and length none is slower (the least
+//     gain, 1 %: 8 x 10234 tokens, 8 / 8 heads, W = 1, where K/V are read once for the summary rows and once for the text).
+enum { kAddrGeneral = 0, kAddrRegular = 1, kAddrMarked = 2, kAddrChunks = 3 };
 
 // RB: 32-row query blocks per wave.  RB = 1: one query head per workgroup, wave w owns rows
 // 32w..32w+31, two workgroups per CU.  RB = 2: two query heads of one kv group per workgroup,
@@ -189,6 +218,157 @@ struct PrefillShape {
     static constexpr int kThreads = 64 * kWaves;
 };
 
+// A row tile of 128 text rows of one chunk (kAddrChunks) and the key tiles its rows see, the same for every row but
+// for the diagonal: [n_pre tiles of the prefix | the text tiles of the window and of the chunk in front of the
+// rows], n_a in all, then - masked - the rest of the prefix (`rem` rows) and the n_diag tiles on the diagonal.
+struct ChunkTile {
+    int p0;        // first row
+    int w0;        // first chunk of the window
+    int pre_rows;  // prefix rows seen
+    int n_pre, rem, n_a, n_diag;
+    // first row of tile d of the diagonal: it ends with the sequence where that is shorter
+    __device__ __forceinline__ int diag0(int d, int Sq) const { return min(p0 + d * kTileN, Sq - kTileN); }
+    // columns of the prefix's last tile that no tile before it holds: at its end, since the tile ends with the last row
+    // seen; a prefix shorter than a tile comes in loads of `rows` rows, of which the last one with new rows ends with
+    // the last row and the ones behind repeat it
+    __device__ __forceinline__ uint64_t pre_bits(int rows) const {
+        if (pre_rows >= kTileN) return ~0ull << (kTileN - rem);
+        if (pre_rows < rows) return ~(~0ull << pre_rows);
+        const int whole = pre_rows / rows * rows, more = pre_rows - whole;
+        return ~(~0ull << whole) | (more ? ~(~0ull << more) << (whole + rows - more) : 0ull);
+    }
+};
+
+__device__ __forceinline__ ChunkTile ksa_chunk_tile(const PrefillParams& p, int mt) {
+    const KsaMask& mk = p.mk;
+    ChunkTile t;
+    const int c = p.by_mt.div(mt), sub = mt - c * (int)p.by_mt.d;
+    t.p0 = c * (mk.C + mk.S) + sub * kTileM;
+    t.w0 = c > mk.W ? c - mk.W : 0;
+    t.pre_rows = mk.skip_old ? 0 : t.w0 * mk.S;
+    t.n_pre = t.pre_rows / kTileN;
+    t.rem = t.pre_rows % kTileN;
+    t.n_a = t.n_pre + (c - t.w0) * (int)p.by_nt.d + sub * (kTileM / kTileN);
+    t.n_diag = mk.Sq - t.p0 > kTileN ? 2 : 1;
+    return t;
+}
+
+// The summary queries of one chunk, one wave per block `cb` of 32 columns (query head of the kv group, summary row): it
+// walks the chunk's C + S rows 32 at a time, with the row maximum moved before the probabilities of every step.  K goes
+// from memory to the operand registers, V through `tile` (32 rows of this wave alone); the rows of the next step are
+// requested before the arithmetic of the current one.
+template <typename T, int D>
+__device__ __forceinline__ void ksa_summary_rows(const PrefillParams& p, int bz, int kvh, int chunk, int cb, int lane,
+                                                 uint16_t* tile) {
+    using Ops = KsaOps<T>;
+    constexpr int KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D;
+    constexpr int NV = 32 * CPR / 64;  // V loads per lane and step
+    const KsaMask& mk = p.mk;
+    const int B = mk.C + mk.S;
+    const int lq = lane & 31, lh = lane >> 5;
+    const int ncol = p.g * mk.S;
+    const int col = cb * 32 + lq, colc = min(col, ncol - 1);
+    const int hg = p.by_S.div(colc), sr = colc - hg * mk.S;
+    const int head = kvh * p.g + hg, row0 = chunk * B, qrow = row0 + mk.C + sr;
+
+    u32x4 qf[KS];
+    const uint16_t* qp = p.q + bz * p.q_bs + (int64_t)qrow * p.q_rs + head * p.q_hs + 8 * lh;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const u32x4*>(qp + 16 * s);
+
+    const uint16_t* kb = p.k + bz * p.kv_bs + kvh * p.kv_hs;
+    const uint16_t* vb = p.v + bz * p.kv_bs + kvh * p.kv_hs;
+    const int nstep = mk.C / 32 + (mk.S + 31) / 32;
+    u32x4 kf[KS], vf[NV];
+    auto request = [&](int i) {
+        const int r0 = row0 + 32 * i;
+        const uint16_t* kp = kb + (int64_t)min(r0 + lq, mk.Sq - 1) * p.kv_rs + 8 * lh;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) kf[s] = *reinterpret_cast<const u32x4*>(kp + 16 * s);
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int idx = j * 64 + lane;
+            vf[j] = *reinterpret_cast<const u32x4*>(vb + (int64_t)min(r0 + idx / CPR, mk.Sq - 1) * p.kv_rs + 8 * (idx % CPR));
+        }
+    };
+    // 64-byte segment s of row r at s ^ vsw(r), as in the walk of the text rows
+    auto vsw = [](int r) { return D >= 128 ? (r & 3) : ((r >> 1) & 1); };
+    floatx16 oacc[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) oacc[b][i] = 0.f;
+    float m_run = -1e30f, l_run = 0.f;
+    request(0);
+    for (int i = 0; i < nstep; ++i) {
+        floatx16 sc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[e] = 0.f;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) sc = Ops::mfma(kf[s], qf[s], sc);
+        ksa_wave_lds_fence();  // the reads of the step before are done
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int idx = j * 64 + lane, r = idx / CPR, c = idx % CPR;
+            *reinterpret_cast<u32x4*>(reinterpret_cast<char*>(tile) + r * ROWB + (c ^ (vsw(r) << 2)) * 16) = vf[j];
+        }
+        ksa_wave_lds_fence();
+        if (i + 1 < nstep) request(i + 1);
+        const int last = mk.C + sr - 32 * i;  // the last row of this step that the column sees
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            if (8 * (e / 4) + 4 * lh + e % 4 > last) sc[e] = -INFINITY;
+            mloc = fmaxf(mloc, sc[e]);
+        }
+        const float m_new = fmaxf(m_run, ksa_pair_max(mloc));
+        const float alpha = ksa_exp2((m_run - m_new) * p.scale_log2), mc = m_new * p.scale_log2;
+        m_run = m_new;
+        l_run *= alpha;
+        u32x4 pf[2];
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            pf[w / 4][w % 4] = Ops::pack2(ksa_exp2(fmaf(sc[2 * w], p.scale_log2, -mc)),
+                                          ksa_exp2(fmaf(sc[2 * w + 1], p.scale_log2, -mc)));
+            l_run = Ops::sum2(pf[w / 4][w % 4], l_run);
+        }
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) oacc[b][e] *= alpha;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                typedef __attribute__((address_space(3))) ksa_short4* lds_ptr;
+                const int t = lq & 15, r = 16 * ks + 4 * lh + (t >> 2);
+                const char* pv = reinterpret_cast<const char*>(tile) + r * ROWB + (b ^ vsw(r)) * 64 + ((lq & 16) + 4 * (t & 3)) * 2;
+                const u32x2 l2 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(pv)));
+                const u32x2 h2 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(pv + 8 * ROWB)));
+                u32x4 f;
+                f[0] = l2[0];
+                f[1] = l2[1];
+                f[2] = h2[0];
+                f[3] = h2[1];
+                oacc[b] = Ops::mfma(f, pf[ks], oacc[b]);
+            }
+        }
+    }
+    const float l_tot = ksa_pair_sum(l_run);
+    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if (col >= ncol) return;
+    uint16_t* ob = p.out + bz * p.o_bs + (int64_t)qrow * p.o_rs + head * p.o_hs + 4 * lh;
+#pragma unroll
+    for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            u32x2 w;
+            w[0] = Ops::pack2(oacc[b][4 * j] * inv, oacc[b][4 * j + 1] * inv);
+            w[1] = Ops::pack2(oacc[b][4 * j + 2] * inv, oacc[b][4 * j + 3] * inv);
+            *reinterpret_cast<u32x2*>(ob + 32 * b + 8 * j) = w;
+        }
+    if (p.lse && lh == 0)
+        p.lse[bz * p.lse_bs + head * p.lse_hs + qrow] = l_tot > 0.f ? m_run * p.scale + logf(l_tot) : -INFINITY;
+}
+
 template <typename T, int D, int kAddr, int RB, int HW>
 __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 128 ? 2 : 1)) void ksa_prefill_kernel(
     const PrefillParams p) {
@@ -202,6 +382,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     constexpr int RSTEP = kThreads / CPR;           // row distance between a thread's loads
     constexpr bool kRegular = kAddr != kAddrGeneral;
     constexpr bool kMarks = kAddr == kAddrMarked;
+    constexpr bool kChunks = kAddr == kAddrChunks;
     constexpr float kTau = 8.f;      // lazy rescale: exponents stay below 2^kTau
 
     // K and V tiles travel global -> LDS directly (global_load_lds), 1 KB per wave
@@ -242,30 +423,67 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         item = s_item;
         if (item < 0) return;  // every queue is empty: a spare workgroup
     }
-    const int bz = p.by_items.div(item);
-    const int id = item - bz * p.n_items;
-    const int rest = p.by_hkv.div(id);
-    const int kvh = id - rest * p.Hkv;
+    // (chunk tiles: the batch element runs next, so that the heavy tiles of all sequences come first)
+    int bz, kvh, rest;
+    if constexpr (kChunks) {
+        const int x = p.by_hkv.div(item);
+        kvh = item - x * p.Hkv;
+        rest = p.by_items.div(x);
+        bz = x - rest * (int)p.by_items.d;
+    } else {
+        bz = p.by_items.div(item);
+        const int id = item - bz * p.n_items;
+        rest = p.by_hkv.div(id);
+        kvh = id - rest * p.Hkv;
+    }
     constexpr int kWavesPerHead = 4 / RB;
 
-    const int up = p.by_gper.div(rest);
-    const int gi = rest - up * (p.g / HW);
-    const int mt = p.M - 1 - up;
+    int up, gi, mt;
+    if (!kChunks || rest < p.rest_units) {
+        up = p.by_gper.div(rest);
+        gi = rest - up * (p.g / HW);
+        mt = p.M - 1 - up;
+    } else {
+        // Groups of as many chunks as the workgroup has waves, the last ones first: their summary rows, a chunk per wave, then
+        // their text rows, which find the group's K/V in the L2.
+        constexpr int kWaves = PrefillShape<RB, HW>::kWaves;
+        const int u = rest - p.rest_units, grp = p.by_group.div(u), r = u - grp * (int)p.by_group.d;
+        const int end = p.n_chunks - grp * kWaves;
+        if (r < p.sum_blocks) {
+            uint16_t* tile = wave / (kWaves / 4) == 0 ? Ks0 : wave / (kWaves / 4) == 1 ? Ks1 : wave / (kWaves / 4) == 2 ? Vs0 : Vs1;
+            if (end - 1 - wave >= 0)
+                ksa_summary_rows<T, D>(p, bz, kvh, end - 1 - wave, r, lane, tile + (kWaves == 8 ? (wave & 1) * 32 * D : 0));
+            return;
+        }
+        up = p.by_gper.div(r - p.sum_blocks);
+        gi = r - p.sum_blocks - up * (p.g / HW);
+        mt = end * (int)p.by_mt.d - 1 - up;
+    }
     // The counts and the first entries of the two lists of tiles are requested before anything else (rows of the
     // index are N entries, zeroed behind the counts): they head the chain of trips to memory in front of the first
     // tile, and with the counts awaited before the entries it was one trip longer (with the divisions gone too, a
     // workgroup starts its walk 3.2 instead of 4.5 us behind its own start at 300 tokens, 4.8 instead of 6.0 at 4k:
     // 38.2 against 39.6 us a launch there, 933 against 955 us at 32k, +1.1 % at 128k).
-    const int32_t* plist = p.mask_idx + (int64_t)mt * p.idx_stride;
-    const int32_t* flist = p.full_idx + (int64_t)mt * p.idx_stride;
-    const int npart = p.mask_cnt[mt];
-    const int nfull = p.full_cnt[mt];
-    const int list_p0 = plist[min(lane, p.idx_stride - 1)];
-    const int list_p1 = plist[min(64 + lane, p.idx_stride - 1)];
-    const int list_f0 = flist[min(lane, p.idx_stride - 1)];
+    const int32_t* plist = nullptr;
+    const int32_t* flist = nullptr;
+    int npart = 0, nfull = 0, list_p0 = 0, list_p1 = 0, list_f0 = 0;
+    if constexpr (!kChunks) {
+        plist = p.mask_idx + (int64_t)mt * p.idx_stride;
+        flist = p.full_idx + (int64_t)mt * p.idx_stride;
+        npart = p.mask_cnt[mt];
+        nfull = p.full_cnt[mt];
+        list_p0 = plist[min(lane, p.idx_stride - 1)];
+        list_p1 = plist[min(64 + lane, p.idx_stride - 1)];
+        list_f0 = flist[min(lane, p.idx_stride - 1)];
+    }
     const int head = kvh * p.g + HW * gi + wave / kWavesPerHead;
-    const int row0 = mt * kTileM + (wave % kWavesPerHead) * 32 * RB;
     const KsaMask mk = p.mk;
+    const ChunkTile ct = kChunks ? ksa_chunk_tile(p, mt) : ChunkTile{};
+    // (chunk tiles, two heads: the second head's waves take the rows in reverse order, so that every SIMD - it holds waves
+    // w and w + 4 - has one wave with work on the second half of the diagonal)
+    const int wrow = wave % kWavesPerHead;
+    const int row0 = (kChunks ? ct.p0 : mt * kTileM) +
+                     (kChunks && HW == 2 && wave >= kWavesPerHead ? kWavesPerHead - 1 - wrow : wrow) * 32 * RB;
     const bool prefix_mode = mk.P > 0;
     const bool phys = p.phys_prefix != 0;
     const int Bblk = mk.C + mk.S;
@@ -278,7 +496,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     for (int r = 0; r < RB; ++r) {
         qrow[r] = row0 + 32 * r + lq;
         const int qrow_c = min(qrow[r], mk.Sq - 1);
-        rv[r] = ksa_row_vis(mk, p.by_block, qrow_c);
+        if constexpr (!kChunks) rv[r] = ksa_row_vis(mk, p.by_block, qrow_c);
         const uint16_t* qp = p.q + bz * p.q_bs + (int64_t)qrow_c * p.q_rs + head * p.q_hs + 8 * lh;
 #pragma unroll
         for (int s = 0; s < KS; ++s) qf[r][s] = *reinterpret_cast<const u32x4*>(qp + 16 * s);
@@ -302,9 +520,14 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     const uint32_t thr_main = (uint32_t)ld_row * rb;
     // in-place prefix: prefix row j lives at in-line row (j / S) * B + C + j % S; when S
     // divides the per-thread row step the rows of one thread differ by a uniform amount
-    const bool s_fast = !phys && p.by_S.mod(RSTEP) == 0;
+    const bool s_fast = kChunks || (!phys && p.by_S.mod(RSTEP) == 0);
+    // (chunk tiles: a prefix of fewer rows than a load repeats its last one)
+    const int pre_row = kChunks ? min(ld_row, max(ct.pre_rows, 1) - 1) : ld_row;
     const uint32_t thr_pre =
-        s_fast ? (uint32_t)(p.by_S.div(ld_row) * Bblk + mk.C + p.by_S.mod(ld_row)) * rb : 0u;
+        s_fast ? (uint32_t)(p.by_S.div(pre_row) * Bblk + mk.C + p.by_S.mod(pre_row)) * rb : 0u;
+    // ... and one of fewer rows than a tile takes the last load's worth of rows again in its later loads
+    const uint32_t pre_last = kChunks && ct.pre_rows < kTileN
+                                  ? (uint32_t)(p.by_S.div(max(ct.pre_rows - RSTEP, 0)) * Bblk) * rb : ~0u;
     const uint32_t step_main = RSTEP * rb;
     const uint32_t step_pre = s_fast ? (uint32_t)p.by_S.div(RSTEP) * Bblk * rb : 0u;
 
@@ -381,7 +604,9 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         } else {
             tile_src(n * kTileN, i, ub, us, vo);
         }
-        fill_from(base + (ub + us * i), vo + (col ^ ((i & 1) ? odd_xor : 0u)), tile, i);
+        uint32_t at = us * i;
+        if constexpr (kChunks) at = min(at, (word & 1u) ? ~0u : pre_last);
+        fill_from(base + (ub + at), vo + (col ^ ((i & 1) ? odd_xor : 0u)), tile, i);
     };
     // the rows of a tile that is not regular, over what the loop's fills put there (which have to have landed):
     // a row of the prefix by the regular rule, a row of the in-line region or the last one where it is cut
@@ -440,14 +665,14 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     };
 
     // ---- walk order ----
-    const int ntiles = npart + nfull;
+    const int ntiles = kChunks ? ct.n_a + (ct.rem ? 1 : 0) + ct.n_diag : npart + nfull;
     int nquick = 0;
     // the marked tile at the end of the prefix, if the row tile lists it: its position in the list
     const int n_mark = kMarks && !phys && mk.P % kTileN != 0 ? mk.P / kTileN : -1;
     int mark_pos = 0;
     bool has_mark = false;
     int c0 = 0, c1 = 0;  // entries [c0, c1) of the list of partial tiles: the uniform in-line tiles described below
-    {
+    if constexpr (!kChunks) {
         const int c_first = p.by_block.div(mt * kTileM);
         const int w_first = c_first > mk.W ? c_first - mk.W : 0;
         // every text row of the tile has xa >= w_first * S and blo >= P >= thr
@@ -503,13 +728,13 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         c0 = max(cnt0, nquick);
         c1 = max(cnt1, c0);
     }
-    const bool last_full_cut = mk.Sk % kTileN != 0 && nfull > 0 && (flist[nfull - 1] + 1) * kTileN > mk.Sk;
+    const bool last_full_cut = !kChunks && mk.Sk % kTileN != 0 && nfull > 0 && (flist[nfull - 1] + 1) * kTileN > mk.Sk;
     const int nfull_a = nfull - (last_full_cut ? 1 : 0);
     // Walk order.  Phase A: the leading prefix tiles, the uniform in-line tiles, the full tiles; phase B:
     // the other partial tiles (those in front of the uniform run, those behind it, a cut full tile; the
     // tile at the end of the prefix last).
     const int ncheap = c1 - c0;
-    const int n_a = nquick + ncheap + nfull_a;
+    const int n_a = kChunks ? ct.n_a : nquick + ncheap + nfull_a;
     // (the marked tile's place among phase B's entries: it is never one of phase A)
     const int mark_j = mark_pos - nquick - (mark_pos >= c1 ? ncheap : 0);
     // Steps of phase A that may run as such: a step requests the tiles of the next two, and the marked ones - the
@@ -545,15 +770,28 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         if (live && a >= (k < 0 ? 64 : 128)) n = k < 0 ? flist[a] : plist[a];
         return live ? n : 0;
     };
-    int seq_cur = first_chunk(0);
-    int seq_nxt = first_chunk(64);
-    uint32_t word_cur = kRegular ? tile_word(seq_cur) : 0u;
-    uint32_t word_nxt = kRegular ? tile_word(seq_nxt) : 0u;
+    // Chunk tiles: the order is known in closed form, only its words are kept
+    auto chunk_word = [&](int i) -> uint32_t {
+        const int t = i - ct.n_pre, d = i - (ntiles - ct.n_diag);
+        if (t < 0 || (i >= n_a && d < 0))  // rows of the prefix; the last tile ends with the last row
+            return (uint32_t)(p.by_S.div(t < 0 ? i * kTileN : max(ct.pre_rows - kTileN, 0)) * Bblk) * rb;
+        const int c = p.by_nt.div(t);
+        const int row = d < 0 ? (ct.w0 + c) * Bblk + (t - c * (int)p.by_nt.d) * kTileN : ct.diag0(d, mk.Sq);
+        return (uint32_t)row * rb | 1u;
+    };
+    auto words_of = [&](int seq_entry, int base) -> uint32_t {
+        if constexpr (kChunks) return chunk_word(min(base + lane, ntiles - 1));
+        return kRegular ? tile_word(seq_entry) : 0u;
+    };
+    int seq_cur = kChunks ? 0 : first_chunk(0);
+    int seq_nxt = kChunks ? 0 : first_chunk(64);
+    uint32_t word_cur = words_of(seq_cur, 0);
+    uint32_t word_nxt = words_of(seq_nxt, 64);
     // Where a tile's first column stands in the period of C text + S summary columns of the
     // in-line region, (n0 - P) mod (C + S) in [0, C + S): computed with the walk order, one
     // division per lane and 64 tiles, so that the masked steps have none.
     auto tile_phase = [&](int n) {
-        return p.by_block.mod(n * kTileN - mk.P + p.phase_shift);
+        return kChunks ? 0 : p.by_block.mod(n * kTileN - mk.P + p.phase_shift);
     };
     int phase_cur = tile_phase(seq_cur);
     int phase_nxt = tile_phase(seq_nxt);
@@ -622,14 +860,15 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     auto step = [&](auto safe_tag, auto general_tag, auto parity_tag, int it, floatx16 (&scur)[RB][2],
                     floatx16 (&snext)[RB][2], bool quick) __attribute__((always_inline)) {
         constexpr bool kSafe = decltype(safe_tag)::value;
-        constexpr bool kGeneral = decltype(general_tag)::value;
+        constexpr bool kGeneral = decltype(general_tag)::value != 0;
+        constexpr bool kLast = decltype(general_tag)::value == 2;
         constexpr int PAR = decltype(parity_tag)::value;
-        const int n0 = seq(it, it) * kTileN;
+        const int n0 = kChunks ? 0 : seq(it, it) * kTileN;
         // Past the end of the walk the pipeline keeps running on the last tile (fills) and
         // on stale LDS contents (scores); those results are never used.
         // fills: K(it+2) and V(it+1), both issued in the first slots of the score stage
         const int ik = min(it + 2, ntiles - 1), iv = min(it + 1, ntiles - 1);
-        const int nk = seq(ik, it), nv = seq(iv, it);
+        const int nk = kChunks ? 0 : seq(ik, it), nv = kChunks ? 0 : seq(iv, it);
         const uint32_t wk = seq_word(ik, it), wv = seq_word(iv, it);
         bool row_vis[RB];
 #pragma unroll
@@ -654,7 +893,7 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         auto vfrag = [&](int j) { return read_v(vsrc, j); };
         __builtin_amdgcn_sched_barrier(0);
 
-        if constexpr (!kGeneral) {
+        if constexpr (!kGeneral && !kChunks) {
             if (quick && it >= nquick) {
                 // a uniform in-line tile (see the walk order): if it holds the group of summary columns of a
                 // chunk, those eight keys are hidden from every row - in the score layout they are four
@@ -683,16 +922,6 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             }
         }
         if constexpr (kGeneral) {  // 64-bit visibility word per row
-            const int kv = n0 + lane;
-            const bool in = kv < mk.Sk;
-            const uint64_t valid = __ballot(in);
-            // text column: its offset in the period is below C.  phase + lane is below two periods
-            // when a period holds a tile's 64 columns (any real chunk size).
-            int o = seq_phase(it, it) + lane;
-            if (Bblk >= kTileN) o -= o >= Bblk ? Bblk : 0;
-            else o %= Bblk;
-            const uint64_t text = valid & __ballot(kv >= mk.P) & __ballot(o < mk.C);
-            const uint64_t fa = prefix_mode ? valid : (valid & ~text);
             // bits [lo, hi) of a 64-bit word, without a branch
             auto range_bits = [](int lo, int hi) {
                 lo = max(lo, 0);
@@ -714,13 +943,35 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
                     sc[i] = __uint_as_float((__float_as_uint(sc[i]) & m) | (0xff800000u & ~m));
                 }
             };
-            // (uniform) a tile of the in-line region behind a prefix: no row's [0, xa) reaches it
-            const bool no_xa = prefix_mode && n0 >= mk.P;
+            uint64_t text = 0ull, valid = 0ull, fa = 0ull;
+            bool no_xa = true;
+            if constexpr (!kChunks) {
+                const int kv = n0 + lane;
+                const bool in = kv < mk.Sk;
+                valid = __ballot(in);
+                // text column: its offset in the period is below C.  phase + lane is below two periods
+                // when a period holds a tile's 64 columns (any real chunk size).
+                int o = seq_phase(it, it) + lane;
+                if (Bblk >= kTileN) o -= o >= Bblk ? Bblk : 0;
+                else o %= Bblk;
+                text = valid & __ballot(kv >= mk.P) & __ballot(o < mk.C);
+                fa = prefix_mode ? valid : (valid & ~text);
+                // (uniform) a tile of the in-line region behind a prefix: no row's [0, xa) reaches it
+                no_xa = prefix_mode && n0 >= mk.P;
+            }
+            // (chunk tiles, uniform) tile of the diagonal, or -1: the last rows of the prefix
+            const int d = kChunks ? it - (ntiles - ct.n_diag) : 0;
 #pragma unroll
             for (int r = 0; r < RB; ++r) {
-                const uint64_t fb = rv[r].b_text ? text : valid;
-                uint64_t bits = range_bits(rv[r].blo - n0, rv[r].bhi - n0) & fb;
-                if (!no_xa) bits |= range_bits(-n0, rv[r].xa - n0) & fa;
+                uint64_t bits;
+                if constexpr (kChunks) {
+                    const int first = ct.p0 + d * kTileN, from = ct.diag0(d, mk.Sq);
+                    bits = d < 0 ? ct.pre_bits(RSTEP) : range_bits(first - from, qrow[r] + 1 - from);
+                } else {
+                    const uint64_t fb = rv[r].b_text ? text : valid;
+                    bits = range_bits(rv[r].blo - n0, rv[r].bhi - n0) & fb;
+                    if (!no_xa) bits |= range_bits(-n0, rv[r].xa - n0) & fa;
+                }
                 // a row that sees nothing of the tile loses it through its reference (infinite:
                 // every probability 0) and does not keep a half from being skipped
                 const bool any = bits != 0ull;
@@ -806,6 +1057,38 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             for (int r = 0; r < RB; ++r) mc[r] = row_vis[r] ? m_ref[r] * c2 : INFINITY;
         }
 
+        // The last tile of a walk over chunk tiles, the second half of the diagonal: there is no next tile to score or to
+        // fetch, and the waves whose rows all lie in front of it have nothing to do.
+        if constexpr (kLast) {
+            bool any = false;
+#pragma unroll
+            for (int r = 0; r < RB; ++r) any = any || row_vis[r];
+            if (__ballot(any) != 0ull) {
+#pragma unroll
+                for (int j = 0; j < kQueue; ++j) fq[j] = vfrag(j);
+#pragma unroll
+                for (int vt = 0; vt < 7; ++vt) prob_slot(vt);  // the first 16 keys' pairs
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < NPV; ++j) {
+#pragma unroll
+                    for (int r = 0; r < RB; ++r)
+                        oacc[r][j % DB] = Ops::mfma(fq[j % kQueue], pf[r][j / DB], oacc[r][j % DB]);
+                    if (j + kQueue < NPV) fq[j % kQueue] = vfrag(j + kQueue);
+                    // (the next 16 keys' pairs between the MFMAs of these)
+#pragma unroll
+                    for (int vt = 7 + 4 * j / DB; vt < 7 + 4 * (j + 1) / DB; ++vt) prob_slot(vt);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+#pragma unroll
+                for (int r = 0; r < RB; ++r) {
+                    if constexpr (!kSafe) bad = bad || l_tile[r] > 16777216.f;
+                    l_run[r] += l_tile[r];
+                }
+            }
+            return;
+        }
+
         // Score MFMAs of the NEXT tile with the probability pairs of THIS tile between them.
         // The fences pin the order; kLead slots run first and cover the first operand reads.
         // The first slots also issue the fills of the two buffers freed by the barrier.
@@ -876,8 +1159,8 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             seq_cur = seq_nxt;
             word_cur = word_nxt;
             phase_cur = phase_nxt;
-            seq_nxt = seq_chunk(it + 1 + 64);
-            word_nxt = kRegular ? tile_word(seq_nxt) : 0u;
+            seq_nxt = kChunks ? 0 : seq_chunk(it + 1 + 64);
+            word_nxt = words_of(seq_nxt, it + 1 + 64);
             phase_nxt = tile_phase(seq_nxt);
         }
     };
@@ -902,13 +1185,15 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
     using Odd = std::integral_constant<int, 1>;
     auto walk = [&](auto safe_tag) __attribute__((always_inline)) {
         constexpr bool kSafe = decltype(safe_tag)::value;
-        using A = std::false_type;
-        using B = std::true_type;
+        using A = std::integral_constant<int, 0>;
+        using B = std::integral_constant<int, 1>;
+        using Last = std::integral_constant<int, 2>;
+        const bool odd = kChunks && !(ntiles & 1);  // the first tile's place in the pairs of buffers
         if constexpr (kSafe) {  // from the start again
-            seq_cur = seq_chunk(0);
-            seq_nxt = seq_chunk(64);
-            word_cur = kRegular ? tile_word(seq_cur) : 0u;
-            word_nxt = kRegular ? tile_word(seq_nxt) : 0u;
+            seq_cur = kChunks ? 0 : seq_chunk(0);
+            seq_nxt = kChunks ? 0 : seq_chunk(64);
+            word_cur = words_of(seq_cur, 0);
+            word_nxt = words_of(seq_nxt, 64);
             phase_cur = tile_phase(seq_cur);
             phase_nxt = tile_phase(seq_nxt);
         }
@@ -923,9 +1208,9 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
         }
         if (ntiles > 0) {  // prologue: K(0), V(0), K(1) in LDS, scores of tile 0
             const int i1 = min(1, ntiles - 1);
-            fill(kbase, Ks0, kcol, seq(0, 0), seq_word(0, 0), kKOdd);
-            fill(vbase, Vs0, vcol, seq(0, 0), seq_word(0, 0), 0u);
-            fill(kbase, Ks1, kcol, seq(i1, 0), seq_word(i1, 0), kKOdd);
+            fill(kbase, odd ? Ks1 : Ks0, kcol, seq(0, 0), seq_word(0, 0), kKOdd);
+            fill(vbase, odd ? Vs1 : Vs0, vcol, seq(0, 0), seq_word(0, 0), 0u);
+            fill(kbase, odd ? Ks0 : Ks1, kcol, seq(i1, 0), seq_word(i1, 0), kKOdd);
             fills_done();
             if constexpr (kMarks) {
                 if ((seq_word(0, 0) | seq_word(i1, 0)) & kSpecialBit) {
@@ -938,9 +1223,9 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
                 }
             }
             __syncthreads();
-            scores(s0, Ks0);
+            scores(s0, odd ? Ks1 : Ks0);
 #pragma unroll
-            for (int j = 0; j < kQueue; ++j) fq[j] = read_k(Ks1, j);  // the first step's first operands
+            for (int j = 0; j < kQueue; ++j) fq[j] = read_k(odd ? Ks0 : Ks1, j);  // the first step's first operands
             // the first step refills K(0)'s buffer at once: every wave must be done reading it
             wg_barrier();
             if constexpr (!kSafe) {
@@ -954,6 +1239,35 @@ __global__ __launch_bounds__((PrefillShape<RB, HW>::kThreads), (RB == 1 && D <= 
             }
         }
         int it = 0;
+        if constexpr (kChunks) {
+            // the last tile is an even step: an odd one first where their number asks for it
+            if (odd && n_a > 0) {
+                step(safe_tag, A{}, Odd{}, it, s0, s1, false);
+                copy_scores();
+                ++it;
+            }
+            for (; it + 2 <= n_a; it += 2) {
+                step(safe_tag, A{}, Even{}, it, s0, s1, false);
+                step(safe_tag, A{}, Odd{}, it + 1, s1, s0, false);
+            }
+            if (it < n_a) {
+                step(safe_tag, A{}, Even{}, it, s0, s1, false);
+                copy_scores();
+                ++it;
+            }
+            if (it + 3 == ntiles) {
+                step(safe_tag, B{}, Even{}, it, s0, s1, false);
+                copy_scores();
+                ++it;
+            }
+            if (it + 2 == ntiles) {
+                step(safe_tag, B{}, Odd{}, it, s0, s1, false);
+                copy_scores();
+                ++it;
+            }
+            step(safe_tag, Last{}, Even{}, it, s0, s1, false);
+            return;
+        }
         for (; it + 2 <= n_run; it += 2) {
             step(safe_tag, A{}, Even{}, it, s0, s1, it < nquick + ncheap);
             step(safe_tag, A{}, Odd{}, it + 1, s1, s0, it + 1 < nquick + ncheap);
@@ -1062,13 +1376,21 @@ int prefill_addr(const PrefillParams& p) {
 template <typename T, int D, int RB, int HW>
 int launch_shape(const PrefillParams& p, int batch, hipStream_t stream) {
     constexpr int kThreads = PrefillShape<RB, HW>::kThreads;
-    const int addr = prefill_addr<D, RB, HW>(p);
-    if (KSA_PREFILL_VARIANT >= 0 && addr != KSA_PREFILL_VARIANT) return KSA_ERR_INVALID;
+    const int addr = p.chunk_tiles ? kAddrChunks : prefill_addr<D, RB, HW>(p);
+    if (KSA_PREFILL_VARIANT < 0 ? addr == kAddrChunks : addr != KSA_PREFILL_VARIANT) return KSA_ERR_INVALID;
     PrefillParams pp = p;
     pp.n_items = p.M * (p.Hq / HW);
+    if (addr == kAddrChunks) {
+        constexpr int kWaves = PrefillShape<RB, HW>::kWaves;
+        const int per_tile = p.g / HW, mt = (int)p.by_mt.d;
+        pp.rest_units = (p.M - p.n_chunks * mt) * per_tile;
+        pp.sum_blocks = (p.g * p.mk.S + 31) / 32;
+        pp.by_group = FastDiv((uint32_t)(pp.sum_blocks + kWaves * mt * per_tile));
+        pp.n_items += (p.n_chunks + kWaves - 1) / kWaves * pp.sum_blocks * p.Hkv;
+    }
     pp.total = pp.n_items * batch;
     pp.n_static = pp.total;
-    pp.by_items = FastDiv((uint32_t)pp.n_items);
+    pp.by_items = FastDiv((uint32_t)(addr == kAddrChunks ? batch : pp.n_items));
     pp.by_hkv = FastDiv((uint32_t)p.Hkv);
     pp.by_gper = FastDiv((uint32_t)(p.g / HW));
     int spare = 0;
@@ -1086,13 +1408,14 @@ int launch_shape(const PrefillParams& p, int batch, hipStream_t stream) {
     dim3 grid(pp.total + spare);
     auto go = [&](auto tag) {
         constexpr int kAddr = decltype(tag)::value;
-        if constexpr ((KSA_PREFILL_VARIANT < 0 || KSA_PREFILL_VARIANT == kAddr) && !(kAddr == kAddrMarked && RB != 1))
+        if constexpr ((KSA_PREFILL_VARIANT < 0 ? kAddr != kAddrChunks : KSA_PREFILL_VARIANT == kAddr) && (kAddr <= kAddrRegular || RB == 1))
             if (addr == kAddr)
                 hipLaunchKernelGGL((ksa_prefill_kernel<T, D, kAddr, RB, HW>), grid, dim3(kThreads), 0, stream, pp);
     };
     go(std::integral_constant<int, kAddrGeneral>{});
     go(std::integral_constant<int, kAddrRegular>{});
     go(std::integral_constant<int, kAddrMarked>{});
+    go(std::integral_constant<int, kAddrChunks>{});
     return ksa_check_launch();
 }
 
@@ -1108,7 +1431,7 @@ int launch(const PrefillParams& p, int batch, hipStream_t stream) {
     return launch_shape<T, D, 1, 1>(p, batch, stream);
 }
 
-#if KSA_PREFILL_UNIT == 0
+#if KSA_PREFILL_UNIT == 0 || KSA_PREFILL_UNIT == 9
 bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 bool stride_ok(int64_t s) { return (s % 8) == 0; }
 #endif
@@ -1123,6 +1446,8 @@ int KSA_PREFILL_D256(bf16, marked);
 int KSA_PREFILL_D256(f16, general);
 int KSA_PREFILL_D256(f16, regular);
 int KSA_PREFILL_D256(f16, marked);
+int KSA_PREFILL_D256(bf16, chunks);
+int KSA_PREFILL_D256(f16, chunks);
 #if KSA_PREFILL_UNIT == 1
 int KSA_PREFILL_D256(bf16, general)
 #elif KSA_PREFILL_UNIT == 2
@@ -1135,13 +1460,17 @@ int KSA_PREFILL_D256(f16, general)
 int KSA_PREFILL_D256(f16, regular)
 #elif KSA_PREFILL_UNIT == 6
 int KSA_PREFILL_D256(f16, marked)
+#elif KSA_PREFILL_UNIT == 7
+int KSA_PREFILL_D256(bf16, chunks)
+#elif KSA_PREFILL_UNIT == 8
+int KSA_PREFILL_D256(f16, chunks)
 #endif
-#if KSA_PREFILL_UNIT >= 1
+#if KSA_PREFILL_UNIT >= 1 && KSA_PREFILL_UNIT <= 8
 {
-    return launch<std::conditional_t<(KSA_PREFILL_UNIT <= 3), KsaBf16, KsaF16>, 256>(
+    return launch<std::conditional_t<(KSA_PREFILL_UNIT <= 3 || KSA_PREFILL_UNIT == 7), KsaBf16, KsaF16>, 256>(
         *static_cast<const PrefillParams*>(params), batch, (hipStream_t)stream);
 }
-#else
+#elif KSA_PREFILL_UNIT == 0
 
 extern "C" int ksa_prefill_fwd(const void* q, const void* k, const void* v, void* out, float* lse,
                                int batch, int Sq, int Hq, int Hkv, int D, int dtype,
@@ -1232,5 +1561,73 @@ extern "C" int ksa_prefill_fwd(const void* q, const void* k, const void* v, void
         }
     }
     return KSA_ERR_UNSUPPORTED;  // other head dimensions: the caller pads to 64 / 128 / 256
+}
+#else
+
+extern "C" int ksa_prefill_chunks_fwd(const void* q, const void* k, const void* v, void* out, float* lse, int batch,
+                                      int Sq, int Hq, int Hkv, int D, int dtype, const int64_t* q_strides,
+                                      const int64_t* kv_strides, const int64_t* out_strides, int C, int S, int W,
+                                      int skip_old, float scale, int shape, int32_t* sched, void* stream) {
+    if (!q || !k || !v || !out || !q_strides || !kv_strides || !out_strides) return KSA_ERR_NULL;
+    if (batch <= 0 || Sq <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0) return KSA_ERR_INVALID;
+    if (C <= 0 || S <= 0 || W < 0 || (int64_t)Sq * 2 >= (1ll << 30)) return KSA_ERR_INVALID;
+    if (dtype != KSA_DTYPE_BF16 && dtype != KSA_DTYPE_F16) return KSA_ERR_UNSUPPORTED;
+    if (D != 64 && D != 128 && D != 256) return KSA_ERR_UNSUPPORTED;
+    if (shape != 0 && shape != 2 && shape != 32) return KSA_ERR_INVALID;
+    // what the kernel takes for granted, see kAddr
+    if (C % kTileM != 0 || C > 512 || (8 % S != 0 && !(S == 16 && D <= 128))) return KSA_ERR_UNSUPPORTED;
+    const int block = C + S, n_chunks = Sq / block, rest = Sq - n_chunks * block;
+    if (Sq < kTileN || rest > C) return KSA_ERR_UNSUPPORTED;
+    if ((int64_t)Sq * kv_strides[1] * 2 >= (1ll << 32)) return KSA_ERR_INVALID;
+    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out)) return KSA_ERR_ALIGN;
+    for (int i = 0; i < 3; ++i)
+        if (!stride_ok(q_strides[i]) || !stride_ok(kv_strides[i]) || !stride_ok(out_strides[i])) return KSA_ERR_ALIGN;
+
+    PrefillParams p{};
+    p.q = (const uint16_t*)q;
+    p.k = (const uint16_t*)k;
+    p.v = (const uint16_t*)v;
+    p.out = (uint16_t*)out;
+    p.lse = lse;
+    p.M = n_chunks * (C / kTileM) + (rest + kTileM - 1) / kTileM;
+    p.Hq = Hq;
+    p.Hkv = Hkv;
+    p.g = Hq / Hkv;
+    p.q_bs = q_strides[0], p.q_rs = q_strides[1], p.q_hs = q_strides[2];
+    p.kv_bs = kv_strides[0], p.kv_rs = kv_strides[1], p.kv_hs = kv_strides[2];
+    p.o_bs = out_strides[0], p.o_rs = out_strides[1], p.o_hs = out_strides[2];
+    p.lse_bs = (int64_t)Hq * Sq;
+    p.lse_hs = Sq;
+    p.mk = KsaMask{C, S, W, n_chunks * S, skip_old ? 1 : 0, Sq, Sq + n_chunks * S};
+    p.scale = scale;
+    p.scale_log2 = scale * 1.4426950408889634f;
+    p.by_block = FastDiv((uint32_t)block);
+    p.by_S = FastDiv((uint32_t)S);
+    p.chunk_tiles = 1;
+    p.n_chunks = n_chunks;
+    p.by_mt = FastDiv((uint32_t)(C / kTileM));
+    p.by_nt = FastDiv((uint32_t)(C / kTileN));
+    p.sched = sched;
+    // Workgroup shape (D = 128, even group size): one head on 4 waves, two workgroups per CU that hide each other's start
+    // and end, until the two-head workgroups would have 128 tile steps per CU to do; then two heads on 8 waves, for which
+    // one K/V tile in LDS serves twice the work.  One / two heads, us (32 / 8 heads, bf16; steps per CU): window of 4
+    // chunks, 4k tokens 57.8 / 62.6 (24), 8k 125.7 / 128.0 (50), 16k 304 / 306 (118), 24k 540 / 528 (200); unbounded window, 4k
+    // 141.6 / 141.8 (70), 9001 tokens 598 / 573 (330), three sequences of that length 1776 / 1698.
+    int64_t steps = 3ll * p.M;
+    {
+        const int64_t n = n_chunks + (rest > 0), far = n > W ? n - W : 0, near = n - far;
+        steps += C / kTileM * (C / kTileN * (near * (near - 1) / 2 + far * near) + (skip_old ? 0 : far * (far + 1) / 2 * S / kTileN));
+    }
+    p.shape = shape ? shape : (steps * (Hq / 2) * batch < 128ll * ksa_cu_count_or(256) ? 32 : 2);
+
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == KSA_DTYPE_BF16) {
+        if (D == 128) return launch<KsaBf16, 128>(p, batch, st);
+        if (D == 64) return launch<KsaBf16, 64>(p, batch, st);
+        return ksa_prefill_launch_d256_bf16_chunks(&p, batch, stream);
+    }
+    if (D == 128) return launch<KsaF16, 128>(p, batch, st);
+    if (D == 64) return launch<KsaF16, 64>(p, batch, st);
+    return ksa_prefill_launch_d256_f16_chunks(&p, batch, stream);
 }
 #endif  // KSA_PREFILL_UNIT

@@ -172,6 +172,20 @@ def pad_head_dim(t: torch.Tensor, Dk: int) -> torch.Tensor:
     return t if t.shape[-1] == Dk else torch.nn.functional.pad(t, (0, Dk - t.shape[-1]))
 
 
+# `shape` of a call on chunk tiles (ksa_prefill_chunks_fwd), and the largest chunk that takes them
+_CHUNK_TILES = 128
+_CHUNK_MAX = 512
+
+
+def _chunk_tiles(Sq: int, D: int, C: int, S: int, P: int, phys: bool) -> bool:
+    """Whether a call runs on tiles laid along the chunks instead of the 128 x 64 grid of the block index: whole row
+    tiles to a chunk, a summary count that divides the rows of a load, every summary row (in line or as the prefix that
+    is read in place) behind its whole chunk."""
+    block = C + S
+    return (C % TILE_M == 0 and C <= _CHUNK_MAX and (8 % S == 0 or (S == 16 and D <= 128)) and not phys
+            and Sq >= TILE_N and Sq % block <= C and P in (0, Sq // block * S))
+
+
 def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P, skip_old, phys_prefix, scale, want_lse,
                     shape):
     b, Sq, Hq, D = q.shape
@@ -182,6 +196,16 @@ def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P,
     # workgroups per CU; a workgroup takes 128 rows of one or two heads)
     sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= 1 << 19 else None
     dims = (0, 1, 2)
+    if shape == _CHUNK_TILES:
+        with _lib.on_device(dev):
+            rc = _lib.lib().ksa_prefill_chunks_fwd(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr() if want_lse else None,
+                b, Sq, Hq, k.shape[2], D, _DTYPES[q.dtype],
+                _lib.strides3(q, dims), _lib.strides3(k, dims), _lib.strides3(out, dims),
+                C, S, W, int(skip_old), scale, 0, sched.data_ptr() if sched is not None else None, _lib.stream_ptr(dev))
+        if rc:
+            _lib.check(rc, "ksa_prefill_chunks_fwd")
+        return out, lse
     with _lib.on_device(dev):
         rc = _lib.lib().ksa_prefill_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
@@ -269,16 +293,22 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     if k.stride() != v.stride():
         v = v.contiguous()
         k = k.contiguous()
-    idx = _cached_index(Sq, C, S, W, P, skip_old_summary, q.device)
     scale = float(D) ** -0.5 if softmax_scale is None else float(softmax_scale)
     Dk = kernel_head_dim(D)
     if Dk != D:   # a head dimension without a kernel of its own: zero-padded copies (see kernel_head_dim)
         q, k, v = pad_head_dim(q, Dk), pad_head_dim(k, Dk), pad_head_dim(v, Dk)
-    forward = _launch_prefill if _lib.direct(q, k, v) else torch.ops.ksa_amd.summary_attn_fwd
+    shape = PREFILL_SHAPE if workgroup_shape is None else int(workgroup_shape)
+    direct = _lib.direct(q, k, v)
+    if shape == 0 and _chunk_tiles(Sq, Dk, C, S, P, phys):
+        shape = _CHUNK_TILES
+    elif shape == _CHUNK_TILES:
+        shape = -1   # no shape that a caller can name: refused by the library
+    # (chunk tiles need no block index; the operator's arguments hold one)
+    idx = (None,) * 4 if direct and shape == _CHUNK_TILES else _cached_index(Sq, C, S, W, P, skip_old_summary, q.device)
+    forward = _launch_prefill if direct else torch.ops.ksa_amd.summary_attn_fwd
     out, lse = forward(
         q, k, v, idx[0], idx[1], idx[2], idx[3], C, S, W, P,
-        bool(skip_old_summary), phys, scale, bool(return_lse),
-        PREFILL_SHAPE if workgroup_shape is None else int(workgroup_shape))
+        bool(skip_old_summary), phys, scale, bool(return_lse), shape)
     if Dk != D:
         out = out[..., :D].contiguous()
     return out, (lse if return_lse else None)

@@ -677,3 +677,60 @@ def test_chunk_longer_than_any_sequence(C):
         want, wlse = ksa_amd.summary_attn_func(q[None].cuda(), k[None].cuda(), v[None].cuda(), Sq, S, 1, return_lse=True)
         assert torch.allclose(out.float(), want.float(), rtol=0, atol=ATOL)
         assert torch.allclose(lse, wlse, rtol=0, atol=5e-2)
+
+
+@pytest.mark.parametrize("D, dtype, heads", [(128, torch.bfloat16, (4, 2)), (128, torch.float16, (3, 1)), (64, torch.bfloat16, (8, 1)),
+                                             (256, torch.bfloat16, (2, 2)), (256, torch.float16, (2, 1))])
+@pytest.mark.parametrize("C, S, W", [(128, 8, 4), (128, 8, 0), (128, 4, 1), (256, 2, 1), (512, 1, 0), (128, 8, 1 << 20), (384, 8, 2)])
+def test_prefill_chunk_tiles(C, S, W, D, dtype, heads):
+    """Tiles laid along the chunks: one row tile with one and with two key tiles on the diagonal, lengths that cut
+    either, chunk counts around the prefix of one load, of one tile and of a tile and a half, every column block of the
+    summary rows (8 heads of 8 rows: two), with the summary rows as the prefix, in line and skipped; and the same calls
+    on the block index.  Against the oracle: 16-bit probabilities, as everywhere in this file."""
+    import ksa_amd
+    from ksa_amd import prefill
+    dev = torch.device("cuda")
+    B = C + S
+    for n in (64, 65, 127, C, B + 1, B + C // 2, (W + 2) * B, (W + 9) * B + 64, (W + 13) * B + 65):
+        if W > 100:
+            n = min(n, 9 * B) - (0 if n < 9 * B else 7 * S)
+        if n > 2600:
+            continue
+        q, k, v = (t.to(dtype) for t in make_qkv(n, *heads, D, seed=n + D, scaled=False))
+        sp = O.summary_positions(n, C, S)
+        assert prefill._chunk_tiles(n, D, C, S, int(sp.sum()), False)
+        for spt, skip in ((sp, False), (None, False), (sp, True)):
+            want, wlse = c_oracle.attention_rows(to_np(q), to_np(k), to_np(v), C, S, W, summary_pos=spt, skip_old=skip)
+            for shape in (0, 32):
+                out, lse = ksa_amd.summary_attn_func(
+                    q[None].to(dev), k[None].to(dev), v[None].to(dev), C, S, W, skip_old_summary=skip, return_lse=True,
+                    summary_pos=None if spt is None else torch.as_tensor(sp, device=dev), workgroup_shape=shape)
+                got = to_np(out[0])
+                assert np.isfinite(got).all(), (n, spt is None, skip, shape)
+                assert np.abs(got - want).max() <= ATOL * max(1.0, np.abs(want).max()), (n, spt is None, skip, shape)
+                assert np.abs(to_np(lse[0]) - wlse).max() <= 5e-2, (n, spt is None, skip, shape)
+
+
+@pytest.mark.parametrize("shape", [2, 32])
+def test_prefill_chunk_tiles_of_both_workgroup_shapes(shape):
+    """The two workgroup shapes of the chunk tiles through the C entry point: a strided batch of three, all rows against
+    the same rows on the block index; the walk with exact references (summary keys of a huge norm) included."""
+    import ksa_amd
+    from ksa_amd import _lib
+    dev = torch.device("cuda")
+    C, S, W, Hq, Hkv, D, n = 128, 8, 3, 8, 2, 128, 21 * 136 + 77
+    g = torch.Generator(device=dev).manual_seed(5)
+    qkv = torch.randn(3, n, Hq + 2 * Hkv, D, generator=g, device=dev).bfloat16()
+    q, k, v = qkv[:, :, :Hq], qkv[:, :, Hq:Hq + Hkv], qkv[:, :, Hq + Hkv:]
+    sp = torch.as_tensor(O.summary_positions(n, C, S), device=dev)
+    for boost in (1.0, 40.0):
+        k[:, sp] *= boost
+        want, wlse = ksa_amd.summary_attn_func(q, k, v, C, S, W, summary_pos=sp, return_lse=True, workgroup_shape=32)
+        out, lse = torch.full_like(want, float("nan")), torch.full_like(wlse, float("nan"))
+        st = lambda t: _lib.strides3(t, (0, 1, 2))  # noqa: E731
+        rc = _lib.lib().ksa_prefill_chunks_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), 3, n,
+                                               Hq, Hkv, D, 0, st(q), st(k), st(out), C, S, W, 0, D ** -0.5, shape, None,
+                                               torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        assert (out.float() - want.float()).abs().max() <= ATOL * max(1.0, float(want.float().abs().max()))
+        assert (lse - wlse).abs().max() <= 0.1 + 1e-3 * float(wlse.abs().max())
