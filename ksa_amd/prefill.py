@@ -258,7 +258,8 @@ def _gathered_prefix(t: torch.Tensor, rows: torch.Tensor, P: int) -> torch.Tenso
 def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
                       summary_pos: Optional[torch.Tensor] = None,
                       skip_old_summary: bool = False, *, return_lse: bool = False,
-                      softmax_scale: Optional[float] = None, workgroup_shape: Optional[int] = None):
+                      softmax_scale: Optional[float] = None, workgroup_shape: Optional[int] = None,
+                      chunk_tiles: bool = True):
     """q [b, Sq, Hq, D]; k, v [b, Sq (+P), Hkv, D]; returns (out [b, Sq, Hq, D], lse or None).
 
     With `summary_pos` (bool [Sq]) the summary rows of k/v form the key prefix, as
@@ -268,9 +269,9 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     a [prefix | in-line] buffer first.  Without `summary_pos`, the first
     `k.shape[1] - q.shape[1]` rows of k/v are taken as an already-built prefix.
     Forward only: tensors that require grad under an enabled grad mode are rejected.
-    `return_lse` / `softmax_scale` / `workgroup_shape` are extensions (the reference returns lse
+    `return_lse` / `softmax_scale` / `workgroup_shape` / `chunk_tiles` are extensions (the reference returns lse
     only for autograd and always uses head_dim ** -0.5; `workgroup_shape` is the tuning knob of
-    `PREFILL_SHAPE`).
+    `PREFILL_SHAPE`; `chunk_tiles=False` keeps a call on the grid of the block index).
     """
     _check_inputs(q, k, v)
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
@@ -299,7 +300,7 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
         q, k, v = pad_head_dim(q, Dk), pad_head_dim(k, Dk), pad_head_dim(v, Dk)
     shape = PREFILL_SHAPE if workgroup_shape is None else int(workgroup_shape)
     direct = _lib.direct(q, k, v)
-    if shape == 0 and _chunk_tiles(Sq, Dk, C, S, P, phys):
+    if shape == 0 and chunk_tiles and _chunk_tiles(Sq, Dk, C, S, P, phys):
         shape = _CHUNK_TILES
     elif shape == _CHUNK_TILES:
         shape = -1   # no shape that a caller can name: refused by the library
