@@ -158,6 +158,32 @@ int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_
                        const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
                        float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
 
+/* ksa_decode_qkv_fwd and the o projection behind it (HF:879) in one launch, for at most 16 sequences: the workgroups of the
+ * product request their weights and wait for the attention of their heads.  Instead of out:
+ *   o_weight [N, Hq D] in the streaming layout (ksa_tile_weights); o_partials fp32 [Hq D / 512][16][N], the product's
+ *   K-split partial sums as ksa_gemm_rows leaves them (rows past batch unwritten)
+ *   workspace: ksa_decode_qkv_o_workspace_bytes(...) bytes, 16-byte aligned, also for one split
+ *   step_workspace: ksa_step_workspace_bytes() bytes, 16-byte aligned, ZEROED ONCE by the caller; it belongs to one device,
+ *   and launches that share it must not overlap.  The launch relies on the order in which workgroups are started, as
+ *   ksa_mlp_rows does, with its wait bounded in the same way: after a launch that gave up, the 8-byte word at
+ *   ksa_step_status_offset() reads 1, the output is unusable, and the caller waits for the device, zeroes the words
+ *   and repeats the work with the separate calls.
+ *   nsplit: ksa_decode_qkv_o_splits(...) of the longest range, or any other count
+ * Hq D a multiple of 512 up to 32768, N a multiple of 16, batch x nsplit <= 64, Hkv <= 128 (KSA_ERR_UNSUPPORTED
+ * otherwise: use the separate calls); the rest as there.  The splits are merged in another order than there: the product's
+ * input may differ in the last place of its 16 bits. */
+size_t ksa_step_workspace_bytes(void);
+size_t ksa_step_status_offset(void);
+int ksa_decode_qkv_o_splits(int batch, int Hq, int Hkv, int D, int max_rows);
+size_t ksa_decode_qkv_o_workspace_bytes(int batch, int Hq, int Hkv, int D, int nsplit);
+int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                         const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                         void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
+                         int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype, const int64_t* k_strides,
+                         const int64_t* v_strides, float scale, int nsplit, const void* o_weight, float* o_partials,
+                         int N, void* workspace, size_t workspace_bytes, void* step_workspace,
+                         size_t step_workspace_bytes, void* stream);
+
 /* ksa_decode_fwd for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
  * Same arguments and results as ksa_decode_fwd without the workspace: the split-K partials go to

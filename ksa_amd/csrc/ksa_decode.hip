@@ -19,13 +19,18 @@
 // of q (kPre): the kernel then does the pre-attention step itself - sums, norm and rotary embedding of the query
 // rows of its group in every workgroup, of the new key and value rows in the one workgroup whose
 // slice holds their cache row - one launch, and one round trip of the rows through memory, less.
+//
+// With kO the launch also holds the o projection behind the attention: see ksa_decode_o_stage.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "ksa_api_internal.h"
 #include "ksa_pre_row.h"
+#include "ksa_rows_mfma.h"
+#include "ksa_rows_sync.h"
 #include "ksa_tile.h"
 
 namespace {
@@ -70,6 +75,15 @@ struct DecodeParams {
     const int32_t* row_seq;     // cache row of the new token per sequence, or null: row0
     int row0;
 };
+// kO: the o projection in the same launch
+struct DecodeOParams : DecodeParams {
+    const uint16_t* o_w;        // streaming layout [o_n / 16][Hq D / 32][1 KB]
+    float* o_part;              // [o_chunks][16][o_n]
+    unsigned long long* sync;
+    int batch, n_attn;          // n_attn: workgroups of the attention
+    int o_n, o_chunks, o_wgs;
+    unsigned spin_limit;
+};
 
 // column lq of column block colblk -> (query token, head in the group); false: no such column
 __device__ __forceinline__ bool ksa_decode_column(const DecodeParams& p, int colblk, int lq, int& qi, int& gi) {
@@ -101,13 +115,170 @@ constexpr int kThreads = 256;
 constexpr int kWaves = 4;
 constexpr int kRows = 32;  // key rows per wave tile
 
+// The o projection (modeling_qwen3sa.py:879) behind the attention of a one-token step, at most 16 rows: a workgroup owns
+// 128 columns (two tiles of 16 per wave) times one chunk of 512 elements of K, i.e. 512 / D heads.  It requests all its
+// weights at once, waits until the attention workgroups of those heads have left their sums, merges the splits of its
+// heads into the rows of x and multiplies.  Against the three launches it stands for the weights (21 MB at 4096 x 2560) move
+// while the attention runs, and two ramps and a trip of the rows through memory are gone; what bounds it is the chain
+// projection sums - scores - sums - merge - product (figures at ksa_decode_qkv_o_splits).  Every workgroup merges for
+// itself, rows x splits x 2 KB of sums, 131 KB at the most (kMaxOSums), which is why it has 128 columns and not fewer.
+constexpr int kMaxOSums = 64;  // rows x splits
+template <typename T, int D>
+__device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int idx, unsigned char* smem) {
+    using Ops = KsaOps<T>;
+    constexpr int HPC = kChunkK / D;   // heads of a chunk
+    constexpr int kCols = 2;           // column tiles of a wave
+    constexpr int kBatch = 16;         // splits requested at a time
+    __shared__ int s_there;
+    unsigned char* xs = smem;                                                    // [16][kRowB]
+    float* s_m = reinterpret_cast<float*>(smem + 16 * kRowB);                    // [rows][HPC][splits]
+    floatx2_ws* s_f = reinterpret_cast<floatx2_ws*>(s_m + kMaxOSums * HPC);      // factor and factor x sum
+    floatx4* s_half = reinterpret_cast<floatx4*>(s_f + kMaxOSums * HPC);         // [128] sums of the second half, their l
+    float* s_half_l = reinterpret_cast<float*>(s_half + 128);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kq = lane >> 4;
+    const int grp = idx / p.o_chunks, chunk = idx - grp * p.o_chunks;
+    const int tiles = p.o_n / 16, steps = p.Hq * D / 32;
+    u32x4 a[kCols][kChunkSteps];
+#pragma unroll
+    for (int t = 0; t < kCols; ++t) {
+        const int tile = min(grp * (kWaves * kCols) + wave * kCols + t, tiles - 1);
+        const char* wt = reinterpret_cast<const char*>(p.o_w) + ((int64_t)tile * steps + chunk * kChunkSteps) * 1024;
+#pragma unroll
+        for (int u = 0; u < kChunkSteps; ++u)
+            a[t][u] = ksa_load_weights<true>(reinterpret_cast<const uint16_t*>(wt + u * 1024 + (uint32_t)(64 * r + 16 * kq)));
+    }
+    const int ns = p.nsplit, M = p.batch;
+    // this thread's maxima and sums (row, head, split) and its piece of four elements of x
+    const uint32_t slot_step = (uint32_t)p.ncols_pad, row_step = (uint32_t)(p.Hkv * ns) * slot_step;
+    const int count = M * HPC * ns;
+    uint32_t ml_off[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int e = min(tid + kThreads * i, count - 1);
+        const int rh = e / ns, sp = e - rh * ns, hh = rh % HPC, head = chunk * HPC + hh;
+        const int kvh = head / p.g;
+        ml_off[i] = ((uint32_t)(rh / HPC) * row_step + (uint32_t)(kvh * ns + sp) * slot_step + (uint32_t)(head - kvh * p.g)) * 8u;
+    }
+    const int piece = tid & 127, half = wave >> 1;
+    const int hh = 4 * piece / D, head = chunk * HPC + hh, kvh = head / p.g;
+    const uint32_t o_off = (((uint32_t)(kvh * ns) * slot_step + (uint32_t)(head - kvh * p.g)) * D + (uint32_t)(4 * piece % D)) * 4u;
+
+    // The entries of a thread: rows half, half + 2, .. with all their splits one after the other; of a single row the two
+    // halves take the even and the odd splits.  Lane j holds entry j: the offset of its sums; the place of its factor and, in
+    // the upper half behind the last split of a row, the row + 1.
+    const bool one = M == 1;
+    const int n = one ? (ns - half + 1) / 2 : (M - half + 1) / 2 * ns;  // at most 64
+    const int erow = one ? 0 : half + 2 * (lane / ns), esp = one ? 2 * lane + half : lane % ns;
+    const uint32_t ent_off = ((uint32_t)erow * row_step + (uint32_t)esp * slot_step) * (uint32_t)(D * 4);
+    const int ent = (erow * HPC * ns + esp) | (!one && esp == ns - 1 ? (erow + 1) << 16 : 0);
+
+    if (wave == 0) {
+        const int kv0 = chunk * HPC / p.g, kv1 = (chunk * HPC + HPC - 1) / p.g;
+        const bool there = ksa_wave_wait(p.sync + kWordStride * (kStepHead0 + min(kv0 + lane, kv1)), lane <= kv1 - kv0,
+                                         (long long)M * ns, p.sync + kWordStride * kStepStatus, p.spin_limit);
+        if (lane == 0) s_there = there;
+    }
+    __syncthreads();
+    if (!s_there) return;
+
+    const uint32_t slots = (uint32_t)M * row_step;
+    const KsaAgentBuffer so(p.ws_o, slots * D * 4u), sml(p.ws_ml, slots * 8u);
+    floatx2_ws ml[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) ml[i] = __builtin_bit_cast(floatx2_ws, sml.ld2(ml_off[i]));
+    floatx4 o[kBatch];
+    auto request = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (j0 + u < n) o[u] = __builtin_bit_cast(floatx4, so.ld4(o_off, (uint32_t)__builtin_amdgcn_readlane((int)ent_off, j0 + u)));
+    };
+    request(0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (tid + kThreads * i < count) s_m[tid + kThreads * i] = ml[i][0];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int e = tid + kThreads * i;
+        if (e < count) {
+            const int e0 = e / ns * ns;
+            float mx = -INFINITY;
+            for (int j = 0; j < ns; ++j) mx = fmaxf(mx, s_m[e0 + j]);
+            const float m = ml[i][0];
+            // (an empty slice leaves its sums unwritten: nothing of it may enter, not even times zero)
+            const float f = m == -INFINITY ? -1.f : ksa_exp2(m - mx);
+            s_f[e] = floatx2_ws{f, m == -INFINITY ? 0.f : f * ml[i][1]};
+        }
+    }
+    __syncthreads();
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+    auto x_store = [&](int row) {
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+        u32x2 w;
+        w[0] = Ops::pack2(acc[0] * inv, acc[1] * inv), w[1] = Ops::pack2(acc[2] * inv, acc[3] * inv);
+        *reinterpret_cast<u32x2*>(xs + row * kRowB + 8 * piece) = w;
+    };
+    for (int j0 = 0; j0 < n; j0 += kBatch) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            if (j0 + u < n) {
+                const int e = __builtin_amdgcn_readlane(ent, j0 + u);
+                const floatx2_ws f = s_f[(e & 0xffff) + hh * ns];
+                const bool live = f[0] >= 0.f;
+                l += f[1];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[i] = fmaf(live ? o[u][i] : 0.f, f[0], acc[i]);
+                if (e >> 16) {
+                    x_store((e >> 16) - 1);
+                    acc = floatx4{0.f, 0.f, 0.f, 0.f}, l = 0.f;
+                }
+            }
+        }
+        if (j0 + kBatch < n) request(j0 + kBatch);
+    }
+    if (one) {
+        if (half) s_half[piece] = acc, s_half_l[piece] = l;
+        __syncthreads();
+        if (!half) {
+            acc += s_half[piece], l += s_half_l[piece];
+            x_store(0);
+        }
+    }
+    __syncthreads();
+    f32x4 c[kCols];
+#pragma unroll
+    for (int t = 0; t < kCols; ++t) c[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const unsigned char* xb = xs + min(r, M - 1) * kRowB + 16 * kq;  // (rows past the last repeat it, nothing of them is stored)
+#pragma unroll
+    for (int u = 0; u < kChunkSteps; ++u) {
+        const u32x4 b = *reinterpret_cast<const u32x4*>(xb + 64 * u);
+#pragma unroll
+        for (int t = 0; t < kCols; ++t) c[t] = mfma16<T>(a[t][u], b, c[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < kCols; ++t) {
+        const int tile = grp * (kWaves * kCols) + wave * kCols + t;
+        if (r < M && tile < tiles)
+            *reinterpret_cast<f32x4*>(p.o_part + ((int64_t)chunk * 16 + r) * p.o_n + 16 * tile + 4 * kq) = c[t];
+    }
+    // (everybody who counts here has seen the sums)
+    if (tid == 0 && add_agent(p.sync + kWordStride * kStepAttnDone, 1ull) == (unsigned long long)p.o_wgs - 1) {
+        for (int h = 0; h < p.Hkv; ++h) add_agent(p.sync + kWordStride * (kStepHead0 + h), -(unsigned long long)(M * ns));
+        st_agent(p.sync + kWordStride * kStepAttnDone, 0ull);
+    }
+}
+
 // kPre against the pre-attention launch in front, a decode step of 8 layers of the 4B shape: batch 1 665 -> 652 us,
 // batch 8 772 -> 759.  The chain of trips that it puts in front of the first scores (row and range, partial sums, LDS)
 // runs next to the loads of the first K / V tile; what it costs is that every split repeats it, and a
 // workgroup that is not among the first on its CU runs it behind full memory queues (who calls it keeps to launches whose
 // workgroups all fit at once).
-template <typename T, int D, bool kPre>
-__global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kernel(const DecodeParams p) {
+template <typename T, int D, bool kPre, bool kO = false>
+__global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kernel(
+    const std::conditional_t<kO, DecodeOParams, DecodeParams> p) {
     using Ops = KsaOps<T>;
     constexpr int KS = D / 16;
     constexpr int DB = D / 32;
@@ -129,9 +300,30 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
     const int lq = lane & 31;
     const int lh = lane >> 5;
 
-    const int split = blockIdx.x;
-    const int kvh = blockIdx.y % p.Hkv;
-    const int bz = blockIdx.z;
+    int split = blockIdx.x, unit = blockIdx.y, bz = blockIdx.z;
+    if constexpr (kO) {  // the same order in one dimension, the o projection behind it
+        if ((int)blockIdx.x >= p.n_attn) {
+            ksa_decode_o_stage<T, D>(p, blockIdx.x - p.n_attn, smem);
+            return;
+        }
+        unit = blockIdx.x / p.nsplit;
+        split = blockIdx.x - unit * p.nsplit;
+        bz = unit / p.Hkv;
+        unit -= bz * p.Hkv;
+    }
+    const int kvh = unit % p.Hkv;
+    // (kO) the sums of this workgroup have left and are counted off
+    auto arrive = [&]() {
+        if constexpr (kO) {
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (tid == 0) add_agent(p.sync + kWordStride * (kStepHead0 + kvh), 1ull);
+        }
+    };
+    auto put = [&](float* dst, float v) {
+        if constexpr (kO) st_agent(dst, v);
+        else *dst = v;
+    };
 
     uint16_t* Kw = reinterpret_cast<uint16_t*>(smem) + wave * kStage;
     uint16_t* Vw = Kw + kRows * KROW;
@@ -142,7 +334,7 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
     // ones, those short blocks held places of a CU for a chain of memory round trips under full load, and the
     // long workgroups that had to wait for the places ended late: +8 us per small-window layer and +27 us
     // per large-window layer of a boundary step.
-    const int colblk_first = p.split_q ? 0 : blockIdx.y / p.Hkv;
+    const int colblk_first = p.split_q ? 0 : unit / p.Hkv;
     const int colblk_last = p.split_q ? p.ncols_pad / 32 - 1 : colblk_first;
     for (int colblk = colblk_first; colblk <= colblk_last; ++colblk) {
     if (colblk != colblk_first) __syncthreads();  // the previous block's merge area becomes staging again
@@ -163,9 +355,10 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
                                     : (colblk == 0 ? p.g : min(32, (p.Q - 1) * p.g - (colblk - 1) * 32));
         if (tid < ncol) {
             const int64_t slot = (((int64_t)bz * p.Hkv + kvh) * p.nsplit + split) * p.ncols_pad + colblk * 32 + tid;
-            p.ws_ml[slot * 2] = -INFINITY;
-            p.ws_ml[slot * 2 + 1] = 0.f;
+            put(p.ws_ml + slot * 2, -INFINITY);
+            put(p.ws_ml + slot * 2 + 1, 0.f);
         }
+        arrive();
         continue;
     }
 
@@ -396,7 +589,7 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
             l += row[D + 1] * f;
         }
         const int cg = colblk * 32 + c;
-        if (p.nsplit == 1) {
+        if (!kO && p.nsplit == 1) {
             int oq, og;
             ksa_decode_column(p, colblk, c, oq, og);
             const float val = l > 0.f ? acc / l : 0.f;
@@ -405,13 +598,14 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
             *op = (uint16_t)(pk & 0xffffu);
         } else {
             const int64_t slot = (((int64_t)bz * p.Hkv + kvh) * p.nsplit + split) * p.ncols_pad + cg;
-            p.ws_o[slot * D + d] = acc;
+            put(p.ws_o + slot * D + d, acc);
             if (d == 0) {
-                p.ws_ml[slot * 2] = mx;
-                p.ws_ml[slot * 2 + 1] = l;
+                put(p.ws_ml + slot * 2, mx);
+                put(p.ws_ml + slot * 2 + 1, l);
             }
         }
     }
+    arrive();
     }  // column blocks of this workgroup
 }
 
@@ -767,15 +961,16 @@ extern "C" int ksa_decode_boundary_fwd(const void* q, const void* kcache, const 
 // A decode step's attention from the K-split partial sums of its fused q | k | v projection: the pre-attention step
 // (HF:660-666) and the attention over the cache (HF:591-612) in one launch.  Arithmetic and results are those of
 // ksa_pre_attention_partials followed by ksa_decode_fwd.
-extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
-                                  const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
-                                  void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
-                                  const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
-                                  const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
-                                  float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
+namespace {
+// `p` filled from the arguments that the two forms share
+int decode_qkv_params(DecodeParams& p, const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                      const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache, void* vcache,
+                      const int32_t* row, int row0, const int32_t* start, const int32_t* end, int start0, int end0,
+                      int batch, int Hq, int Hkv, int D, int dtype, const int64_t* k_strides, const int64_t* v_strides,
+                      float scale, int nsplit, void* workspace) {
     if (!qkv_partials || !q_weight || !k_weight || !cos || !sin || !kcache || !vcache || !k_strides || !v_strides)
         return KSA_ERR_NULL;
-    if (!out || !out_strides || (start == nullptr) != (end == nullptr)) return KSA_ERR_NULL;
+    if ((start == nullptr) != (end == nullptr)) return KSA_ERR_NULL;
     if (batch <= 0 || batch > kMaxPartialRows || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Hq / Hkv > 32 || qkv_ksplit < 1 ||
         qkv_ksplit > 64 || nsplit < 1 || nsplit > 64 || !(eps >= 0.f))
         return KSA_ERR_INVALID;
@@ -789,7 +984,6 @@ extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, con
     for (int i = 0; i < 3; ++i)
         if ((k_strides[i] % 8) || (v_strides[i] % 8)) return KSA_ERR_ALIGN;
     if (cos_batch_stride % 8) return KSA_ERR_ALIGN;
-    DecodeParams p{};
     p.qkv = qkv_partials, p.qkv_ksplit = qkv_ksplit, p.qkv_prows = ksa_partial_rows(batch);
     p.wq = (const uint16_t*)q_weight, p.wk = (const uint16_t*)k_weight;
     p.cos = (const uint16_t*)cos, p.sin = (const uint16_t*)sin, p.c_bs = cos_batch_stride;
@@ -797,7 +991,6 @@ extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, con
     p.k = p.kw = (uint16_t*)kcache;
     p.v = p.vw = (uint16_t*)vcache;
     p.row_seq = row, p.row0 = row0;
-    p.out = (uint16_t*)out;
     p.start = start, p.end = end, p.start0 = start0, p.end0 = end0;
     p.Hq = Hq, p.Hkv = Hkv, p.g = Hq / Hkv, p.Q = 1;
     p.ncols = p.g;
@@ -805,8 +998,25 @@ extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, con
     p.nsplit = nsplit;
     p.k_bs = k_strides[0], p.k_hs = k_strides[1], p.k_rs = k_strides[2];
     p.v_bs = v_strides[0], p.v_hs = v_strides[1], p.v_rs = v_strides[2];
-    p.o_bs = out_strides[0], p.o_qs = out_strides[1], p.o_hs = out_strides[2];
     p.scale_log2 = scale * 1.4426950408889634f;
+    return KSA_OK;
+}
+}  // namespace
+
+extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                                  const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                  void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                                  const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                  const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                                  float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!out || !out_strides) return KSA_ERR_NULL;
+    DecodeParams p{};
+    const int rc = decode_qkv_params(p, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache,
+                                     vcache, row, row0, start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides,
+                                     v_strides, scale, nsplit, workspace);
+    if (rc != KSA_OK) return rc;
+    p.out = (uint16_t*)out;
+    p.o_bs = out_strides[0], p.o_qs = out_strides[1], p.o_hs = out_strides[2];
     if (nsplit > 1) {
         if (!workspace || workspace_bytes < ksa_decode_workspace_bytes(batch, Hq, Hkv, 1, D, nsplit)) return KSA_ERR_WORKSPACE;
         p.ws_o = (float*)workspace;
@@ -814,6 +1024,67 @@ extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, con
     }
     hipStream_t st = (hipStream_t)stream;
     return dtype == KSA_DTYPE_BF16 ? launch_head_dim<KsaBf16>(p, D, batch, st) : launch_head_dim<KsaF16>(p, D, batch, st);
+}
+
+// ksa_decode_qkv_fwd and the o projection behind it (modeling_qwen3sa.py:879) in one launch: see ksa_decode_o_stage.
+extern "C" size_t ksa_decode_qkv_o_workspace_bytes(int batch, int Hq, int Hkv, int D, int nsplit) {
+    if (batch <= 0 || Hkv <= 0 || Hq % Hkv != 0 || D <= 0 || nsplit < 1) return 0;
+    return (size_t)batch * Hkv * nsplit * (size_t)pad_cols(Hq / Hkv) * (D + 2) * sizeof(float);
+}
+
+extern "C" size_t ksa_step_workspace_bytes(void) { return (size_t)kStepWords * kWordStride * 8; }
+extern "C" size_t ksa_step_status_offset(void) { return (size_t)kWordStride * kStepStatus * 8; }
+
+// Splits for the one launch: five attention workgroups to eight CUs, so that those of the product find places next to them, but
+// no more than the count for the attention alone, nor than the sums that a workgroup of the product merges.  Attention
+// + product at 32 / 8 heads of 128, 4096 x 2560, us: the separate launches / this form with their count / with this one: 1 sequence of
+// 700 / 4100 / 16000 rows 17.6 / 14.9 / 14.9, 21.4 / 19.7 / 18.3, 27.2 / 26.7 / 26.5; 2 of 700 18.0 / 17.2 / 16.7, 4 of 700
+// 20.6 / 19.8 / 18.9, 8 of 700 / 4100 22.0 / 22.9 / 19.9, 40.7 / 39.3 / 36.5; 16 of 700 / 4100 26.6 / 26.3 / 23.6, 60.8 / 57.9 / 56.3.
+extern "C" int ksa_decode_qkv_o_splits(int batch, int Hq, int Hkv, int D, int max_rows) {
+    if (batch <= 0 || batch > 16 || Hkv <= 0) return 1;
+    const int units = batch * Hkv, cus = ksa_cu_count_or(256);
+    int n = (cus * 5 / 8 + units - 1) / units;
+    n = min(n, min(ksa_decode_splits(batch, Hq, Hkv, 1, D, max_rows), kMaxOSums / batch));
+    return n < 1 ? 1 : n;
+}
+
+extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                                    const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                    void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
+                                    int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                    const int64_t* k_strides, const int64_t* v_strides, float scale, int nsplit,
+                                    const void* o_weight, float* o_partials, int N, void* workspace, size_t workspace_bytes,
+                                    void* step_workspace, size_t step_workspace_bytes, void* stream) {
+    if (!o_weight || !o_partials || !workspace || !step_workspace) return KSA_ERR_NULL;
+    if (N <= 0) return KSA_ERR_INVALID;
+    DecodeOParams p{};
+    const int rc = decode_qkv_params(p, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache,
+                                     vcache, row, row0, start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides,
+                                     v_strides, scale, nsplit, workspace);
+    if (rc != KSA_OK) return rc;
+    if (batch > 16 || batch * nsplit > kMaxOSums || Hkv > kStepMaxHeads || Hq * D % kChunkK != 0 || Hq * D > 64 * kChunkK ||
+        N % 16 != 0)
+        return KSA_ERR_UNSUPPORTED;
+    for (const void* ptr : {o_weight, (const void*)o_partials, (const void*)step_workspace})
+        if (reinterpret_cast<uintptr_t>(ptr) & 15) return KSA_ERR_ALIGN;
+    if (workspace_bytes < ksa_decode_qkv_o_workspace_bytes(batch, Hq, Hkv, D, nsplit)) return KSA_ERR_WORKSPACE;
+    if (step_workspace_bytes < ksa_step_workspace_bytes()) return KSA_ERR_WORKSPACE;
+    p.ws_o = (float*)workspace;
+    p.ws_ml = p.ws_o + (size_t)batch * Hkv * nsplit * p.ncols_pad * D;
+    p.o_w = (const uint16_t*)o_weight, p.o_part = o_partials;
+    p.sync = (unsigned long long*)step_workspace;
+    p.batch = batch, p.n_attn = batch * Hkv * nsplit;
+    p.o_n = N, p.o_chunks = Hq * D / kChunkK;
+    p.o_wgs = (N / 16 + 2 * kWaves - 1) / (2 * kWaves) * p.o_chunks;
+    p.spin_limit = 1u << 19;  // polls of a microsecond or two: about a second
+    const dim3 grid(p.n_attn + p.o_wgs), block(kThreads);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, p);
+        return ksa_check_launch();
+    };
+    if (dtype == KSA_DTYPE_BF16)
+        return D == 128 ? go(ksa_decode_kernel<KsaBf16, 128, true, true>) : go(ksa_decode_kernel<KsaBf16, 64, true, true>);
+    return D == 128 ? go(ksa_decode_kernel<KsaF16, 128, true, true>) : go(ksa_decode_kernel<KsaF16, 64, true, true>);
 }
 
 extern "C" size_t ksa_decode_noalloc_max_workspace_bytes(void) { return kNoAllocScratchBytes; }

@@ -39,12 +39,12 @@
 #include "ksa_api_internal.h"
 #include "ksa_cvt.h"
 #include "ksa_rows_mfma.h"
+#include "ksa_rows_sync.h"
 
 namespace {
 
 constexpr int kSlices = 4;        // K slices of the hidden size = waves per gate / up half
 constexpr int kTileCols = 16;     // columns of the activation per gate | up workgroup (8: same time, twice the reads of x)
-constexpr int kWordStride = 64;   // 64-bit words are 512 bytes apart
 // words: [0] launches so far, [1] down workgroups done, [2] status, [3] rows of the norm stages of all past
 // launches (a launch may have any number of rows, and one without a norm stage has none: the target of a
 // wait is this word plus the rows of the launch itself), [4 .. 11] rows of the norm stage done (eight copies,
@@ -57,14 +57,8 @@ constexpr int kSyncWords = kWordStride * (kWordChunk0 + kMaxChunks);
 
 struct MlpParams {
     const uint16_t* x;        // h rows [M][H]; null: they come from the norm stage of this launch
-    const float* o_part;      // norm stage: [o_ksplit][16][H] partial sums of the o projection
-    const uint16_t* res;      // norm stage: residual rows [M][H]
-    const uint16_t* norm_w;   // norm stage: weight [H]
-    uint16_t* out_sum;        // norm stage: residual + o projection [M][H]
-    unsigned long long* hbuf; // norm stage: its rows for the gate | up workgroups, [M][H / 4]
-    int64_t res_rs, sum_rs;
-    int o_ksplit, head;       // head: workgroups of the norm stage (M, or 0)
-    float eps;
+    KsaNormStage norm;        // norm stage: from the partial sums of the o projection
+    int head;                 // workgroups of the norm stage (M, or 0)
     const uint16_t* w_gu;     // [2 I][H]
     const uint16_t* w_dn;     // [H][I]
     float* dn_part;           // [KC][16][H]
@@ -76,15 +70,6 @@ struct MlpParams {
     unsigned spin_limit;
 };
 
-__device__ __forceinline__ unsigned long long ld_agent(const unsigned long long* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_agent(unsigned long long* p, unsigned long long v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned long long add_agent(unsigned long long* p, unsigned long long v) {
-    return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // 16 bytes written by another workgroup of this launch: a load that is not served from this XCD's
 // L2 (the cache-control bit the compiler sets for agent-scope atomic loads; those stop at 8 bytes).
 // Assembly with the wait inside the statement: the compiler does not know that the value of a bare
@@ -112,65 +97,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 
     if ((int)blockIdx.x < p.head) {
-        // ---- norm stage, one workgroup per row: x' = residual + sum of the o_proj partial sums (plain
-        // store, for later launches), h = norm(x') w (for the gate | up workgroups of this launch).
-        // Arithmetic and summation order of ksa_add_rmsnorm_partials. ----
-        const int row = blockIdx.x;
-        const int items = p.H / 8;  // at most 512: one per thread
-        float* s_ss = reinterpret_cast<float*>(lds);
-        float ss = 0.f;
-        u32x4 rsum = {0u, 0u, 0u, 0u}, wv = {0u, 0u, 0u, 0u};
-        if (tid < items) {
-            wv = *reinterpret_cast<const u32x4*>(p.norm_w + 8 * tid);
-            const u32x4 q = *reinterpret_cast<const u32x4*>(p.res + (int64_t)row * p.res_rs + 8 * tid);
-            float ac[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            for (int sp0 = 0; sp0 < p.o_ksplit; sp0 += 4) {  // (four slices requested at a time: registers)
-                f32x4 lo[4], hi[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float* src = p.o_part + ((int64_t)min(sp0 + k, p.o_ksplit - 1) * 16 + row) * p.H + 8 * tid;
-                    lo[k] = *reinterpret_cast<const f32x4*>(src);
-                    hi[k] = *reinterpret_cast<const f32x4*>(src + 4);
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    if (sp0 + k < p.o_ksplit) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) ac[i] += lo[k][i], ac[4 + i] += hi[k][i];
-                    }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t x = C::down2(ac[2 * i], ac[2 * i + 1]);
-                rsum[i] = C::down2(C::lo(x) + C::lo(q[i]), C::hi(x) + C::hi(q[i]));
-                const float a_ = C::lo(rsum[i]), b_ = C::hi(rsum[i]);
-                ss = fmaf(a_, a_, ss);
-                ss = fmaf(b_, b_, ss);
-            }
-            *reinterpret_cast<u32x4*>(p.out_sum + (int64_t)row * p.sum_rs + 8 * tid) = rsum;
-        }
-#pragma unroll
-        for (int m = 32; m >= 1; m >>= 1) ss += __shfl_xor(ss, m);
-        if (lane == 0) s_ss[wave] = ss;
-        __syncthreads();
-        ss = 0.f;
-        for (int w = 0; w < (items + 63) / 64; ++w) ss += s_ss[w];
-        const float inv = rsqrtf(ss / (float)p.H + p.eps);
-        if (tid < items) {
-            uint32_t o[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t y = C::down2(C::lo(rsum[i]) * inv, C::hi(rsum[i]) * inv);
-                o[i] = C::down2(C::lo(wv[i]) * C::lo(y), C::hi(wv[i]) * C::hi(y));
-            }
-            unsigned long long* hp = p.hbuf + (int64_t)row * (p.H / 4) + 2 * tid;
-            st_agent(hp, (unsigned long long)o[0] | ((unsigned long long)o[1] << 32));
-            st_agent(hp + 1, (unsigned long long)o[2] | ((unsigned long long)o[3] << 32));
-        }
-        // Every thread waits until its own stores have left (they write through to memory), and only then
-        // joins the barrier: the barrier itself does not wait for the stores of the other waves.
-        __builtin_amdgcn_s_waitcnt(0);
+        // ---- norm stage, one workgroup per row (four slices requested at a time: registers) ----
+        ksa_norm_row<T, 4>(p.norm, p.H, blockIdx.x, tid, reinterpret_cast<float*>(lds));
         __syncthreads();
         if (tid < kHeadCopies) add_agent(p.sync + kWordStride * (kWordHead0 + tid), 1ull);
         return;
@@ -224,7 +152,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
             const int per_row = p.H / 4;  // 8-byte words (agent-scope loads the compiler tracks: several in flight)
             for (int e = tid; e < p.M * per_row; e += blockDim.x) {
                 const int m = e / per_row, j = e - m * per_row;
-                *reinterpret_cast<unsigned long long*>(lds + m * rowb + 8 * j) = ld_agent(p.hbuf + (int64_t)m * per_row + j);
+                *reinterpret_cast<unsigned long long*>(lds + m * rowb + 8 * j) = ld_agent(p.norm.hbuf + (int64_t)m * per_row + j);
             }
         } else {
             const int per_row = p.H / 8;
@@ -419,7 +347,7 @@ int mlp_rows_launch(const void* x, long long x_row_stride, const float* o_partia
     p.dn_part = down_partials;
     p.sync = (unsigned long long*)workspace;
     p.act = p.sync + kSyncWords;
-    p.hbuf = p.act + (size_t)16 * I / 4;
+    p.norm.hbuf = p.act + (size_t)16 * I / 4;
     p.wgu_rs = w_gate_up_row_stride, p.wdn_rs = w_down_row_stride;
     p.M = M, p.H = H, p.I = I;
     p.UB = I / kTileCols;
@@ -437,13 +365,13 @@ int mlp_rows_launch(const void* x, long long x_row_stride, const float* o_partia
         if (H > 4096) return KSA_ERR_UNSUPPORTED;  // a norm row is one 16-byte item per thread
         if (bad(o_partials) || bad(residual) || bad(norm_weight) || bad(out_sum)) return KSA_ERR_ALIGN;
         if (residual_row_stride % 8 || sum_row_stride % 8) return KSA_ERR_ALIGN;
-        p.o_part = o_partials;
-        p.o_ksplit = o_ksplit;
-        p.res = (const uint16_t*)residual;
-        p.norm_w = (const uint16_t*)norm_weight;
-        p.out_sum = (uint16_t*)out_sum;
-        p.res_rs = residual_row_stride, p.sum_rs = sum_row_stride;
-        p.eps = eps;
+        p.norm.part = o_partials;
+        p.norm.ksplit = o_ksplit;
+        p.norm.res = (const uint16_t*)residual;
+        p.norm.w = (const uint16_t*)norm_weight;
+        p.norm.out_sum = (uint16_t*)out_sum;
+        p.norm.res_rs = residual_row_stride, p.norm.sum_rs = sum_row_stride;
+        p.norm.eps = eps;
         p.head = M;
     }
     hipLaunchKernelGGL(kern, dim3(p.head + p.UB + p.GR * p.KC), dim3(128 * kSlices), lds, (hipStream_t)stream, p);

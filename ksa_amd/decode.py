@@ -136,14 +136,8 @@ def decode_qkv_pays(kcache: torch.Tensor, Hq: int, start, end) -> bool:
         return b * Hkv * n <= 2 * max(1, L.ksa_device_cu_count())
 
 
-def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
-                   eps: float, kcache: torch.Tensor, vcache: torch.Tensor, Hq: int, row, start, end,
-                   scale: Optional[float] = None, nsplit: Optional[int] = None) -> torch.Tensor:
-    """`pre_attention_partials` + `ksa_decode` of one new token per sequence in one launch (`ksa_decode_qkv_fwd`).
-
-    qkv: the deferred q | k | v projection (`SplitKPartials` [b, 1, (Hq + 2 Hkv) D]); cos / sin [1 or b, 1, D].  The
-    token's key and value go to `row` of the caches and are attended with the rest of [start, end), which has
-    to hold that row (each an int, or an int32 GPU tensor [b]).  Returns [b, 1, Hq D]."""
+def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end):
+    """What the two forms of the one-launch step share: the checked arguments, and the longest range."""
     from .gemm import SplitKPartials
     assert isinstance(qkv, SplitKPartials) and qkv.dtype in _DTYPES and qkv.dtype == kcache.dtype == vcache.dtype
     b, Hkv, rows, D = kcache.shape
@@ -168,6 +162,21 @@ def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor
     else:
         r0 = int(row)
         assert 0 <= r0 < rows and (t_start is not None or s0 <= r0 < e0), "the new row must lie in the attended range"
+    return cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows
+
+
+def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                   eps: float, kcache: torch.Tensor, vcache: torch.Tensor, Hq: int, row, start, end,
+                   scale: Optional[float] = None, nsplit: Optional[int] = None) -> torch.Tensor:
+    """`pre_attention_partials` + `ksa_decode` of one new token per sequence in one launch (`ksa_decode_qkv_fwd`).
+
+    qkv: the deferred q | k | v projection (`SplitKPartials` [b, 1, (Hq + 2 Hkv) D]); cos / sin [1 or b, 1, D].  The
+    token's key and value go to `row` of the caches and are attended with the rest of [start, end), which has
+    to hold that row (each an int, or an int32 GPU tensor [b]).  Returns [b, 1, Hq D]."""
+    cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows = _qkv_arguments(
+        qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end)
+    b, Hkv, _, D = kcache.shape
+    dev, dt = qkv.device, qkv.dtype
     L = _lib.lib()
     ptr = lambda t: None if t is None else t.data_ptr()
     with _lib.on_device(dev):
@@ -187,6 +196,45 @@ def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor
             float(D) ** -0.5 if scale is None else float(scale), nsplit, ptr(ws), ws_bytes, _lib.stream_ptr(dev))
     _lib.check(rc, "ksa_decode_qkv_fwd")
     return out.view(b, 1, Hq * D)
+
+
+def decode_qkv_o_supported(kcache: torch.Tensor, Hq: int, N: int) -> bool:
+    b, Hkv, _, D = kcache.shape
+    return (b <= 16 and Hkv <= 128 and decode_qkv_supported(Hq, Hkv, D) and Hq * D % 512 == 0 and Hq * D <= 32768
+            and N % 16 == 0)
+
+
+def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
+                     eps: float, kcache: torch.Tensor, vcache: torch.Tensor, Hq: int, row, start, end, o_weight, ws,
+                     scale: Optional[float] = None, nsplit: Optional[int] = None):
+    """`ksa_decode_qkv` and the o projection behind it (modeling_qwen3sa.py:879) in one launch
+    (`ksa_decode_qkv_o_fwd`), for at most 16 sequences: o_weight a `gemm.TiledWeight` [N, Hq D], ws the step's
+    `gemm.MlpRowsWorkspace`.  Returns the product's `SplitKPartials` [b, 1, N]."""
+    from .gemm import SplitKPartials, TiledWeight
+    cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows = _qkv_arguments(
+        qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end)
+    b, Hkv, _, D = kcache.shape
+    dev, dt = qkv.device, qkv.dtype
+    N = o_weight.shape[0]
+    assert isinstance(o_weight, TiledWeight) and o_weight.shape == (N, Hq * D) and o_weight.dtype == dt
+    L = _lib.lib()
+    ptr = lambda t: None if t is None else t.data_ptr()
+    with _lib.on_device(dev):
+        if nsplit is None:
+            nsplit = L.ksa_decode_qkv_o_splits(b, Hq, Hkv, D, max_rows)
+        ws_bytes = L.ksa_decode_qkv_o_workspace_bytes(b, Hq, Hkv, D, nsplit)
+        sums = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        ks = Hq * D // 512
+        part = torch.empty(ks * 16 * N, dtype=torch.float32, device=dev)
+        dims = (0, 1, 2)
+        rc = L.ksa_decode_qkv_o_fwd(
+            qkv.workspace.data_ptr(), qkv.ksplit, qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+            D if cos.shape[0] > 1 else 0, float(eps), kcache.data_ptr(), vcache.data_ptr(), ptr(t_row), r0,
+            ptr(t_start), ptr(t_end), s0, e0, b, Hq, Hkv, D, _DTYPES[dt], _lib.strides3(kcache, dims),
+            _lib.strides3(vcache, dims), float(D) ** -0.5 if scale is None else float(scale), nsplit, o_weight.data_ptr(),
+            part.data_ptr(), N, sums.data_ptr(), ws_bytes, ws.step.data_ptr(), ws.step.numel(), _lib.stream_ptr(dev))
+    _lib.check(rc, "ksa_decode_qkv_o_fwd")
+    return SplitKPartials(part.view(torch.uint8), ks, b, (b, 1, N), dt)
 
 
 def ksa_decode_boundary(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor, text_start, text_end,

@@ -132,6 +132,9 @@ class MlpRowsWorkspace:
         self.H, self.I = H, I
         self.buf = torch.zeros(L.ksa_mlp_rows_workspace_bytes(H, I), dtype=torch.uint8, device=device)
         self._status = self.buf[L.ksa_mlp_rows_status_offset():][:8].view(torch.int64)
+        # ... and the counting words of the step's other one-launch form, `decode.ksa_decode_qkv_o`
+        self.step = torch.zeros(L.ksa_step_workspace_bytes(), dtype=torch.uint8, device=device)
+        self._step_status = self.step[L.ksa_step_status_offset():][:8].view(torch.int64)
 
     def failed(self) -> bool:
         """True if a launch gave up waiting inside the kernel.  Waits for the whole device to be idle
@@ -139,9 +142,10 @@ class MlpRowsWorkspace:
         cleared); after a failure the workspace is zeroed again so that it can be used further.
         Recorded graphs that launch on it stay valid (the buffer does not move)."""
         torch.cuda.synchronize(self.buf.device)
-        bad = bool(self._status.item() != 0)
+        bad = bool(self._status.item() != 0) or bool(self._step_status.item() != 0)
         if bad:
             self.buf.zero_()
+            self.step.zero_()
             torch.cuda.synchronize(self.buf.device)
         return bad
 

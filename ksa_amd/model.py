@@ -192,6 +192,23 @@ class HipOps:
         return self._decode_mod.ksa_decode_qkv(qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end,
                                                scale=scale)
 
+    def _step_ws(self, H, device):
+        """The workspace of the one-launch forms for this hidden size, if `prepare_mlp_rows` has made one."""
+        return next((ws for (d, h, _), ws in self._mlp_ws.items() if d == str(device) and h == H), None)
+
+    def decode_qkv_o(self, qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end, scale, o_weight):
+        """`decode_qkv` and the o projection behind it in one launch: the projection's partial sums; None where
+        the two have to do it."""
+        if not self.mlp_one_launch or not isinstance(qkv, self._gemm.SplitKPartials):
+            return None
+        ws = self._step_ws(o_weight.shape[0], kbuf.device)
+        takes = ws is not None and self._decode_mod.decode_qkv_o_supported(kbuf, Hq, o_weight.shape[0])
+        tiled = self._streaming(o_weight) if takes else None
+        if not isinstance(tiled, self._gemm.TiledWeight):
+            return None
+        return self._decode_mod.ksa_decode_qkv_o(qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end,
+                                                 tiled, ws, scale=scale)
+
     def argmax(self, logits):
         """Greedy token choice over the last dimension (lowest index among equal values)."""
         if (logits.dtype in (torch.bfloat16, torch.float16) and logits.stride(-1) == 1 and logits.dim() == 2
@@ -450,13 +467,28 @@ class KsaQwen3ForCausalLM:
                              (vc if in_cache else vs, vc, S, 0, rows["append"])])
         return attn
 
-    def _text_attention(self, lw, h, cos, sin, kc, vc, row, start, end, slots):
-        """Projection, q / k norm, rotary embedding and attention of one text token per sequence, its key and
-        value written to `row` of the caches (`slots`: the same as arguments of `pre_attention`):
-        [b, 1, Hq D]."""
+    def _norm_qkv(self, lw, delta, x):
+        """The residual add and norm in front of a layer at a decode step, and its q | k | v projection:
+        (x', deferred q | k | v)."""
+        x, h = self._add_norm(delta, x, lw["input_layernorm"])
+        return x, self.ops.linear(h, lw["qkv_proj"], defer=True)
+
+    def _text_attention(self, lw, qkv, cos, sin, kc, vc, row, start, end, slots):
+        """q / k norm, rotary embedding and attention of one text token per sequence from its deferred q | k | v
+        projection, its key and value written to `row` of the caches (`slots`: the same as arguments of
+        `pre_attention`), and the o projection: [b, 1, H], deferred."""
+        ops = self.ops
+        if hasattr(ops, "decode_qkv_o"):
+            o = ops.decode_qkv_o(qkv, lw["q_norm"], lw["k_norm"], cos, sin, self.config.rms_norm_eps, kc, vc,
+                                 self.config.num_attention_heads, row, start, end, self.scaling, lw["o_proj"])
+            if o is not None:
+                return o
+        return ops.linear(self._text_heads(lw, qkv, cos, sin, kc, vc, row, start, end, slots), lw["o_proj"], defer=True)
+
+    def _text_heads(self, lw, qkv, cos, sin, kc, vc, row, start, end, slots):
+        """`_text_attention` without the o projection: [b, 1, Hq D]."""
         cfg, ops = self.config, self.ops
         Hq, Hkv, D = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
-        qkv = ops.linear(h, lw["qkv_proj"], defer=True)
         if hasattr(ops, "decode_qkv"):
             attn = ops.decode_qkv(qkv, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps, kc, vc, Hq, row, start, end,
                                   self.scaling)
@@ -469,12 +501,11 @@ class KsaQwen3ForCausalLM:
             q, _, _ = ops.pre_attention_partials(qkv, Hq, Hkv, D, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps,
                                                  **slots)
         attn = ops.decode(q.transpose(1, 2), kc, vc, start, end, self.scaling)
-        return attn.reshape(h.shape[0], 1, -1)
+        return attn.reshape(kc.shape[0], 1, -1)
 
-    def _post_attention(self, lw, attn, x):
-        """The second half of a layer at a decode step, from the attention output: (x', delta) with
-        x' = x + o_proj(attn) and delta = mlp(post_attention_layernorm(x')) (deferred sums)."""
-        o = self.ops.linear(attn, lw["o_proj"], defer=True)
+    def _post_attention(self, lw, o, x):
+        """The second half of a layer at a decode step, from the output o of its o projection: (x', delta) with
+        x' = x + o and delta = mlp(post_attention_layernorm(x')) (deferred sums)."""
         if hasattr(self.ops, "add_norm_mlp_rows"):
             out = self.ops.add_norm_mlp_rows(o, x, lw["post_attention_layernorm"], self.config.rms_norm_eps,
                                              lw["gate_up_proj"], lw["down_proj"])
@@ -629,15 +660,17 @@ class KsaQwen3ForCausalLM:
         delta = None
         tables = {}   # boundary step: (text row, first summary row) -> row table on the device
         for li, lw in enumerate(self.w["layers"]):
-            x, h = self._add_norm(delta, x, lw["input_layernorm"])
-            if not boundary:
+            if boundary:
+                x, h = self._add_norm(delta, x, lw["input_layernorm"])
+            else:
+                x, qkv = self._norm_qkv(lw, delta, x)
                 k_slot, v_slot = cache.text_slots(li, b, Hkv, D, self.dtype, self.device)
                 a, e = cache.attention_range(li)
                 # (a text token's row: the last one of a large window, the first one of a small one)
-                attn = self._text_attention(lw, h, cos, sin, cache.key_cache[li], cache.value_cache[li],
-                                            e - 1 if cache.is_large_window[li] else a, a, e,
-                                            dict(k_out=k_slot, v_out=v_slot))
-            else:
+                o = self._text_attention(lw, qkv, cos, sin, cache.key_cache[li], cache.value_cache[li],
+                                         e - 1 if cache.is_large_window[li] else a, a, e,
+                                         dict(k_out=k_slot, v_out=v_slot))
+            if boundary:
                 fused = hasattr(ops, "decode_boundary") and cache.boundary_fits_one_piece(li)
                 if fused:
                     # fused operators: the cache only does the bookkeeping and names the rows
@@ -674,7 +707,7 @@ class KsaQwen3ForCausalLM:
                                       lw["post_attention_layernorm"])
                 delta = self._mlp(lw, h, defer=True)
             else:
-                x, delta = self._post_attention(lw, attn, x)
+                x, delta = self._post_attention(lw, o, x)
         cache.reset_chunk_counter()
         if not boundary:
             return self._logits(x, delta)
@@ -696,13 +729,15 @@ class KsaQwen3ForCausalLM:
         for li, lw in enumerate(self.w["layers"]):
             kind = 1 if cache.is_large_window[li] else 0
             if li or h is None:
-                x, h = self._add_norm(delta, x, lw["input_layernorm"])
+                x, qkv = self._norm_qkv(lw, delta, x)
+            else:
+                qkv = ops.linear(h, lw["qkv_proj"], defer=True)
             # k and v go straight to the cache row the device-side cursor names
             slots = dict(k_out=cache.key_cache[li][:, :, :1].transpose(1, 2),
                          v_out=cache.value_cache[li][:, :, :1].transpose(1, 2), kv_out_row=st["cur"][kind, 0])
-            attn = self._text_attention(lw, h, cos, sin, cache.key_cache[li], cache.value_cache[li], *st["cur"][kind],
-                                        slots)
-            x, delta = self._post_attention(lw, attn, x)
+            o = self._text_attention(lw, qkv, cos, sin, cache.key_cache[li], cache.value_cache[li], *st["cur"][kind],
+                                     slots)
+            x, delta = self._post_attention(lw, o, x)
         return self._logits(x, delta)
 
     def _boundary_step_body(self, st, cache):

@@ -372,6 +372,80 @@ def test_decode_qkv_with_a_range_row_and_position_per_sequence(dtype, b, Hq, Hkv
     assert np.abs(to_np(got).reshape(ref.shape) - ref).max() <= ATOL * max(1.0, np.abs(ref).max())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,Hq,Hkv,D,N,nsplit", [
+    (1, 32, 8, 128, 2560, None),
+    (1, 32, 8, 128, 256, 1),       # no split: nothing for the second half of a workgroup to merge
+    (1, 16, 2, 128, 144, 39),      # odd count, several requests; the last workgroup has one tile
+    (1, 8, 4, 64, 16, 64),         # eight heads of several kv heads in a chunk
+    (2, 32, 8, 128, 272, 32),      # a row's splits end with a request
+    (3, 8, 8, 64, 128, 21),        # rows 0 and 2 / row 1 over two requests each
+    (5, 4, 2, 128, 512, 7),
+    (8, 32, 8, 128, 2560, 8),
+    (16, 32, 8, 128, 1024, 4),
+])
+def test_decode_qkv_o_equals_separate_launches(dtype, b, Hq, Hkv, D, N, nsplit):
+    """Attention and o projection of a step in one launch against the two launches (three with the merge) it stands for, with
+    ranges from one row to all (later splits empty), several launches on one workspace, fresh data each.  The
+    splits are merged in another order: a head's output may move by one unit in the last place (2^-8 / 2^-11 of it),
+    a random share of which reaches a product of K terms - bound: 2 units x sqrt(K) times the mean term; most are equal."""
+    from ksa_amd import _lib, decode, gemm
+    rows = 4100 if nsplit is None or nsplit > 16 else 1100
+    auto = _lib.lib().ksa_decode_qkv_o_splits(b, Hq, Hkv, D, rows)   # (another count rounds other probabilities)
+    g = torch.Generator(device="cuda").manual_seed(b * 10 + N)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    H, width, K = 1536, (Hq + 2 * Hkv) * D, Hq * D
+    wo = (rnd(N, K) * K ** -0.5).to(dtype)
+    tiled, ws = gemm.TiledWeight(wo), gemm.MlpRowsWorkspace(N, 64, torch.device("cuda"))
+    qw, kw = (1 + 0.1 * rnd(D)).to(dtype), (1 + 0.1 * rnd(D)).to(dtype)
+    ang = rnd(b, 1, D // 2)
+    ang = torch.cat((ang, ang), -1)
+    cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+    w = (rnd(width, H) * H ** -0.5).to(dtype)
+    forms = [(0, rows, rows - 1), (7, 1031, 7), (128, 129, 128), (3, 40, 20), (0, 300, 127)]
+    dev = lambda v: torch.as_tensor(v, device="cuda", dtype=torch.int32)
+    for rep in range(3):
+        lo, hi, row = (dev([forms[(i + rep) % len(forms)][j] for i in range(b)]) for j in range(3))
+        qkv = gemm.linear_rows(rnd(b, 1, H).to(dtype), w, defer=True)
+        caches = [rnd(b, Hkv, rows, D).to(dtype) for _ in range(2)]
+        kc, vc = (c.clone() for c in caches)
+        kr, vr = (c.clone() for c in caches)
+        attn = decode.ksa_decode_qkv(qkv, qw, kw, cos, sin, 1e-6, kr, vr, Hq, row, lo, hi, nsplit=nsplit or auto)
+        got = decode.ksa_decode_qkv_o(qkv, qw, kw, cos, sin, 1e-6, kc, vc, Hq, row, lo, hi, tiled, ws, nsplit=nsplit)
+        torch.cuda.synchronize()
+        assert not ws.failed() and int(ws.step.view(torch.int64).abs().sum().item()) == 0
+        assert torch.equal(kc, kr) and torch.equal(vc, vr)
+        got = got.workspace.view(torch.float32).view(K // 512, 16, N)[:, :b].sum(0)
+        want = attn.view(b, K).double() @ wo.double().t()
+        ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        term = (attn.view(b, K).double().square() @ wo.double().t().square() / K).sqrt()
+        assert ((got - want).abs() <= 2 * ulp * K ** 0.5 * term + 1e-5 * want.abs().max()).all()
+        assert (got - want).square().mean() <= (0.25 * ulp) ** 2 * (K * term.square()).mean()
+
+
+@pytest.mark.gpu
+def test_decode_qkv_o_bounded_wait_gives_up_and_recovers():
+    """The give-up path of the wait for the attention, forced from the host: the counts are set far below zero.  The first
+    workgroup to exhaust its bounded wait (about a second) sets the status word, the others leave, the launch ends;
+    `failed()` reports it and zeroes the words, and the next launch equals one on a fresh workspace."""
+    from ksa_amd import decode, gemm
+    g = torch.Generator(device="cuda").manual_seed(4)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    qkv = gemm.linear_rows(rnd(2, 1, 1024), rnd(8 * 128, 1024), defer=True)
+    kc, vc, tiled = rnd(2, 2, 300, 128), rnd(2, 2, 300, 128), gemm.TiledWeight(rnd(256, 512))
+    one, ws = torch.ones(128, device="cuda").bfloat16(), gemm.MlpRowsWorkspace(256, 64, torch.device("cuda"))
+    call = lambda w: decode.ksa_decode_qkv_o(qkv, one, one, one, one, 1e-6, kc, vc, 4, 5, 0, 300, tiled, w, nsplit=2)
+    ws.step.view(torch.int64)[4 * 64::64] = -(1 << 40)
+    torch.cuda.synchronize()
+    call(ws)
+    assert ws.failed() and not ws.failed()
+    assert int(ws.step.view(torch.int64).abs().sum().item()) == 0
+    a, b = call(ws), call(gemm.MlpRowsWorkspace(256, 64, torch.device("cuda")))
+    assert not ws.failed()
+    assert torch.equal(*(t.workspace.view(torch.float32).view(1, 16, 256)[:, :2] for t in (a, b)))
+
+
 @pytest.mark.parametrize("Hkv,D,nsplit", [(2, 256, None), (4, 256, 64), (2, 256, 33), (1, 128, 100), (1, 64, 150), (2, 256, 32),
                                           (2, 128, 32), (2, 128, 33), (1, 64, 32), (1, 64, 33)])
 def test_decode_merge_of_more_splits_than_one_pass_takes(Hkv, D, nsplit):
