@@ -172,7 +172,7 @@ int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_
  * Hq D a multiple of 512 up to 32768, N a multiple of 16, batch x nsplit <= 64, Hkv <= 128 (KSA_ERR_UNSUPPORTED
  * otherwise: use the separate calls); the rest as there.  The splits are merged in another order than there: the product's
  * input may differ in the last place of its 16 bits. */
-size_t ksa_step_workspace_bytes(void);
+size_t ksa_step_workspace_bytes(void);  /* (ksa_add_rmsnorm_gemm_rows shares it) */
 size_t ksa_step_status_offset(void);
 int ksa_decode_qkv_o_splits(int batch, int Hq, int Hkv, int D, int max_rows);
 size_t ksa_decode_qkv_o_workspace_bytes(int batch, int Hq, int Hkv, int D, int nsplit);
@@ -440,6 +440,20 @@ int ksa_add_rmsnorm_mlp_rows(const float* o_partials, int o_ksplit, const void* 
                              int H, int I, long long residual_row_stride, long long sum_row_stride,
                              long long w_gate_up_row_stride, long long w_down_row_stride, int dtype, float eps,
                              void* workspace, size_t workspace_bytes, void* stream);
+
+/* The residual add + RMSNorm between two layers and the product behind it (HF:950-952, the next layer's HF:938, :660-662) for
+ * at most 4 rows as one launch:
+ *   x' = residual + sum of partials (out_sum), out_partials[c] = (norm(x') norm_weight)[:, 512 c : 512 c + 512] W[:, same]^T
+ * partials fp32 [ksplit][16][H]; weight [N, H] in the streaming layout; out_partials fp32 [ceil(H / 512)][16][N].  Results
+ * are those of ksa_add_rmsnorm_partials and ksa_gemm_rows.  step_workspace and the bounded wait inside the launch as at
+ * ksa_decode_qkv_o_fwd, whose workspace it may share on one stream.  H a multiple of 32 up to 4096, N of 16 (KSA_ERR_UNSUPPORTED
+ * otherwise).  ksa_add_rmsnorm_gemm_rows_splits: ceil(H / 512), or 0 where the two calls are to be used instead: sizes that
+ * it does not take, or more workgroups than the device has CUs. */
+int ksa_add_rmsnorm_gemm_rows_splits(int M, int N, int H);
+int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, const void* residual, const void* norm_weight,
+                              void* out_sum, const void* weight, float* out_partials, int M, int N, int H,
+                              long long residual_row_stride, long long sum_row_stride, int dtype, float eps,
+                              void* step_workspace, size_t step_workspace_bytes, void* stream);
 
 /* Host-side diagnostic: number of key columns in [a, b) visible to query row q under the
  * closed-form rule the kernels use (no GPU involved). */

@@ -14,7 +14,7 @@ SOURCES = ["ksa_prefill_d256_bf16_regular.hip", "ksa_prefill_d256_bf16_general.h
            "ksa_prefill_d256_f16_general.hip", "ksa_prefill_d256_bf16_marked.hip", "ksa_prefill_d256_f16_marked.hip",
            "ksa_prefill_d256_bf16_chunks.hip", "ksa_prefill_d256_f16_chunks.hip",
            "ksa_prefill.hip", "ksa_prefill_chunks.hip", "ksa_api.hip", "ksa_index.hip", "ksa_decode.hip", "ksa_decode_weights.hip", "ksa_cache.hip",
-           "ksa_pre.hip", "ksa_elementwise.hip", "ksa_gemm_rows.hip", "ksa_mlp_rows.hip"]
+           "ksa_pre.hip", "ksa_elementwise.hip", "ksa_gemm_rows.hip", "ksa_mlp_rows.hip", "ksa_norm_gemm_rows.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

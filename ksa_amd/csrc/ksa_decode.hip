@@ -1032,7 +1032,7 @@ extern "C" size_t ksa_decode_qkv_o_workspace_bytes(int batch, int Hq, int Hkv, i
     return (size_t)batch * Hkv * nsplit * (size_t)pad_cols(Hq / Hkv) * (D + 2) * sizeof(float);
 }
 
-extern "C" size_t ksa_step_workspace_bytes(void) { return (size_t)kStepWords * kWordStride * 8; }
+extern "C" size_t ksa_step_workspace_bytes(void) { return kStepBytes; }
 extern "C" size_t ksa_step_status_offset(void) { return (size_t)kWordStride * kStepStatus * 8; }
 
 // Splits for the one launch: five attention workgroups to eight CUs, so that those of the product find places next to them, but

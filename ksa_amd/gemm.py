@@ -132,7 +132,8 @@ class MlpRowsWorkspace:
         self.H, self.I = H, I
         self.buf = torch.zeros(L.ksa_mlp_rows_workspace_bytes(H, I), dtype=torch.uint8, device=device)
         self._status = self.buf[L.ksa_mlp_rows_status_offset():][:8].view(torch.int64)
-        # ... and the counting words of the step's other one-launch form, `decode.ksa_decode_qkv_o`
+        # ... and the counting words of the step's other one-launch forms, `decode.ksa_decode_qkv_o` and
+        # `add_rmsnorm_linear_rows`
         self.step = torch.zeros(L.ksa_step_workspace_bytes(), dtype=torch.uint8, device=device)
         self._step_status = self.step[L.ksa_step_status_offset():][:8].view(torch.int64)
 
@@ -204,3 +205,47 @@ def add_rmsnorm_mlp_rows(o_partials: SplitKPartials, residual: torch.Tensor, nor
                                         float(eps), ws.buf.data_ptr(), ws.buf.numel(), _lib.stream_ptr(r2.device))
     _lib.check(rc, "ksa_add_rmsnorm_mlp_rows")
     return out_sum.view(residual.shape), SplitKPartials(part.view(torch.uint8), ks, M, residual.shape, dt)
+
+
+def add_rmsnorm_linear_rows_supported(M: int, N: int, H: int, device) -> bool:
+    """Whether `add_rmsnorm_linear_rows` takes these sizes: up to 4 rows, and all its workgroups run at once."""
+    with _lib.on_device(device):
+        return _lib.lib().ksa_add_rmsnorm_gemm_rows_splits(M, N, H) > 0
+
+
+def add_rmsnorm_linear_rows_pays(M: int, H: int, ksplit: int) -> bool:
+    """Whether it is the faster way: every workgroup adds up the rows for itself, which long rows of many slices make up
+    for longer.  `add_rmsnorm` + `linear_rows` / one launch, us: H 2560, N 6144, 19 slices, 1 / 2 / 3 / 4 rows 11.8 / 8.6,
+    12.0 / 10.2, 12.0 / 11.4, 12.2 / 12.1; the same without the hold-back of the weights, 8 slices 10.3 / 9.2, 10.4 / 9.8,
+    10.6 / 10.6; H 4096, N 2048, 19 slices, 1 / 3 rows 11.0 / 7.8, 11.5 / 9.3, 8 slices 9.0 / 7.6, 9.4 / 9.0; H 1024,
+    N 4096, 19 slices 7.3 / 6.9, 7.6 / 8.1, 8 slices 6.2 / 6.6."""
+    if H < 2048:
+        return M == 1 and ksplit > 16
+    return M <= (3 if ksplit > 16 else 2)
+
+
+def add_rmsnorm_linear_rows(delta: SplitKPartials, residual: torch.Tensor, norm_weight: torch.Tensor, eps: float,
+                            weight: TiledWeight, ws: MlpRowsWorkspace):
+    """One launch for `x' = residual + delta; y = norm(x') W^T` at a decode step (`ksa_add_rmsnorm_gemm_rows`;
+    modeling_qwen3sa.py:950-952 and the next layer's :938, :660-662).  Returns (x', y), y as `SplitKPartials`;
+    bit-identical to `add_rmsnorm` and `linear_rows`."""
+    M, H, N, dt = delta.rows, delta.shape[-1], weight.shape[0], delta.dtype
+    assert isinstance(weight, TiledWeight) and _weight_ok(weight, N, H, dt)
+    r2 = residual.reshape(-1, H)
+    if r2.stride(1) != 1:
+        r2 = r2.contiguous()
+    assert r2.shape[0] == M and r2.dtype == dt
+    w = norm_weight.to(dt).contiguous()
+    assert w.shape == (H,)
+    L = _lib.lib()
+    with _lib.on_device(r2.device):
+        ks = L.ksa_add_rmsnorm_gemm_rows_splits(M, N, H)
+        assert ks > 0, "sizes outside of add_rmsnorm_linear_rows_supported"
+        out_sum = torch.empty(M, H, dtype=dt, device=r2.device)
+        part = torch.empty(ks * 16 * N, dtype=torch.float32, device=r2.device)
+        rc = L.ksa_add_rmsnorm_gemm_rows(delta.workspace.data_ptr(), delta.ksplit, r2.data_ptr(), w.data_ptr(),
+                                         out_sum.data_ptr(), weight.data_ptr(), part.data_ptr(), M, N, H, r2.stride(0), H,
+                                         _DT[dt], float(eps), ws.step.data_ptr(), ws.step.numel(),
+                                         _lib.stream_ptr(r2.device))
+    _lib.check(rc, "ksa_add_rmsnorm_gemm_rows")
+    return out_sum.view(residual.shape), SplitKPartials(part.view(torch.uint8), ks, M, (*residual.shape[:-1], N), dt)

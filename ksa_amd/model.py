@@ -246,6 +246,19 @@ class HipOps:
         return self._gemm.add_rmsnorm_mlp_rows(o_partials, residual, norm_weight, eps, self._streaming(w_gate_up, 32),
                                                self._streaming(w_down), self.prepare_mlp_rows(H, I, residual.device))
 
+    def add_norm_linear(self, delta, residual, norm_weight, eps, weight):
+        """(residual + delta, norm of that sum times weight^T, deferred) in one launch from the K-split partial sums
+        delta; None where `add_rmsnorm` and `linear` have to do it."""
+        if not self.mlp_one_launch or not isinstance(delta, self._gemm.SplitKPartials):
+            return None
+        ws = self._step_ws(residual.shape[-1], residual.device)
+        takes = (ws is not None and self._gemm.add_rmsnorm_linear_rows_pays(delta.rows, weight.shape[1], delta.ksplit)
+                 and self._gemm.add_rmsnorm_linear_rows_supported(delta.rows, *weight.shape, residual.device))
+        tiled = self._streaming(weight) if takes else None
+        if not isinstance(tiled, self._gemm.TiledWeight):
+            return None
+        return self._gemm.add_rmsnorm_linear_rows(delta, residual, norm_weight, eps, tiled, ws)
+
     def mlp_rows_failed(self):
         """True if a `mlp_rows` launch gave up waiting since the last call (waits for the device; every
         workspace is looked at and, where needed, cleared: see `MlpRowsWorkspace.failed`)."""
@@ -470,6 +483,10 @@ class KsaQwen3ForCausalLM:
     def _norm_qkv(self, lw, delta, x):
         """The residual add and norm in front of a layer at a decode step, and its q | k | v projection:
         (x', deferred q | k | v)."""
+        if hasattr(self.ops, "add_norm_linear"):
+            out = self.ops.add_norm_linear(delta, x, lw["input_layernorm"], self.config.rms_norm_eps, lw["qkv_proj"])
+            if out is not None:
+                return out
         x, h = self._add_norm(delta, x, lw["input_layernorm"])
         return x, self.ops.linear(h, lw["qkv_proj"], defer=True)
 

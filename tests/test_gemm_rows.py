@@ -301,6 +301,70 @@ def test_gpu_mlp_rows_bounded_wait_gives_up_and_recovers():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,N,ksplit", [
+    (2560, 6144, 19),   # the 4B shape
+    (160, 16, 1),       # one short chunk, one tile in the only workgroup
+    (544, 272, 3),      # a second chunk of one step, a last workgroup of one tile
+    (4096, 1024, 64),   # the longest row, several requests of slices
+    (1024, 128, 20),
+])
+def test_gpu_add_rmsnorm_linear_rows_one_launch(dtype, H, N, ksplit):
+    """Residual add + norm + product in one launch against the two launches it stands for: the row sums bit for bit, the
+    product as the same partial sums of the same rows where that launch splits K into chunks of 512 too, and otherwise to
+    fp32 rounding (each of H products and sums is off by 2^-24 at the most: 2 sqrt(H) 2^-24 of the terms' root sum of
+    squares, generously).  Launches of changing row counts on one workspace, fresh data each."""
+    from ksa_amd import add_rmsnorm
+    from ksa_amd.gemm import (MlpRowsWorkspace, SplitKPartials, TiledWeight, add_rmsnorm_linear_rows,
+                              add_rmsnorm_linear_rows_supported, linear_rows)
+    dev = torch.device("cuda")
+    g = torch.Generator(device="cuda").manual_seed(H + N)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    w, nw = (rnd(N, H) * 0.03).to(dtype), (1 + 0.1 * rnd(H)).to(dtype)
+    tiled, ws = TiledWeight(w), MlpRowsWorkspace(H, 64, dev)
+    assert not add_rmsnorm_linear_rows_supported(5, N, H, dev) and not add_rmsnorm_linear_rows_supported(1, 1 << 20, H, dev)
+    for M in (1, 4, 2, 3, 3, 4, 1):
+        assert add_rmsnorm_linear_rows_supported(M, N, H, dev)
+        delta = SplitKPartials((rnd(ksplit, 16, H) * ksplit ** -0.5).view(-1).view(torch.uint8), ksplit, M, (1, M, H), dtype)
+        res = rnd(1, M, H).to(dtype)
+        x_ref, h = add_rmsnorm(delta, res, nw, 1e-6)
+        x_new, y = add_rmsnorm_linear_rows(delta, res, nw, 1e-6, tiled, ws)
+        ref = linear_rows(h, tiled, defer=True)
+        torch.cuda.synchronize()
+        assert not ws.failed() and int(ws.step.view(torch.int64).abs().sum().item()) == 0, M
+        assert torch.equal(x_new, x_ref), M
+        parts = lambda p: p.workspace.view(torch.float32).view(p.ksplit, 16, N)[:, :M]
+        assert y.shape == (1, M, N) and y.ksplit == -(-H // 512)
+        if isinstance(ref, SplitKPartials) and ref.ksplit == y.ksplit and H % 512 == 0:
+            assert torch.equal(parts(y), parts(ref)), M
+        want = h[0].double() @ w.double().t()
+        terms = (h[0].double().square() @ w.double().t().square()).sqrt()
+        assert ((parts(y).double().sum(0) - want).abs() <= 2 * H ** 0.5 * 2.0 ** -24 * terms).all(), M
+
+
+@pytest.mark.gpu
+def test_gpu_add_rmsnorm_linear_rows_bounded_wait_gives_up_and_recovers():
+    """The give-up path of the wait for the other chunks' sums, forced from the host: the status word is set, which every
+    workgroup that waits looks at; whether one of them had to wait or not, `failed()` reports it and zeroes the words."""
+    from ksa_amd.gemm import MlpRowsWorkspace, SplitKPartials, TiledWeight, add_rmsnorm_linear_rows
+    dev = torch.device("cuda")
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rnd = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    H, N, M = 1024, 2048, 4
+    tiled, ws = TiledWeight(rnd(N, H).bfloat16()), MlpRowsWorkspace(H, 64, dev)
+    delta = SplitKPartials(rnd(2, 16, H).view(-1).view(torch.uint8), 2, M, (1, M, H), torch.bfloat16)
+    res, one = rnd(1, M, H).bfloat16(), torch.ones(H, device="cuda").bfloat16()
+    call = lambda w: add_rmsnorm_linear_rows(delta, res, one, 1e-6, tiled, w)[1].workspace.view(torch.float32).view(2, 16, N)[:, :M]
+    ws._step_status.fill_(1)
+    torch.cuda.synchronize()
+    call(ws)
+    assert ws.failed() and not ws.failed()
+    assert int(ws.step.view(torch.int64).abs().sum().item()) == 0
+    a, b = call(ws), call(MlpRowsWorkspace(H, 64, dev))
+    assert not ws.failed() and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gpu_streaming_weight_layout(dtype):
     """`TiledWeight` (`ksa_tile_weights`): [ceil(N / 16)][K / 32][16][32] with zero rows past N, from a
     matrix and from a row slice of a larger one; and every few-rows kernel gives bit for bit the result
