@@ -442,13 +442,12 @@ int ksa_add_rmsnorm_mlp_rows(const float* o_partials, int o_ksplit, const void* 
                              void* workspace, size_t workspace_bytes, void* stream);
 
 /* The residual add + RMSNorm between two layers and the product behind it (HF:950-952, the next layer's HF:938, :660-662) for
- * at most 4 rows as one launch:
+ * at most 8 rows as one launch:
  *   x' = residual + sum of partials (out_sum), out_partials[c] = (norm(x') norm_weight)[:, 512 c : 512 c + 512] W[:, same]^T
  * partials fp32 [ksplit][16][H]; weight [N, H] in the streaming layout; out_partials fp32 [ceil(H / 512)][16][N].  Results
  * are those of ksa_add_rmsnorm_partials and ksa_gemm_rows.  step_workspace and the bounded wait inside the launch as at
  * ksa_decode_qkv_o_fwd, whose workspace it may share on one stream.  H a multiple of 32 up to 4096, N of 16 (KSA_ERR_UNSUPPORTED
- * otherwise).  ksa_add_rmsnorm_gemm_rows_splits: ceil(H / 512), or 0 where the two calls are to be used instead: sizes that
- * it does not take, or more workgroups than the device has CUs. */
+ * otherwise).  ksa_add_rmsnorm_gemm_rows_splits: ceil(H / 512), or 0 for sizes that it does not take. */
 int ksa_add_rmsnorm_gemm_rows_splits(int M, int N, int H);
 int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, const void* residual, const void* norm_weight,
                               void* out_sum, const void* weight, float* out_partials, int M, int N, int H,

@@ -58,8 +58,8 @@ __device__ __forceinline__ bool ksa_wave_wait(const unsigned long long* word, bo
     }
 }
 
-// Words of the workspace of ksa_decode_qkv_o_fwd and ksa_add_rmsnorm_gemm_rows.  They are zero between launches: the last
-// workgroup of a launch to have seen them clears them.
+// Words of the workspace of ksa_decode_qkv_o_fwd and ksa_add_rmsnorm_gemm_rows, the latter's rows behind them.  The words
+// are zero between launches: the last workgroup of a launch to have seen them clears them.
 enum {
     kStepStatus = 0,
     kStepAttnDone = 1,       // workgroups of the o projection that are through with their wait
@@ -69,10 +69,10 @@ enum {
     kStepNormDone0 = kStepHead0 + kStepMaxHeads,       // workgroups that have read a copy of the norm's sums
     kStepNorm0 = kStepNormDone0 + kStepNormCopies,     // a copy: 2^32 | sum of squares, [chunk of 512 columns][row]
     kStepWords = kStepNorm0 + kStepNormCopies,
-    kStepNormRows = 4,
-    kStepMaxHidden = 4096,
+    kStepNormRows = 8,
+    kStepMaxHidden = kWordStride / kStepNormRows * 512,
 };
-constexpr size_t kStepBytes = (size_t)kStepWords * kWordStride * 8;
+constexpr size_t kStepBytes = (size_t)kStepWords * kWordStride * 8 + (size_t)kStepNormRows * kStepMaxHidden * 2;
 
 // ---- residual add + RMSNorm of one row by the 512 threads of a workgroup ----
 // x' = residual + rounded sum of the K-split partial sums (plain store, for later launches), h = norm(x') w (for the

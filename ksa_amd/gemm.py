@@ -208,20 +208,17 @@ def add_rmsnorm_mlp_rows(o_partials: SplitKPartials, residual: torch.Tensor, nor
 
 
 def add_rmsnorm_linear_rows_supported(M: int, N: int, H: int, device) -> bool:
-    """Whether `add_rmsnorm_linear_rows` takes these sizes: up to 4 rows, and all its workgroups run at once."""
+    """Whether `add_rmsnorm_linear_rows` takes these sizes."""
     with _lib.on_device(device):
         return _lib.lib().ksa_add_rmsnorm_gemm_rows_splits(M, N, H) > 0
 
 
-def add_rmsnorm_linear_rows_pays(M: int, H: int, ksplit: int) -> bool:
-    """Whether it is the faster way: every workgroup adds up the rows for itself, which long rows of many slices make up
-    for longer.  `add_rmsnorm` + `linear_rows` / one launch, us: H 2560, N 6144, 19 slices, 1 / 2 / 3 / 4 rows 11.8 / 8.6,
-    12.0 / 10.2, 12.0 / 11.4, 12.2 / 12.1; the same without the hold-back of the weights, 8 slices 10.3 / 9.2, 10.4 / 9.8,
-    10.6 / 10.6; H 4096, N 2048, 19 slices, 1 / 3 rows 11.0 / 7.8, 11.5 / 9.3, 8 slices 9.0 / 7.6, 9.4 / 9.0; H 1024,
-    N 4096, 19 slices 7.3 / 6.9, 7.6 / 8.1, 8 slices 6.2 / 6.6."""
-    if H < 2048:
-        return M == 1 and ksplit > 16
-    return M <= (3 if ksplit > 16 else 2)
+def add_rmsnorm_linear_rows_pays(H: int, ksplit: int) -> bool:
+    """Whether it is the faster way: not for short rows of few slices, whose norm alone takes little.  `add_rmsnorm` +
+    `linear_rows` / one launch, us: H 2560, N 6144, 8 slices, 1 / 8 rows 10.3 / 8.7, 10.9 / 10.4 (19 slices: 11.7 / 8.7, 12.6 /
+    11.3); H 4096, N 2048, 8 slices 8.9 / 7.0, 9.7 / 9.1; H 1024, N 4096, 19 slices 7.4 / 6.4, 8.0 / 7.4, 8 slices 6.3 /
+    6.3, 6.8 / 7.2."""
+    return H >= 2048 or ksplit > 16
 
 
 def add_rmsnorm_linear_rows(delta: SplitKPartials, residual: torch.Tensor, norm_weight: torch.Tensor, eps: float,

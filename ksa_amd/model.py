@@ -252,7 +252,7 @@ class HipOps:
         if not self.mlp_one_launch or not isinstance(delta, self._gemm.SplitKPartials):
             return None
         ws = self._step_ws(residual.shape[-1], residual.device)
-        takes = (ws is not None and self._gemm.add_rmsnorm_linear_rows_pays(delta.rows, weight.shape[1], delta.ksplit)
+        takes = (ws is not None and self._gemm.add_rmsnorm_linear_rows_pays(weight.shape[1], delta.ksplit)
                  and self._gemm.add_rmsnorm_linear_rows_supported(delta.rows, *weight.shape, residual.device))
         tiled = self._streaming(weight) if takes else None
         if not isinstance(tiled, self._gemm.TiledWeight):
