@@ -180,10 +180,10 @@ _CHUNK_MAX = 512
 def _chunk_tiles(Sq: int, D: int, C: int, S: int, P: int, phys: bool) -> bool:
     """Whether a call runs on tiles laid along the chunks instead of the 128 x 64 grid of the block index: whole row
     tiles to a chunk, a summary count that divides the rows of a load, every summary row (in line or as the prefix that
-    is read in place) behind its whole chunk."""
+    is read in place) behind its whole chunk, and no more rows than the library takes in this form."""
     block = C + S
     return (C % TILE_M == 0 and C <= _CHUNK_MAX and (8 % S == 0 or (S == 16 and D <= 128)) and not phys
-            and Sq >= TILE_N and Sq % block <= C and P in (0, Sq // block * S))
+            and TILE_N <= Sq < 1 << 29 and Sq % block <= C and P in (0, Sq // block * S))
 
 
 def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P, skip_old, phys_prefix, scale, want_lse,
