@@ -71,7 +71,7 @@ int ksa_block_index(int Sq, int Sk, int C, int S, int W, int P, int skip_old, in
  *       rows * row stride * 2 bytes must stay below 4 GiB.
  *   out [batch, Sq, Hq, D]; lse fp32 [batch, Hq, Sq] (natural log) or NULL.
  *   mask_cnt .. full_idx: output of ksa_block_index(Sq, Sq+P, ..., 128, 64), idx_stride = N.
- *   scale: soft-max scale (the reference uses head_dim^-0.5).
+ *   scale: soft-max scale, positive, here and in every call below (the reference uses head_dim^-0.5).
  *   shape: workgroup shape, a tuning knob with no effect on the result beyond the tolerance of
  *       the tests.  KSA_PREFILL_SHAPE_AUTO lets the library choose from the launch size and the
  *       device's CU count; the others apply to head_dim 128 with an even Hq / Hkv and fall back

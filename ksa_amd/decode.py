@@ -17,7 +17,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from .prefill import kernel_head_dim, pad_head_dim
+from .prefill import fold_scale, kernel_head_dim, pad_head_dim
 
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
 
@@ -92,8 +92,7 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
         e0 = rows if end is None else int(end)
         assert 0 <= s0 < e0 <= rows, "row range out of bounds"
         max_rows = e0 - s0
-    if scale is None:
-        scale = float(D) ** -0.5
+    q, scale = fold_scale(q, float(D) ** -0.5 if scale is None else float(scale))
     if nsplit is None:
         nsplit = _lib.lib().ksa_decode_splits(b, q.shape[1], kcache.shape[1], q.shape[2], D, max_rows)
     Dk = kernel_head_dim(D)
@@ -109,10 +108,10 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
             lo, hi, s0, e0 = s0, e0, 0, e0 - s0
         kcache, vcache = pad_head_dim(kcache[:, :, lo:hi], Dk), pad_head_dim(vcache[:, :, lo:hi], Dk)
         out = torch.ops.ksa_amd.decode_fwd(pad_head_dim(q, Dk), kcache, vcache, t_start, t_end, s0, e0,
-                                           float(scale), int(nsplit))
+                                           scale, int(nsplit))
         return out[..., :D].contiguous()
     forward = _launch_decode if _lib.direct(q, kcache, vcache, t_start, t_end) else torch.ops.ksa_amd.decode_fwd
-    return forward(q, kcache, vcache, t_start, t_end, s0, e0, float(scale), int(nsplit))
+    return forward(q, kcache, vcache, t_start, t_end, s0, e0, scale, int(nsplit))
 
 
 def decode_qkv_supported(Hq: int, Hkv: int, D: int) -> bool:
@@ -136,8 +135,9 @@ def decode_qkv_pays(kcache: torch.Tensor, Hq: int, start, end) -> bool:
         return b * Hkv * n <= 2 * max(1, L.ksa_device_cu_count())
 
 
-def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end):
-    """What the two forms of the one-launch step share: the checked arguments, and the longest range."""
+def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end, scale):
+    """What the two forms of the one-launch step share: the checked arguments, and the longest range.  (The queries are
+    linear in their norm weight, which takes the sign of the scale.)"""
     from .gemm import SplitKPartials
     assert isinstance(qkv, SplitKPartials) and qkv.dtype in _DTYPES and qkv.dtype == kcache.dtype == vcache.dtype
     b, Hkv, rows, D = kcache.shape
@@ -146,7 +146,8 @@ def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, 
     assert kcache.stride(-1) == 1 and vcache.stride(-1) == 1, "cache rows must be contiguous"
     dt = qkv.dtype
     cos, sin = (t.to(dt).reshape(-1, D).contiguous() for t in (cos, sin))
-    qw, kw = q_norm_weight.to(dt).contiguous(), k_norm_weight.to(dt).contiguous()
+    qw, scale = fold_scale(q_norm_weight.to(dt).contiguous(), float(D) ** -0.5 if scale is None else float(scale))
+    kw = k_norm_weight.to(dt).contiguous()
     assert cos.shape == sin.shape and cos.shape[0] in (1, b) and qw.shape == (D,) and kw.shape == (D,)
     t_row = t_start = t_end = None
     s0, e0, r0 = 0, 1, 0
@@ -162,7 +163,7 @@ def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, 
     else:
         r0 = int(row)
         assert 0 <= r0 < rows and (t_start is not None or s0 <= r0 < e0), "the new row must lie in the attended range"
-    return cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows
+    return cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows, scale
 
 
 def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
@@ -173,8 +174,8 @@ def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor
     qkv: the deferred q | k | v projection (`SplitKPartials` [b, 1, (Hq + 2 Hkv) D]); cos / sin [1 or b, 1, D].  The
     token's key and value go to `row` of the caches and are attended with the rest of [start, end), which has
     to hold that row (each an int, or an int32 GPU tensor [b]).  Returns [b, 1, Hq D]."""
-    cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows = _qkv_arguments(
-        qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end)
+    cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows, scale = _qkv_arguments(
+        qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end, scale)
     b, Hkv, _, D = kcache.shape
     dev, dt = qkv.device, qkv.dtype
     L = _lib.lib()
@@ -193,7 +194,7 @@ def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor
             D if cos.shape[0] > 1 else 0, float(eps), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), ptr(t_row), r0,
             ptr(t_start), ptr(t_end), s0, e0, b, Hq, Hkv, D, _DTYPES[dt], _lib.strides3(kcache, dims),
             _lib.strides3(vcache, dims), _lib.strides3(out, dims),
-            float(D) ** -0.5 if scale is None else float(scale), nsplit, ptr(ws), ws_bytes, _lib.stream_ptr(dev))
+            scale, nsplit, ptr(ws), ws_bytes, _lib.stream_ptr(dev))
     _lib.check(rc, "ksa_decode_qkv_fwd")
     return out.view(b, 1, Hq * D)
 
@@ -211,8 +212,8 @@ def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tens
     (`ksa_decode_qkv_o_fwd`), for at most 16 sequences: o_weight a `gemm.TiledWeight` [N, Hq D], ws the step's
     `gemm.MlpRowsWorkspace`.  Returns the product's `SplitKPartials` [b, 1, N]."""
     from .gemm import SplitKPartials, TiledWeight
-    cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows = _qkv_arguments(
-        qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end)
+    cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows, scale = _qkv_arguments(
+        qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end, scale)
     b, Hkv, _, D = kcache.shape
     dev, dt = qkv.device, qkv.dtype
     N = o_weight.shape[0]
@@ -231,7 +232,7 @@ def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tens
             qkv.workspace.data_ptr(), qkv.ksplit, qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(),
             D if cos.shape[0] > 1 else 0, float(eps), kcache.data_ptr(), vcache.data_ptr(), ptr(t_row), r0,
             ptr(t_start), ptr(t_end), s0, e0, b, Hq, Hkv, D, _DTYPES[dt], _lib.strides3(kcache, dims),
-            _lib.strides3(vcache, dims), float(D) ** -0.5 if scale is None else float(scale), nsplit, o_weight.data_ptr(),
+            _lib.strides3(vcache, dims), scale, nsplit, o_weight.data_ptr(),
             part.data_ptr(), N, sums.data_ptr(), ws_bytes, ws.step.data_ptr(), ws.step.numel(), _lib.stream_ptr(dev))
     _lib.check(rc, "ksa_decode_qkv_o_fwd")
     return SplitKPartials(part.view(torch.uint8), ks, b, (b, 1, N), dt)
@@ -262,8 +263,7 @@ def ksa_decode_boundary(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
         return None, None, int(lo), int(hi)
     ts, te, ts0, te0 = pair(text_start, text_end)
     ss, se, ss0, se0 = pair(sum_start, sum_end)
-    if scale is None:
-        scale = float(D) ** -0.5
+    q, scale = fold_scale(q, float(D) ** -0.5 if scale is None else float(scale))
     lib = _lib.lib()
     if nsplit is None:   # (the count by the slices: ksa_decode_splits is for one range, not for two of different lengths)
         nsplit = lib.ksa_decode_auto_splits(b, Hkv, rows if ts is not None else te0 - ts0)
@@ -278,7 +278,7 @@ def ksa_decode_boundary(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
             q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), ptr(ts), ptr(te), ts0, te0,
             ptr(ss), ptr(se), ss0, se0, b, Hq, Hkv, Q, D, _DTYPES[q.dtype], _lib.strides3(q, (0, 1, 2)),
             _lib.strides3(kcache, (0, 1, 2)), _lib.strides3(vcache, (0, 1, 2)), _lib.strides3(out, (0, 1, 2)),
-            float(scale), int(nsplit), ptr(ws), ws_bytes, _lib.stream_ptr(q.device))
+            scale, int(nsplit), ptr(ws), ws_bytes, _lib.stream_ptr(q.device))
     _lib.check(rc, "ksa_decode_boundary_fwd")
     return out
 

@@ -172,6 +172,14 @@ def pad_head_dim(t: torch.Tensor, Dk: int) -> torch.Tensor:
     return t if t.shape[-1] == Dk else torch.nn.functional.pad(t, (0, Dk - t.shape[-1]))
 
 
+def fold_scale(q: torch.Tensor, scale: float):
+    """(q', scale') with q' scale' = q scale, exactly, and scale' positive: the kernels hide a key by a score of -inf in
+    front of the factor, which a negative one would turn into +inf and zero into NaN."""
+    if scale < 0:
+        return -q, -scale
+    return (torch.zeros_like(q), 1.0) if scale == 0 else (q, scale)
+
+
 # `shape` of a call on chunk tiles (ksa_prefill_chunks_fwd), and the largest chunk that takes them
 _CHUNK_TILES = 128
 _CHUNK_MAX = 512
@@ -294,7 +302,7 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     if k.stride() != v.stride():
         v = v.contiguous()
         k = k.contiguous()
-    scale = float(D) ** -0.5 if softmax_scale is None else float(softmax_scale)
+    q, scale = fold_scale(q, float(D) ** -0.5 if softmax_scale is None else float(softmax_scale))
     Dk = kernel_head_dim(D)
     if Dk != D:   # a head dimension without a kernel of its own: zero-padded copies (see kernel_head_dim)
         q, k, v = pad_head_dim(q, Dk), pad_head_dim(k, Dk), pad_head_dim(v, Dk)

@@ -424,6 +424,26 @@ def test_decode_qkv_o_equals_separate_launches(dtype, b, Hq, Hkv, D, N, nsplit):
         assert (got - want).square().mean() <= (0.25 * ulp) ** 2 * (K * term.square()).mean()
 
 
+@pytest.mark.parametrize("scale", [-0.3, 0.0])
+def test_decode_scale_that_is_not_positive(scale):
+    """Ranges that end inside a tile (hidden rows) with one split and with several; the one-launch step against the oracle
+    on the rows that it wrote."""
+    from ksa_amd import decode, gemm
+    q, k, v = _mk(2, 4, 2, 1, 128, 700, seed=8)
+    for nsplit in (1, 3):
+        _check(q, k, v, [3, 0], [77, 690], nsplit, scale=scale)
+    dev = torch.device("cuda")
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    qkv = gemm.linear_rows(rnd(2, 1, 1024), rnd(8 * 128, 1024), defer=True)
+    kc, vc, one, zero = k.to(dev), v.to(dev), torch.ones(128, device=dev).bfloat16(), torch.zeros(128, device=dev).bfloat16()
+    got = decode.ksa_decode_qkv(qkv, one, one, one, zero, 1e-6, kc, vc, 4, 76, 3, 77, scale=scale)
+    x = qkv.workspace.view(torch.float32).view(qkv.ksplit, 16, 1024)[:, :2].sum(0).bfloat16().float().view(2, 8, 128)
+    qn = (x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6))[:, :4, None]
+    want = c_oracle.decode(to_np(qn), to_np(kc), to_np(vc), 3, 77, scale=scale)
+    assert np.abs(to_np(got).reshape(want.shape) - want).max() <= ATOL * max(1.0, np.abs(want).max())
+
+
 @pytest.mark.gpu
 def test_decode_qkv_o_bounded_wait_gives_up_and_recovers():
     """The give-up path of the wait for the attention, forced from the host: the counts are set far below zero.  The first

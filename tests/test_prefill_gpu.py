@@ -734,3 +734,22 @@ def test_prefill_chunk_tiles_of_both_workgroup_shapes(shape):
         assert rc == 0
         assert (out.float() - want.float()).abs().max() <= ATOL * max(1.0, float(want.float().abs().max()))
         assert (lse - wlse).abs().max() <= 0.1 + 1e-3 * float(wlse.abs().max())
+
+
+@pytest.mark.parametrize("scale", [-0.3, 0.0])
+@pytest.mark.parametrize("chunk_tiles", [True, False])
+def test_prefill_scale_that_is_not_positive(scale, chunk_tiles):
+    """A negative scale prefers the keys that a positive one avoids, zero weighs every visible key the same; hidden keys
+    stay hidden.  Text and summary rows, tiles with and without hidden keys."""
+    import ksa_amd
+    dev = torch.device("cuda")
+    C, S, W, n = 128, 8, 2, 5 * 136 + 70
+    q, k, v = make_qkv(n, 4, 2, 128, seed=77, scaled=False)
+    sp = O.summary_positions(n, C, S)
+    want, wlse = c_oracle.attention_rows(to_np(q), to_np(k), to_np(v), C, S, W, summary_pos=sp, scale=scale)
+    out, lse = ksa_amd.summary_attn_func(q[None].to(dev), k[None].to(dev), v[None].to(dev), C, S, W, return_lse=True,
+                                         summary_pos=torch.as_tensor(sp, device=dev), softmax_scale=scale,
+                                         chunk_tiles=chunk_tiles)
+    assert np.isfinite(to_np(out)).all()
+    assert np.abs(to_np(out[0]) - want).max() <= ATOL * max(1.0, np.abs(want).max())
+    assert np.abs(to_np(lse[0]) - wlse).max() <= 5e-2
