@@ -1,7 +1,7 @@
 """The helper operators around the two attention paths as `torch.library.custom_op`s with fake
 (shape-only) kernels, so that a caller may trace or `torch.compile` code that contains them:
 `torch.ops.ksa_amd.{pre_attention, rmsnorm, add_rmsnorm, add_rmsnorm_partials, silu_mul, linear_rows,
-gate_up_silu_rows, mlp_rows, argmax_rows}`.  (`summary_attn_fwd` and `decode_fwd` are registered where
+gate_up_silu_rows, mlp_rows, argmax_rows}`.  (`summary_attn_fwd`, `summary_attn_chunks_fwd` and `decode_fwd` are registered where
 they are defined, `prefill.py` and `decode.py`.)
 
 They take and return plain tensors and allocate their outputs; the forms that write into a caller's

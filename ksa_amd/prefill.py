@@ -180,9 +180,7 @@ def fold_scale(q: torch.Tensor, scale: float):
     return (torch.zeros_like(q), 1.0) if scale == 0 else (q, scale)
 
 
-# `shape` of a call on chunk tiles (ksa_prefill_chunks_fwd), and the largest chunk that takes them
-_CHUNK_TILES = 128
-_CHUNK_MAX = 512
+_CHUNK_MAX = 512   # the largest chunk that takes tiles laid along the chunks (ksa_prefill_chunks_fwd)
 
 
 def _chunk_tiles(Sq: int, D: int, C: int, S: int, P: int, phys: bool) -> bool:
@@ -194,26 +192,39 @@ def _chunk_tiles(Sq: int, D: int, C: int, S: int, P: int, phys: bool) -> bool:
             and TILE_N <= Sq < 1 << 29 and Sq % block <= C and P in (0, Sq // block * S))
 
 
-def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P, skip_old, phys_prefix, scale, want_lse,
-                    shape):
-    b, Sq, Hq, D = q.shape
+def _outputs(q, want_lse):
+    b, Sq, Hq, _ = q.shape
     dev = q.device
     out = torch.empty_like(q)
     lse = torch.empty((b, Hq, Sq), dtype=torch.float32, device=dev) if want_lse else None
     # work queues of this call alone, for a launch long enough to use them (the library's own bound is 32
     # workgroups per CU; a workgroup takes 128 rows of one or two heads)
     sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= 1 << 19 else None
+    return out, lse, sched
+
+
+def _launch_chunks(q, k, v, C, S, W, skip_old, scale, want_lse):
+    b, Sq, Hq, D = q.shape
+    dev = q.device
+    out, lse, sched = _outputs(q, want_lse)
     dims = (0, 1, 2)
-    if shape == _CHUNK_TILES:
-        with _lib.on_device(dev):
-            rc = _lib.lib().ksa_prefill_chunks_fwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr() if want_lse else None,
-                b, Sq, Hq, k.shape[2], D, _DTYPES[q.dtype],
-                _lib.strides3(q, dims), _lib.strides3(k, dims), _lib.strides3(out, dims),
-                C, S, W, int(skip_old), scale, 0, sched.data_ptr() if sched is not None else None, _lib.stream_ptr(dev))
-        if rc:
-            _lib.check(rc, "ksa_prefill_chunks_fwd")
-        return out, lse
+    with _lib.on_device(dev):
+        rc = _lib.lib().ksa_prefill_chunks_fwd(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr() if want_lse else None,
+            b, Sq, Hq, k.shape[2], D, _DTYPES[q.dtype],
+            _lib.strides3(q, dims), _lib.strides3(k, dims), _lib.strides3(out, dims),
+            C, S, W, int(skip_old), scale, 0, sched.data_ptr() if sched is not None else None, _lib.stream_ptr(dev))
+    if rc:
+        _lib.check(rc, "ksa_prefill_chunks_fwd")
+    return out, lse
+
+
+def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P, skip_old, phys_prefix, scale, want_lse,
+                    shape):
+    b, Sq, Hq, D = q.shape
+    dev = q.device
+    out, lse, sched = _outputs(q, want_lse)
+    dims = (0, 1, 2)
     with _lib.on_device(dev):
         rc = _lib.lib().ksa_prefill_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
@@ -242,6 +253,20 @@ def _summary_attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 @_summary_attn_fwd.register_fake
 def _(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P, skip_old, phys_prefix, scale,
       want_lse, shape):
+    b, Sq, Hq, _ = q.shape
+    return torch.empty_like(q), q.new_empty((b, Hq, Sq) if want_lse else (0,), dtype=torch.float32)
+
+
+@torch.library.custom_op("ksa_amd::summary_attn_chunks_fwd", mutates_args=())
+def _summary_attn_chunks_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, C: int, S: int, W: int, skip_old: bool,
+                             scale: float, want_lse: bool) -> Tuple[torch.Tensor, torch.Tensor]:
+    assert k.shape[1] == q.shape[1], "chunk tiles: the summary rows lie in line, k and v have the rows of q"
+    out, lse = _launch_chunks(q, k, v, C, S, W, skip_old, scale, want_lse)
+    return out, torch.empty(0, dtype=torch.float32, device=q.device) if lse is None else lse
+
+
+@_summary_attn_chunks_fwd.register_fake
+def _(q, k, v, C, S, W, skip_old, scale, want_lse):
     b, Sq, Hq, _ = q.shape
     return torch.empty_like(q), q.new_empty((b, Hq, Sq) if want_lse else (0,), dtype=torch.float32)
 
@@ -309,15 +334,14 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     shape = PREFILL_SHAPE if workgroup_shape is None else int(workgroup_shape)
     direct = _lib.direct(q, k, v)
     if shape == 0 and chunk_tiles and _chunk_tiles(Sq, Dk, C, S, P, phys):
-        shape = _CHUNK_TILES
-    elif shape == _CHUNK_TILES:
-        shape = -1   # no shape that a caller can name: refused by the library
-    # (chunk tiles need no block index; the operator's arguments hold one)
-    idx = (None,) * 4 if direct and shape == _CHUNK_TILES else _cached_index(Sq, C, S, W, P, skip_old_summary, q.device)
-    forward = _launch_prefill if direct else torch.ops.ksa_amd.summary_attn_fwd
-    out, lse = forward(
-        q, k, v, idx[0], idx[1], idx[2], idx[3], C, S, W, P,
-        bool(skip_old_summary), phys, scale, bool(return_lse), shape)
+        forward = _launch_chunks if direct else torch.ops.ksa_amd.summary_attn_chunks_fwd
+        out, lse = forward(q, k, v, C, S, W, bool(skip_old_summary), scale, bool(return_lse))
+    else:
+        idx = _cached_index(Sq, C, S, W, P, skip_old_summary, q.device)
+        forward = _launch_prefill if direct else torch.ops.ksa_amd.summary_attn_fwd
+        out, lse = forward(
+            q, k, v, idx[0], idx[1], idx[2], idx[3], C, S, W, P,
+            bool(skip_old_summary), phys, scale, bool(return_lse), shape)
     if Dk != D:
         out = out[..., :D].contiguous()
     return out, (lse if return_lse else None)

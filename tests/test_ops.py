@@ -191,6 +191,34 @@ def test_direct_calls_step_aside_for_modes_and_subclasses():
     assert not _lib.direct(q.detach().requires_grad_())
 
 
+@pytest.mark.gpu
+def test_prefill_operators_refuse_what_they_do_not_take():
+    """The operator of the block index knows the shapes of the library and no other, the one of the chunk tiles takes no
+    built prefix and no layout outside of the library's rule; a call through each equals the direct call."""
+    import ksa_amd
+    from ksa_amd import _lib, prefill
+    ns = torch.ops.ksa_amd
+    g = torch.Generator(device="cuda").manual_seed(1)
+    C, S, W, n = 128, 8, 1, 3 * 136 + 70
+    q, k, v = (torch.randn(1, n, h, 64, generator=g, device="cuda").bfloat16() for h in (4, 2, 2))
+    pos = torch.arange(n, device="cuda") % (C + S) >= C
+    built = [torch.cat((t[:, pos], t), dim=1) for t in (k, v)]
+    idx = prefill.compute_block_sparsity(n, n + 3 * S, C, S, W)
+    for bad in (128, 1, -1):
+        with pytest.raises(_lib.KsaError):
+            ns.summary_attn_fwd(q, *built, *idx, C, S, W, 3 * S, False, True, 0.125, False, bad)
+        with pytest.raises(_lib.KsaError):
+            ksa_amd.summary_attn_func(q, *built, C, S, W, workgroup_shape=bad)
+    with pytest.raises(AssertionError):
+        ns.summary_attn_chunks_fwd(q, *built, C, S, W, False, 0.125, False)
+    with pytest.raises(_lib.KsaError):
+        ns.summary_attn_chunks_fwd(q, k, v, 100, S, W, False, 0.125, False)
+    args = (q, k, v, C, S, W, False, 0.125, True)
+    for got, want in zip(ns.summary_attn_chunks_fwd(*args), ksa_amd.summary_attn_func(*args[:6], pos, return_lse=True)):
+        assert torch.equal(got, want)
+    torch.library.opcheck(ns.summary_attn_chunks_fwd, args, test_utils=("test_schema", "test_faketensor"))
+
+
 def test_direct_calls_step_aside_for_transforms_and_negative_views():
     """... nor inside `torch.func` transforms and function modes, nor for views whose negative bit is set."""
     from torch.overrides import TorchFunctionMode
