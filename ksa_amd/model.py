@@ -129,7 +129,12 @@ def convert_weights(weights: dict, device, dtype) -> dict:
 
 
 class HipOps:
-    """The attention-side operators of the model, bound to this package's HIP kernels."""
+    """The attention-side operators of the model, bound to this package's HIP kernels.
+
+    The one-launch forms of a decode step count on words in device memory (`MlpRowsWorkspace`), kept here by (device, hidden
+    size, MLP size): decoders of different sizes have words of their own, but steps of decoders of equal sizes on one
+    operator set - one model's steps with two caches among them - must not run on two streams at once.  A program
+    that does so gives each stream its operator set."""
 
     def __init__(self):
         from . import cache, decode, elementwise, gemm, pre, prefill
@@ -192,16 +197,18 @@ class HipOps:
         return self._decode_mod.ksa_decode_qkv(qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end,
                                                scale=scale)
 
-    def _step_ws(self, H, device):
-        """The workspace of the one-launch forms for this hidden size, if `prepare_mlp_rows` has made one."""
-        return next((ws for (d, h, _), ws in self._mlp_ws.items() if d == str(device) and h == H), None)
+    def _step_ws(self, rows, H, I, device):
+        """The counting words of the step's other one-launch forms: those of the one-launch MLP of this decoder (hidden
+        size, MLP size) and step, if `prepare_mlp_rows` has made them.  Where the MLP itself runs as separate launches
+        there are none, so that two steps share words here only if they share them there."""
+        return self._mlp_ws.get((str(device), H, I)) if self._gemm.mlp_rows_supported(rows, H, I) else None
 
-    def decode_qkv_o(self, qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end, scale, o_weight):
-        """`decode_qkv` and the o projection behind it in one launch: the projection's partial sums; None where
-        the two have to do it."""
+    def decode_qkv_o(self, qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end, scale, o_weight, mlp_size):
+        """`decode_qkv` and the o projection behind it in one launch, for a decoder of this MLP size: the projection's
+        partial sums; None where the two have to do it."""
         if not self.mlp_one_launch or not isinstance(qkv, self._gemm.SplitKPartials):
             return None
-        ws = self._step_ws(o_weight.shape[0], kbuf.device)
+        ws = self._step_ws(kbuf.shape[0], o_weight.shape[0], mlp_size, kbuf.device)
         takes = ws is not None and self._decode_mod.decode_qkv_o_supported(kbuf, Hq, o_weight.shape[0])
         tiled = self._streaming(o_weight) if takes else None
         if not isinstance(tiled, self._gemm.TiledWeight):
@@ -246,12 +253,12 @@ class HipOps:
         return self._gemm.add_rmsnorm_mlp_rows(o_partials, residual, norm_weight, eps, self._streaming(w_gate_up, 32),
                                                self._streaming(w_down), self.prepare_mlp_rows(H, I, residual.device))
 
-    def add_norm_linear(self, delta, residual, norm_weight, eps, weight):
+    def add_norm_linear(self, delta, residual, norm_weight, eps, weight, mlp_size):
         """(residual + delta, norm of that sum times weight^T, deferred) in one launch from the K-split partial sums
-        delta; None where `add_rmsnorm` and `linear` have to do it."""
+        delta, for a decoder of this MLP size; None where `add_rmsnorm` and `linear` have to do it."""
         if not self.mlp_one_launch or not isinstance(delta, self._gemm.SplitKPartials):
             return None
-        ws = self._step_ws(residual.shape[-1], residual.device)
+        ws = self._step_ws(delta.rows, residual.shape[-1], mlp_size, residual.device)
         takes = (ws is not None and self._gemm.add_rmsnorm_linear_rows_pays(weight.shape[1], delta.ksplit)
                  and self._gemm.add_rmsnorm_linear_rows_supported(delta.rows, *weight.shape, residual.device))
         tiled = self._streaming(weight) if takes else None
@@ -484,7 +491,8 @@ class KsaQwen3ForCausalLM:
         """The residual add and norm in front of a layer at a decode step, and its q | k | v projection:
         (x', deferred q | k | v)."""
         if hasattr(self.ops, "add_norm_linear"):
-            out = self.ops.add_norm_linear(delta, x, lw["input_layernorm"], self.config.rms_norm_eps, lw["qkv_proj"])
+            out = self.ops.add_norm_linear(delta, x, lw["input_layernorm"], self.config.rms_norm_eps, lw["qkv_proj"],
+                                           self.config.intermediate_size)
             if out is not None:
                 return out
         x, h = self._add_norm(delta, x, lw["input_layernorm"])
@@ -497,7 +505,8 @@ class KsaQwen3ForCausalLM:
         ops = self.ops
         if hasattr(ops, "decode_qkv_o"):
             o = ops.decode_qkv_o(qkv, lw["q_norm"], lw["k_norm"], cos, sin, self.config.rms_norm_eps, kc, vc,
-                                 self.config.num_attention_heads, row, start, end, self.scaling, lw["o_proj"])
+                                 self.config.num_attention_heads, row, start, end, self.scaling, lw["o_proj"],
+                                 self.config.intermediate_size)
             if o is not None:
                 return o
         return ops.linear(self._text_heads(lw, qkv, cos, sin, kc, vc, row, start, end, slots), lw["o_proj"], defer=True)

@@ -438,6 +438,38 @@ def _mlp_rows_config():
                        summary_sliding_chunk_num=[1, 1 << 20, 1], vocab_size=1000, summary_token_begin=1000)
 
 
+def test_one_launch_forms_count_on_the_words_of_their_own_decoder(monkeypatch):
+    """Two decoders of one hidden size and different MLP sizes on one operator set: each gets the workspace that its own
+    one-launch MLP uses, whichever was made first, so that their steps may overlap; none where that MLP takes other launches
+    (16 rows of 5120).  Host logic: the launches themselves are replaced by what they were given."""
+    from ksa_amd import decode, gemm
+    from ksa_amd.model import HipOps
+    given = []
+    monkeypatch.setattr(gemm, "MlpRowsWorkspace", lambda H, I, device: (H, I))
+    monkeypatch.setattr(gemm, "add_rmsnorm_linear_rows", lambda *a: (given.append(a[-1]), (None, None))[1])
+    monkeypatch.setattr(decode, "ksa_decode_qkv_o", lambda *a, **k: (given.append(a[-1]), "o")[1])
+    monkeypatch.setattr(HipOps, "_streaming", lambda self, w, multiple=16: object.__new__(gemm.TiledWeight))
+    ops = HipOps()
+    for H, b, sizes in ((2048, 2, (512, 1024)), (5120, 16, (512,))):
+        models = []
+        for I in sizes:
+            cfg = tiny_config(hidden_size=H, intermediate_size=I, num_attention_heads=8, num_hidden_layers=1,
+                              summary_sliding_chunk_num=1)
+            models.append(KsaQwen3ForCausalLM(cfg, init_weights(cfg, "cpu", torch.bfloat16), ops))
+            ops.prepare_mlp_rows(H, I, torch.device("cpu"))
+        for model, I in list(zip(models, sizes))[::-1]:
+            lw = model.w["layers"][0]
+            part = lambda n: gemm.SplitKPartials(torch.zeros(17 * 16 * n * 4, dtype=torch.uint8), 17, b, (b, 1, n), torch.bfloat16)
+            kc = torch.zeros(b, 2, 32, 64, dtype=torch.bfloat16)
+            given.clear()
+            if H == 2048:
+                model._norm_qkv(lw, part(H), torch.zeros(b, 1, H, dtype=torch.bfloat16))
+                assert model._text_attention(lw, part(12 * 64), None, None, kc, kc, 3, 0, 9, {}) == "o"
+                assert given == [(H, I)] * 2
+            else:
+                assert ops.decode_qkv_o(part(12 * 64), *[None] * 5, kc, kc, 8, 3, 0, 9, 1.0, lw["o_proj"], I) is None
+
+
 @pytest.mark.gpu
 def test_gpu_one_model_serves_changing_batch_sizes():
     """Batch 8, then 2, then 8, then 1 on ONE model (one operator set, hence one workspace of the
