@@ -175,6 +175,7 @@ int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_
 size_t ksa_step_workspace_bytes(void);  /* (ksa_add_rmsnorm_gemm_rows shares it) */
 size_t ksa_step_status_offset(void);
 int ksa_decode_qkv_o_splits(int batch, int Hq, int Hkv, int D, int max_rows);
+int ksa_decode_qkv_o_pays(int batch, int Hq, int Hkv, int D, int N, int max_rows);  /* 1: faster than the separate calls */
 size_t ksa_decode_qkv_o_workspace_bytes(int batch, int Hq, int Hkv, int D, int nsplit);
 int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
                          const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,

@@ -73,6 +73,7 @@ _SIGNATURES = {
     "ksa_step_workspace_bytes": (ctypes.c_size_t, []),
     "ksa_step_status_offset": (ctypes.c_size_t, []),
     "ksa_decode_qkv_o_splits": (_int, [_int] * 5),
+    "ksa_decode_qkv_o_pays": (_int, [_int] * 6),
     "ksa_decode_qkv_o_workspace_bytes": (ctypes.c_size_t, [_int] * 5),
     "ksa_decode_qkv_o_fwd": (_int, [_vp, _int] + [_vp] * 4 + [ctypes.c_longlong, ctypes.c_float] + [_vp] * 3 + [_int]
                              + [_vp] * 2 + [_int] * 7 + [_i64p] * 2 + [ctypes.c_float, _int, _vp, _vp, _int, _vp,

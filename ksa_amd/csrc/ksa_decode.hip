@@ -1035,17 +1035,36 @@ extern "C" size_t ksa_decode_qkv_o_workspace_bytes(int batch, int Hq, int Hkv, i
 extern "C" size_t ksa_step_workspace_bytes(void) { return kStepBytes; }
 extern "C" size_t ksa_step_status_offset(void) { return (size_t)kWordStride * kStepStatus * 8; }
 
-// Splits for the one launch: five attention workgroups to eight CUs, so that those of the product find places next to them, but
-// no more than the count for the attention alone, nor than the sums that a workgroup of the product merges.  Attention
-// + product at 32 / 8 heads of 128, 4096 x 2560, us: the separate launches / this form with their count / with this one: 1 sequence of
-// 700 / 4100 / 16000 rows 17.6 / 14.9 / 14.9, 21.4 / 19.7 / 18.3, 27.2 / 26.7 / 26.5; 2 of 700 18.0 / 17.2 / 16.7, 4 of 700
-// 20.6 / 19.8 / 18.9, 8 of 700 / 4100 22.0 / 22.9 / 19.9, 40.7 / 39.3 / 36.5; 16 of 700 / 4100 26.6 / 26.3 / 23.6, 60.8 / 57.9 / 56.3.
+// Splits for the one launch.  The count for the attention alone as long as its workgroups leave every CU room for one of the
+// product (units * n <= CUs) and the sums to merge stay few; otherwise five attention workgroups to eight CUs, so that those of the
+// product find places next to them.  One sequence of 32768 rows and more takes every split that a workgroup of the product
+// merges, 64: there the attention is all of the time.  Attention + product at 32 / 8 heads of 128, N 2560, us, separate launches /
+// five to eight CUs / this rule where it differs: 1 sequence of 4096 / 32768 / 131072 rows 19.5 / 18.1 / 17.9, 38.3 / 36.6 / 36.5,
+// 101.3 / 101.3 / 99.0; N 4096, 65536 rows 60.3 / 61.5 / 58.5; 4 of 700 18.7 / 18.8 / 17.6; N 4096, 8 of 400 21.4 / 22.2 / 21.3.
+// The rule kept at five to eight, separate / it / the count alone: 8 of 4096 / 32768 39.0 / 35.6 / 37.1, 180.5 / 168.2 / 176.3; 16 of
+// 4096 60.0 / 55.2 / 57.6; 1 of 16384 28.2 / 27.0 / 27.3.
 extern "C" int ksa_decode_qkv_o_splits(int batch, int Hq, int Hkv, int D, int max_rows) {
     if (batch <= 0 || batch > 16 || Hkv <= 0) return 1;
     const int units = batch * Hkv, cus = ksa_cu_count_or(256);
-    int n = (cus * 5 / 8 + units - 1) / units;
-    n = min(n, min(ksa_decode_splits(batch, Hq, Hkv, 1, D, max_rows), kMaxOSums / batch));
+    int n = min(ksa_decode_splits(batch, Hq, Hkv, 1, D, max_rows), kMaxOSums / batch);
+    if (!(batch == 1 && max_rows >= 32768) && (units * n > cus || batch * n > 32)) n = min(n, (cus * 5 / 8 + units - 1) / units);
     return n < 1 ? 1 : n;
+}
+
+// Whether the one launch is the faster way.  Its gain is two ramps and a trip of the rows, 1 to 3 us, and the time of o's
+// weights where they are many; its price the merge of batch * n sums in every workgroup of the product, fewer splits, and the
+// attention's places on the CUs that the product holds.  Measured over 1675 shapes (1 to 16 sequences of 400 to 131072 rows, 8 to
+// 64 heads of 128 and 64, 1 to 32 kv heads, N 1024 to 5120): 326 are taken, at 0.92 of the separate launches on average and 1.02 at the
+// worst.  Outside: 16 sequences with 1 kv head, 64 sums, 4 splits where the attention alone has 32: 400 / 131072 rows 1.05 / 1.92;
+// 2 kv heads, 8 sequences 1.01 to 1.12; head_dim 64 from 4096 rows on 1.05 to 1.6 (a split is half the work and as many trips);
+// 16 heads (16 KB of a column's weights instead of 32) with more than 20 sums up to 1.13; 64 heads, N 5120, 640 workgroups of
+// the product 1.00 to 1.14; 32 kv heads up to 1.08.  Some of the shapes left out gain, e.g. 32 / 4 heads, 16 sequences 0.94 to 0.98.
+extern "C" int ksa_decode_qkv_o_pays(int batch, int Hq, int Hkv, int D, int N, int max_rows) {
+    if (batch <= 0 || batch > 16 || Hkv <= 0 || Hkv > 8 || Hq % Hkv != 0 || N <= 0 || max_rows <= 0) return 0;
+    if ((N + 127) / 128 * (int64_t)(Hq * D / kChunkK) > ksa_cu_count_or(256)) return 0;
+    const int n = ksa_decode_qkv_o_splits(batch, Hq, Hkv, D, max_rows);
+    if (n > 1 && batch * n <= 20 && n == ksa_decode_splits(batch, Hq, Hkv, 1, D, max_rows)) return 1;
+    return D == 128 && Hq * D >= 4096 && (batch * n <= 32 || (batch == 1 && max_rows >= 32768));
 }
 
 extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,

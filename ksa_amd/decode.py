@@ -205,6 +205,16 @@ def decode_qkv_o_supported(kcache: torch.Tensor, Hq: int, N: int) -> bool:
             and N % 16 == 0)
 
 
+def decode_qkv_o_pays(kcache: torch.Tensor, Hq: int, N: int, start, end) -> bool:
+    """Whether `ksa_decode_qkv_o` is the faster way (`ksa_decode_qkv_o_pays`, by the longest possible range where the ranges
+    are on the device)."""
+    b, Hkv, rows, D = kcache.shape
+    if not (isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor)):
+        rows = max(1, int(end) - int(start))
+    with _lib.on_device(kcache.device):
+        return _lib.lib().ksa_decode_qkv_o_pays(b, Hq, Hkv, D, N, rows) != 0
+
+
 def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                      eps: float, kcache: torch.Tensor, vcache: torch.Tensor, Hq: int, row, start, end, o_weight, ws,
                      scale: Optional[float] = None, nsplit: Optional[int] = None):

@@ -209,7 +209,8 @@ class HipOps:
         if not self.mlp_one_launch or not isinstance(qkv, self._gemm.SplitKPartials):
             return None
         ws = self._step_ws(kbuf.shape[0], o_weight.shape[0], mlp_size, kbuf.device)
-        takes = ws is not None and self._decode_mod.decode_qkv_o_supported(kbuf, Hq, o_weight.shape[0])
+        takes = (ws is not None and self._decode_mod.decode_qkv_o_supported(kbuf, Hq, o_weight.shape[0])
+                 and self._decode_mod.decode_qkv_o_pays(kbuf, Hq, o_weight.shape[0], start, end))
         tiled = self._streaming(o_weight) if takes else None
         if not isinstance(tiled, self._gemm.TiledWeight):
             return None

@@ -393,3 +393,36 @@ def test_decode_splits_of_column_blocks(b, hq, hkv, q, D):
         assert 1 <= n <= 64 and (n == 1 or (n - 1) * 128 < rows) and (n == 1 or (n - 1) * slices < 512)
         if rows >= 4096 and a * slices <= 512:
             assert n % a == 0 or n < a
+
+
+def test_attention_and_o_projection_in_one_launch_where_it_is_faster():
+    """The rule for the one launch at 256 CUs, both sides of each of its lines, and the split counts that it rests on (the
+    counts of the attention alone beside them): what measured slower goes to the separate launches."""
+    import ksa_amd._lib as _lib
+    L = _lib.lib()
+    if L.ksa_device_cu_count() not in (0, 256):
+        pytest.skip("the figures are those of 256 CUs")
+    for (b, Hq, Hkv, D, N, rows), alone, n, pays in [
+        ((1, 32, 8, 128, 2560, 400), 4, 4, 1),
+        ((1, 32, 8, 128, 2560, 4096), 32, 32, 1),
+        ((1, 32, 8, 128, 2560, 16384), 64, 20, 1),
+        ((1, 32, 8, 128, 2560, 131072), 64, 64, 1),
+        ((8, 32, 8, 128, 2560, 131072), 8, 3, 1),
+        ((16, 32, 8, 128, 4096, 4096), 4, 2, 1),
+        ((1, 32, 1, 128, 2560, 16384), 64, 64, 0),    # too many sums
+        ((1, 32, 1, 128, 2560, 32768), 64, 64, 1),    # ... for a range below this
+        ((8, 32, 2, 128, 2560, 32768), 32, 8, 0),     # few kv heads: too few splits
+        ((16, 32, 1, 128, 2560, 131072), 32, 4, 0),
+        ((2, 16, 4, 128, 2048, 1400), 11, 11, 0),     # 22 sums at 16 heads
+        ((1, 16, 4, 128, 2048, 2500), 20, 20, 1),
+        ((1, 16, 8, 128, 2048, 16384), 64, 20, 0),
+        ((1, 32, 8, 64, 2048, 2500), 20, 20, 1),
+        ((1, 32, 8, 64, 2048, 4096), 32, 32, 0),
+        ((1, 64, 8, 128, 5120, 400), 4, 4, 0),        # 640 workgroups of the product
+        ((1, 32, 32, 128, 4096, 400), 4, 4, 0),
+        ((17, 32, 8, 128, 2560, 400), 1, 1, 0),
+        ((1, 32, 8, 128, 2560, 0), 1, 1, 0),
+    ]:
+        got = (L.ksa_decode_splits(b, Hq, Hkv, 1, D, rows), L.ksa_decode_qkv_o_splits(b, Hq, Hkv, D, rows),
+               L.ksa_decode_qkv_o_pays(b, Hq, Hkv, D, N, rows))
+        assert got == (alone, n, pays), (b, Hq, Hkv, D, N, rows, got)

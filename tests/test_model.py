@@ -449,6 +449,7 @@ def test_one_launch_forms_count_on_the_words_of_their_own_decoder(monkeypatch):
     monkeypatch.setattr(gemm, "add_rmsnorm_linear_rows", lambda *a: (given.append(a[-1]), (None, None))[1])
     monkeypatch.setattr(decode, "ksa_decode_qkv_o", lambda *a, **k: (given.append(a[-1]), "o")[1])
     monkeypatch.setattr(HipOps, "_streaming", lambda self, w, multiple=16: object.__new__(gemm.TiledWeight))
+    monkeypatch.setattr(decode, "decode_qkv_o_pays", lambda *a: True)
     ops = HipOps()
     for H, b, sizes in ((2048, 2, (512, 1024)), (5120, 16, (512,))):
         models = []
