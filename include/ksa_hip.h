@@ -450,6 +450,7 @@ int ksa_add_rmsnorm_mlp_rows(const float* o_partials, int o_ksplit, const void* 
  * ksa_decode_qkv_o_fwd, whose workspace it may share on one stream.  H a multiple of 32 up to 4096, N of 16 (KSA_ERR_UNSUPPORTED
  * otherwise).  ksa_add_rmsnorm_gemm_rows_splits: ceil(H / 512), or 0 for sizes that it does not take. */
 int ksa_add_rmsnorm_gemm_rows_splits(int M, int N, int H);
+int ksa_add_rmsnorm_gemm_rows_pays(int M, int N, int H, int ksplit);  /* 1: faster than the two calls */
 int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, const void* residual, const void* norm_weight,
                               void* out_sum, const void* weight, float* out_partials, int M, int N, int H,
                               long long residual_row_stride, long long sum_row_stride, int dtype, float eps,

@@ -194,6 +194,24 @@ extern "C" int ksa_add_rmsnorm_gemm_rows_splits(int M, int N, int H) {
     return chunks_of(H);
 }
 
+// Whether the one launch is the faster way.  It saves the norm's launch, which takes longer with long rows and many slices, and
+// pays with the hand-over, which takes longer with many rows.  Timed against add_rmsnorm + ksa_gemm_rows at 23 shapes (H 544 to
+// 4096, N 16 to 16384), 4 to 37 slices, 1 to 8 rows, 1610 in all: taken ones 0.86 of the two launches on average, 1.04 at the worst
+// (8 rows of 3072 x 5120, 12 slices).  Outside, by line: short rows of few slices (1024 x 4096, 8 slices, 1 / 8 rows 1.00 / 1.07); more
+// slices than are requested at once, which then come one behind the other (37 slices of 2560 x 6144, 4 / 8 rows 1.00 / 1.07; 24 of 3072 x
+// 5120, 8 rows 1.09, but of 4096 x 6144 0.91); a product wide against its rows (2560 x 16384 1.03 to 1.15, 2048 x 16384, 24 slices 0.98
+// to 1.10); more than 4 rows of few slices (2560 x 12288, 8 rows, 4 slices 1.04), or up to 16 where a few workgroups of the product
+// come in a second round (3840 x 4352, 272 of them, 9 slices 1.03 to 1.09).
+extern "C" int ksa_add_rmsnorm_gemm_rows_pays(int M, int N, int H, int ksplit) {
+    const int cus = ksa_cu_count_or(256);
+    if (ksa_add_rmsnorm_gemm_rows_splits(M, N, H) == 0) return 0;
+    const int wgs = groups_of(N) * chunks_of(H);
+    if (wgs > 3 * cus || N > 5 * H) return 0;
+    if (M <= 4) return ksplit <= 28 && ksplit > (H >= 2048 ? 0 : 16);
+    const bool few_more = wgs > cus && 4 * wgs <= 5 * cus;
+    return ksplit > (H >= 2048 && !few_more ? 8 : 16) && ksplit <= (M <= 6 || H > 3584 ? 24 : 20);
+}
+
 extern "C" int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, const void* residual, const void* norm_weight,
                                          void* out_sum, const void* weight, float* out_partials, int M, int N, int H,
                                          long long residual_row_stride, long long sum_row_stride, int dtype, float eps,
@@ -220,11 +238,12 @@ extern "C" int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, cons
     p.M = M, p.H = H, p.N = N;
     p.chunks = chunks_of(H), p.wgs = groups_of(N) * p.chunks;
     // as few rows to a workgroup of the sums as leave every workgroup a CU of its own (4 / 8 rows of 2560 x 6144: 20 / 40
-    // workgroups next to the 240 of the product 10.7 / 11.7 us, 10 / 15 of them 9.7 / 11.3)
+    // workgroups next to the 240 of the product 10.7 / 11.7 us, 10 / 15 of them 9.7 / 11.3); one where no number does (3584 x 4608, 252 of
+    // the product, 24 slices: 4 rows in one workgroup 14.8 us, one each 12.8)
     const int cus = ksa_cu_count_or(256);
     auto heads = [&](int rows) { return (M + rows - 1) / rows * p.chunks; };
     p.head_rows = 1;
-    while (p.head_rows < 4 && heads(p.head_rows) + p.wgs > cus && heads(4) + p.wgs <= cus + p.chunks) ++p.head_rows;
+    while (p.head_rows < 4 && heads(p.head_rows) + p.wgs > cus && heads(4) + p.wgs <= cus) ++p.head_rows;
     p.heads = heads(p.head_rows);
     p.spin_limit = 1u << 19;  // polls of a microsecond or two: about a second
     const dim3 grid(p.heads + p.wgs), block(kThreads);

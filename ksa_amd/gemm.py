@@ -213,12 +213,10 @@ def add_rmsnorm_linear_rows_supported(M: int, N: int, H: int, device) -> bool:
         return _lib.lib().ksa_add_rmsnorm_gemm_rows_splits(M, N, H) > 0
 
 
-def add_rmsnorm_linear_rows_pays(H: int, ksplit: int) -> bool:
-    """Whether it is the faster way: not for short rows of few slices, whose norm alone takes little.  `add_rmsnorm` +
-    `linear_rows` / one launch, us: H 2560, N 6144, 8 slices, 1 / 8 rows 10.3 / 8.7, 10.9 / 10.4 (19 slices: 11.7 / 8.7, 12.6 /
-    11.3); H 4096, N 2048, 8 slices 8.9 / 7.0, 9.7 / 9.1; H 1024, N 4096, 19 slices 7.4 / 6.4, 8.0 / 7.4, 8 slices 6.3 /
-    6.3, 6.8 / 7.2."""
-    return H >= 2048 or ksplit > 16
+def add_rmsnorm_linear_rows_pays(M: int, N: int, H: int, ksplit: int, device) -> bool:
+    """Whether it is the faster way for partial sums of `ksplit` slices (`ksa_add_rmsnorm_gemm_rows_pays`)."""
+    with _lib.on_device(device):
+        return _lib.lib().ksa_add_rmsnorm_gemm_rows_pays(M, N, H, ksplit) != 0
 
 
 def add_rmsnorm_linear_rows(delta: SplitKPartials, residual: torch.Tensor, norm_weight: torch.Tensor, eps: float,

@@ -260,8 +260,8 @@ class HipOps:
         if not self.mlp_one_launch or not isinstance(delta, self._gemm.SplitKPartials):
             return None
         ws = self._step_ws(delta.rows, residual.shape[-1], mlp_size, residual.device)
-        takes = (ws is not None and self._gemm.add_rmsnorm_linear_rows_pays(weight.shape[1], delta.ksplit)
-                 and self._gemm.add_rmsnorm_linear_rows_supported(delta.rows, *weight.shape, residual.device))
+        takes = ws is not None and self._gemm.add_rmsnorm_linear_rows_pays(delta.rows, *weight.shape, delta.ksplit,
+                                                                           residual.device)
         tiled = self._streaming(weight) if takes else None
         if not isinstance(tiled, self._gemm.TiledWeight):
             return None

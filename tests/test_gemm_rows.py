@@ -308,6 +308,7 @@ def test_gpu_mlp_rows_bounded_wait_gives_up_and_recovers():
     (4096, 1024, 64),   # the longest row, several requests of slices
     (1024, 128, 20),
     (512, 32768 + 16, 21),   # more workgroups than CUs
+    (3584, 4608, 24),   # too few CUs left for the rows: one to a workgroup of the sums
 ])
 def test_gpu_add_rmsnorm_linear_rows_one_launch(dtype, H, N, ksplit):
     """Residual add + norm + product in one launch against the two launches it stands for: the row sums bit for bit, the

@@ -426,3 +426,22 @@ def test_attention_and_o_projection_in_one_launch_where_it_is_faster():
         got = (L.ksa_decode_splits(b, Hq, Hkv, 1, D, rows), L.ksa_decode_qkv_o_splits(b, Hq, Hkv, D, rows),
                L.ksa_decode_qkv_o_pays(b, Hq, Hkv, D, N, rows))
         assert got == (alone, n, pays), (b, Hq, Hkv, D, N, rows, got)
+
+
+def test_norm_and_product_in_one_launch_where_it_is_faster():
+    """The rule for the residual add + norm in front of a product at 256 CUs, both sides of each of its lines."""
+    import ksa_amd._lib as _lib
+    L = _lib.lib()
+    if L.ksa_device_cu_count() not in (0, 256):
+        pytest.skip("the figures are those of 256 CUs")
+    for (M, N, H, ksplit), pays in [
+        ((1, 6144, 2560, 19), 1), ((8, 6144, 2560, 19), 1), ((9, 6144, 2560, 19), 0),
+        ((4, 6144, 2560, 28), 1), ((4, 6144, 2560, 29), 0), ((8, 6144, 2560, 24), 0), ((6, 6144, 2560, 24), 1),
+        ((8, 6144, 4096, 24), 1), ((8, 6144, 4096, 25), 0),
+        ((4, 2560, 2048, 4), 1), ((5, 2560, 2048, 8), 0), ((5, 2560, 2048, 9), 1),
+        ((1, 4096, 1024, 16), 0), ((1, 4096, 1024, 17), 1), ((8, 4096, 1024, 17), 1),
+        ((1, 16384, 2560, 19), 0), ((1, 12288, 4096, 19), 1), ((1, 16384, 4096, 19), 0), ((1, 16384, 1024, 20), 0),
+        ((4, 4352, 3840, 9), 1), ((5, 4352, 3840, 16), 0), ((5, 4352, 3840, 17), 1),
+        ((1, 6144, 2561, 19), 0), ((1, 6144, 4128, 19), 0),
+    ]:
+        assert L.ksa_add_rmsnorm_gemm_rows_pays(M, N, H, ksplit) == pays, (M, N, H, ksplit)
