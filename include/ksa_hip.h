@@ -456,6 +456,12 @@ int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, const void* res
                               long long residual_row_stride, long long sum_row_stride, int dtype, float eps,
                               void* step_workspace, size_t step_workspace_bytes, void* stream);
 
+/* Test aid: the product's workgroups of ksa_add_rmsnorm_gemm_rows alone (contiguous rows).  Nothing that they wait for comes, every wait
+ * runs out after some 200 polls, and the launch ends by its give-up path: status word set, out_partials untouched. */
+int ksa_debug_norm_gemm_rows_give_up(const float* partials, int ksplit, const void* residual, const void* norm_weight,
+                                     void* out_sum, const void* weight, float* out_partials, int M, int N, int H, int dtype,
+                                     float eps, void* step_workspace, size_t step_workspace_bytes, void* stream);
+
 /* Host-side diagnostic: number of key columns in [a, b) visible to query row q under the
  * closed-form rule the kernels use (no GPU involved). */
 long long ksa_debug_count_visible(long long q, long long a, long long b, int C, int S, int W,

@@ -82,6 +82,7 @@ _SIGNATURES = {
     "ksa_add_rmsnorm_gemm_rows_pays": (_int, [_int] * 4),
     "ksa_add_rmsnorm_gemm_rows": (_int, [_vp, _int] + [_vp] * 5 + [_int] * 3 + [ctypes.c_longlong] * 2
                                   + [_int, ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
+    "ksa_debug_norm_gemm_rows_give_up": (_int, [_vp, _int] + [_vp] * 5 + [_int] * 4 + [ctypes.c_float, _vp, ctypes.c_size_t, _vp]),
     "ksa_debug_count_visible": (ctypes.c_longlong, [ctypes.c_longlong] * 3 + [_int] * 7),
 }
 

@@ -212,10 +212,12 @@ extern "C" int ksa_add_rmsnorm_gemm_rows_pays(int M, int N, int H, int ksplit) {
     return ksplit > (H >= 2048 && !few_more ? 8 : 16) && ksplit <= (M <= 6 || H > 3584 ? 24 : 20);
 }
 
-extern "C" int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, const void* residual, const void* norm_weight,
-                                         void* out_sum, const void* weight, float* out_partials, int M, int N, int H,
-                                         long long residual_row_stride, long long sum_row_stride, int dtype, float eps,
-                                         void* step_workspace, size_t step_workspace_bytes, void* stream) {
+namespace {
+// `spin_limit` polls of a microsecond or two at the most; without `sums` nobody leaves what the product waits for
+int norm_gemm_rows(const float* partials, int ksplit, const void* residual, const void* norm_weight, void* out_sum,
+                   const void* weight, float* out_partials, int M, int N, int H, long long residual_row_stride,
+                   long long sum_row_stride, int dtype, float eps, void* step_workspace, size_t step_workspace_bytes,
+                   bool sums, unsigned spin_limit, void* stream) {
     if (!partials || !residual || !norm_weight || !out_sum || !weight || !out_partials || !step_workspace) return KSA_ERR_NULL;
     if (M <= 0 || N <= 0 || H <= 0 || ksplit < 1 || ksplit > 64 || !(eps >= 0.f)) return KSA_ERR_INVALID;
     if (dtype != KSA_DTYPE_BF16 && dtype != KSA_DTYPE_F16) return KSA_ERR_UNSUPPORTED;
@@ -245,11 +247,30 @@ extern "C" int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, cons
     p.head_rows = 1;
     while (p.head_rows < 4 && heads(p.head_rows) + p.wgs > cus && heads(4) + p.wgs <= cus) ++p.head_rows;
     p.heads = heads(p.head_rows);
-    p.spin_limit = 1u << 19;  // polls of a microsecond or two: about a second
+    if (!sums) p.heads = 0;
+    p.spin_limit = spin_limit;
     const dim3 grid(p.heads + p.wgs), block(kThreads);
     if (dtype == KSA_DTYPE_BF16)
         hipLaunchKernelGGL(ksa_norm_gemm_rows_kernel<KsaBf16>, grid, block, 0, (hipStream_t)stream, p);
     else
         hipLaunchKernelGGL(ksa_norm_gemm_rows_kernel<KsaF16>, grid, block, 0, (hipStream_t)stream, p);
     return ksa_check_launch();
+}
+}  // namespace
+
+extern "C" int ksa_add_rmsnorm_gemm_rows(const float* partials, int ksplit, const void* residual, const void* norm_weight,
+                                         void* out_sum, const void* weight, float* out_partials, int M, int N, int H,
+                                         long long residual_row_stride, long long sum_row_stride, int dtype, float eps,
+                                         void* step_workspace, size_t step_workspace_bytes, void* stream) {
+    return norm_gemm_rows(partials, ksplit, residual, norm_weight, out_sum, weight, out_partials, M, N, H,
+                          residual_row_stride, sum_row_stride, dtype, eps, step_workspace, step_workspace_bytes, true,
+                          1u << 19, stream);  // (about a second)
+}
+
+extern "C" int ksa_debug_norm_gemm_rows_give_up(const float* partials, int ksplit, const void* residual,
+                                                const void* norm_weight, void* out_sum, const void* weight,
+                                                float* out_partials, int M, int N, int H, int dtype, float eps,
+                                                void* step_workspace, size_t step_workspace_bytes, void* stream) {
+    return norm_gemm_rows(partials, ksplit, residual, norm_weight, out_sum, weight, out_partials, M, N, H, H, H, dtype, eps,
+                          step_workspace, step_workspace_bytes, false, 200, stream);
 }

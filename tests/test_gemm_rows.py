@@ -345,8 +345,10 @@ def test_gpu_add_rmsnorm_linear_rows_one_launch(dtype, H, N, ksplit):
 
 @pytest.mark.gpu
 def test_gpu_add_rmsnorm_linear_rows_bounded_wait_gives_up_and_recovers():
-    """The give-up path of the wait for the other chunks' sums, forced from the host: the status word is set, which every
-    workgroup that waits looks at; whether one of them had to wait or not, `failed()` reports it and zeroes the words."""
+    """The give-up path of the wait for the other chunks' sums: a launch whose workgroups of the sums stay out, so that every
+    wait runs out after a few polls.  The kernel sets the status word, no workgroup stores anything, `failed()` reports it
+    and zeroes the words, and the next launch equals one on a fresh workspace."""
+    from ksa_amd import _lib
     from ksa_amd.gemm import MlpRowsWorkspace, SplitKPartials, TiledWeight, add_rmsnorm_linear_rows
     dev = torch.device("cuda")
     g = torch.Generator(device="cuda").manual_seed(3)
@@ -356,9 +358,13 @@ def test_gpu_add_rmsnorm_linear_rows_bounded_wait_gives_up_and_recovers():
     delta = SplitKPartials(rnd(2, 16, H).view(-1).view(torch.uint8), 2, M, (1, M, H), torch.bfloat16)
     res, one = rnd(1, M, H).bfloat16(), torch.ones(H, device="cuda").bfloat16()
     call = lambda w: add_rmsnorm_linear_rows(delta, res, one, 1e-6, tiled, w)[1].workspace.view(torch.float32).view(2, 16, N)[:, :M]
-    ws._step_status.fill_(1)
+    out, part = torch.full((M, H), 3.0, device="cuda").bfloat16(), torch.full((2, 16, N), 3.0, device="cuda")
+    assert int(ws._step_status.item()) == 0
+    rc = _lib.lib().ksa_debug_norm_gemm_rows_give_up(
+        delta.workspace.data_ptr(), 2, res.data_ptr(), one.data_ptr(), out.data_ptr(), tiled.data_ptr(), part.data_ptr(), M, N, H,
+        0, 1e-6, ws.step.data_ptr(), ws.step.numel(), _lib.stream_ptr(dev))
     torch.cuda.synchronize()
-    call(ws)
+    assert rc == 0 and int(ws._step_status.item()) == 1 and bool((out == 3).all()) and bool((part == 3).all())
     assert ws.failed() and not ws.failed()
     assert int(ws.step.view(torch.int64).abs().sum().item()) == 0
     a, b = call(ws), call(MlpRowsWorkspace(H, 64, dev))
