@@ -277,14 +277,15 @@ def test_prefill_cfg1_sampled_rows(wave_rows):
     assert np.abs(lse[:, rows] - wlse).max() <= 2e-3
 
 
-def test_prefill_cfg2_sampled_rows():
+@pytest.mark.parametrize("chunk_tiles", [True, False])
+def test_prefill_cfg2_sampled_rows(chunk_tiles):
     """cfg 2 (128k text tokens, 1024 chunks, 32/8 heads), the benchmark's shape: every row of the
     first and last two chunks, offsets {0, C-1, C, B-1} of 32 random chunks and 256 random rows
-    against the oracle."""
+    against the oracle; on chunk tiles, and on the grid of the block index, whose longest walks these are."""
     Sq, Hq, Hkv, D, C, S, W = 139264, 32, 8, 128, 128, 8, 4
     q, k, v = make_qkv(Sq, Hq, Hkv, D, seed=0)
     sp = O.summary_positions(Sq, C, S)
-    got, lse = _run_prefill(q, k, v, C, S, W, sp)
+    got, lse = _run_prefill(q, k, v, C, S, W, sp, chunk_tiles=chunk_tiles)
     rng = np.random.default_rng(2)
     B = C + S
     rows = set(range(0, 2 * B)) | set(range(Sq - 2 * B, Sq))
@@ -297,10 +298,11 @@ def test_prefill_cfg2_sampled_rows():
     assert np.abs(lse[:, rows] - wlse).max() <= 2e-3
 
 
-def test_prefill_dense_causal_layer_batch8_sampled_rows():
+@pytest.mark.parametrize("chunk_tiles", [True, False])
+def test_prefill_dense_causal_layer_batch8_sampled_rows(chunk_tiles):
     """The launch an unbounded-window ("full attention") layer of the end-to-end prefill makes: batch 8,
     34816 expanded rows (32k text), 32 / 8 heads, window larger than the sequence, so every text row
-    sees all earlier text and no summary, and 97 % of the listed tiles are masked ones.  Sequences 0, 3
+    sees all earlier text and no summary, and 97 % of the tiles that the block index lists are masked ones.  Sequences 0, 3
     and 7 of the batch (different data each) against the oracle on the first and last chunk's rows,
     chunk-edge offsets of 16 random chunks and 256 random rows."""
     import ksa_amd
@@ -310,7 +312,8 @@ def test_prefill_dense_causal_layer_batch8_sampled_rows():
     sp = O.summary_positions(Sq, C, S)
     qkv = [make_qkv(Sq, Hq, Hkv, D, seed=50 + b) for b in range(bsz)]
     q, k, v = (torch.stack([t[i] for t in qkv]).to(dev) for i in range(3))
-    out, _ = ksa_amd.summary_attn_func(q, k, v, C, S, W, summary_pos=torch.as_tensor(sp, device=dev))
+    out, _ = ksa_amd.summary_attn_func(q, k, v, C, S, W, summary_pos=torch.as_tensor(sp, device=dev),
+                                       chunk_tiles=chunk_tiles)
     rng = np.random.default_rng(5)
     rows = set(range(0, B)) | set(range(Sq - B, Sq))
     for c in rng.choice(Sq // B, 16, replace=False):
@@ -323,7 +326,8 @@ def test_prefill_dense_causal_layer_batch8_sampled_rows():
         _compare(to_np(out[b])[rows], want, f"dense causal, sequence {b}")
 
 
-def test_prefill_work_queues_equal_fixed_split():
+@pytest.mark.parametrize("chunk_tiles", [True, False])
+def test_prefill_work_queues_equal_fixed_split(chunk_tiles):
     """A long launch (32 workgroups per CU and more) hands out its last work items from per-XCD
     queues; a short one gives workgroup i item i.  Three copies of a 32k-row sequence in one batch
     take the first path, one copy the second: every copy must equal it bit for bit (an item
@@ -336,17 +340,18 @@ def test_prefill_work_queues_equal_fixed_split():
     q, k, v = make_qkv(Sq, Hq, Hkv, D, seed=21)
     sp = torch.as_tensor(O.summary_positions(Sq, C, S), device=dev)
     q1, k1, v1 = q[None].to(dev), k[None].to(dev), v[None].to(dev)
-    one, _ = ksa_amd.summary_attn_func(q1, k1, v1, C, S, W, summary_pos=sp)
+    one, _ = ksa_amd.summary_attn_func(q1, k1, v1, C, S, W, summary_pos=sp, chunk_tiles=chunk_tiles)
     assert Sq // 128 * (Hq // 2) < 32 * _lib.lib().ksa_device_cu_count() <= 3 * (Sq // 128) * (Hq // 2)
     q3, k3, v3 = (t.expand(3, -1, -1, -1).contiguous() for t in (q1, k1, v1))
     for _ in range(2):
-        three, _ = ksa_amd.summary_attn_func(q3, k3, v3, C, S, W, summary_pos=sp)
+        three, _ = ksa_amd.summary_attn_func(q3, k3, v3, C, S, W, summary_pos=sp, chunk_tiles=chunk_tiles)
         torch.cuda.synchronize()
         for b in range(3):
             assert torch.equal(three[b], one[0]), b
 
 
-def test_prefill_cfg2_visibility_probe_all_rows():
+@pytest.mark.parametrize("chunk_tiles", [True, False])
+def test_prefill_cfg2_visibility_probe_all_rows(chunk_tiles):
     """Every row of the 128k shape: with Q = K = 0 and V = one-hot of (position mod 128) the
     output is count-of-class / n_i over the row's visible set.  All probabilities are exactly 1,
     so the only error is the final rounding to bf16 and one wrongly (un)masked key moves a value
@@ -372,7 +377,7 @@ def test_prefill_cfg2_visibility_probe_all_rows():
     k = torch.zeros(Sq, Hkv, D, dtype=torch.bfloat16)
     v = torch.zeros(Sq, Hkv, D, dtype=torch.bfloat16)
     v[torch.arange(Sq), 0, torch.from_numpy(cls)] = 1.0
-    got, lse = _run_prefill(q, k, v, C, S, W, O.summary_positions(Sq, C, S))
+    got, lse = _run_prefill(q, k, v, C, S, W, O.summary_positions(Sq, C, S), chunk_tiles=chunk_tiles)
     for h in range(Hq):
         err = np.abs(got[:, h] - want)
         assert (err <= want * 2.0 ** -8 + 1e-7).all(), (h, float(err.max()))
@@ -612,7 +617,8 @@ def test_prefill_marked_tiles(Sq, D, shape):
     for W in (0, 2, 1000):
         for spt in (torch.as_tensor(sp, device=dev), None):
             out, lse = ksa_amd.summary_attn_func(q[None].to(dev), k[None].to(dev), v[None].to(dev), C, S, W,
-                                                 summary_pos=spt, return_lse=True, workgroup_shape=shape)
+                                                 summary_pos=spt, return_lse=True, workgroup_shape=shape,
+                                                 chunk_tiles=False)
             want, wlse = c_oracle.attention_rows(to_np(q), to_np(k), to_np(v), C, S, W,
                                                  summary_pos=None if spt is None else sp)
             got = to_np(out[0])
@@ -652,7 +658,7 @@ def test_prefill_marked_tiles_of_long_lists(D, shape, mode, C):
             kk, vv, spt = torch.cat([k[st], k]), torch.cat([v[st], v]), None
         for W in (4, 1 << 20):
             out, lse = ksa_amd.summary_attn_func(q[None].to(dev), kk[None].to(dev), vv[None].to(dev), C, S, W, summary_pos=spt,
-                                                 return_lse=True, workgroup_shape=shape)
+                                                 return_lse=True, workgroup_shape=shape, chunk_tiles=False)
             got, glse = to_np(out[0]), to_np(lse[0])
             want, wlse = c_oracle.attention_rows(to_np(q), to_np(k), to_np(v), C, S, W, summary_pos=osp, rows=rows)
             assert np.isfinite(got).all() and np.isfinite(glse).all(), (peaked, W)
@@ -681,7 +687,8 @@ def test_chunk_longer_than_any_sequence(C):
 
 @pytest.mark.parametrize("D, dtype, heads", [(128, torch.bfloat16, (4, 2)), (128, torch.float16, (3, 1)), (64, torch.bfloat16, (8, 1)),
                                              (256, torch.bfloat16, (2, 2)), (256, torch.float16, (2, 1))])
-@pytest.mark.parametrize("C, S, W", [(128, 8, 4), (128, 8, 0), (128, 4, 1), (256, 2, 1), (512, 1, 0), (128, 8, 1 << 20), (384, 8, 2)])
+@pytest.mark.parametrize("C, S, W", [(128, 8, 4), (128, 8, 0), (128, 4, 1), (256, 2, 1), (512, 1, 0), (128, 8, 1 << 20), (384, 8, 2),
+                                     (128, 16, 4), (256, 16, 0)])
 def test_prefill_chunk_tiles(C, S, W, D, dtype, heads):
     """Tiles laid along the chunks: one row tile with one and with two key tiles on the diagonal, lengths that cut
     either, chunk counts around the prefix of one load, of one tile and of a tile and a half, every column block of the
@@ -689,6 +696,9 @@ def test_prefill_chunk_tiles(C, S, W, D, dtype, heads):
     on the block index.  Against the oracle: 16-bit probabilities, as everywhere in this file."""
     import ksa_amd
     from ksa_amd import prefill
+    if S == 16 and D == 256:   # (a load has 8 rows there)
+        assert not prefill._chunk_tiles(C + S, D, C, S, S, False)
+        return
     dev = torch.device("cuda")
     B = C + S
     for n in (64, 65, 127, C, B + 1, B + C // 2, (W + 2) * B, (W + 9) * B + 64, (W + 13) * B + 65):
@@ -712,13 +722,16 @@ def test_prefill_chunk_tiles(C, S, W, D, dtype, heads):
 
 
 @pytest.mark.parametrize("shape", [2, 32])
-def test_prefill_chunk_tiles_of_both_workgroup_shapes(shape):
+@pytest.mark.parametrize("C, S, W", [(128, 8, 3), (128, 16, 2), (256, 16, 1), (384, 2, 1), (512, 4, 0)])
+def test_prefill_chunk_tiles_of_both_workgroup_shapes(shape, C, S, W):
     """The two workgroup shapes of the chunk tiles through the C entry point: a strided batch of three, all rows against
-    the same rows on the block index; the walk with exact references (summary keys of a huge norm) included."""
+    the same rows on the block index; the walk with exact references (summary keys of a huge norm) included.  One to four row
+    tiles per chunk, prefixes of fewer rows than a load of either shape, than a tile, of whole tiles and between."""
     import ksa_amd
     from ksa_amd import _lib
     dev = torch.device("cuda")
-    C, S, W, Hq, Hkv, D, n = 128, 8, 3, 8, 2, 128, 21 * 136 + 77
+    Hq, Hkv, D = 8, 2, 128
+    n = 2870 // (C + S) * (C + S) + 77
     g = torch.Generator(device=dev).manual_seed(5)
     qkv = torch.randn(3, n, Hq + 2 * Hkv, D, generator=g, device=dev).bfloat16()
     q, k, v = qkv[:, :, :Hq], qkv[:, :, Hq:Hq + Hkv], qkv[:, :, Hq + Hkv:]
