@@ -1053,18 +1053,24 @@ extern "C" int ksa_decode_qkv_o_splits(int batch, int Hq, int Hkv, int D, int ma
 
 // Whether the one launch is the faster way.  Its gain is two ramps and a trip of the rows, 1 to 3 us, and the time of o's
 // weights where they are many; its price the merge of batch * n sums in every workgroup of the product, fewer splits, and the
-// attention's places on the CUs that the product holds.  Measured over 1675 shapes (1 to 16 sequences of 400 to 131072 rows, 8 to
-// 64 heads of 128 and 64, 1 to 32 kv heads, N 1024 to 5120): 326 are taken, at 0.92 of the separate launches on average and 1.02 at the
-// worst.  Outside: 16 sequences with 1 kv head, 64 sums, 4 splits where the attention alone has 32: 400 / 131072 rows 1.05 / 1.92;
-// 2 kv heads, 8 sequences 1.01 to 1.12; head_dim 64 from 4096 rows on 1.05 to 1.6 (a split is half the work and as many trips);
-// 16 heads (16 KB of a column's weights instead of 32) with more than 20 sums up to 1.13; 64 heads, N 5120, 640 workgroups of
-// the product 1.00 to 1.14; 32 kv heads up to 1.08.  Some of the shapes left out gain, e.g. 32 / 4 heads, 16 sequences 0.94 to 0.98.
+// attention's places on the CUs that the product holds.  By a sweep over 1675 shapes (1 to 16 sequences of 400 to 131072 rows, 8 to
+// 64 heads of 128 and 64, 1 to 32 kv heads, N 1024 to 5120) three kinds are taken, 461 of
+// them, at 0.94 of the separate launches on average and 1.02 at the worst; one launch / separate ones at the lines' other sides:
+//   as many splits as the attention alone takes, but few sums: 16 / 4 heads, 2 x 1400 rows (22 sums) 0.94, 4 x 1400 (40) 1.06, 8 x 700 (40)
+//     1.13; one split, where there is no merge to save, at head_dim 64 1.00 to 1.07
+//   32 heads of 128 and more: 32 / 2 heads, 8 sequences (64 sums) 1.01 to 1.12, 32 / 1, 16 (64 sums, 4 splits instead of 32) 1.05 to 1.92;
+//     16 / 8 heads, 1 or 2 x 8192 1.04; head_dim 64 from 4096 rows on 1.05 to 1.65 (a split is half the work and as many trips)
+//   many workgroups of the attention: 24 / 8 heads, 8 x 400 rows 1.02, 4 x 4096 1.03; 16 / 8, 8 x 5000 1.03 to 1.05
+// and none with far more workgroups of the product than CUs (64 heads, N 5120, 640 of them, 1.00 to 1.14) or more than 8 kv heads
+// (32 / 32 0.89 to 1.12).
 extern "C" int ksa_decode_qkv_o_pays(int batch, int Hq, int Hkv, int D, int N, int max_rows) {
     if (batch <= 0 || batch > 16 || Hkv <= 0 || Hkv > 8 || Hq % Hkv != 0 || N <= 0 || max_rows <= 0) return 0;
-    if ((N + 127) / 128 * (int64_t)(Hq * D / kChunkK) > ksa_cu_count_or(256)) return 0;
-    const int n = ksa_decode_qkv_o_splits(batch, Hq, Hkv, D, max_rows);
-    if (n > 1 && batch * n <= 20 && n == ksa_decode_splits(batch, Hq, Hkv, 1, D, max_rows)) return 1;
-    return D == 128 && Hq * D >= 4096 && (batch * n <= 32 || (batch == 1 && max_rows >= 32768));
+    const int64_t product = (N + 127) / 128 * (int64_t)(Hq * D / kChunkK), cus = ksa_cu_count_or(256);
+    const int n = ksa_decode_qkv_o_splits(batch, Hq, Hkv, D, max_rows), sums = batch * n;
+    if (product <= cus && n > 1 && sums <= 20 && n == ksa_decode_splits(batch, Hq, Hkv, 1, D, max_rows)) return 1;
+    if (D != 128) return 0;
+    if (product <= cus && Hq * D >= 4096 && (sums <= 32 || (batch == 1 && max_rows >= 32768))) return 1;
+    return product <= 2 * cus && batch * Hkv >= (Hq >= 24 ? 64 : 96) && max_rows >= 1400 && sums <= 32;
 }
 
 extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,

@@ -196,20 +196,19 @@ extern "C" int ksa_add_rmsnorm_gemm_rows_splits(int M, int N, int H) {
 
 // Whether the one launch is the faster way.  It saves the norm's launch, which takes longer with long rows and many slices, and
 // pays with the hand-over, which takes longer with many rows.  Timed against add_rmsnorm + ksa_gemm_rows at 23 shapes (H 544 to
-// 4096, N 16 to 16384), 4 to 37 slices, 1 to 8 rows, 1610 in all: taken ones 0.86 of the two launches on average, 1.04 at the worst
-// (8 rows of 3072 x 5120, 12 slices).  Outside, by line: short rows of few slices (1024 x 4096, 8 slices, 1 / 8 rows 1.00 / 1.07); more
-// slices than are requested at once, which then come one behind the other (37 slices of 2560 x 6144, 4 / 8 rows 1.00 / 1.07; 24 of 3072 x
-// 5120, 8 rows 1.09, but of 4096 x 6144 0.91); a product wide against its rows (2560 x 16384 1.03 to 1.15, 2048 x 16384, 24 slices 0.98
-// to 1.10); more than 4 rows of few slices (2560 x 12288, 8 rows, 4 slices 1.04), or up to 16 where a few workgroups of the product
-// come in a second round (3840 x 4352, 272 of them, 9 slices 1.03 to 1.09).
+// 4096, N 16 to 16384), 4 to 37 slices, 1 to 8 rows, 1610 in all: 1018 are taken, at 0.87 of the two launches on average, 1.04 at
+// the worst (8 rows of 3072 x 5120, 12 slices).  Outside, by line: short rows of few slices (1024 x 4096, 8 slices, 1 / 8 rows 1.00 / 1.07); more slices than are requested at once, which then come one behind the other (37 slices of 2560 x
+// 6144, 4 / 8 rows 1.00 / 1.07; 24 of 3072 x 5120, 8 rows 1.09, but of 4096 x 6144 0.91); a product wide against its rows (2560 x 16384
+// 1.03 to 1.15, 2048 x 16384, 24 slices 0.98 to 1.10); more than 4 rows of few slices (2560 x 12288, 8 rows, 4 slices 1.04), or up to 16
+// where a few workgroups of the product come in a second round (3840 x 4352, 272 of them, 9 slices 1.03 to 1.09).
 extern "C" int ksa_add_rmsnorm_gemm_rows_pays(int M, int N, int H, int ksplit) {
     const int cus = ksa_cu_count_or(256);
     if (ksa_add_rmsnorm_gemm_rows_splits(M, N, H) == 0) return 0;
     const int wgs = groups_of(N) * chunks_of(H);
-    if (wgs > 3 * cus || N > 5 * H) return 0;
-    if (M <= 4) return ksplit <= 28 && ksplit > (H >= 2048 ? 0 : 16);
+    if (wgs > 3 * cus || N > 6 * H || ksplit > (M <= 6 || H > 3584 ? 28 : 20)) return 0;
+    if (M <= 4) return ksplit > (H >= 2048 ? 0 : 16);
     const bool few_more = wgs > cus && 4 * wgs <= 5 * cus;
-    return ksplit > (H >= 2048 && !few_more ? 8 : 16) && ksplit <= (M <= 6 || H > 3584 ? 24 : 20);
+    return ksplit > (H >= 2048 && !few_more ? 8 : 16);
 }
 
 namespace {

@@ -198,8 +198,10 @@ __device__ __forceinline__ RowVis ksa_row_vis(const KsaMask& mk, const FastDiv& 
 //     Tiles per row tile at C = 128, S = 8, W = 4: 73.9 instead of 75.7 at 128k tokens, 25.8 instead of 27.7 at 32k, and 6 % fewer row tiles.
 //     Measured, grid / chunks, us: 32 / 8 heads in bf16, W = 4, 300 tokens 15.0 / 12.7, 32k 896 / 795, 128k 8903 / 8123; 16 / 8
 //     heads, 4k 36.6 / 33.1; unbounded window, 3 x 9001 tokens in fp16 2119 / 1765; head_dim 64, 2 x 11013 tokens 309 / 232; head_dim
-//     256, 8 x 2608 tokens 787 / 625.  Of 140 shapes drawn over batch, heads, window and length none is slower (the least
-//     gain, 1 %: 8 x 10234 tokens, 8 / 8 heads, W = 1, where K/V are read once for the summary rows and once for the text).
+//     256, 8 x 2608 tokens 787 / 625.  Of 140 shapes drawn over batch, heads, head_dim, window and length none is
+//     slower: 0.54 to 0.96 of the grid's time (the least gain met, 1 %: 8 x 10234 tokens, 8 / 8 heads, W = 1, where K/V are read once
+//     for the summary rows and once for the text).  The probabilities are rounded against another first tile than on the grid: over 60 shapes
+//     the output lies 0.97 to 1.01 times as far from 64 bits as there (summary rows 0.9 times).
 enum { kAddrGeneral = 0, kAddrRegular = 1, kAddrMarked = 2, kAddrChunks = 3 };
 
 // RB: 32-row query blocks per wave.  RB = 1: one query head per workgroup, wave w owns rows

@@ -177,10 +177,13 @@ class HipOps:
             hit = self._tiled[key] = (weight, self._gemm.TiledWeight(weight))
         return hit[1]
 
-    # Up to this many rows a prompt's attention stays on the grid of the block index.  Chunk tiles round a prompt's logits
-    # differently by about a unit in their last place, which can tip the greedy token where the two best logits lie that
-    # close (5 of 108 prompts of random weights), and win next to nothing in a short prefill: 4 layers of the 4B shape, grid /
-    # chunk tiles, 300 / 1000 / 4096 / 16384 tokens 1.62 / 1.62, 1.95 / 1.95, 4.36 / 4.31, 16.8 / 16.4 ms.
+    # Up to this many rows a prompt's attention stays on the grid of the block index, and its logits what they are there bit for
+    # bit: chunk tiles round them differently by about a unit in their last place, which can tip the greedy token where the two
+    # best logits lie that close (5 of 108 prompts of random weights).  Neither form is the more accurate one - distance of the
+    # logits from fp32 behind 4 layers, 15 prompts of 150 to 1500 tokens, 1.720 % on the grid and 1.725 % on chunk tiles, of keys and
+    # values 1.517 and 1.515 % - so this is a choice for unchanged results where they cost little, not a line that the kernels draw:
+    # 4 layers of the 4B shape, grid / chunk tiles, 300 / 1000 / 2 x 3000 / 4096 / 8192 / 16384 tokens 1.65 / 1.64, 2.00 / 1.98, 5.87 /
+    # 5.77, 4.51 / 4.46, 8.22 / 8.07, 17.0 / 16.5 ms.
     GRID_ROWS = 4608
 
     def summary_attn_func(self, q, k, v, *args, **kwargs):

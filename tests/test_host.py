@@ -420,6 +420,14 @@ def test_attention_and_o_projection_in_one_launch_where_it_is_faster():
         ((1, 32, 8, 64, 2048, 4096), 32, 32, 0),
         ((1, 64, 8, 128, 5120, 400), 4, 4, 0),        # 640 workgroups of the product
         ((1, 32, 32, 128, 4096, 400), 4, 4, 0),
+        ((8, 24, 8, 128, 3072, 1300), 8, 3, 0),
+        ((8, 24, 8, 128, 3072, 1400), 8, 3, 1),       # 64 workgroups to a split
+        ((4, 24, 8, 128, 3072, 4096), 16, 5, 0),
+        ((8, 48, 8, 128, 4096, 4096), 8, 3, 1),
+        ((8, 16, 8, 128, 2048, 4096), 8, 3, 0),
+        ((12, 16, 8, 128, 2048, 4096), 5, 2, 1),
+        ((8, 64, 8, 128, 5120, 4096), 8, 3, 0),
+        ((16, 32, 4, 128, 2560, 4096), 8, 3, 0),      # 48 sums
         ((17, 32, 8, 128, 2560, 400), 1, 1, 0),
         ((1, 32, 8, 128, 2560, 0), 1, 1, 0),
     ]:
@@ -436,11 +444,11 @@ def test_norm_and_product_in_one_launch_where_it_is_faster():
         pytest.skip("the figures are those of 256 CUs")
     for (M, N, H, ksplit), pays in [
         ((1, 6144, 2560, 19), 1), ((8, 6144, 2560, 19), 1), ((9, 6144, 2560, 19), 0),
-        ((4, 6144, 2560, 28), 1), ((4, 6144, 2560, 29), 0), ((8, 6144, 2560, 24), 0), ((6, 6144, 2560, 24), 1),
-        ((8, 6144, 4096, 24), 1), ((8, 6144, 4096, 25), 0),
+        ((6, 6144, 2560, 28), 1), ((4, 6144, 2560, 29), 0), ((7, 6144, 2560, 20), 1), ((7, 6144, 2560, 21), 0),
+        ((8, 6144, 4096, 28), 1), ((8, 6144, 4096, 29), 0),
         ((4, 2560, 2048, 4), 1), ((5, 2560, 2048, 8), 0), ((5, 2560, 2048, 9), 1),
         ((1, 4096, 1024, 16), 0), ((1, 4096, 1024, 17), 1), ((8, 4096, 1024, 17), 1),
-        ((1, 16384, 2560, 19), 0), ((1, 12288, 4096, 19), 1), ((1, 16384, 4096, 19), 0), ((1, 16384, 1024, 20), 0),
+        ((1, 16384, 2560, 19), 0), ((1, 12288, 4096, 19), 1), ((1, 16384, 4096, 19), 0), ((1, 16384, 1024, 20), 0), ((1, 12288, 2048, 19), 1), ((1, 12416, 2048, 19), 0),
         ((4, 4352, 3840, 9), 1), ((5, 4352, 3840, 16), 0), ((5, 4352, 3840, 17), 1),
         ((1, 6144, 2561, 19), 0), ((1, 6144, 4128, 19), 0),
     ]:
