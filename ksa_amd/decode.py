@@ -92,7 +92,9 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
         e0 = rows if end is None else int(end)
         assert 0 <= s0 < e0 <= rows, "row range out of bounds"
         max_rows = e0 - s0
-    q, scale = fold_scale(q, float(D) ** -0.5 if scale is None else float(scale))
+    scale = float(D) ** -0.5 if scale is None else float(scale)
+    if scale <= 0:
+        q, scale = fold_scale(q, scale)
     if nsplit is None:
         nsplit = _lib.lib().ksa_decode_splits(b, q.shape[1], kcache.shape[1], q.shape[2], D, max_rows)
     Dk = kernel_head_dim(D)
@@ -146,8 +148,10 @@ def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, 
     assert kcache.stride(-1) == 1 and vcache.stride(-1) == 1, "cache rows must be contiguous"
     dt = qkv.dtype
     cos, sin = (t.to(dt).reshape(-1, D).contiguous() for t in (cos, sin))
-    qw, scale = fold_scale(q_norm_weight.to(dt).contiguous(), float(D) ** -0.5 if scale is None else float(scale))
-    kw = k_norm_weight.to(dt).contiguous()
+    qw, kw = q_norm_weight.to(dt).contiguous(), k_norm_weight.to(dt).contiguous()
+    scale = float(D) ** -0.5 if scale is None else float(scale)
+    if scale <= 0:
+        qw, scale = fold_scale(qw, scale)
     assert cos.shape == sin.shape and cos.shape[0] in (1, b) and qw.shape == (D,) and kw.shape == (D,)
     t_row = t_start = t_end = None
     s0, e0, r0 = 0, 1, 0
@@ -273,7 +277,9 @@ def ksa_decode_boundary(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Ten
         return None, None, int(lo), int(hi)
     ts, te, ts0, te0 = pair(text_start, text_end)
     ss, se, ss0, se0 = pair(sum_start, sum_end)
-    q, scale = fold_scale(q, float(D) ** -0.5 if scale is None else float(scale))
+    scale = float(D) ** -0.5 if scale is None else float(scale)
+    if scale <= 0:
+        q, scale = fold_scale(q, scale)
     lib = _lib.lib()
     if nsplit is None:   # (the count by the slices: ksa_decode_splits is for one range, not for two of different lengths)
         nsplit = lib.ksa_decode_auto_splits(b, Hkv, rows if ts is not None else te0 - ts0)

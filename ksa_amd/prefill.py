@@ -173,11 +173,9 @@ def pad_head_dim(t: torch.Tensor, Dk: int) -> torch.Tensor:
 
 
 def fold_scale(q: torch.Tensor, scale: float):
-    """(q', scale') with q' scale' = q scale, exactly, and scale' positive: the kernels hide a key by a score of -inf in
-    front of the factor, which a negative one would turn into +inf and zero into NaN."""
-    if scale < 0:
-        return -q, -scale
-    return (torch.zeros_like(q), 1.0) if scale == 0 else (q, scale)
+    """For a scale that is not positive: (q', scale') with q' scale' = q scale, exactly, and scale' positive.  The kernels
+    hide a key by a score of -inf in front of the factor, which a negative one would turn into +inf and zero into NaN."""
+    return (-q, -scale) if scale < 0 else (torch.zeros_like(q), 1.0)
 
 
 _CHUNK_MAX = 512   # the largest chunk that takes tiles laid along the chunks (ksa_prefill_chunks_fwd)
@@ -192,21 +190,14 @@ def _chunk_tiles(Sq: int, D: int, C: int, S: int, P: int, phys: bool) -> bool:
             and TILE_N <= Sq < 1 << 29 and Sq % block <= C and P in (0, Sq // block * S))
 
 
-def _outputs(q, want_lse):
-    b, Sq, Hq, _ = q.shape
+def _launch_chunks(q, k, v, C, S, W, skip_old, scale, want_lse):
+    b, Sq, Hq, D = q.shape
     dev = q.device
     out = torch.empty_like(q)
     lse = torch.empty((b, Hq, Sq), dtype=torch.float32, device=dev) if want_lse else None
     # work queues of this call alone, for a launch long enough to use them (the library's own bound is 32
     # workgroups per CU; a workgroup takes 128 rows of one or two heads)
     sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= 1 << 19 else None
-    return out, lse, sched
-
-
-def _launch_chunks(q, k, v, C, S, W, skip_old, scale, want_lse):
-    b, Sq, Hq, D = q.shape
-    dev = q.device
-    out, lse, sched = _outputs(q, want_lse)
     dims = (0, 1, 2)
     with _lib.on_device(dev):
         rc = _lib.lib().ksa_prefill_chunks_fwd(
@@ -223,7 +214,9 @@ def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P,
                     shape):
     b, Sq, Hq, D = q.shape
     dev = q.device
-    out, lse, sched = _outputs(q, want_lse)
+    out = torch.empty_like(q)
+    lse = torch.empty((b, Hq, Sq), dtype=torch.float32, device=dev) if want_lse else None
+    sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= 1 << 19 else None  # as in _launch_chunks
     dims = (0, 1, 2)
     with _lib.on_device(dev):
         rc = _lib.lib().ksa_prefill_fwd(
@@ -327,7 +320,9 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     if k.stride() != v.stride():
         v = v.contiguous()
         k = k.contiguous()
-    q, scale = fold_scale(q, float(D) ** -0.5 if softmax_scale is None else float(softmax_scale))
+    scale = float(D) ** -0.5 if softmax_scale is None else float(softmax_scale)
+    if scale <= 0:
+        q, scale = fold_scale(q, scale)
     Dk = kernel_head_dim(D)
     if Dk != D:   # a head dimension without a kernel of its own: zero-padded copies (see kernel_head_dim)
         q, k, v = pad_head_dim(q, Dk), pad_head_dim(k, Dk), pad_head_dim(v, Dk)
