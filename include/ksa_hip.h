@@ -243,6 +243,24 @@ int ksa_copy_rows_multi(int n_moves, const void* const* src, void* const* dst,
                         const int* nrows, int batch, int heads, int D, const int64_t* src_strides,
                         const int64_t* dst_strides, void* stream);
 
+/* ksa_copy_rows_multi with source rows by a closed form: dst[m] row (dst_start[m] + i) <- src[m] row
+ * (offset[m] + (first[m] + i) / run[m] * period + (first[m] + i) % run[m]), i < nrows[m].  With period = C + S and
+ * run = C or (offset C) run = S these are the text and the summary rows of a prompt with its summary tokens in line:
+ * HF:209-302 (reorganize_after_prefill) as one launch per layer. */
+int ksa_copy_rows_runs(int n_moves, const void* const* src, void* const* dst, const int* offset, const int* first,
+                       const int* run, int period, const int* dst_start, const int* nrows, int batch, int heads, int D,
+                       const int64_t* src_strides, const int64_t* dst_strides, void* stream);
+
+/* Head of a prefill.  Replaces HF:1080-1177 (_expand_input_with_summary_tokens) and HF:1018-1032
+ * (Qwen3RotaryEmbedding.forward) for ids int64 [batch, n] (rows ids_row_stride apart), L = n + n / C * S:
+ *   out_ids int64 [batch, L]: the ids with summary_begin .. summary_begin + S - 1 behind every whole chunk
+ *   is_summary uint8 [L], cos / sin 16-bit [L, D] (16-byte aligned; D a multiple of 16)
+ * of position (float) times inv_freq [D / 2], fp32.  inner_chunk: text positions start again at every chunk;
+ * summary_kind 0 / 1 / 2: position ids "zeros" / "last_chunk_slice_left" / "last_chunk_slice_right". */
+int ksa_expand_prompt(const long long* ids, long long ids_row_stride, int batch, int n, int C, int S,
+                      long long summary_begin, int inner_chunk, int summary_kind, const float* inv_freq, int D,
+                      long long* out_ids, void* cos, void* sin, void* is_summary, int dtype, void* stream);
+
 /* Pre-attention step: per-head RMSNorm of q and k, rotary embedding, layout write of q, k, v.
  * Replaces HF:660-666 (q_norm / k_norm = Qwen3RMSNorm HF:64-79 on head_dim, the three
  * .transpose(1, 2), apply_rotary_pos_emb HF:523-554 in its rotate_half form) and the

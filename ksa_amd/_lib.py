@@ -43,6 +43,9 @@ _SIGNATURES = {
     "ksa_decode_boundary_fwd": (_int, [_vp] * 6 + [_int, _int, _vp, _vp] + [_int] * 8 + [_i64p] * 4
                                 + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
     "ksa_copy_rows_multi": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp, _vp, _vp]),
+    "ksa_copy_rows_runs": (_int, [_int] + [_vp] * 5 + [_int] + [_vp] * 2 + [_int] * 3 + [_vp] * 3),
+    "ksa_expand_prompt": (_int, [_vp, ctypes.c_longlong] + [_int] * 4 + [ctypes.c_longlong, _int, _int, _vp, _int]
+                          + [_vp] * 4 + [_int, _vp]),
     "ksa_copy_rows": (_int, [_vp] * 4 + [_int] * 6 + [_i64p] * 2 + [_vp]),
     "ksa_pre_attention": (_int, [_vp] * 10 + [_int] * 6 + [_i64p] * 7 + [_vp, _int, ctypes.c_float, _vp]),
     "ksa_pre_attention_partials": (_int, [_vp, _int] + [_vp] * 7 + [_int] * 6 + [_i64p] * 4

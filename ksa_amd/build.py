@@ -13,7 +13,7 @@ LIB = os.path.join(HERE, "libksa_hip.so")
 SOURCES = ["ksa_prefill_d256_bf16_regular.hip", "ksa_prefill_d256_bf16_general.hip", "ksa_prefill_d256_f16_regular.hip",
            "ksa_prefill_d256_f16_general.hip", "ksa_prefill_d256_bf16_marked.hip", "ksa_prefill_d256_f16_marked.hip",
            "ksa_prefill_d256_bf16_chunks.hip", "ksa_prefill_d256_f16_chunks.hip",
-           "ksa_prefill.hip", "ksa_prefill_chunks.hip", "ksa_api.hip", "ksa_index.hip", "ksa_decode.hip", "ksa_decode_weights.hip", "ksa_cache.hip",
+           "ksa_prefill.hip", "ksa_prefill_chunks.hip", "ksa_api.hip", "ksa_index.hip", "ksa_decode.hip", "ksa_decode_weights.hip", "ksa_cache.hip", "ksa_prompt.hip",
            "ksa_pre.hip", "ksa_elementwise.hip", "ksa_gemm_rows.hip", "ksa_mlp_rows.hip", "ksa_norm_gemm_rows.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

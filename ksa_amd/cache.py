@@ -88,6 +88,30 @@ def _move_rows_multi(moves) -> None:
     _lib.check(rc, "ksa_copy_rows_multi")
 
 
+def _move_runs(moves, period: int) -> None:
+    """Up to 8 independent row moves as one launch, source rows by a closed form (`ksa_copy_rows_runs`): row i of a
+    move (src, dst, nrows, offset, first, run, dst_start) is row offset + (first + i) // run * period + (first + i) % run
+    of its source.  All tensors [bsz, heads, rows, D] of one shape class."""
+    moves = [m for m in moves if m[2] > 0]
+    if not moves:
+        return
+    import ctypes
+    n = len(moves)
+    bsz, heads, _, D = moves[0][1].shape
+    for src, dst, *_ in moves:
+        assert src.is_cuda and dst.is_cuda and src.dtype == dst.dtype and src.element_size() == 2
+        assert src.shape[:2] == dst.shape[:2] == (bsz, heads) and src.shape[3] == dst.shape[3] == D
+        assert src.stride(3) == dst.stride(3) == 1
+    ptrs = lambda j: (ctypes.c_void_p * n)(*[m[j].data_ptr() for m in moves])
+    ints = lambda j: (ctypes.c_int * n)(*[int(m[j]) for m in moves])
+    strides = lambda j: (ctypes.c_int64 * (3 * n))(*[v for m in moves for v in m[j].stride()[:3]])
+    dev = moves[0][1].device
+    with _lib.on_device(dev):
+        rc = _lib.lib().ksa_copy_rows_runs(n, ptrs(0), ptrs(1), ints(3), ints(4), ints(5), int(period), ints(6), ints(2), bsz,
+                                           heads, D, strides(0), strides(1), _lib.stream_ptr(dev))
+    _lib.check(rc, "ksa_copy_rows_runs")
+
+
 class Qwen3RingBufferCache:
     is_compileable = False
     _SUMMARY_INIT_CAP = 512
@@ -120,6 +144,7 @@ class Qwen3RingBufferCache:
         self._reorganized = False
         self._reorg_done = set()   # layers already in the ring layout (`reorganize_layer`)
         self._reorg_rows = None    # (text rows, summary rows, counts) of the prefill, made once
+        self._reorg_in_line = None  # text rows of a prefill whose summaries lie in line, see `prompt_in_line`
 
     # ---- queries -------------------------------------------------------------------
     def __len__(self):
@@ -226,6 +251,12 @@ class Qwen3RingBufferCache:
         return (self.key_cache[layer_idx][:, :, row:row + 1, :].transpose(1, 2),
                 self.value_cache[layer_idx][:, :, row:row + 1, :].transpose(1, 2))
 
+    def prompt_in_line(self, n_text: int):
+        """Says in front of `reorganize_layer` that the prefill's mask is the periodic one, `summary_token_num` rows
+        behind every whole chunk of its `n_text` text rows: the rows are then closed forms, and neither the mask is
+        read nor the host made to wait for it."""
+        self._reorg_in_line = n_text
+
     def reorganize_after_prefill(self, summary_mask: torch.Tensor):
         """Prefill order -> ring layout for every layer.  summary_mask: bool [bsz, prefill_len]."""
         if self._reorganized:
@@ -243,20 +274,27 @@ class Qwen3RingBufferCache:
             return
         self._reorg_done.add(layer)
         C, S = self.summary_chunk_size, self.summary_token_num
-        if self._reorg_rows is None:
+        if self._reorg_in_line is not None:
+            n_text = self._reorg_in_line
+            n_sum = n_text // C * S
+        elif self._reorg_rows is None:
             sm = summary_mask[0]
             self._reorg_rows = (torch.nonzero(~sm, as_tuple=False).flatten().to(torch.int32),
                                 torch.nonzero(sm, as_tuple=False).flatten().to(torch.int32))
-        text_rows, sum_rows = self._reorg_rows
-        n_text, n_sum = text_rows.numel(), sum_rows.numel()
+        if self._reorg_in_line is None:
+            text_rows, sum_rows = self._reorg_rows
+            n_text, n_sum = text_rows.numel(), sum_rows.numel()
         n_complete, n_partial = divmod(n_text, C)
 
         old_k, old_v = self.key_cache[layer], self.value_cache[layer]
         if self.is_large_window[layer]:
             cap = n_text + self._APPEND_HEADROOM
             new_k, new_v = self._alloc(old_k, cap), self._alloc(old_v, cap)
-            self._move_rows(old_k, new_k, n_text, src_index=text_rows)
-            self._move_rows(old_v, new_v, n_text, src_index=text_rows)
+            if self._reorg_in_line is not None:
+                _move_runs([(old, new, n_text, 0, 0, C, 0) for old, new in ((old_k, new_k), (old_v, new_v))], C + S)
+            else:
+                self._move_rows(old_k, new_k, n_text, src_index=text_rows)
+                self._move_rows(old_v, new_v, n_text, src_index=text_rows)
             self._text_len[layer] = n_text
         else:
             ws, scn = self.window_sizes[layer], self.sliding_chunk_nums[layer]
@@ -264,7 +302,12 @@ class Qwen3RingBufferCache:
             cap = S + C + ws + n_sum + max(self._SUMMARY_INIT_CAP, n_sum + 256)
             new_k, new_v = self._alloc(old_k, cap), self._alloc(old_v, cap)
             first_win = n_complete * C - n_win
-            for old, new in ((old_k, new_k), (old_v, new_v)):
+            if self._reorg_in_line is not None:
+                _move_runs([m for old, new in ((old_k, new_k), (old_v, new_v))
+                            for m in ((old, new, n_partial, 0, n_complete * C, C, S + C - n_partial),
+                                      (old, new, n_win, 0, first_win, C, S + C),
+                                      (old, new, n_sum, C, 0, S, S + C + ws))], C + S)
+            for old, new in ((old_k, new_k), (old_v, new_v)) if self._reorg_in_line is None else ():
                 # trailing partial chunk, right-aligned in the chunk region
                 self._move_rows(old, new, n_partial, dst_start=S + C - n_partial,
                                 src_index=text_rows[n_complete * C:])

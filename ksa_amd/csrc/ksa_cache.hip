@@ -64,7 +64,65 @@ __global__ __launch_bounds__(256) void ksa_copy_rows_multi_kernel(const MultiCop
     }
 }
 
+// The same with a source row that is a closed form: row i of a move is row offset + (first + i) / run * period + (first +
+// i) % run of its source - the text rows (run = C) or the summary rows (run = S) of a prompt with its summary tokens in line
+// (period = C + S).  What a layer keeps of a prompt, the cut chunk, the window and the summaries of K and of V, is then one
+// launch where it was six through index lists, which a mask had to be turned into first.
+struct RunParams : CopyParams {
+    int first, run, period;
+};
+struct MultiRunParams {
+    RunParams mv[kMaxMoves];
+};
+
+__global__ __launch_bounds__(256) void ksa_copy_rows_runs_kernel(const MultiRunParams mp, int heads) {
+    const int which = blockIdx.y / heads, h = blockIdx.y % heads, b = blockIdx.z;
+    const RunParams& p = mp.mv[which];
+    const unsigned total = (unsigned)p.nrows * p.cpr;
+    const uint16_t* sb = p.src + b * p.s_bs + h * p.s_hs;
+    uint16_t* db = p.dst + b * p.d_bs + h * p.d_hs;
+    for (unsigned u = blockIdx.x * 256u + threadIdx.x; u < total; u += gridDim.x * 256u) {
+        const unsigned i = u / (unsigned)p.cpr, c = u % (unsigned)p.cpr, j = (unsigned)p.first + i;
+        const int64_t sr = p.src_start + (int64_t)(j / (unsigned)p.run) * p.period + j % (unsigned)p.run;
+        *reinterpret_cast<u32x4*>(db + (int64_t)(p.dst_start + (int)i) * p.d_rs + 8 * c) =
+            __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(sb + sr * p.s_rs + 8 * c));
+    }
+}
+
 }  // namespace
+
+extern "C" int ksa_copy_rows_runs(int n_moves, const void* const* src, void* const* dst, const int* offset, const int* first,
+                                  const int* run, int period, const int* dst_start, const int* nrows, int batch, int heads,
+                                  int D, const int64_t* src_strides, const int64_t* dst_strides, void* stream) {
+    if (!src || !dst || !offset || !first || !run || !dst_start || !nrows || !src_strides || !dst_strides) return KSA_ERR_NULL;
+    if (n_moves <= 0 || n_moves > kMaxMoves || batch <= 0 || heads <= 0 || D <= 0 || D % 8 != 0) return KSA_ERR_INVALID;
+    MultiRunParams mp{};
+    int64_t most = 0;
+    for (int m = 0; m < n_moves; ++m) {
+        if (!src[m] || !dst[m]) return KSA_ERR_NULL;
+        if (nrows[m] < 0 || offset[m] < 0 || first[m] < 0 || run[m] <= 0 || period < run[m] || dst_start[m] < 0)
+            return KSA_ERR_INVALID;
+        if ((reinterpret_cast<uintptr_t>(src[m]) | reinterpret_cast<uintptr_t>(dst[m])) & 15) return KSA_ERR_ALIGN;
+        for (int i = 0; i < 3; ++i)
+            if ((src_strides[3 * m + i] % 8) || (dst_strides[3 * m + i] % 8)) return KSA_ERR_ALIGN;
+        RunParams& p = mp.mv[m];
+        p.src = (const uint16_t*)src[m];
+        p.dst = (uint16_t*)dst[m];
+        p.src_start = offset[m], p.dst_start = dst_start[m], p.nrows = nrows[m];
+        p.first = first[m], p.run = run[m], p.period = period;
+        p.cpr = D / 8;
+        p.s_bs = src_strides[3 * m], p.s_hs = src_strides[3 * m + 1], p.s_rs = src_strides[3 * m + 2];
+        p.d_bs = dst_strides[3 * m], p.d_hs = dst_strides[3 * m + 1], p.d_rs = dst_strides[3 * m + 2];
+        const int64_t total = (int64_t)nrows[m] * p.cpr;
+        if (total >= (1ll << 31) || (int64_t)first[m] + nrows[m] >= (1ll << 31)) return KSA_ERR_INVALID;
+        if (total > most) most = total;
+    }
+    if (most == 0) return KSA_OK;
+    int gx = (int)((most + 255) / 256);
+    if (gx > 1024) gx = 1024;
+    hipLaunchKernelGGL(ksa_copy_rows_runs_kernel, dim3(gx, heads * n_moves, batch), dim3(256), 0, (hipStream_t)stream, mp, heads);
+    return ksa_check_launch();
+}
 
 // n_moves <= 8 moves, move m: dst[m] row (dst_start[m] (+ dst_start_seq[m][sequence] instead, if given) + i)
 // <- src[m] row (src_start[m] + i), i < nrows[m], for every (sequence, head).  The moves must not

@@ -137,11 +137,13 @@ class HipOps:
     that does so gives each stream its operator set."""
 
     def __init__(self):
-        from . import cache, decode, elementwise, gemm, pre, prefill
+        from . import _lib, cache, decode, elementwise, gemm, pre, prefill
+        self._lib = _lib
         self.cache_cls = cache.Qwen3RingBufferCache
         self.pre_attention = pre.pre_attention
         self.pre_attention_partials = pre.pre_attention_partials
         self._summary_attn = prefill.summary_attn_func
+        self._summary_attn_in_line = prefill.summary_attn_in_line
         self.add_rmsnorm = elementwise.add_rmsnorm
         self.silu_mul = elementwise.silu_mul
         self.embed_rmsnorm = elementwise.embed_rmsnorm       # the head of a recorded step in one launch
@@ -188,6 +190,37 @@ class HipOps:
 
     def summary_attn_func(self, q, k, v, *args, **kwargs):
         return self._summary_attn(q, k, v, *args, chunk_tiles=q.shape[1] > self.GRID_ROWS, **kwargs)
+
+    def summary_attn_in_line(self, q, k, v, C, S, W):
+        """`summary_attn_func` with the mask of `expand_prompt`."""
+        return self._summary_attn_in_line(q, k, v, C, S, W, chunk_tiles=q.shape[1] > self.GRID_ROWS)
+
+    def expand_prompt(self, input_ids, config, inv_freq, dtype):
+        """`expand_with_summary_tokens` and the rotary rows of its positions in one launch (`ksa_expand_prompt`): (ids
+        [b, L], cos, sin [1, L, D], mask [L]); None where those have to do it."""
+        text = {"origin": 0, "inner_chunk": 1}.get(config.summary_chunk_position_ids_type)
+        summary = {"zeros": 0, "last_chunk_slice_left": 1, "last_chunk_slice_right": 2}.get(
+            config.summary_token_position_ids_type)
+        D = config.head_dim
+        if (text is None or summary is None or dtype not in (torch.bfloat16, torch.float16) or D % 16
+                or input_ids.dtype != torch.long or input_ids.dim() != 2 or not input_ids.is_cuda or input_ids.numel() == 0
+                or inv_freq.dtype != torch.float32 or inv_freq.shape != (D // 2,) or not inv_freq.is_contiguous()):
+            return None
+        C, S, dev = config.summary_chunk_size, config.summary_token_num, input_ids.device
+        if input_ids.stride(1) != 1:
+            input_ids = input_ids.contiguous()
+        b, n = input_ids.shape
+        L = n // C * S + n
+        ids = torch.empty(b, L, dtype=torch.long, device=dev)
+        rope = torch.empty(2, 1, L, D, dtype=dtype, device=dev)
+        mask = torch.empty(L, dtype=torch.bool, device=dev)
+        with self._lib.on_device(dev):
+            rc = self._lib.lib().ksa_expand_prompt(
+                input_ids.data_ptr(), input_ids.stride(0), b, n, C, S, config.summary_token_begin, text, summary,
+                inv_freq.data_ptr(), D, ids.data_ptr(), rope[0].data_ptr(), rope[1].data_ptr(), mask.data_ptr(),
+                0 if dtype == torch.bfloat16 else 1, self._lib.stream_ptr(dev))
+        self._lib.check(rc, "ksa_expand_prompt")
+        return ids, rope[0], rope[1], mask
 
     def decode(self, q, kbuf, vbuf, start, end, scale):
         return self._decode(q, kbuf, vbuf, start, end, scale=scale)
@@ -618,12 +651,21 @@ class KsaQwen3ForCausalLM:
         """input_ids [b, n] -> (logits [b, 1, vocab] of the last prompt token, cache)."""
         cfg, ops = self.config, self.ops
         C, S = cfg.summary_chunk_size, cfg.summary_token_num
-        ids, pos, is_sum = expand_with_summary_tokens(input_ids.to(self.device), cfg)
+        input_ids = input_ids.to(self.device)
+        head = ops.expand_prompt(input_ids, cfg, self.inv_freq_dev, self.dtype) if hasattr(ops, "expand_prompt") else None
+        if head is not None:
+            ids, cos, sin, is_sum = head
+        else:
+            ids, pos, is_sum = expand_with_summary_tokens(input_ids, cfg)
+            cos, sin = self._rope_tables(pos)
         b, L = ids.shape
-        n_sum = int(is_sum.sum().item())
-        sum_rows = torch.nonzero(is_sum).flatten()
-        cos, sin = self._rope_tables(pos)
+        n_sum = input_ids.shape[1] // C * S
+        sum_rows = torch.nonzero(is_sum).flatten() if cfg.summary_independent_parameters else None
         cache = ops.cache_cls(cfg, self.scns)
+        if head is not None and hasattr(cache, "prompt_in_line"):
+            cache.prompt_in_line(L - n_sum)
+        # (an operator set with an attention of its own gets the mask)
+        in_line = head is not None and getattr(ops.summary_attn_func, "__func__", None) is HipOps.summary_attn_func
         x = self.w["embed_tokens"][ids]
         delta = None     # output of the previous MLP, added to the residual stream by the next norm
         Hkv, D = cfg.num_key_value_heads, cfg.head_dim
@@ -634,7 +676,8 @@ class KsaQwen3ForCausalLM:
             q, k, v = ops.pre_attention(q, k, v, lw["q_norm"], lw["k_norm"], cos, sin, cfg.rms_norm_eps,
                                         k_out=k_slot, v_out=v_slot)
             self._blend_summary(lw, h, sum_rows, cos, sin, q, k, v)
-            attn, _ = ops.summary_attn_func(q, k, v, C, S, self.scns[li], summary_pos=is_sum)
+            attn, _ = (ops.summary_attn_in_line(q, k, v, C, S, self.scns[li]) if in_line else
+                       ops.summary_attn_func(q, k, v, C, S, self.scns[li], summary_pos=is_sum))
             del q, k, v, k_slot, v_slot
             if hasattr(cache, "reorganize_layer"):   # the layer's K/V in prompt order are not needed any more
                 cache.reorganize_layer(li, is_sum[None])

@@ -299,6 +299,34 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     only for autograd and always uses head_dim ** -0.5; `workgroup_shape` is the tuning knob of
     `PREFILL_SHAPE`; `chunk_tiles=False` keeps a call on the grid of the block index).
     """
+    def layout(Sq, C, S, k, v):
+        if summary_pos is not None:
+            assert k.shape[1] == Sq, "with summary_pos, k/v must have the same length as q"
+            P, periodic, rows = _analyse_summary_pos(summary_pos, Sq, C, S)
+            if P > 0 and not periodic:
+                return P, True, _gathered_prefix(k, rows, P), _gathered_prefix(v, rows, P)
+            return P, False, k, v
+        P = k.shape[1] - Sq
+        assert P >= 0, "k/v must be at least as long as q"
+        return P, P > 0, k, v
+
+    return _forward(q, k, v, chunk_size, summary_num, sliding_chunk_num, layout, skip_old_summary, return_lse,
+                    softmax_scale, workgroup_shape, chunk_tiles)
+
+
+def summary_attn_in_line(q, k, v, chunk_size, summary_num, sliding_chunk_num, *, chunk_tiles: bool = True):
+    """`summary_attn_func` for a prompt whose summary rows the caller itself has put behind every whole chunk: with the
+    `summary_pos` of that layout, without the host waiting for an analysis of it."""
+    def layout(Sq, C, S, k, v):
+        assert k.shape[1] == Sq and Sq % (C + S) <= C, "k/v have the rows of q, summary rows stand behind whole chunks"
+        return Sq // (C + S) * S, False, k, v
+
+    return _forward(q, k, v, chunk_size, summary_num, sliding_chunk_num, layout, False, False, None, None, chunk_tiles)
+
+
+def _forward(q, k, v, chunk_size, summary_num, sliding_chunk_num, layout, skip_old_summary, return_lse, softmax_scale,
+             workgroup_shape, chunk_tiles):
+    """`layout(Sq, C, S, k, v)` -> (rows of the key prefix, whether k and v hold it as rows of their own, k, v)."""
     _check_inputs(q, k, v)
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
         raise NotImplementedError("ksa_amd implements the prefill forward only; call it under torch.no_grad()")
@@ -306,17 +334,7 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     C, S, W = int(chunk_size), int(summary_num), int(sliding_chunk_num)
     assert C > 0 and S > 0 and W >= 0, "chunk_size/summary_num must be positive, sliding_chunk_num >= 0"
     q, k, v = _lastdim_contig(q), _lastdim_contig(k), _lastdim_contig(v)
-    phys = False
-    if summary_pos is not None:
-        assert k.shape[1] == Sq, "with summary_pos, k/v must have the same length as q"
-        P, periodic, rows = _analyse_summary_pos(summary_pos, Sq, C, S)
-        if P > 0 and not periodic:
-            k, v = _gathered_prefix(k, rows, P), _gathered_prefix(v, rows, P)
-            phys = True
-    else:
-        P = k.shape[1] - Sq
-        assert P >= 0, "k/v must be at least as long as q"
-        phys = P > 0
+    P, phys, k, v = layout(Sq, C, S, k, v)
     if k.stride() != v.stride():
         v = v.contiguous()
         k = k.contiguous()

@@ -208,3 +208,28 @@ def test_move_rows_multi_equals_single_moves():
         torch.cuda.synchronize()
         for x, r in zip(bufs, ref):
             assert torch.equal(x, r)
+
+
+@pytest.mark.parametrize("C,S,D,n_text", [(8, 1, 64, 5), (8, 2, 128, 8), (16, 3, 64, 37), (128, 8, 128, 127), (128, 8, 128, 1300)])
+def test_reorganize_in_line_equals_index_lists(C, S, D, n_text):
+    """The rows of a prompt with its summaries in line by closed form (`ksa_copy_rows_runs`) and through the mask."""
+    import ksa_amd
+    cfg = types.SimpleNamespace(summary_chunk_size=C, summary_token_num=S, num_hidden_layers=2)
+    L = n_text // C * S + n_text
+    mask = torch.from_numpy(O.summary_positions(L, C, S))[None].cuda()
+    g = torch.Generator(device="cuda").manual_seed(0)
+    k, v = (torch.randn(2, 3, L, D, generator=g, device="cuda").bfloat16() for _ in range(2))
+    views = []
+    for in_line in (False, True):
+        cache = ksa_amd.Qwen3RingBufferCache(cfg, [3, 10 ** 6])
+        for layer in range(2):
+            for slot, t in zip(cache.prefill_slots(layer, 2, 3, L, D, k.dtype, k.device, n_text // C * S), (k, v)):
+                slot.copy_(t.transpose(1, 2))
+        if in_line:
+            cache.prompt_in_line(n_text)
+        cache.reorganize_after_prefill(mask)
+        views.append([t for layer in range(2) for t in cache.get_attention_kv(layer)])
+        views[-1] += [getattr(cache, n) for n in ("_text_len", "_n_valid_window", "_window_write_ptr", "_chunk_buf_len",
+                                                  "_n_summaries", "_capacity", "_total_chunks", "cur_chunk_sizes")]
+    for a, b in zip(*views):
+        assert torch.equal(a, b) if torch.is_tensor(a) else a == b

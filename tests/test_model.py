@@ -68,6 +68,26 @@ def test_expand_positions_brute_force(kind, n):
     assert is_sum.tolist() == exp_sum
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["last_chunk_slice_right", "last_chunk_slice_left", "zeros"])
+@pytest.mark.parametrize("text,C,S,D", [("origin", 128, 8, 128), ("inner_chunk", 100, 7, 64), ("origin", 5, 3, 16)])
+def test_gpu_expand_prompt_equals_host_form(text, C, S, D, kind, dtype):
+    from ksa_amd.model import HipOps
+    cfg = tiny_config(head_dim=D, summary_chunk_size=C, summary_token_num=S, summary_token_position_ids_type=kind,
+                      summary_chunk_position_ids_type=text)
+    inv = (1.0 / (1e6 ** (torch.arange(0, D, 2).float() / D))).cuda()
+    for b, n in ((1, 1), (9, C - 1), (2, C), (2, 7 * C + 3), (1, 60 * C)):
+        ids = torch.randint(0, 200, (b, 2 * n), device="cuda")[:, ::2]   # (a view with a stride)
+        got_ids, cos, sin, mask = HipOps().expand_prompt(ids, cfg, inv, dtype)
+        want_ids, pos, want_mask = expand_with_summary_tokens(ids, cfg)
+        assert torch.equal(got_ids, want_ids) and torch.equal(mask, want_mask)
+        angle = pos[0].float()[:, None] * torch.cat((inv, inv))[None]
+        for got, want in ((cos, angle.cos()), (sin, angle.sin())):   # one rounding of the same fp32 function
+            assert got.shape == (1, want.shape[0], D)
+            torch.testing.assert_close(got[0], want.to(dtype), rtol=2.0 ** (-7 if dtype == torch.bfloat16 else -10), atol=1e-6)
+
+
 def test_expand_known_values():
     cfg = tiny_config(summary_token_num=2)
     ids, pos, is_sum = expand_with_summary_tokens(torch.arange(17)[None], cfg)
