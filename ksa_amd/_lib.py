@@ -13,6 +13,10 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # KSA_AMD_LIB selects another build of the same library (e.g. a profiling variant)
 LIB_PATH = os.environ.get("KSA_AMD_LIB") or os.path.join(_HERE, "libksa_hip.so")
 _lib = None
+# the native front of the hottest calls (csrc/ksa_fast.cpp); what it calls, in the order of its `bind`
+fast = None
+_FAST = ("ksa_block_index", "ksa_decode_splits", "ksa_decode_workspace_bytes", "ksa_decode_fwd", "ksa_prefill_chunks_fwd",
+         "ksa_pre_attention")
 
 _i32p = ctypes.POINTER(ctypes.c_int32)
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -97,7 +101,7 @@ class KsaError(RuntimeError):
 
 
 def lib():
-    global _lib
+    global _lib, fast
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise KsaError(
@@ -108,6 +112,13 @@ def lib():
             fn = getattr(L, name)
             fn.restype = res
             fn.argtypes = args
+        try:
+            from . import _fast
+        except ImportError as e:
+            raise KsaError(f"ksa_amd/_fast.so is missing or was built for another PyTorch: build it with `python "
+                           f"ksa_amd/build.py` ({e})") from e
+        _fast.bind(*[ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _FAST])
+        fast = _fast
         _lib = L
     return _lib
 

@@ -1,4 +1,5 @@
-"""Build recipe for libksa_hip.so (hipcc, gfx950 only)."""
+"""Build recipe for libksa_hip.so (hipcc, gfx950 only) and _fast.so (the native front of the hottest calls, g++ against the
+installed PyTorch)."""
 from __future__ import annotations
 
 import os
@@ -9,6 +10,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libksa_hip.so")
+FAST = os.path.join(HERE, "_fast.so")
 # (the slowest units first: they run next to the others)
 SOURCES = ["ksa_prefill_d256_bf16_regular.hip", "ksa_prefill_d256_bf16_general.hip", "ksa_prefill_d256_f16_regular.hip",
            "ksa_prefill_d256_f16_general.hip", "ksa_prefill_d256_bf16_marked.hip", "ksa_prefill_d256_f16_marked.hip",
@@ -23,6 +25,20 @@ FLAGS = [
     # canonicalising v_max
     "-fno-honor-nans",
 ]
+
+
+def _fast_command() -> list:
+    import sysconfig
+    import torch
+    at = os.path.dirname(os.path.abspath(torch.__file__))
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"))))
+    include = [os.path.join(at, "include"), os.path.join(at, "include", "torch", "csrc", "api", "include"),
+               os.path.join(rocm, "include"), sysconfig.get_paths()["include"], os.path.join(os.path.dirname(HERE), "include")]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",  # what the headers of ROCm and of PyTorch ask for
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(a for d in include for a in ("-isystem", d)),
+            os.path.join(CSRC, "ksa_fast.cpp"), "-o", FAST, "-L" + os.path.join(at, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu",
+            "-ltorch_hip", "-ltorch", "-ltorch_python", "-Wl,-rpath," + os.path.join(at, "lib")]
 
 
 def _run(cmd, verbose):
@@ -47,6 +63,8 @@ def build(verbose: bool = False, extra_flags=(), out: str = LIB, csrc: str = CSR
     objs = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in SOURCES]
     cmds = [[hipcc, *FLAGS, *extra_flags, "-I", csrc, "-c", os.path.join(csrc, s), "-o", o]
             for s, o in zip(SOURCES, objs)]
+    if out == LIB:
+        cmds.append(_fast_command())
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
         list(pool.map(lambda c: _run(c, verbose), cmds))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *objs], verbose)

@@ -73,6 +73,10 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     """q [b, Hq, Q, D]; kcache/vcache [b, Hkv, rows, D] (any batch/head/row strides);
     rows [start, end) are attended: ints for every sequence, or int32 device tensors [b]
     per sequence; default is the whole row axis.  Returns [b, Q, Hq, D]."""
+    if not torch.compiler.is_compiling():
+        out = _lib.fast.decode(q, kcache, vcache, start, end, scale, nsplit)
+        if out is not None:
+            return out
     assert q.is_cuda and kcache.is_cuda and vcache.is_cuda, "inputs must be on a GPU"
     assert q.dtype in _DTYPES and q.dtype == kcache.dtype == vcache.dtype, "inputs must share a 16-bit float dtype"
     assert q.dim() == 4 and kcache.dim() == 4 and kcache.shape == vcache.shape
@@ -383,7 +387,7 @@ def decode_attention_forward(module, query: torch.Tensor, key: torch.Tensor, val
     as the reference's SDPA variant ignores it (it passes attn_mask=None); dropout must be 0."""
     if dropout:
         raise NotImplementedError("decode attention is inference-only (dropout must be 0)")
-    g = query.shape[1] // key.shape[1]
+    g = query.size(1) // key.size(1)
     mg = getattr(module, "num_key_value_groups", g)
     assert mg == g, "module.num_key_value_groups does not match the tensor shapes"
     return ksa_decode(query, key, value, scale=scaling), None

@@ -39,6 +39,10 @@ def pre_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm_weig
     [b, S] it names the output row of every token's k and v outright (k_out / v_out then only give
     the base address and the strides: pass the view that starts at row 0).
     """
+    if not torch.compiler.is_compiling():
+        out = _lib.fast.pre_attention(q, k, v, q_norm_weight, k_norm_weight, cos, sin, eps, q_out, k_out, v_out, kv_out_row)
+        if out is not None:
+            return out
     assert q.dtype in _DT and k.dtype == q.dtype and v.dtype == q.dtype, "q, k, v must share bf16 or fp16"
     assert q.is_cuda and k.is_cuda and v.is_cuda, "inputs must be on a GPU"
     b, S, Hq, D = q.shape

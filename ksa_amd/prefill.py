@@ -47,6 +47,11 @@ def compute_block_sparsity(seqlen_q: int, seqlen_k: int, chunk_size: int, summar
                            device=None) -> BlockSparseIndex:
     """Builds the four int32 index tensors on the GPU (bit-exact with the reference's
     BlockSparsityKernel, flash_attn/cute/compute_block_sparsity.py:189-274)."""
+    if device is None and torch.cuda.is_initialized() and not torch.compiler.is_compiling():
+        out = _lib.fast.block_index(seqlen_q, seqlen_k, chunk_size, summary_num, sliding_chunk_num, skip_old_summary, tile_m,
+                                    tile_n)
+        if out is not None:
+            return BlockSparseIndex(out)
     device = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
     if device.type != "cuda":
         raise AssertionError("compute_block_sparsity runs on the GPU only")
@@ -299,6 +304,13 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
     only for autograd and always uses head_dim ** -0.5; `workgroup_shape` is the tuning knob of
     `PREFILL_SHAPE`; `chunk_tiles=False` keeps a call on the grid of the block index).
     """
+    if chunk_tiles and not (PREFILL_SHAPE if workgroup_shape is None else workgroup_shape) \
+            and not torch.compiler.is_compiling():
+        out = _lib.fast.prefill(q, k, v, chunk_size, summary_num, sliding_chunk_num, skip_old_summary, softmax_scale, return_lse,
+                                summary_pos, _analyse_summary_pos)
+        if out is not None:
+            return out
+
     def layout(Sq, C, S, k, v):
         if summary_pos is not None:
             assert k.shape[1] == Sq, "with summary_pos, k/v must have the same length as q"

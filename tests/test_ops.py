@@ -327,3 +327,144 @@ def test_prefill_under_vmap():
     f = lambda a, b, c: ksa_amd.summary_attn_func(a, b, c, 32, 4, 1)[0]
     got = torch.func.vmap(f)(q, k, v)
     assert torch.equal(got, torch.stack([f(q[i], k[i], v[i]) for i in range(2)]))
+
+
+class _Front:
+    """`_lib.fast` with a record of which calls it took (`general`: takes none)."""
+
+    def __init__(self, real, general=False):
+        self.real, self.general, self.took = real, general, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            out = None if self.general else getattr(self.real, name)(*args)
+            self.took.append(out is not None)
+            return out
+        return call
+
+
+def _front_calls():
+    """(name, whether the native front takes the call, the call) over the forms of the four functions."""
+    import ksa_amd
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rnd = lambda dt, *s: torch.randn(*s, generator=g, device="cuda").to(dt)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    for dt in (torch.bfloat16, torch.float16):
+        for D, taken in ((64, True), (128, True), (256, True), (72, False)):
+            q, kc, vc = rnd(dt, 3, 8, 1, D), rnd(dt, 3, 2, 300, D), rnd(dt, 3, 2, 300, D)
+            q9 = rnd(dt, 3, 9, 8, D).transpose(1, 2)
+            wide = rnd(dt, 3, 300, 4, D).transpose(1, 2)   # rows and heads in the other order, keys next to values
+            dec = ksa_amd.ksa_decode
+            yield "decode", taken, lambda: dec(q, kc, vc)
+            yield "decode ints", taken, lambda: dec(q, kc, vc, 7, 233)
+            yield "decode views", taken, lambda: dec(q9, wide[:, :2, 5:299], wide[:, 2:, 5:299], scale=0.1)
+            yield "decode ranges", taken, lambda: dec(q, kc, vc, i32(0, 3, 299), i32(300, 4, 300), nsplit=3)
+            yield "decode one range", False, lambda: dec(q, kc, vc, None, i32(300, 4, 17))
+            yield "decode strided range", False, lambda: dec(q, kc, vc, i32(0, 9, 3, 9, 2, 9)[::2], i32(300, 4, 17))
+            yield "decode long range", False, lambda: dec(q, kc, vc, i32(0, 3, 2).long(), i32(300, 4, 17))
+            yield "decode scale", False, lambda: dec(q, kc, vc, scale=-0.1)
+            yield "decode int scale", False, lambda: dec(q, kc, vc, scale=1)
+            yield "decode strided q", False, lambda: dec(q.repeat(1, 1, 1, 2)[..., ::2], kc, vc)
+            n = 3 * 136 + 71
+            pos = torch.arange(n, device="cuda") % 136 >= 128
+            odd = pos.roll(1)
+            qkv = rnd(dt, 2, n, 8, D)
+            a = (qkv[:, :, :4], qkv[:, :, 4:6], qkv[:, :, 6:])
+            own = tuple(t.contiguous() for t in a)
+            sa = ksa_amd.summary_attn_func
+            yield "prefill", taken, lambda: sa(*a, 128, 8, 1, pos, return_lse=True)
+            yield "prefill own", taken, lambda: sa(*own, 128, 8, 2, summary_pos=pos, skip_old_summary=True)
+            yield "prefill no prefix", taken, lambda: sa(*own, 128, 8, 2, softmax_scale=0.2)
+            yield "prefill other chunk", False, lambda: sa(*own, 64, 8, 2)
+            yield "prefill grid", False, lambda: sa(*own, 128, 8, 2, pos, chunk_tiles=False)
+            yield "prefill shape", False, lambda: sa(*own, 128, 8, 2, pos, workgroup_shape=32)
+            yield "prefill other mask", False, lambda: sa(*own, 128, 8, 2, odd)
+            yield "prefill strides", False, lambda: sa(a[0], a[1], own[2], 128, 8, 2, pos)
+            yield "prefill built prefix", False, lambda: sa(own[0], *(torch.cat((t[:, pos], t), 1) for t in own[1:]), 128, 8, 2)
+            if D in (64, 128):
+                w = [torch.nn.Parameter(rnd(dt, D)) for _ in range(2)]
+                cos, sin = rnd(dt, 1, n, D), rnd(dt, 1, n, D)
+                pre = ksa_amd.pre_attention
+                cache = lambda: [torch.zeros(2, 2, n + 9, D, dtype=dt, device="cuda") for _ in range(2)]
+
+                def into(rows, S):
+                    c = cache()
+                    o = [t[:, :, :S].transpose(1, 2) for t in c]
+                    return pre(*(t[:, :S] for t in a), *w, cos[:, :S].contiguous(), sin[:, :S].contiguous(), 1e-5, k_out=o[0],
+                               v_out=o[1], kv_out_row=rows)[:1] + tuple(c)
+                yield "pre", True, lambda: pre(*a, *w, cos, sin)
+                yield "pre rope per sequence", True, lambda: pre(*own, *w, cos.repeat(2, 1, 1), sin.repeat(2, 1, 1), 1e-4)
+                yield "pre rows", True, lambda: into(i32(3, 0), 5)
+                yield "pre row per token", True, lambda: into(i32(3, 0, 9, 5, 5, 1, 2, 7).view(2, 4)[:, :3].contiguous(), 3)
+                yield "pre into", True, lambda: into(None, n)
+                yield "pre 2-d rope", False, lambda: pre(*a, *w, cos[0], sin[0])
+                yield "pre fp32 rope", False, lambda: pre(*a, *w, cos.float(), sin)
+    for args in ((400, 400, 128, 8, 2), (409, 433, 128, 8, 0, True), (1000, 1056, 100, 7, 3, False, 64, 32)):
+        yield "index", True, lambda: ksa_amd.compute_block_sparsity(*args)
+    yield "index device", False, lambda: ksa_amd.compute_block_sparsity(400, 400, 128, 8, 2, device="cuda:0")
+
+
+@pytest.mark.gpu
+def test_native_front_equals_general_way(monkeypatch):
+    """Every form of the four calls: taken where it should be, and the same tensors (values, shapes, strides) either way."""
+    from ksa_amd import _lib
+    real = _lib.fast
+    flat = lambda o: [t for t in (o if isinstance(o, tuple) else (o,)) if t is not None]
+    for name, taken, call in _front_calls():
+        front = _Front(real)
+        monkeypatch.setattr(_lib, "fast", front)
+        got = flat(call())
+        assert front.took == [True] if taken else not any(front.took), name
+        monkeypatch.setattr(_lib, "fast", _Front(real, general=True))
+        want = flat(call())
+        assert len(got) == len(want), name
+        for x, y in zip(got, want):
+            assert torch.equal(x, y) and x.stride() == y.stride() and x.dtype == y.dtype, name
+
+
+@pytest.mark.gpu
+def test_native_front_steps_aside():
+    """... for everybody whom `_lib.direct` steps aside for, for other devices and types, and for arguments out of range."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from ksa_amd import _lib
+    q = torch.randn(2, 4, 1, 64, device="cuda", dtype=torch.bfloat16)
+    kc, vc = (torch.randn(2, 2, 40, 64, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    ask = lambda a=q, k=kc, v=vc, *r: _lib.fast.decode(a, k, v, *(r or (None, None, None, None))) is not None
+    assert ask()
+    assert not ask(q.cpu()) and not ask(q.float()) and not ask(q.half()) and not ask(torch.nn.Parameter(q)) and not ask(q[0])
+    assert not ask(q.detach().requires_grad_()) and not ask(q, kc[:, :, :39]) and not ask(q, kc[:1], vc[:1])
+    assert not ask(q[:, :3]) and not ask(q[:0], kc[:0], vc[:0])
+    with torch.no_grad():
+        assert ask(q.detach().requires_grad_())
+    for r in ((-1, 9, None, None), (9, 9, None, None), (0, 41, None, None), (0.0, 9, None, None), (None, None, 0.0, None),
+              (None, None, float("nan"), None), (None, None, None, -1), (None, None, None, 0)):
+        assert not ask(q, kc, vc, *r), r
+    seen = []
+
+    def note(a):
+        seen.append(ask(a))
+        return a * 1
+    torch.func.vmap(lambda a: (seen.append(_lib.fast.decode(a, kc, vc, None, None, None, None) is not None), a)[1])(q[None])
+    torch.func.jvp(note, (q,), (q,))
+    torch.func.functionalize(note)(q)
+    torch.func.grad(lambda a: note(a).sum())(q)
+    with torch.autograd.forward_ad.dual_level():
+        note(torch.autograd.forward_ad.make_dual(q, q))
+
+    class Fn(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Op(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+    for context in (Fn(), Op(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]),
+                    torch.autograd.profiler.profile()):
+        with context:
+            note(q)
+    note(torch._to_functional_tensor(q))
+    note(torch._efficientzerotensor((2, 4, 1, 64), dtype=q.dtype, device="cuda"))
+    assert len(seen) == 11 and not any(seen), seen
+    assert ask()
