@@ -39,24 +39,33 @@ static inline KsaMask ksa_make_mask(int C, int S, int W, int P, int skip_old, in
     return KsaMask{ksa_imin(C, longest), ksa_imin(S, longest), W, P, skip_old ? 1 : 0, Sq, Sk};
 }
 
+// Division by C + S, as the counts below take it: this one, or FastDiv in a kernel.
+struct KsaPlainDiv {
+    int32_t d;
+    KSA_HD int32_t div(int32_t n) const { return n / d; }
+};
+
 // number of text rows (offset < C) among in-line rows [0, x), x >= 0
-KSA_HD int32_t ksa_text_below(int32_t x, int C, int B) {
-    const int32_t r = x % B;
-    return (x / B) * C + (r < C ? r : C);
+template <typename Div>
+KSA_HD int32_t ksa_text_below(int32_t x, int C, int B, const Div& by_block) {
+    const int32_t n = by_block.div(x), r = x - n * B;
+    return n * C + (r < C ? r : C);
 }
 
 // number of text rows among in-line rows [lo, hi)
-KSA_HD int32_t ksa_text_in(int32_t lo, int32_t hi, int C, int B) {
+template <typename Div>
+KSA_HD int32_t ksa_text_in(int32_t lo, int32_t hi, int C, int B, const Div& by_block) {
     if (lo < 0) lo = 0;
     if (hi <= lo) return 0;
-    return ksa_text_below(hi, C, B) - ksa_text_below(lo, C, B);
+    return ksa_text_below(hi, C, B, by_block) - ksa_text_below(lo, C, B, by_block);
 }
 
 // Number of key columns in [a, b) (already clipped to [0, Sk)) visible to row q.
-KSA_HD int32_t ksa_count_visible(const KsaMask& mk, int32_t q, int32_t a, int32_t b) {
+template <typename Div>
+KSA_HD int32_t ksa_count_visible(const KsaMask& mk, int32_t q, int32_t a, int32_t b, const Div& by_block) {
     const int B = mk.C + mk.S;
-    const int32_t c = q / B;
-    const int32_t o = q % B;
+    const int32_t c = by_block.div(q);
+    const int32_t o = q - c * B;
     const int32_t P = mk.P;
     if (o >= mk.C) {  // summary row: own chunk, causal
         const int32_t lo = ksa_imax(a, P + c * B), hi = ksa_imin(b, P + q + 1);
@@ -73,20 +82,35 @@ KSA_HD int32_t ksa_count_visible(const KsaMask& mk, int32_t q, int32_t a, int32_
         // window text + own text, kv >= max(P + w0*B, X)
         const int32_t lo = ksa_imax(ksa_imax(a, P + w0 * B), X) - P;
         const int32_t hi = ksa_imin(b, P + q + 1) - P;
-        n += ksa_text_in(lo, hi, mk.C, B);
+        n += ksa_text_in(lo, hi, mk.C, B, by_block);
     } else {
         const int32_t hi_all = ksa_imin(b, q + 1);
         // window text + own text
-        n += ksa_text_in(ksa_imax(a, w0 * B), hi_all, mk.C, B);
+        n += ksa_text_in(ksa_imax(a, w0 * B), hi_all, mk.C, B, by_block);
         if (!mk.skip_old) {  // in-line summary rows of chunks < w0
             const int32_t lo = a, hi = ksa_imin(hi_all, w0 * B);
-            if (hi > lo) n += (hi - lo) - ksa_text_in(lo, hi, mk.C, B);
+            if (hi > lo) n += (hi - lo) - ksa_text_in(lo, hi, mk.C, B, by_block);
         }
     }
     return n;
 }
 
 #if defined(__HIPCC__)
+// n / d for 0 <= n < 2^31 with d fixed per launch: one multiplication, where the compiler's division by
+// a number it does not know is some 35 instructions - a workgroup has about twenty of them in front of
+// its first tile.  With p = 31 + ceil(log2 d) and m = ceil(2^p / d), m d - 2^p < d <= 2^(p - 31), hence
+// floor(n m / 2^p) = floor(n / d); m < 2^32 and 2 n < 2^32, so n m / 2^p is (2 n m / 2^32) / 2^ceil(log2 d).
+struct FastDiv {
+    uint32_t d, m, s;
+    FastDiv() = default;
+    explicit FastDiv(uint32_t n) : d(n), s(0) {
+        while ((1ull << s) < d) ++s;
+        m = (uint32_t)(((1ull << (31 + s)) + d - 1) / d);
+    }
+    __device__ __forceinline__ int div(int n) const { return (int)(__umulhi(2u * (uint32_t)n, m) >> s); }
+    __device__ __forceinline__ int mod(int n) const { return n - div(n) * (int)d; }
+};
+
 // bits t in [lo, hi) of a 64-bit tile mask
 __device__ __forceinline__ uint64_t ksa_range_bits(int lo, int hi) {
     if (lo < 0) lo = 0;

@@ -72,21 +72,6 @@
 
 namespace {
 
-// n / d for 0 <= n < 2^31 with d fixed per launch: one multiplication, where the compiler's division by
-// a number it does not know is some 35 instructions - a workgroup has about twenty of them in front of
-// its first tile.  With p = 31 + ceil(log2 d) and m = ceil(2^p / d), m d - 2^p < d <= 2^(p - 31), hence
-// floor(n m / 2^p) = floor(n / d); m < 2^32 and 2 n < 2^32, so n m / 2^p is (2 n m / 2^32) / 2^ceil(log2 d).
-struct FastDiv {
-    uint32_t d, m, s;
-    FastDiv() = default;
-    explicit FastDiv(uint32_t n) : d(n), s(0) {
-        while ((1ull << s) < d) ++s;
-        m = (uint32_t)(((1ull << (31 + s)) + d - 1) / d);
-    }
-    __device__ __forceinline__ int div(int n) const { return (int)(__umulhi(2u * (uint32_t)n, m) >> s); }
-    __device__ __forceinline__ int mod(int n) const { return n - div(n) * (int)d; }
-};
-
 struct PrefillParams {
     const uint16_t* q;
     const uint16_t* k;
