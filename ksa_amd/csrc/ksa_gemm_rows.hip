@@ -516,13 +516,13 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) vo
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[(wave * 16 + r) * 17 + 4 * kq + i] = acc[i];
     __syncthreads();
-    if (threadIdx.x < 256) {
-        const int m = threadIdx.x >> 4, n = n0 + (threadIdx.x & 15);
+    for (int e = threadIdx.x; e < 256; e += blockDim.x) {  // (one chunk of K: a workgroup has 128 threads)
+        const int m = e >> 4, c = e & 15, n = n0 + c;
         if (m < p.M && n < p.I) {
             float g = 0.f, u = 0.f;
             for (int sl = 0; sl < p.S; ++sl) {
-                g += red[(sl * 16 + m) * 17 + (threadIdx.x & 15)];
-                u += red[((p.S + sl) * 16 + m) * 17 + (threadIdx.x & 15)];
+                g += red[(sl * 16 + m) * 17 + c];
+                u += red[((p.S + sl) * 16 + m) * 17 + c];
             }
             g = C::up(C::down(g));
             u = C::up(C::down(u));

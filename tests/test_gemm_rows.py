@@ -141,6 +141,14 @@ def test_gpu_gate_up_silu_one_launch(dtype, M, I, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,I,K", [(9, 40, 96), (16, 64, 128), (12, 200, 512), (16, 64, 544)])
+def test_gpu_gate_up_silu_of_one_chunk(dtype, M, I, K):
+    """Nine rows and more with a K of one chunk, whose workgroups have fewer threads than a tile has elements."""
+    test_gpu_gate_up_silu_one_launch(dtype, M, I, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M,H,I", [(8, 2560, 9728), (1, 2560, 9728), (16, 1024, 768), (3, 256, 256), (5, 4096, 512),
                                    (8, 768, 2304), (16, 2560, 1024)])
 def test_gpu_mlp_rows_one_launch(dtype, M, H, I):
