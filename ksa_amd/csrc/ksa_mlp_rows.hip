@@ -81,11 +81,21 @@ __device__ __forceinline__ u32x4 ld_agent_x4_wait(const void* p) {
 }
 
 // kTiled: both matrices in the streaming layout (what decides how they are loaded)
-template <typename T, bool kTiled>
+// kTight: x lies in LDS without padding, 16-byte piece j of row m at piece j ^ m instead, which keeps the reads of 16 rows apart as
+// well, and the outcome of a wait where x comes to lie.  Where that makes room for one more workgroup per CU: 16 rows of
+// 2560 are half a CU's LDS to the byte, 38.3 -> 36.1 us, 8 rows a quarter, 32.4 -> 31.7.  Elsewhere it costs the
+// exclusive-or of every read: 1 / 4 / 12 rows 29.3 / 30.4 / 34.7 -> 29.5 / 30.6 / 35.2 us.
+template <typename T, bool kTiled, bool kTight>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) void ksa_mlp_rows_kernel(const MlpParams p) {
     using C = KsaCvt<T>;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    __shared__ int s_fail;
+    int* s_fail;
+    if constexpr (kTight) {
+        s_fail = reinterpret_cast<int*>(lds);
+    } else {
+        __shared__ int own;
+        s_fail = &own;
+    }
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: what depends on it stays in scalar registers
@@ -97,8 +107,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 
     if ((int)blockIdx.x < p.head) {
-        // ---- norm stage, one workgroup per row (four slices requested at a time: registers) ----
-        ksa_norm_row<T, 4>(p.norm, p.H, blockIdx.x, tid, reinterpret_cast<float*>(lds));
+        // ---- norm stage, one workgroup per row (eight slices requested at a time; four: +0.5 us) ----
+        ksa_norm_row<T, 8>(p.norm, p.H, blockIdx.x, tid, reinterpret_cast<float*>(lds));
         __syncthreads();
         if (tid < kHeadCopies) add_agent(p.sync + kWordStride * (kWordHead0 + tid), 1ull);
         return;
@@ -111,7 +121,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
         const int half = wave / kSlices;  // 0: gate rows of w, 1: up rows
         const int slice = wave - half * kSlices;
         const int sl_steps = p.H / 32 / kSlices;  // K steps of a slice (H is a multiple of 128)
-        const int rowb = (p.H + 8) * 2;
+        const int rowb = kTight ? p.H * 2 : (p.H + 8) * 2;
         static_assert(kTileCols == 16, "a workgroup's columns are one tile of the streaming weight layout");
         KsaWeightLane wl = ksa_weight_lane(p.w_gu, p.wgu_rs, p.H, (int64_t)half * p.I + kTileCols * u, r, kq,
                                            (int64_t)(half + 1) * p.I);
@@ -145,20 +155,35 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
                         break;
                     }
                 }
-                s_fail = fail;
+                *s_fail = fail;
             }
             __syncthreads();
-            if (s_fail) return;
-            const int per_row = p.H / 4;  // 8-byte words (agent-scope loads the compiler tracks: several in flight)
-            for (int e = tid; e < p.M * per_row; e += blockDim.x) {
-                const int m = e / per_row, j = e - m * per_row;
-                *reinterpret_cast<unsigned long long*>(lds + m * rowb + 8 * j) = ld_agent(p.norm.hbuf + (int64_t)m * per_row + j);
+            const int failed = *s_fail;
+            if constexpr (kTight) __syncthreads();
+            if (failed) return;
+            // Five 16-byte loads in flight: one trip for 8 rows of 2560.  (One 8-byte load after the other made ten of it: 8 / 12 / 16 rows
+            // 34.4 / 40.3 / 46.9 us a launch, 32.6 / 35.7 / 38.5 like this; eight in flight spill, +6 us.)
+            constexpr int kX = 5;
+            const int per_row = p.H / 8, n = p.M * per_row;
+            const KsaAgentBuffer hb(p.norm.hbuf, (uint32_t)n * 16u);
+            int t1 = tid;  // (opaque: nothing of this lives across the wait above)
+            asm volatile("" : "+v"(t1));
+            for (int base = 0; base < n; base += kX * 512) {
+                u32x4 v[kX];
+#pragma unroll
+                for (int i = 0; i < kX; ++i)
+                    if (base + 512 * i < n) v[i] = hb.ld4((uint32_t)min(base + 512 * i + t1, n - 1) * 16u);
+#pragma unroll
+                for (int i = 0; i < kX; ++i) {
+                    const int e = base + 512 * i + t1, m = e / per_row, j = e - m * per_row;
+                    if (e < n) *reinterpret_cast<u32x4*>(lds + m * rowb + 16 * (kTight ? j ^ m : j)) = v[i];
+                }
             }
         } else {
             const int per_row = p.H / 8;
             for (int e = tid; e < p.M * per_row; e += blockDim.x) {
                 const int m = e / per_row, j = e - m * per_row;
-                *reinterpret_cast<u32x4*>(lds + m * rowb + 16 * j) =
+                *reinterpret_cast<u32x4*>(lds + m * rowb + 16 * (kTight ? j ^ m : j)) =
                     *reinterpret_cast<const u32x4*>(p.x + (int64_t)m * p.x_rs + 8 * j);
             }
         }
@@ -166,10 +191,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
         for (int s0 = 0; s0 < sl_steps; s0 += kB) {
             if (s0 != 0) load_steps(s0);
             const int nst = min(kB, sl_steps - s0);
-            const unsigned char* xb = lds + xrow * rowb + (slice * sl_steps + s0) * 64 + 16 * kq;
+            const int st0 = slice * sl_steps + s0, flip = kTight ? xrow >> 2 : 0;
+            const unsigned char* xb = lds + xrow * rowb + (kTight ? 16 * (kq ^ (xrow & 3)) : st0 * 64 + 16 * kq);
 #pragma unroll
             for (int k = 0; k < kB; ++k) {
-                if (k < nst) acc = mfma16<T>(a[k], *reinterpret_cast<const u32x4*>(xb + 64 * k), acc);
+                if (k < nst) acc = mfma16<T>(a[k], *reinterpret_cast<const u32x4*>(xb + 64 * (kTight ? (st0 + k) ^ flip : k)), acc);
             }
         }
         __syncthreads();  // x is no longer read: its place takes the partial sums
@@ -246,10 +272,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
                 break;
             }
         }
-        s_fail = fail;
+        *s_fail = fail;
     }
     __syncthreads();
-    if (s_fail == 0) {
+    const int failed = __builtin_amdgcn_readfirstlane(*s_fail);
+    if constexpr (kTight) __syncthreads();
+    if (failed == 0) {
         // the chunk of the activation: [M][512] through cache-bypassing loads into LDS
         const int per_row = nst * 4;  // 16-byte items
         int t1 = tid;  // (an opaque copy: what is derived from it does not live across the wait above)
@@ -290,8 +318,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
     }
 }
 
-size_t mlp_lds_bytes(int M, int H) {
-    const size_t xb = (size_t)M * (H + 8) * 2;
+size_t mlp_lds_bytes(int M, int H, bool tight) {
+    const size_t xb = (size_t)M * (tight ? H : H + 8) * 2;
     const size_t red = (size_t)2 * kSlices * 16 * 17 * sizeof(float);
     const size_t xd = (size_t)M * kRowB;
     size_t n = xb > red ? xb : red;
@@ -332,11 +360,19 @@ int mlp_rows_launch(const void* x, long long x_row_stride, const float* o_partia
     if (bad(w_gate_up) || bad(w_down) || bad(down_partials) || bad(workspace)) return KSA_ERR_ALIGN;
     if ((w_gate_up_row_stride != kWTiled && w_gate_up_row_stride % 8) || (w_down_row_stride != kWTiled && w_down_row_stride % 8))
         return KSA_ERR_ALIGN;
-    const size_t lds = mlp_lds_bytes(M, H);
-    if (lds > 160 * 1024) return KSA_ERR_UNSUPPORTED;
+    constexpr size_t kLds = 160 * 1024;
+    if (mlp_lds_bytes(M, H, false) > kLds) return KSA_ERR_UNSUPPORTED;
+    // (more than four workgroups do not run on a CU anyway)
+    auto per_cu = [&](size_t bytes) { return bytes * 4 <= kLds ? 4 : kLds / bytes; };
+    const bool tight = per_cu(mlp_lds_bytes(M, H, true)) > per_cu(mlp_lds_bytes(M, H, false) + sizeof(int));
+    const size_t lds = mlp_lds_bytes(M, H, tight);
     const bool tiled = w_gate_up_row_stride == kWTiled && w_down_row_stride == kWTiled;
-    auto kern = dtype == KSA_DTYPE_BF16 ? (tiled ? ksa_mlp_rows_kernel<KsaBf16, true> : ksa_mlp_rows_kernel<KsaBf16, false>)
-                                        : (tiled ? ksa_mlp_rows_kernel<KsaF16, true> : ksa_mlp_rows_kernel<KsaF16, false>);
+    auto pick = [&](auto t) {
+        using T = decltype(t);
+        return tight ? (tiled ? ksa_mlp_rows_kernel<T, true, true> : ksa_mlp_rows_kernel<T, false, true>)
+                     : (tiled ? ksa_mlp_rows_kernel<T, true, false> : ksa_mlp_rows_kernel<T, false, false>);
+    };
+    auto kern = dtype == KSA_DTYPE_BF16 ? pick(KsaBf16{}) : pick(KsaF16{});
     if (lds > 64 * 1024 &&
         hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)lds) != hipSuccess)

@@ -228,6 +228,18 @@ def test_gpu_add_rmsnorm_mlp_rows_one_launch(dtype, M, H, I):
             mlp_rows(h_ref, w_gu, w_dn, ws)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,H,I", [(2, 4096, 64), (7, 2560, 96), (9, 1152, 512), (10, 4096, 512), (13, 1152, 96), (16, 128, 64),
+                                   (16, 2560, 512), (16, 4096, 512)])
+def test_gpu_mlp_rows_in_lds(dtype, M, H, I):
+    """Rows of x with and without padding in LDS (10 x 4096 and 16 x 2560 are half a CU's to the byte), whole and cut batches of the
+    rows that the norm stage hands over."""
+    test_gpu_mlp_rows_one_launch(dtype, M, H, I)
+    if H <= 1024 or H >= 2560:
+        test_gpu_add_rmsnorm_mlp_rows_one_launch(dtype, M, H, I)
+
+
 def _o_partials(M, H, dtype, dev, g):
     """The K-split partial sums of an o projection for M rows, as `linear_rows(..., defer=True)` leaves them."""
     from ksa_amd.gemm import SplitKPartials, linear_rows
