@@ -126,6 +126,16 @@ int ksa_decode_fwd(const void* q, const void* kcache, const void* vcache, void* 
                    const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
                    float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same in workgroups of eight waves of 64 rows each, one to a CU, for Q Hq / Hkv <= 16 and head_dim 64 or 128: what the
+ * Python mirror calls where no split count is named.  Results agree to the rounding of the probabilities; workspace as above.
+ * ksa_decode_wide_splits: the count to call it with, or 0 where ksa_decode_fwd is the faster one (or the only one). */
+int ksa_decode_wide_fwd(const void* q, const void* kcache, const void* vcache, void* out,
+                        const int32_t* start, const int32_t* end, int start0, int end0, int batch,
+                        int Hq, int Hkv, int Q, int D, int dtype, const int64_t* q_strides,
+                        const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                        float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
+int ksa_decode_wide_splits(int batch, int Hq, int Hkv, int Q, int D, int max_rows);
+
 /* Chunk-boundary decode step in one launch (HF:831-876, the two calls of the decode attention
  * function and the torch.cat behind them): query token 0 (the chunk's last text token) attends rows
  * [text_start, text_end), query tokens 1 .. Q - 1 (its summary tokens) attend [sum_start, sum_end),
@@ -152,6 +162,13 @@ int ksa_decode_boundary_fwd(const void* q, const void* kcache, const void* vcach
  *   16-byte aligned
  * batch <= 128, head_dim 64 or 128, Hq / Hkv <= 32, nsplit <= 64. */
 int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                       const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                       void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                       const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                       const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                       float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
+/* ... in workgroups of eight waves, as ksa_decode_wide_fwd (Hq / Hkv <= 16) */
+int ksa_decode_qkv_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
                        const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
                        void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
                        const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,

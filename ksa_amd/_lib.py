@@ -16,7 +16,7 @@ _lib = None
 # the native front of the hottest calls (csrc/ksa_fast.cpp); what it calls, in the order of its `bind`
 fast = None
 _FAST = ("ksa_block_index", "ksa_decode_splits", "ksa_decode_workspace_bytes", "ksa_decode_fwd", "ksa_prefill_chunks_fwd",
-         "ksa_pre_attention")
+         "ksa_pre_attention", "ksa_decode_wide_splits", "ksa_decode_wide_fwd")
 
 _i32p = ctypes.POINTER(ctypes.c_int32)
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -38,6 +38,11 @@ _SIGNATURES = {
     "ksa_decode_fwd": (_int, [_vp] * 6 + [_int] * 8 + [_i64p] * 4
                        + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
     "ksa_decode_qkv_fwd": (_int, [_vp, _int] + [_vp] * 4 + [ctypes.c_longlong, ctypes.c_float] + [_vp] * 4 + [_int]
+                           + [_vp] * 2 + [_int] * 7 + [_i64p] * 3 + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
+    "ksa_decode_wide_splits": (_int, [_int] * 6),
+    "ksa_decode_wide_fwd": (_int, [_vp] * 6 + [_int] * 8 + [_i64p] * 4
+                       + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
+    "ksa_decode_qkv_wide_fwd": (_int, [_vp, _int] + [_vp] * 4 + [ctypes.c_longlong, ctypes.c_float] + [_vp] * 4 + [_int]
                            + [_vp] * 2 + [_int] * 7 + [_i64p] * 3 + [ctypes.c_float, _int, _vp, ctypes.c_size_t, _vp]),
     "ksa_decode_noalloc_max_workspace_bytes": (ctypes.c_size_t, []),
     "ksa_decode_fwd_noalloc": (_int, [_vp] * 6 + [_int] * 8 + [_i64p] * 4 + [ctypes.c_float, _int, _vp]),

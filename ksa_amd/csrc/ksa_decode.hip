@@ -54,6 +54,7 @@ struct DecodeParams {
     float* ws_ml;  // [B,Hkv,nsplit,ncols_pad,2]  (max in log2 units, sum)
     int ncols_pad;
     float scale_log2;
+    int wide;      // workgroups of eight waves (ksa_decode_wide_kernel)
     // Chunk-boundary form (split_q != 0): query token 0 (the chunk's last text token) attends the rows
     // [start, end) and has column block 0 to itself (g columns); the other Q - 1 query tokens (the
     // chunk's summary tokens) attend [start2, end2) and fill the column blocks behind it.
@@ -271,6 +272,64 @@ __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int i
     }
 }
 
+// (kPre) Row `it` of a workgroup's new rows - the query heads of its group, then the key and the value row, which also go to the
+// cache - from the projection's partial sums: eight elements (lane t of D / 8).  Requested in this order: the partial sums (first
+// eight slices), the rotary row and the weight, what `then` requests - the sums are worked on while that is on its way.
+template <typename T, int D, typename Then>
+__device__ __forceinline__ u32x4 ksa_decode_new_row(const DecodeParams& p, int bz, int kvh, int it, int new_row, int t, Then then) {
+    using C = KsaCvt<T>;
+    constexpr int LPR = D / 8;
+    const int width = (p.Hq + 2 * p.Hkv) * D;
+                const int hrow = it < p.g ? kvh * p.g + it : p.Hq + (it - p.g) * p.Hkv + kvh;
+                const float* src = p.qkv + (int64_t)bz * width + (int64_t)hrow * D + 8 * t;
+                const int64_t pitch = (int64_t)p.qkv_prows * width;
+                f32x4 lo[8], hi[8];
+    #pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const float* sp = src + pitch * min(u, p.qkv_ksplit - 1);
+                    lo[u] = *reinterpret_cast<const f32x4*>(sp);
+                    hi[u] = *reinterpret_cast<const f32x4*>(sp + 4);
+                }
+                const u32x4 w = *reinterpret_cast<const u32x4*>((it < p.g ? p.wq : p.wk) + 8 * t);
+                const u32x4 cr = *reinterpret_cast<const u32x4*>(p.cos + bz * p.c_bs + 8 * t);
+                const u32x4 sr = *reinterpret_cast<const u32x4*>(p.sin + bz * p.c_bs + 8 * t);
+                then();
+                float ac[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // summed and rounded as ksa_sum_partials8
+    #pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    if (u < p.qkv_ksplit) {
+    #pragma unroll
+                        for (int i = 0; i < 4; ++i) ac[i] += lo[u][i], ac[4 + i] += hi[u][i];
+                    }
+                }
+                for (int u = 8; u < p.qkv_ksplit; ++u) {
+                    const f32x4 l4 = *reinterpret_cast<const f32x4*>(src + pitch * u);
+                    const f32x4 h4 = *reinterpret_cast<const f32x4*>(src + pitch * u + 4);
+    #pragma unroll
+                    for (int i = 0; i < 4; ++i) ac[i] += l4[i], ac[4 + i] += h4[i];
+                }
+                u32x4 raw;
+    #pragma unroll
+                for (int i = 0; i < 4; ++i) raw[i] = C::down2(ac[2 * i], ac[2 * i + 1]);
+                const uint32_t sgn = t < LPR / 2 ? 0x80008000u : 0u;
+                uint32_t wl[4], wh[4], cl[4], ch[4], sl[4], sh[4];
+    #pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    wl[i] = w[i] & 0xffffu, wh[i] = w[i] & 0xffff0000u;
+                    cl[i] = cr[i] & 0xffffu, ch[i] = cr[i] & 0xffff0000u;
+                    sl[i] = (sr[i] ^ sgn) & 0xffffu, sh[i] = (sr[i] ^ sgn) & 0xffff0000u;
+                }
+                const u32x4 z = ksa_row_scale<T>(raw, ksa_row_inv_rms<T, LPR>(raw, p.eps), wl, wh);
+                const u32x4 rot = ksa_row_rope<T, LPR>(z, cl, ch, sl, sh);
+                const u32x4 val = it == p.g + 1 ? raw : rot;  // (the value row changes its place only)
+    if (it >= p.g) {
+        uint16_t* dst = it == p.g ? p.kw + bz * p.k_bs + kvh * p.k_hs + (int64_t)new_row * p.k_rs
+                                  : p.vw + bz * p.v_bs + kvh * p.v_hs + (int64_t)new_row * p.v_rs;
+        __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst + 8 * t));
+    }
+    return val;
+}
+
 // kPre against the pre-attention launch in front, a decode step of 8 layers of the 4B shape: batch 1 665 -> 652 us,
 // batch 8 772 -> 759.  The chain of trips that it puts in front of the first scores (row and range, partial sums, LDS)
 // runs next to the loads of the first K / V tile; what it costs is that every split repeats it, and a
@@ -410,68 +469,20 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
         }
         if (row0 < s1) load_tile(row0);
     } else {
-        using C = KsaCvt<T>;
         constexpr int LPR = D / 8;      // lanes per head row
         constexpr int RPW = 64 / LPR;   // head rows per wave
         const int t = lane % LPR;
         new_row = p.row_seq ? p.row_seq[bz] : p.row0;
         if (new_row < s0 || new_row >= s1) new_row = -1;
         const int rows_here = p.g + (new_row >= 0 ? 2 : 0);  // query rows, then the key and the value row
-        const int width = (p.Hq + 2 * p.Hkv) * D;
         bool loaded = false;
         for (int i0 = wave * RPW; i0 < rows_here; i0 += kWaves * RPW) {  // (at most once for up to 14 query rows of 128)
             const int it = min(i0 + lane / LPR, rows_here - 1);          // (lanes past the last row repeat it)
-            const int hrow = it < p.g ? kvh * p.g + it : p.Hq + (it - p.g) * p.Hkv + kvh;
-            // requested in this order: the partial sums (first eight slices), the rotary row and the weight, the
-            // first K / V tile - the sums are then worked on while the tile is on its way
-            const float* src = p.qkv + (int64_t)bz * width + (int64_t)hrow * D + 8 * t;
-            const int64_t pitch = (int64_t)p.qkv_prows * width;
-            f32x4 lo[8], hi[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const float* sp = src + pitch * min(u, p.qkv_ksplit - 1);
-                lo[u] = *reinterpret_cast<const f32x4*>(sp);
-                hi[u] = *reinterpret_cast<const f32x4*>(sp + 4);
-            }
-            const u32x4 w = *reinterpret_cast<const u32x4*>((it < p.g ? p.wq : p.wk) + 8 * t);
-            const u32x4 cr = *reinterpret_cast<const u32x4*>(p.cos + bz * p.c_bs + 8 * t);
-            const u32x4 sr = *reinterpret_cast<const u32x4*>(p.sin + bz * p.c_bs + 8 * t);
-            if (!loaded && row0 < s1) load_tile(row0);
-            loaded = true;
-            float ac[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // summed and rounded as ksa_sum_partials8
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (u < p.qkv_ksplit) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) ac[i] += lo[u][i], ac[4 + i] += hi[u][i];
-                }
-            }
-            for (int u = 8; u < p.qkv_ksplit; ++u) {
-                const f32x4 l4 = *reinterpret_cast<const f32x4*>(src + pitch * u);
-                const f32x4 h4 = *reinterpret_cast<const f32x4*>(src + pitch * u + 4);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) ac[i] += l4[i], ac[4 + i] += h4[i];
-            }
-            u32x4 raw;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) raw[i] = C::down2(ac[2 * i], ac[2 * i + 1]);
-            const uint32_t sgn = t < LPR / 2 ? 0x80008000u : 0u;
-            uint32_t wl[4], wh[4], cl[4], ch[4], sl[4], sh[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                wl[i] = w[i] & 0xffffu, wh[i] = w[i] & 0xffff0000u;
-                cl[i] = cr[i] & 0xffffu, ch[i] = cr[i] & 0xffff0000u;
-                sl[i] = (sr[i] ^ sgn) & 0xffffu, sh[i] = (sr[i] ^ sgn) & 0xffff0000u;
-            }
-            const u32x4 z = ksa_row_scale<T>(raw, ksa_row_inv_rms<T, LPR>(raw, p.eps), wl, wh);
-            const u32x4 rot = ksa_row_rope<T, LPR>(z, cl, ch, sl, sh);
-            const u32x4 val = it == p.g + 1 ? raw : rot;  // (the value row changes its place only)
+            const u32x4 val = ksa_decode_new_row<T, D>(p, bz, kvh, it, new_row, t, [&]() {
+                if (!loaded && row0 < s1) load_tile(row0);
+                loaded = true;
+            });
             *reinterpret_cast<u32x4*>(s_new + (it < p.g ? it : 32 + it - p.g) * D + 8 * t) = val;
-            if (it >= p.g) {
-                uint16_t* dst = it == p.g ? p.kw + bz * p.k_bs + kvh * p.k_hs + (int64_t)new_row * p.k_rs
-                                          : p.vw + bz * p.v_bs + kvh * p.v_hs + (int64_t)new_row * p.v_rs;
-                __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst + 8 * t));
-            }
         }
         if (!loaded && row0 < s1) load_tile(row0);
         __syncthreads();
@@ -681,11 +692,241 @@ __global__ __launch_bounds__(kThreads) void ksa_decode_merge_kernel(const Decode
     }
 }
 
+// The same in workgroups of eight waves, one to a CU, for up to 16 columns (query tokens x heads of a group) at head_dim 64 and
+// 128: what a call takes that does not name a split count (ksa_decode_wide_splits).  A round of the kernel above is a chain of
+// trips - a tile's loads, LDS, scores, sums - with 64 KB on its way, and a launch of few sequences is some of them and a merge.
+// Here a wave takes 64 rows at once on 16x16x32 products: with 16 columns instead of 32 the sums take half the registers, K goes
+// from memory straight to the operand registers (64 bytes of 16 rows an instruction), V through LDS, and a round's 256 KB are
+// requested before the round in front is worked on.  What bounds it is what one CU fetches, 50 GB/s of its own and
+// 27 when all do, and the chain once per launch; the split counts follow that (ksa_decode_wide_splits).
+// Attention and merge of calls behind one another in a graph, 32 / 8 heads of 128, in the kernel above -> here, us: 1 sequence of 150 / 300 /
+// 1500 / 9000 rows 6.4 / 7.7 / 8.7 / 15.3 -> 5.6 / 7.0 / 8.7 / 13.0; 4 of 300 / 3000 9.9 / 16.7 -> 7.5 / 14.6; 8 of 1500 18.0 ->
+// 14.6; 16 of 737 / 3000 15.9 / 39.9 -> 13.3 / 35.2; 24 of 737 / 1500 / 9000 20.5 / 37.5 / 178 -> 15.7 / 26.8 / 138; 32 of 737 / 9000
+// 23.8 / 188 -> 18.4 / 179; 48 of 1100 / 9000 46.8 / 301 -> 39.6 / 264; 64 of 1100 / 9000 49.7 / 359 -> 46.7 / 348.
+// kPre as above; the new key goes to the operand registers, the new value to the tile.
+constexpr int kWideWaves = 8, kWideRows = 64, kWideColumns = 16;
+template <typename T, int D, bool kPre>
+__global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const DecodeParams p) {
+    using Ops = KsaOps<T>;
+    constexpr int KS = D / 32, DB = D / 16, NB = kWideRows / 16, NT = kWideRows / 32, CPR = D / 8;
+    constexpr int VLD = kWideRows * CPR / 64;  // V loads per lane and round
+    constexpr int VROW = D + 16;
+    constexpr int kStage = kWideRows * VROW;   // elements of one wave's V tile
+    __shared__ __attribute__((aligned(16))) uint16_t smem[kWideWaves * kStage];
+    // (kPre) the query rows of the group, then the new key and value row
+    __shared__ __attribute__((aligned(16))) uint16_t s_new[kPre ? (16 + 2) * D : 8];
+    static_assert(kWideWaves * 16 * (D + 2) * 4 <= sizeof(smem), "the merge reuses the tiles");
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, kq = lane >> 4;
+    const int split = blockIdx.x, kvh = blockIdx.y, bz = blockIdx.z;
+    const int r_first = p.start ? p.start[bz] : p.start0;
+    const int r_last = p.end ? p.end[bz] : p.end0;
+    // rows per split: whole tiles of a wave
+    const int per = ((max(r_last - r_first, 0) + p.nsplit - 1) / p.nsplit + kWideRows - 1) / kWideRows * kWideRows;
+    const int r_begin = r_first + split * per, r_end = min(r_last, r_begin + per);
+    const int last_row = max(r_end - 1, r_first);
+    const int64_t slot0 = (((int64_t)bz * p.Hkv + kvh) * p.nsplit + split) * p.ncols_pad;
+    if (p.nsplit > 1 && r_begin >= r_end) {  // an empty slice: the merge does not read its sums
+        if (tid < p.ncols) p.ws_ml[(slot0 + tid) * 2] = -INFINITY, p.ws_ml[(slot0 + tid) * 2 + 1] = 0.f;
+        return;
+    }
+    const uint16_t* kbase = p.k + bz * p.k_bs + kvh * p.k_hs + 8 * kq;
+    const uint16_t* vbase = p.v + bz * p.v_bs + kvh * p.v_hs + 8 * (lane % CPR);
+    uint16_t* Vw = smem + wave * kStage;
+
+    u32x4 kreg[NB][KS], vreg[VLD];
+    auto load_k = [&](int row0) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            // (plain loads: the other half of the line is the next instruction's)
+            const uint16_t* kp = kbase + (int64_t)min(row0 + 16 * b + r, last_row) * p.k_rs;
+#pragma unroll
+            for (int s = 0; s < KS; ++s) kreg[b][s] = *reinterpret_cast<const u32x4*>(kp + 32 * s);
+        }
+    };
+    auto load_v = [&](int row0, int i) {
+        const int row = min(row0 + (lane + 64 * i) / CPR, last_row);
+        vreg[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vbase + (int64_t)row * p.v_rs));
+    };
+    int row0 = r_begin + wave * kWideRows;
+    auto load_first = [&]() {
+        if (row0 < r_end) {
+            load_k(row0);
+#pragma unroll
+            for (int i = 0; i < VLD; ++i) load_v(row0, i);
+        }
+    };
+    int qi, gi;
+    const bool col_ok = ksa_decode_column(p, 0, r, qi, gi);
+    if (!col_ok) qi = 0, gi = 0;
+    u32x4 qf[KS];
+    int new_row = -1;  // (kPre) the new token's cache row, if it lies in this slice
+    if constexpr (!kPre) {
+        load_first();
+        const uint16_t* qp = p.q + bz * p.q_bs + (kvh * p.g + gi) * p.q_hs + qi * p.q_qs + 8 * kq;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) qf[s] = col_ok ? *reinterpret_cast<const u32x4*>(qp + 32 * s) : u32x4{0u, 0u, 0u, 0u};
+    } else {
+        new_row = p.row_seq ? p.row_seq[bz] : p.row0;
+        if (new_row < r_begin || new_row >= r_end) new_row = -1;
+        const int rows_here = p.g + (new_row >= 0 ? 2 : 0);
+        constexpr int LPR = D / 8, RPW = 64 / LPR;
+        static_assert(kWideWaves * RPW >= 18, "one pass over the rows");
+        if (wave * RPW < rows_here) {
+            const int it = min(wave * RPW + lane / LPR, rows_here - 1);
+            const u32x4 val = ksa_decode_new_row<T, D>(p, bz, kvh, it, new_row, lane % LPR, load_first);
+            *reinterpret_cast<u32x4*>(s_new + (it < p.g ? it : 16 + it - p.g) * D + 8 * (lane % LPR)) = val;
+        } else {
+            load_first();
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+            qf[s] = col_ok ? *reinterpret_cast<const u32x4*>(s_new + gi * D + 32 * s + 8 * kq) : u32x4{0u, 0u, 0u, 0u};
+    }
+
+    f32x4 oacc[DB];
+#pragma unroll
+    for (int b = 0; b < DB; ++b) oacc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_run = -INFINITY, l_run = 0.f;
+    const float c2 = p.scale_log2;
+    for (; row0 < r_end; row0 += kWideWaves * kWideRows) {
+        const int next = row0 + kWideWaves * kWideRows;
+        const bool has_next = next < r_end;
+        const int at = new_row - row0;  // (kPre) place of the new row in the tile
+        if constexpr (kPre) {
+            if (at >= 0 && at < kWideRows) {
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+#pragma unroll
+                    for (int s = 0; s < KS; ++s)
+                        if (16 * b + r == at) kreg[b][s] = *reinterpret_cast<const u32x4*>(s_new + 16 * D + 32 * s + 8 * kq);
+            }
+        }
+        f32x4 sacc[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            sacc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < KS; ++s) sacc[b] = mfma16<T>(kreg[b][s], qf[s], sacc[b]);
+        }
+        if (has_next) load_k(next);
+        ksa_wave_lds_fence();  // the reads of the round before are done
+#pragma unroll
+        for (int i = 0; i < VLD; ++i) {
+            const int u = lane + 64 * i;
+            *reinterpret_cast<u32x4*>(Vw + (u / CPR) * VROW + 8 * (u % CPR)) = vreg[i];
+            if (has_next) load_v(next, i);
+        }
+        if constexpr (kPre) {
+            // over what the cache held in its place - and, where it is the last one, over its repetitions in the rows
+            // past the end (their probabilities are 0, so they have to be finite)
+            if (at >= 0 && at < kWideRows) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(s_new + 17 * D + 8 * (lane % CPR));
+                const int end = new_row == last_row ? kWideRows : at + 1;
+                for (int j = at + lane / CPR; j < end; j += 64 / CPR) *reinterpret_cast<u32x4*>(Vw + j * VROW + 8 * (lane % CPR)) = v;
+            }
+        }
+        ksa_wave_lds_fence();
+        // lane: column r, rows 16 b + 4 kq + i of the tile
+        if (row0 + kWideRows > r_end) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (row0 + 16 * b + 4 * kq + i >= r_end) sacc[b][i] = -INFINITY;
+        }
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mloc = fmaxf(mloc, sacc[b][i]);
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
+        const float m_new = fmaxf(m_run, mloc);  // finite: every tile has at least one row
+        const float alpha = ksa_exp2((m_run - m_new) * c2), mc = m_new * c2;
+        m_run = m_new;
+        float rowsum = 0.f;
+        u32x4 pf[NT];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {
+                const float p0 = ksa_exp2(fmaf(sacc[b][i], c2, -mc)), p1 = ksa_exp2(fmaf(sacc[b][i + 1], c2, -mc));
+                rowsum += p0 + p1;
+                pf[b / 2][2 * (b % 2) + i / 2] = Ops::pack2(p0, p1);
+            }
+        l_run = l_run * alpha + rowsum;
+        if (__any(alpha != 1.f)) {
+#pragma unroll
+            for (int b = 0; b < DB; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) oacc[b][i] *= alpha;
+        }
+        // contraction element 8 kq + 4 a + j of step t is row 32 t + 16 a + 4 kq + j: what this lane holds of the probabilities
+        typedef __attribute__((address_space(3))) ksa_short4* lds_ptr;
+        const uint16_t* vp = Vw + (4 * kq + (r >> 2)) * VROW + 4 * (r & 3);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int b = 0; b < DB; ++b) {
+                const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(vp + 32 * t * VROW + 16 * b)));
+                const u32x2 hi =
+                    __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(vp + (32 * t + 16) * VROW + 16 * b)));
+                oacc[b] = mfma16<T>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pf[t], oacc[b]);
+            }
+    }
+
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+    __syncthreads();  // the tiles are dead from here on
+    float* mg = reinterpret_cast<float*>(smem);  // [wave][column 16][D + 2]
+    if (col_ok) {
+        float* row = mg + (wave * 16 + r) * (D + 2);
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) row[16 * b + 4 * kq + i] = oacc[b][i];
+        if (kq == 0) row[D] = m_run * c2, row[D + 1] = l_run;  // (log2 units; -inf of a wave without rows)
+    }
+    __syncthreads();
+    for (int e = tid; e < p.ncols * D; e += 64 * kWideWaves) {
+        const int c = e / D, d = e % D;
+        const float* row = mg + c * (D + 2);
+        float mx = -INFINITY, acc = 0.f, l = 0.f;
+#pragma unroll
+        for (int w = 0; w < kWideWaves; ++w) mx = fmaxf(mx, row[w * 16 * (D + 2) + D]);
+#pragma unroll
+        for (int w = 0; w < kWideWaves; ++w) {
+            const float m = row[w * 16 * (D + 2) + D];
+            const float f = m == -INFINITY ? 0.f : ksa_exp2(m - mx);
+            acc += row[w * 16 * (D + 2) + d] * f;
+            l += row[w * 16 * (D + 2) + D + 1] * f;
+        }
+        if (p.nsplit > 1) {
+            p.ws_o[(slot0 + c) * D + d] = acc;
+            if (d == 0) p.ws_ml[(slot0 + c) * 2] = mx, p.ws_ml[(slot0 + c) * 2 + 1] = l;
+            continue;
+        }
+        int oq, og;
+        ksa_decode_column(p, 0, c, oq, og);
+        p.out[bz * p.o_bs + oq * p.o_qs + (kvh * p.g + og) * p.o_hs + d] = (uint16_t)(Ops::pack2(l > 0.f ? acc / l : 0.f, 0.f) & 0xffffu);
+    }
+}
+
 template <typename T, int D>
 int launch(const DecodeParams& p, int batch, hipStream_t stream) {
     const int colblks = p.split_q ? 1 : p.ncols_pad / 32;  // (boundary form: a workgroup walks its column blocks)
     dim3 grid(p.nsplit, p.Hkv * colblks, batch);
-    if (p.qkv) {
+    if (p.wide) {
+        if constexpr (D <= 128) {
+            auto kern = p.qkv ? ksa_decode_wide_kernel<T, D, true> : ksa_decode_wide_kernel<T, D, false>;
+            hipLaunchKernelGGL(kern, grid, dim3(64 * kWideWaves), 0, stream, p);
+        } else {
+            return KSA_ERR_UNSUPPORTED;
+        }
+    } else if (p.qkv) {
         if constexpr (D <= 128)
             hipLaunchKernelGGL((ksa_decode_kernel<T, D, true>), grid, dim3(kThreads), 0, stream, p);
         else
@@ -829,6 +1070,39 @@ extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int m
     return n < 1 ? 1 : (int)n;
 }
 
+// Number of splits for ksa_decode_wide_fwd, or 0 where ksa_decode_fwd is the one to call: more than 16 columns, head_dim 256, and
+// more pairs of sequence and kv head than CUs over few rows, where two of its workgroups share a CU (48 / 64 sequences of
+// 8 kv heads, 150 / 300 / 500 rows 11.3 / 16.6 / 21.5 against 12.3 / 17.0 / 24.0 us, 12.3 / 19.0 / 25.3 against 13.2 / 19.2 / 25.8;
+// 737 rows 33.6 against 30.9, 35.2 against 34.2).
+// The count is the one with the least time by what was measured of one workgroup to a CU, for 1 to 64 sequences of 150 to 9000 rows:
+// 3 us for the start of each round of workgroups, 10.2 ns a row of head_dim 128 and CU when the other CUs are idle and 9.4 more when all
+// are at work, 2.4 to 4 us for the merge.  Of those shapes the count is within 4 % of the best of twelve counts but for 16
+// sequences of 1100 rows and 2 of 500.
+extern "C" int ksa_decode_wide_splits(int batch, int Hq, int Hkv, int Q, int D, int max_rows) {
+    if (batch <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || Q <= 0 || max_rows <= 0 || (D != 64 && D != 128)) return 0;
+    const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
+    if ((int64_t)Q * (Hq / Hkv) > kWideColumns || (units > cus && max_rows <= 600)) return 0;
+    const int64_t tiles = ((int64_t)max_rows + kWideRows - 1) / kWideRows;
+    int64_t most = 4 * cus / units;
+    most = most < tiles ? most : tiles;
+    most = most < 1 ? 1 : most < 64 ? most : 64;
+    const double row = D / 128.0 * 0.0102, load = D / 128.0 * 0.0094;
+    int best = 1, before = 0;
+    double least = 1e30;
+    for (int64_t n = 1; n <= most; ++n) {
+        const int64_t per = (tiles + n - 1) / n;
+        const int used = (int)((tiles + per - 1) / per);  // slices that have rows
+        if (used == before) continue;
+        before = used;
+        const int64_t wgs = units * used, full = wgs / cus, rest = wgs % cus;
+        double us = full * (3.0 + per * kWideRows * (row + load));
+        if (rest) us += 3.0 + per * kWideRows * (row + load * rest / cus);
+        if (used > 1) us += 2.4 + (full ? 1.6 : 1.6 * rest / cus);
+        if (us < least) least = us, best = used;
+    }
+    return best;
+}
+
 namespace {
 
 template <typename T>
@@ -845,7 +1119,7 @@ int decode_fwd_impl(const void* q, const void* kcache, const void* vcache, void*
                     const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
                     float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream,
                     bool boundary = false, const int32_t* start2 = nullptr, const int32_t* end2 = nullptr,
-                    int start20 = 0, int end20 = 0) {
+                    int start20 = 0, int end20 = 0, bool wide = false) {
     if (!q || !kcache || !vcache || !out || !q_strides || !k_strides || !v_strides || !out_strides)
         return KSA_ERR_NULL;
     if ((start == nullptr) != (end == nullptr)) return KSA_ERR_NULL;
@@ -879,6 +1153,8 @@ int decode_fwd_impl(const void* q, const void* kcache, const void* vcache, void*
     p.ncols = Q * p.g;
     p.ncols_pad = boundary ? pad_cols_boundary(Q, p.g) : pad_cols(p.ncols);
     p.split_q = boundary ? 1 : 0;
+    p.wide = wide;
+    if (wide && p.ncols > kWideColumns) return KSA_ERR_UNSUPPORTED;
     p.start2 = start2, p.end2 = end2, p.start20 = start20, p.end20 = end20;
     p.nsplit = nsplit;
     p.q_bs = q_strides[0], p.q_hs = q_strides[1], p.q_qs = q_strides[2];
@@ -934,6 +1210,18 @@ extern "C" int ksa_decode_fwd(const void* q, const void* kcache, const void* vca
     return decode_fwd_impl(q, kcache, vcache, out, start, end, start0, end0, batch, Hq, Hkv, Q, D, dtype,
                            q_strides, k_strides, v_strides, out_strides, scale, nsplit, workspace,
                            workspace_bytes, stream);
+}
+
+// ksa_decode_fwd in workgroups of eight waves, see ksa_decode_wide_kernel: Q Hq / Hkv <= 16, head_dim 64 or 128.
+extern "C" int ksa_decode_wide_fwd(const void* q, const void* kcache, const void* vcache, void* out, const int32_t* start,
+                                   const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int Q, int D, int dtype,
+                                   const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                                   const int64_t* out_strides, float scale, int nsplit, void* workspace, size_t workspace_bytes,
+                                   void* stream) {
+    if (D != 64 && D != 128) return KSA_ERR_UNSUPPORTED;
+    return decode_fwd_impl(q, kcache, vcache, out, start, end, start0, end0, batch, Hq, Hkv, Q, D, dtype, q_strides, k_strides,
+                           v_strides, out_strides, scale, nsplit, workspace, workspace_bytes, stream, false, nullptr, nullptr, 0, 0,
+                           true);
 }
 
 // Chunk-boundary step (HF:831-876): the chunk's last text token and its summary tokens in one launch.
@@ -1003,7 +1291,8 @@ int decode_qkv_params(DecodeParams& p, const float* qkv_partials, int qkv_ksplit
 }
 }  // namespace
 
-extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+namespace {
+int decode_qkv_impl(bool wide, const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
                                   const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
                                   void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
                                   const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
@@ -1015,6 +1304,8 @@ extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, con
                                      vcache, row, row0, start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides,
                                      v_strides, scale, nsplit, workspace);
     if (rc != KSA_OK) return rc;
+    p.wide = wide;
+    if (wide && p.ncols > kWideColumns) return KSA_ERR_UNSUPPORTED;
     p.out = (uint16_t*)out;
     p.o_bs = out_strides[0], p.o_qs = out_strides[1], p.o_hs = out_strides[2];
     if (nsplit > 1) {
@@ -1024,6 +1315,30 @@ extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, con
     }
     hipStream_t st = (hipStream_t)stream;
     return dtype == KSA_DTYPE_BF16 ? launch_head_dim<KsaBf16>(p, D, batch, st) : launch_head_dim<KsaF16>(p, D, batch, st);
+}
+}  // namespace
+
+extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                                  const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                  void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                                  const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                  const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                                  float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
+    return decode_qkv_impl(false, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache, vcache, out, row,
+                           row0, start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides, v_strides, out_strides, scale,
+                           nsplit, workspace, workspace_bytes, stream);
+}
+
+// ... in workgroups of eight waves
+extern "C" int ksa_decode_qkv_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                                  const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                  void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                                  const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                  const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                                  float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
+    return decode_qkv_impl(true, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache, vcache, out, row,
+                           row0, start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides, v_strides, out_strides, scale,
+                           nsplit, workspace, workspace_bytes, stream);
 }
 
 // ksa_decode_qkv_fwd and the o projection behind it (modeling_qwen3sa.py:879) in one launch: see ksa_decode_o_stage.

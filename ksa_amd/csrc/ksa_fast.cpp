@@ -36,6 +36,8 @@ struct Library {
     decltype(&ksa_decode_fwd) decode_fwd;
     decltype(&ksa_prefill_chunks_fwd) prefill_chunks_fwd;
     decltype(&ksa_pre_attention) pre_attention;
+    decltype(&ksa_decode_wide_splits) decode_wide_splits;
+    decltype(&ksa_decode_wide_fwd) decode_wide_fwd;
 } lib{};
 
 // Nobody records, traces, transforms or profiles (`_lib.direct`, which says why for each).  Whoever steps in front of the
@@ -138,7 +140,12 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int rc;
     {
         Unlocked u;
-        if (a[6] == Py_None) nsplit = lib.decode_splits((int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, most);
+        auto forward = lib.decode_fwd;
+        if (a[6] == Py_None) {
+            nsplit = lib.decode_wide_splits((int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, most);
+            if (nsplit > 0) forward = lib.decode_wide_fwd;
+            else nsplit = lib.decode_splits((int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, most);
+        }
         out = at::empty({b, Q, Hq, D}, q->options());
         at::Tensor ws;
         size_t ws_bytes = 0;
@@ -147,9 +154,9 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
             ws = bytes(ws_bytes, *q);
         }
         const Strides qs = first3(*q), ks = first3(*k), vs = first3(*v), os = first3(out);
-        rc = lib.decode_fwd(q->const_data_ptr(), k->const_data_ptr(), v->const_data_ptr(), out.mutable_data_ptr(), start, end, s0,
-                            e0, (int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, dt, qs.data(), ks.data(), vs.data(), os.data(), scale,
-                            nsplit, ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream_of(dev));
+        rc = forward(q->const_data_ptr(), k->const_data_ptr(), v->const_data_ptr(), out.mutable_data_ptr(), start, end, s0, e0,
+                     (int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, dt, qs.data(), ks.data(), vs.data(), os.data(), scale, nsplit,
+                     ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream_of(dev));
     }
     if (rc != 0) Py_RETURN_NONE;  // rejected in front of the launch: the general way says why
     return THPVariable_Wrap(out);
@@ -311,12 +318,14 @@ PyObject* block_index(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // bind(addresses of ksa_block_index, ksa_decode_splits, ksa_decode_workspace_bytes, ksa_decode_fwd, ksa_prefill_chunks_fwd,
-// ksa_pre_attention)
+// ksa_pre_attention, ksa_decode_wide_splits, ksa_decode_wide_fwd)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void** slots[] = {(void**)&lib.block_index, (void**)&lib.decode_splits, (void**)&lib.decode_workspace_bytes,
-                      (void**)&lib.decode_fwd, (void**)&lib.prefill_chunks_fwd, (void**)&lib.pre_attention};
-    if (n != 6) return PyErr_Format(PyExc_TypeError, "bind takes six addresses");
-    for (int i = 0; i < 6; ++i) {
+                      (void**)&lib.decode_fwd, (void**)&lib.prefill_chunks_fwd, (void**)&lib.pre_attention,
+                      (void**)&lib.decode_wide_splits, (void**)&lib.decode_wide_fwd};
+    constexpr Py_ssize_t kSlots = sizeof(slots) / sizeof(slots[0]);
+    if (n != kSlots) return PyErr_Format(PyExc_TypeError, "bind takes %zd addresses", kSlots);
+    for (Py_ssize_t i = 0; i < kSlots; ++i) {
         *slots[i] = PyLong_AsVoidPtr(a[i]);
         if (PyErr_Occurred()) return nullptr;
     }

@@ -22,7 +22,7 @@ from .prefill import fold_scale, kernel_head_dim, pad_head_dim
 _DTYPES = {torch.bfloat16: 0, torch.float16: 1}
 
 
-def _launch_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
+def _launch_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit, wide=False):
     b, Hq, Q, D = q.shape
     Hkv = kcache.shape[1]
     dev = q.device
@@ -35,7 +35,7 @@ def _launch_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     dims = (0, 1, 2)
     with _lib.on_device(dev):
-        rc = lib.ksa_decode_fwd(
+        rc = (lib.ksa_decode_wide_fwd if wide else lib.ksa_decode_fwd)(
             q.data_ptr(), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(),
             start.data_ptr() if start is not None else None,
             end.data_ptr() if end is not None else None, start0, end0,
@@ -43,8 +43,12 @@ def _launch_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
             _lib.strides3(q, dims), _lib.strides3(kcache, dims), _lib.strides3(vcache, dims), _lib.strides3(out, dims),
             scale, nsplit, ws.data_ptr() if ws is not None else None, ws_bytes, _lib.stream_ptr(dev))
     if rc:
-        _lib.check(rc, "ksa_decode_fwd")
+        _lib.check(rc, "ksa_decode_wide_fwd" if wide else "ksa_decode_fwd")
     return out
+
+
+def _launch_wide_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
+    return _launch_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit, wide=True)
 
 
 @torch.library.custom_op("ksa_amd::decode_fwd", mutates_args=())
@@ -58,6 +62,24 @@ def _decode_fwd(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
 def _(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
     b, Hq, Q, D = q.shape
     return q.new_empty((b, Q, Hq, D))
+
+
+@torch.library.custom_op("ksa_amd::wide_decode_fwd", mutates_args=())
+def _wide_decode_fwd(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
+                     start: Optional[torch.Tensor], end: Optional[torch.Tensor], start0: int, end0: int,
+                     scale: float, nsplit: int) -> torch.Tensor:
+    return _launch_wide_decode(q, kcache, vcache, start, end, start0, end0, scale, nsplit)
+
+
+@_wide_decode_fwd.register_fake
+def _(q, kcache, vcache, start, end, start0, end0, scale, nsplit):
+    b, Hq, Q, D = q.shape
+    return q.new_empty((b, Q, Hq, D))
+
+
+def _wide_splits(b, Hq, Hkv, Q, D, max_rows) -> int:
+    """Split count of a call that names none, if it takes the workgroups of eight waves (`ksa_decode_wide_fwd`); else 0."""
+    return _lib.lib().ksa_decode_wide_splits(b, Hq, Hkv, Q, D, max_rows)
 
 
 def _bound(v, default: int, b: int, device) -> torch.Tensor:
@@ -99,8 +121,14 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
     scale = float(D) ** -0.5 if scale is None else float(scale)
     if scale <= 0:
         q, scale = fold_scale(q, scale)
+    wide = False
     if nsplit is None:
-        nsplit = _lib.lib().ksa_decode_splits(b, q.shape[1], kcache.shape[1], q.shape[2], D, max_rows)
+        with _lib.on_device(q.device):
+            nsplit = _wide_splits(b, Hq, kcache.shape[1], Q, kernel_head_dim(D), max_rows)
+            wide = nsplit > 0
+            if not wide:
+                nsplit = _lib.lib().ksa_decode_splits(b, Hq, kcache.shape[1], Q, D, max_rows)
+    op = torch.ops.ksa_amd.wide_decode_fwd if wide else torch.ops.ksa_amd.decode_fwd
     Dk = kernel_head_dim(D)
     if Dk != D:
         # A head dimension without a kernel of its own (the kernels are built for 64 / 128 / 256): the
@@ -113,10 +141,11 @@ def ksa_decode(q: torch.Tensor, kcache: torch.Tensor, vcache: torch.Tensor,
         else:
             lo, hi, s0, e0 = s0, e0, 0, e0 - s0
         kcache, vcache = pad_head_dim(kcache[:, :, lo:hi], Dk), pad_head_dim(vcache[:, :, lo:hi], Dk)
-        out = torch.ops.ksa_amd.decode_fwd(pad_head_dim(q, Dk), kcache, vcache, t_start, t_end, s0, e0,
+        out = op(pad_head_dim(q, Dk), kcache, vcache, t_start, t_end, s0, e0,
                                            scale, int(nsplit))
         return out[..., :D].contiguous()
-    forward = _launch_decode if _lib.direct(q, kcache, vcache, t_start, t_end) else torch.ops.ksa_amd.decode_fwd
+    direct = _lib.direct(q, kcache, vcache, t_start, t_end)
+    forward = (_launch_wide_decode if wide else _launch_decode) if direct else op
     return forward(q, kcache, vcache, t_start, t_end, s0, e0, scale, int(nsplit))
 
 
@@ -124,9 +153,18 @@ def decode_qkv_supported(Hq: int, Hkv: int, D: int) -> bool:
     return D in (64, 128) and Hq % Hkv == 0 and Hq // Hkv <= 32
 
 
+def _qkv_splits(b: int, Hq: int, Hkv: int, D: int, max_rows: int) -> Tuple[int, bool]:
+    """(splits, whether in workgroups of eight waves) of a `ksa_decode_qkv` call that names no count, on the current GPU.  Of the
+    wide ones no more than a workgroup per CU, so that all run at once."""
+    L = _lib.lib()
+    cus = max(1, L.ksa_device_cu_count())
+    n = _wide_splits(b, Hq, Hkv, 1, D, max_rows) if b * Hkv <= cus else 0
+    return (min(n, cus // (b * Hkv)), True) if n else (L.ksa_decode_splits(b, Hq, Hkv, 1, D, max_rows), False)
+
+
 def decode_qkv_pays(kcache: torch.Tensor, Hq: int, start, end) -> bool:
     """Whether `ksa_decode_qkv` takes the place of `pre_attention_partials` and `ksa_decode`: where all its workgroups
-    run at once (two per CU).  A workgroup that starts later pays for its query rows behind the others' loads:
+    run at once (two per CU, one of the wide ones).  A workgroup that starts later pays for its query rows behind the others' loads:
     a decode step of 4 layers, 8 kv heads, separate -> one launch: 1 / 16 / 32 / 64 sequences
     402 -> 393 / 563 -> 552 / 597 -> 589 / 800 -> 774 us, but 24 (576 workgroups) 577 -> 582 and 48 (768) 684 -> 702.
     The two calls alone over 200 to 4000 rows of 1 to 32 sequences, in time of the separate launches: head_dim 64, 32 / 8 heads
@@ -137,8 +175,8 @@ def decode_qkv_pays(kcache: torch.Tensor, Hq: int, start, end) -> bool:
     L = _lib.lib()
     device = isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor)
     with _lib.on_device(kcache.device):
-        n = L.ksa_decode_splits(b, Hq, Hkv, 1, D, rows if device else max(1, int(end) - int(start)))
-        return b * Hkv * n <= 2 * max(1, L.ksa_device_cu_count())
+        n, wide = _qkv_splits(b, Hq, Hkv, D, rows if device else max(1, int(end) - int(start)))
+        return wide or b * Hkv * n <= 2 * max(1, L.ksa_device_cu_count())
 
 
 def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end, scale):
@@ -189,15 +227,16 @@ def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor
     L = _lib.lib()
     ptr = lambda t: None if t is None else t.data_ptr()
     with _lib.on_device(dev):
+        wide = False
         if nsplit is None:
-            nsplit = L.ksa_decode_splits(b, Hq, Hkv, 1, D, max_rows)
+            nsplit, wide = _qkv_splits(b, Hq, Hkv, D, max_rows)
         ws = None
         ws_bytes = L.ksa_decode_workspace_bytes(b, Hq, Hkv, 1, D, nsplit)
         if nsplit > 1:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         out = torch.empty((b, 1, Hq, D), dtype=dt, device=dev)
         dims = (0, 1, 2)
-        rc = L.ksa_decode_qkv_fwd(
+        rc = (L.ksa_decode_qkv_wide_fwd if wide else L.ksa_decode_qkv_fwd)(
             qkv.workspace.data_ptr(), qkv.ksplit, qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(),
             D if cos.shape[0] > 1 else 0, float(eps), kcache.data_ptr(), vcache.data_ptr(), out.data_ptr(), ptr(t_row), r0,
             ptr(t_start), ptr(t_end), s0, e0, b, Hq, Hkv, D, _DTYPES[dt], _lib.strides3(kcache, dims),

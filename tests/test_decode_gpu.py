@@ -501,3 +501,40 @@ def test_decode_workspace_on_a_four_byte_border(D, nsplit):
                               *strides, D ** -0.5, nsplit, ws.data_ptr() + shift, need, _lib.stream_ptr(q.device))
         assert rc == 0 and torch.equal(out, want)
         assert (ws[:shift] == 0xff).all() and (ws[shift + need:] == 0xff).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("b,Hq,Hkv,Q,rows,nsplit", [(1, 32, 8, 1, 1, 1), (2, 16, 1, 1, 63, 1), (3, 8, 8, 1, 65, 2), (2, 10, 2, 3, 512, 1),
+                                                    (1, 32, 8, 4, 513, 3), (5, 12, 4, 1, 1100, 5), (1, 4, 1, 1, 4500, 64)])
+def test_decode_wide_workgroups(dtype, D, b, Hq, Hkv, Q, rows, nsplit):
+    """Workgroups of eight waves of 64 rows: one row to several rounds, whole and cut tiles, waves and slices without rows, columns
+    up to 16, a range per sequence (an empty one among them) on strided caches, against the oracle."""
+    import ksa_amd  # noqa: F401
+    g = torch.Generator().manual_seed(rows + D)
+    q = torch.randn(b, Q, Hq, D, generator=g).to(dtype)
+    kv = torch.randn(b, rows + 3, 2 * Hkv, D, generator=g).to(dtype)
+    lo = np.array([(7 * i) % max(1, rows // 2) for i in range(b)], np.int32)
+    hi = np.array([max(lo[i] + 1, rows - 61 * i) for i in range(b)], np.int32)
+    if b == 5:
+        hi[2] = lo[2]
+    kvd = kv.cuda().transpose(1, 2)
+    k, v = kvd[:, :Hkv, :rows], kvd[:, Hkv:, :rows]
+    dev = lambda a: torch.as_tensor(a, device="cuda")
+    got = torch.ops.ksa_amd.wide_decode_fwd(q.cuda().transpose(1, 2), k, v, dev(lo), dev(hi), 0, 0, D ** -0.5, nsplit)
+    kept = np.maximum(hi, lo + 1)
+    want = c_oracle.decode(to_np(q.transpose(1, 2)), to_np(kv.transpose(1, 2)[:, :Hkv]), to_np(kv.transpose(1, 2)[:, Hkv:]), lo, kept)
+    if b == 5:
+        want[2] = 0
+    assert np.abs(to_np(got).reshape(want.shape) - want).max() <= ATOL * max(1.0, np.abs(want).max())
+
+
+def test_decode_wide_workgroups_refuse_what_they_do_not_take():
+    import ksa_amd  # noqa: F401
+    from ksa_amd import _lib
+    for Hq, D in ((17, 64), (4, 256), (4, 32)):
+        q = torch.randn(1, Hq, 1, D, device="cuda").bfloat16()
+        k = torch.randn(1, 1, 40, D, device="cuda").bfloat16()
+        assert _lib.lib().ksa_decode_wide_splits(1, Hq, 1, 1, D, 40) == 0
+        with pytest.raises(_lib.KsaError):
+            torch.ops.ksa_amd.wide_decode_fwd(q, k, k, None, None, 0, 40, 0.1, 1)
