@@ -202,6 +202,18 @@ int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* 
                          int N, void* workspace, size_t workspace_bytes, void* step_workspace,
                          size_t step_workspace_bytes, void* stream);
 
+/* ... in workgroups of eight waves, as ksa_decode_wide_fwd (Hq / Hkv <= 16).  _splits: the count to call it with, 0 where it does
+ * not take the sizes; _pays: whether it is faster than ksa_decode_qkv_wide_fwd and ksa_gemm_rows behind it. */
+int ksa_decode_qkv_o_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                         const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                         void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
+                         int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype, const int64_t* k_strides,
+                         const int64_t* v_strides, float scale, int nsplit, const void* o_weight, float* o_partials,
+                         int N, void* workspace, size_t workspace_bytes, void* step_workspace,
+                         size_t step_workspace_bytes, void* stream);
+int ksa_decode_qkv_o_wide_splits(int batch, int Hq, int Hkv, int D, int N, int max_rows);
+int ksa_decode_qkv_o_wide_pays(int batch, int Hq, int Hkv, int D, int N, int max_rows);
+
 /* ksa_decode_fwd for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
  * Same arguments and results as ksa_decode_fwd without the workspace: the split-K partials go to

@@ -90,6 +90,11 @@ _SIGNATURES = {
     "ksa_decode_qkv_o_fwd": (_int, [_vp, _int] + [_vp] * 4 + [ctypes.c_longlong, ctypes.c_float] + [_vp] * 3 + [_int]
                              + [_vp] * 2 + [_int] * 7 + [_i64p] * 2 + [ctypes.c_float, _int, _vp, _vp, _int, _vp,
                                                                        ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]),
+    "ksa_decode_qkv_o_wide_fwd": (_int, [_vp, _int] + [_vp] * 4 + [ctypes.c_longlong, ctypes.c_float] + [_vp] * 3 + [_int]
+                             + [_vp] * 2 + [_int] * 7 + [_i64p] * 2 + [ctypes.c_float, _int, _vp, _vp, _int, _vp,
+                                                                       ctypes.c_size_t, _vp, ctypes.c_size_t, _vp]),
+    "ksa_decode_qkv_o_wide_splits": (_int, [_int] * 6),
+    "ksa_decode_qkv_o_wide_pays": (_int, [_int] * 6),
     "ksa_add_rmsnorm_gemm_rows_splits": (_int, [_int] * 3),
     "ksa_add_rmsnorm_gemm_rows_pays": (_int, [_int] * 4),
     "ksa_add_rmsnorm_gemm_rows": (_int, [_vp, _int] + [_vp] * 5 + [_int] * 3 + [ctypes.c_longlong] * 2

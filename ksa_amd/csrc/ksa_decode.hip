@@ -123,19 +123,23 @@ constexpr int kRows = 32;  // key rows per wave tile
 // while the attention runs, and two ramps and a trip of the rows through memory are gone; what bounds it is the chain
 // projection sums - scores - sums - merge - product (figures at ksa_decode_qkv_o_splits).  Every workgroup merges for
 // itself, rows x splits x 2 KB of sums, 131 KB at the most (kMaxOSums), which is why it has 128 columns and not fewer.
+// In a launch of workgroups of NW = 8 waves, of which a CU holds one, a workgroup owns 256 columns: half as many of them hold
+// a CU back from the attention.
 constexpr int kMaxOSums = 64;  // rows x splits
-template <typename T, int D>
+template <typename T, int D, int NW>
 __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int idx, unsigned char* smem) {
     using Ops = KsaOps<T>;
     constexpr int HPC = kChunkK / D;   // heads of a chunk
     constexpr int kCols = 2;           // column tiles of a wave
     constexpr int kBatch = 16;         // splits requested at a time
+    constexpr int kParts = NW / 2;     // groups of 128 threads, a piece of four elements of x each
+    constexpr int kMl = (kMaxOSums * HPC + 64 * NW - 1) / (64 * NW);  // maxima and sums of a thread
     __shared__ int s_there;
     unsigned char* xs = smem;                                                    // [16][kRowB]
     float* s_m = reinterpret_cast<float*>(smem + 16 * kRowB);                    // [rows][HPC][splits]
     floatx2_ws* s_f = reinterpret_cast<floatx2_ws*>(s_m + kMaxOSums * HPC);      // factor and factor x sum
-    floatx4* s_half = reinterpret_cast<floatx4*>(s_f + kMaxOSums * HPC);         // [128] sums of the second half, their l
-    float* s_half_l = reinterpret_cast<float*>(s_half + 128);
+    floatx4* s_part = reinterpret_cast<floatx4*>(s_f + kMaxOSums * HPC);         // [kParts - 1][128] sums of the other parts, their l
+    float* s_part_l = reinterpret_cast<float*>(s_part + (kParts - 1) * 128);
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kq = lane >> 4;
@@ -144,7 +148,7 @@ __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int i
     u32x4 a[kCols][kChunkSteps];
 #pragma unroll
     for (int t = 0; t < kCols; ++t) {
-        const int tile = min(grp * (kWaves * kCols) + wave * kCols + t, tiles - 1);
+        const int tile = min(grp * (NW * kCols) + wave * kCols + t, tiles - 1);
         const char* wt = reinterpret_cast<const char*>(p.o_w) + ((int64_t)tile * steps + chunk * kChunkSteps) * 1024;
 #pragma unroll
         for (int u = 0; u < kChunkSteps; ++u)
@@ -154,24 +158,24 @@ __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int i
     // this thread's maxima and sums (row, head, split) and its piece of four elements of x
     const uint32_t slot_step = (uint32_t)p.ncols_pad, row_step = (uint32_t)(p.Hkv * ns) * slot_step;
     const int count = M * HPC * ns;
-    uint32_t ml_off[2];
+    uint32_t ml_off[kMl];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int e = min(tid + kThreads * i, count - 1);
+    for (int i = 0; i < kMl; ++i) {
+        const int e = min(tid + 64 * NW * i, count - 1);
         const int rh = e / ns, sp = e - rh * ns, hh = rh % HPC, head = chunk * HPC + hh;
         const int kvh = head / p.g;
         ml_off[i] = ((uint32_t)(rh / HPC) * row_step + (uint32_t)(kvh * ns + sp) * slot_step + (uint32_t)(head - kvh * p.g)) * 8u;
     }
-    const int piece = tid & 127, half = wave >> 1;
+    const int piece = tid & 127, part = wave >> 1;
     const int hh = 4 * piece / D, head = chunk * HPC + hh, kvh = head / p.g;
     const uint32_t o_off = (((uint32_t)(kvh * ns) * slot_step + (uint32_t)(head - kvh * p.g)) * D + (uint32_t)(4 * piece % D)) * 4u;
 
-    // The entries of a thread: rows half, half + 2, .. with all their splits one after the other; of a single row the two
-    // halves take the even and the odd splits.  Lane j holds entry j: the offset of its sums; the place of its factor and, in
+    // The entries of a thread: rows part, part + kParts, .. with all their splits one after the other; of a single row the parts take
+    // every kParts-th split.  Lane j holds entry j: the offset of its sums; the place of its factor and, in
     // the upper half behind the last split of a row, the row + 1.
     const bool one = M == 1;
-    const int n = one ? (ns - half + 1) / 2 : (M - half + 1) / 2 * ns;  // at most 64
-    const int erow = one ? 0 : half + 2 * (lane / ns), esp = one ? 2 * lane + half : lane % ns;
+    const int n = one ? (ns - part + kParts - 1) / kParts : (M - part + kParts - 1) / kParts * ns;  // at most 64
+    const int erow = one ? 0 : part + kParts * (lane / ns), esp = one ? kParts * lane + part : lane % ns;
     const uint32_t ent_off = ((uint32_t)erow * row_step + (uint32_t)esp * slot_step) * (uint32_t)(D * 4);
     const int ent = (erow * HPC * ns + esp) | (!one && esp == ns - 1 ? (erow + 1) << 16 : 0);
 
@@ -186,9 +190,9 @@ __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int i
 
     const uint32_t slots = (uint32_t)M * row_step;
     const KsaAgentBuffer so(p.ws_o, slots * D * 4u), sml(p.ws_ml, slots * 8u);
-    floatx2_ws ml[2];
+    floatx2_ws ml[kMl];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) ml[i] = __builtin_bit_cast(floatx2_ws, sml.ld2(ml_off[i]));
+    for (int i = 0; i < kMl; ++i) ml[i] = __builtin_bit_cast(floatx2_ws, sml.ld2(ml_off[i]));
     floatx4 o[kBatch];
     auto request = [&](int j0) {
 #pragma unroll
@@ -197,12 +201,12 @@ __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int i
     };
     request(0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-        if (tid + kThreads * i < count) s_m[tid + kThreads * i] = ml[i][0];
+    for (int i = 0; i < kMl; ++i)
+        if (tid + 64 * NW * i < count) s_m[tid + 64 * NW * i] = ml[i][0];
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int e = tid + kThreads * i;
+    for (int i = 0; i < kMl; ++i) {
+        const int e = tid + 64 * NW * i;
         if (e < count) {
             const int e0 = e / ns * ns;
             float mx = -INFINITY;
@@ -241,10 +245,11 @@ __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int i
         if (j0 + kBatch < n) request(j0 + kBatch);
     }
     if (one) {
-        if (half) s_half[piece] = acc, s_half_l[piece] = l;
+        if (part) s_part[(part - 1) * 128 + piece] = acc, s_part_l[(part - 1) * 128 + piece] = l;
         __syncthreads();
-        if (!half) {
-            acc += s_half[piece], l += s_half_l[piece];
+        if (!part) {
+#pragma unroll
+            for (int i = 0; i < kParts - 1; ++i) acc += s_part[i * 128 + piece], l += s_part_l[i * 128 + piece];
             x_store(0);
         }
     }
@@ -261,7 +266,7 @@ __device__ __forceinline__ void ksa_decode_o_stage(const DecodeOParams& p, int i
     }
 #pragma unroll
     for (int t = 0; t < kCols; ++t) {
-        const int tile = grp * (kWaves * kCols) + wave * kCols + t;
+        const int tile = grp * (NW * kCols) + wave * kCols + t;
         if (r < M && tile < tiles)
             *reinterpret_cast<f32x4*>(p.o_part + ((int64_t)chunk * 16 + r) * p.o_n + 16 * tile + 4 * kq) = c[t];
     }
@@ -362,7 +367,7 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
     int split = blockIdx.x, unit = blockIdx.y, bz = blockIdx.z;
     if constexpr (kO) {  // the same order in one dimension, the o projection behind it
         if ((int)blockIdx.x >= p.n_attn) {
-            ksa_decode_o_stage<T, D>(p, blockIdx.x - p.n_attn, smem);
+            ksa_decode_o_stage<T, D, kWaves>(p, blockIdx.x - p.n_attn, smem);
             return;
         }
         unit = blockIdx.x / p.nsplit;
@@ -703,11 +708,17 @@ __global__ __launch_bounds__(kThreads) void ksa_decode_merge_kernel(const Decode
 // 1500 / 9000 rows 6.4 / 7.7 / 8.7 / 15.3 -> 5.6 / 7.0 / 8.7 / 13.0; 4 of 300 / 3000 9.9 / 16.7 -> 7.5 / 14.6; 8 of 1500 18.0 ->
 // 14.6; 16 of 737 / 3000 15.9 / 39.9 -> 13.3 / 35.2; 24 of 737 / 1500 / 9000 20.5 / 37.5 / 178 -> 15.7 / 26.8 / 138; 32 of 737 / 9000
 // 23.8 / 188 -> 18.4 / 179; 48 of 1100 / 9000 46.8 / 301 -> 39.6 / 264; 64 of 1100 / 9000 49.7 / 359 -> 46.7 / 348.
-// kPre as above; the new key goes to the operand registers, the new value to the tile.
+// The probabilities enter the second product as two 16-bit parts, value and remainder: a wave's first tile of 64 rows fixes its
+// reference, where the kernel above has more of them, and a row at its reference has no rounding; with one part the output lay 1.3 %
+// further from 64 bits than the kernel above (60 shapes, up to 5 %), with two 12 % nearer (0.76 to 1.0 times), for 0.2 us a launch.
+// kPre as above; the new key goes to the operand registers, the new value to the tile.  kO as above; a decode step's attention and o
+// projection, 32 / 8 heads of 128, N 2560, in the kernel above -> here: 1 sequence of 737 / 4097 rows 15.8 / 18.2 -> 11.7 / 14.6 us, 8
+// of 737 / 4097 21.3 / 38.6 -> 16.2 / 34.9, 16 of 737 / 4097 26.4 / 61.7 -> 22.2 / 54.6.
 constexpr int kWideWaves = 8, kWideRows = 64, kWideColumns = 16;
-template <typename T, int D, bool kPre>
-__global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const DecodeParams p) {
+template <typename T, int D, bool kPre, bool kO = false>
+__global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const std::conditional_t<kO, DecodeOParams, DecodeParams> p) {
     using Ops = KsaOps<T>;
+    using C = KsaCvt<T>;
     constexpr int KS = D / 32, DB = D / 16, NB = kWideRows / 16, NT = kWideRows / 32, CPR = D / 8;
     constexpr int VLD = kWideRows * CPR / 64;  // V loads per lane and round
     constexpr int VROW = D + 16;
@@ -719,7 +730,29 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, kq = lane >> 4;
-    const int split = blockIdx.x, kvh = blockIdx.y, bz = blockIdx.z;
+    int split = blockIdx.x, kvh = blockIdx.y, bz = blockIdx.z;
+    if constexpr (kO) {
+        if ((int)blockIdx.x >= p.n_attn) {
+            ksa_decode_o_stage<T, D, kWideWaves>(p, blockIdx.x - p.n_attn, reinterpret_cast<unsigned char*>(smem));
+            return;
+        }
+        kvh = blockIdx.x / p.nsplit;
+        split = blockIdx.x - kvh * p.nsplit;
+        bz = kvh / p.Hkv;
+        kvh -= bz * p.Hkv;
+    }
+    // (kO) the sums of this workgroup have left and are counted off
+    auto arrive = [&]() {
+        if constexpr (kO) {
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();
+            if (tid == 0) add_agent(p.sync + kWordStride * (kStepHead0 + kvh), 1ull);
+        }
+    };
+    auto put = [&](float* dst, float v) {
+        if constexpr (kO) st_agent(dst, v);
+        else *dst = v;
+    };
     const int r_first = p.start ? p.start[bz] : p.start0;
     const int r_last = p.end ? p.end[bz] : p.end0;
     // rows per split: whole tiles of a wave
@@ -728,7 +761,8 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const 
     const int last_row = max(r_end - 1, r_first);
     const int64_t slot0 = (((int64_t)bz * p.Hkv + kvh) * p.nsplit + split) * p.ncols_pad;
     if (p.nsplit > 1 && r_begin >= r_end) {  // an empty slice: the merge does not read its sums
-        if (tid < p.ncols) p.ws_ml[(slot0 + tid) * 2] = -INFINITY, p.ws_ml[(slot0 + tid) * 2 + 1] = 0.f;
+        if (tid < p.ncols) put(p.ws_ml + (slot0 + tid) * 2, -INFINITY), put(p.ws_ml + (slot0 + tid) * 2 + 1, 0.f);
+        arrive();
         return;
     }
     const uint16_t* kbase = p.k + bz * p.k_bs + kvh * p.k_hs + 8 * kq;
@@ -848,14 +882,16 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const 
         const float alpha = ksa_exp2((m_run - m_new) * c2), mc = m_new * c2;
         m_run = m_new;
         float rowsum = 0.f;
-        u32x4 pf[NT];
+        u32x4 pf[NT], pl[NT];  // the probabilities in 16 bits, and what that leaves of them
 #pragma unroll
         for (int b = 0; b < NB; ++b)
 #pragma unroll
             for (int i = 0; i < 4; i += 2) {
                 const float p0 = ksa_exp2(fmaf(sacc[b][i], c2, -mc)), p1 = ksa_exp2(fmaf(sacc[b][i + 1], c2, -mc));
                 rowsum += p0 + p1;
-                pf[b / 2][2 * (b % 2) + i / 2] = Ops::pack2(p0, p1);
+                const uint32_t pk = Ops::pack2(p0, p1);
+                pf[b / 2][2 * (b % 2) + i / 2] = pk;
+                pl[b / 2][2 * (b % 2) + i / 2] = Ops::pack2(p0 - C::lo(pk), p1 - C::hi(pk));
             }
         l_run = l_run * alpha + rowsum;
         if (__any(alpha != 1.f)) {
@@ -874,7 +910,9 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const 
                 const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(vp + 32 * t * VROW + 16 * b)));
                 const u32x2 hi =
                     __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(vp + (32 * t + 16) * VROW + 16 * b)));
-                oacc[b] = mfma16<T>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pf[t], oacc[b]);
+                const u32x4 a = {lo[0], lo[1], hi[0], hi[1]};
+                oacc[b] = mfma16<T>(a, pf[t], oacc[b]);
+                oacc[b] = mfma16<T>(a, pl[t], oacc[b]);
             }
     }
 
@@ -904,15 +942,16 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const 
             acc += row[w * 16 * (D + 2) + d] * f;
             l += row[w * 16 * (D + 2) + D + 1] * f;
         }
-        if (p.nsplit > 1) {
-            p.ws_o[(slot0 + c) * D + d] = acc;
-            if (d == 0) p.ws_ml[(slot0 + c) * 2] = mx, p.ws_ml[(slot0 + c) * 2 + 1] = l;
+        if (kO || p.nsplit > 1) {
+            put(p.ws_o + (slot0 + c) * D + d, acc);
+            if (d == 0) put(p.ws_ml + (slot0 + c) * 2, mx), put(p.ws_ml + (slot0 + c) * 2 + 1, l);
             continue;
         }
         int oq, og;
         ksa_decode_column(p, 0, c, oq, og);
         p.out[bz * p.o_bs + oq * p.o_qs + (kvh * p.g + og) * p.o_hs + d] = (uint16_t)(Ops::pack2(l > 0.f ? acc / l : 0.f, 0.f) & 0xffffu);
     }
+    arrive();
 }
 
 template <typename T, int D>
@@ -1388,7 +1427,11 @@ extern "C" int ksa_decode_qkv_o_pays(int batch, int Hq, int Hkv, int D, int N, i
     return product <= 2 * cus && batch * Hkv >= (Hq >= 24 ? 64 : 96) && max_rows >= 1400 && sums <= 32;
 }
 
-extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+namespace {
+// workgroups of the o projection in a launch of workgroups of so many waves
+int o_workgroups(int N, int chunks, int waves) { return (N / 16 + 2 * waves - 1) / (2 * waves) * chunks; }
+
+int decode_qkv_o_impl(bool wide, const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
                                     const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
                                     void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
                                     int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
@@ -1398,12 +1441,13 @@ extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, c
     if (!o_weight || !o_partials || !workspace || !step_workspace) return KSA_ERR_NULL;
     if (N <= 0) return KSA_ERR_INVALID;
     DecodeOParams p{};
+    p.wide = wide;
     const int rc = decode_qkv_params(p, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache,
                                      vcache, row, row0, start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides,
                                      v_strides, scale, nsplit, workspace);
     if (rc != KSA_OK) return rc;
     if (batch > 16 || batch * nsplit > kMaxOSums || Hkv > kStepMaxHeads || Hq * D % kChunkK != 0 || Hq * D > 64 * kChunkK ||
-        N % 16 != 0)
+        N % 16 != 0 || (wide && p.ncols > kWideColumns))
         return KSA_ERR_UNSUPPORTED;
     for (const void* ptr : {o_weight, (const void*)o_partials, (const void*)step_workspace})
         if (reinterpret_cast<uintptr_t>(ptr) & 15) return KSA_ERR_ALIGN;
@@ -1415,16 +1459,92 @@ extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, c
     p.sync = (unsigned long long*)step_workspace;
     p.batch = batch, p.n_attn = batch * Hkv * nsplit;
     p.o_n = N, p.o_chunks = Hq * D / kChunkK;
-    p.o_wgs = (N / 16 + 2 * kWaves - 1) / (2 * kWaves) * p.o_chunks;
+    const int waves = wide ? kWideWaves : kWaves;
+    p.o_wgs = o_workgroups(N, p.o_chunks, waves);
     p.spin_limit = 1u << 19;  // polls of a microsecond or two: about a second
-    const dim3 grid(p.n_attn + p.o_wgs), block(kThreads);
+    const dim3 grid(p.n_attn + p.o_wgs), block(64 * waves);
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, block, 0, (hipStream_t)stream, p);
         return ksa_check_launch();
     };
+    if (wide) {
+        if (dtype == KSA_DTYPE_BF16)
+            return D == 128 ? go(ksa_decode_wide_kernel<KsaBf16, 128, true, true>) : go(ksa_decode_wide_kernel<KsaBf16, 64, true, true>);
+        return D == 128 ? go(ksa_decode_wide_kernel<KsaF16, 128, true, true>) : go(ksa_decode_wide_kernel<KsaF16, 64, true, true>);
+    }
     if (dtype == KSA_DTYPE_BF16)
         return D == 128 ? go(ksa_decode_kernel<KsaBf16, 128, true, true>) : go(ksa_decode_kernel<KsaBf16, 64, true, true>);
     return D == 128 ? go(ksa_decode_kernel<KsaF16, 128, true, true>) : go(ksa_decode_kernel<KsaF16, 64, true, true>);
+}
+}  // namespace
+
+extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                                    const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                    void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
+                                    int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                    const int64_t* k_strides, const int64_t* v_strides, float scale, int nsplit,
+                                    const void* o_weight, float* o_partials, int N, void* workspace, size_t workspace_bytes,
+                                    void* step_workspace, size_t step_workspace_bytes, void* stream) {
+    return decode_qkv_o_impl(false, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache, vcache, row, row0,
+                             start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides, v_strides, scale, nsplit, o_weight,
+                             o_partials, N, workspace, workspace_bytes, step_workspace, step_workspace_bytes, stream);
+}
+
+// ... in workgroups of eight waves
+extern "C" int ksa_decode_qkv_o_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
+                                    const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                    void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
+                                    int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                    const int64_t* k_strides, const int64_t* v_strides, float scale, int nsplit,
+                                    const void* o_weight, float* o_partials, int N, void* workspace, size_t workspace_bytes,
+                                    void* step_workspace, size_t step_workspace_bytes, void* stream) {
+    return decode_qkv_o_impl(true, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache, vcache, row, row0,
+                             start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides, v_strides, scale, nsplit, o_weight,
+                             o_partials, N, workspace, workspace_bytes, step_workspace, step_workspace_bytes, stream);
+}
+
+// Splits of ksa_decode_qkv_o_wide_fwd, or 0 where it does not take the call.  The terms of ksa_decode_wide_splits without rounds (one
+// workgroup to a CU), 30 ns for every row and split that a workgroup of the product merges, and 4 us more where the product's
+// workgroups have to wait for a CU: 32 / 8 heads of 128, N 2560, 8 sequences of 737 / 1100 / 4097 rows in 2 / 4 splits 16.2 / 19.2 / 38.7
+// and 19.2 / 20.5 / 34.9 us (176 CUs are left to the attention, 64 slices a split).
+extern "C" int ksa_decode_qkv_o_wide_splits(int batch, int Hq, int Hkv, int D, int N, int max_rows) {
+    if (batch <= 0 || batch > 16 || Hkv <= 0 || Hkv > kStepMaxHeads || Hq <= 0 || Hq % Hkv != 0 || Hq / Hkv > kWideColumns || N <= 0 ||
+        N % 16 != 0 || max_rows <= 0 || (D != 64 && D != 128) || Hq * D % kChunkK != 0 || Hq * D > 64 * kChunkK)
+        return 0;
+    const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
+    const int64_t room = cus - o_workgroups(N, Hq * D / kChunkK, kWideWaves);
+    const int64_t tiles = ((int64_t)max_rows + kWideRows - 1) / kWideRows;
+    int64_t most = cus / units;
+    most = most < kMaxOSums / batch ? most : kMaxOSums / batch;
+    most = most < tiles ? most : tiles;
+    const double row = D / 128.0 * 0.0102, load = D / 128.0 * 0.0094;
+    int best = 0, before = 0;
+    double least = 1e30;
+    for (int64_t n = 1; n <= most; ++n) {
+        const int64_t per = (tiles + n - 1) / n;
+        const int used = (int)((tiles + per - 1) / per);
+        if (used == before) continue;
+        before = used;
+        const double us = per * kWideRows * (row + load * (double)(units * used) / cus) + 0.03 * batch * used +
+                          (units * used > room ? 4.0 : 0.0);
+        if (us < least) least = us, best = used;
+    }
+    return best;
+}
+
+// Whether ksa_decode_qkv_o_wide_fwd is faster than ksa_decode_qkv_wide_fwd and ksa_gemm_rows behind it: 499 shapes timed (17 of heads, head_dim
+// and N, 1 to 16 sequences of 300 to 16384 rows; graphs), 360 taken, 0.89 of the two launches on average, 1.05 at the worst.
+// Left to the two: a product of more workgroups than CUs (64 heads, N 5120 up to 1.20); few kv heads over long ranges (16 / 2
+// heads, 4097 rows and more up to 1.19), whose count the sums limit; half a CU's worth of slices and more of few heads (16 / 8,
+// 16 x 300 rows 1.06) or of any (32 / 32, 8 x 300 1.15); at head_dim 64 few rows (1.05 to 1.15), many slices (1.1 to 1.46) and
+// long ranges (1.01 to 1.09).
+extern "C" int ksa_decode_qkv_o_wide_pays(int batch, int Hq, int Hkv, int D, int N, int max_rows) {
+    if (ksa_decode_qkv_o_wide_splits(batch, Hq, Hkv, D, N, max_rows) == 0) return 0;
+    const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
+    if (o_workgroups(N, Hq * D / kChunkK, kWideWaves) > cus) return 0;
+    if (Hkv < 4 && (Hq * D < 4096 || max_rows > 2048)) return 0;
+    if (D == 128) return 2 * units < cus || (2 * units == cus && Hq * D >= 4096);
+    return 8 * units <= 3 * cus && max_rows >= 600 && max_rows <= 8192;
 }
 
 extern "C" size_t ksa_decode_noalloc_max_workspace_bytes(void) { return kNoAllocScratchBytes; }

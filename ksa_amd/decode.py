@@ -214,12 +214,13 @@ def _qkv_arguments(qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, 
 
 def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                    eps: float, kcache: torch.Tensor, vcache: torch.Tensor, Hq: int, row, start, end,
-                   scale: Optional[float] = None, nsplit: Optional[int] = None) -> torch.Tensor:
+                   scale: Optional[float] = None, nsplit: Optional[int] = None, wide: bool = False) -> torch.Tensor:
     """`pre_attention_partials` + `ksa_decode` of one new token per sequence in one launch (`ksa_decode_qkv_fwd`).
 
     qkv: the deferred q | k | v projection (`SplitKPartials` [b, 1, (Hq + 2 Hkv) D]); cos / sin [1 or b, 1, D].  The
     token's key and value go to `row` of the caches and are attended with the rest of [start, end), which has
-    to hold that row (each an int, or an int32 GPU tensor [b]).  Returns [b, 1, Hq D]."""
+    to hold that row (each an int, or an int32 GPU tensor [b]).  `wide`: a named count of splits is one of workgroups of eight
+    waves (`ksa_decode_qkv_wide_fwd`).  Returns [b, 1, Hq D]."""
     cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows, scale = _qkv_arguments(
         qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end, scale)
     b, Hkv, _, D = kcache.shape
@@ -227,7 +228,6 @@ def ksa_decode_qkv(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor
     L = _lib.lib()
     ptr = lambda t: None if t is None else t.data_ptr()
     with _lib.on_device(dev):
-        wide = False
         if nsplit is None:
             nsplit, wide = _qkv_splits(b, Hq, Hkv, D, max_rows)
         ws = None
@@ -253,21 +253,22 @@ def decode_qkv_o_supported(kcache: torch.Tensor, Hq: int, N: int) -> bool:
 
 
 def decode_qkv_o_pays(kcache: torch.Tensor, Hq: int, N: int, start, end) -> bool:
-    """Whether `ksa_decode_qkv_o` is the faster way (`ksa_decode_qkv_o_pays`, by the longest possible range where the ranges
-    are on the device)."""
+    """Whether `ksa_decode_qkv_o` is the faster way (`ksa_decode_qkv_o_wide_pays`, for groups of more than 16 heads, which the wide
+    form does not take, `ksa_decode_qkv_o_pays`; by the longest possible range where the ranges are on the device)."""
     b, Hkv, rows, D = kcache.shape
     if not (isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor)):
         rows = max(1, int(end) - int(start))
     with _lib.on_device(kcache.device):
-        return _lib.lib().ksa_decode_qkv_o_pays(b, Hq, Hkv, D, N, rows) != 0
+        L = _lib.lib()
+        return (L.ksa_decode_qkv_o_wide_pays if Hq // Hkv <= 16 else L.ksa_decode_qkv_o_pays)(b, Hq, Hkv, D, N, rows) != 0
 
 
 def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                      eps: float, kcache: torch.Tensor, vcache: torch.Tensor, Hq: int, row, start, end, o_weight, ws,
-                     scale: Optional[float] = None, nsplit: Optional[int] = None):
+                     scale: Optional[float] = None, nsplit: Optional[int] = None, wide: bool = False):
     """`ksa_decode_qkv` and the o projection behind it (modeling_qwen3sa.py:879) in one launch
     (`ksa_decode_qkv_o_fwd`), for at most 16 sequences: o_weight a `gemm.TiledWeight` [N, Hq D], ws the step's
-    `gemm.MlpRowsWorkspace`.  Returns the product's `SplitKPartials` [b, 1, N]."""
+    `gemm.MlpRowsWorkspace`.  `wide`: in workgroups of eight waves where they take the call (`ksa_decode_qkv_o_wide_fwd`).  Returns the product's `SplitKPartials` [b, 1, N]."""
     from .gemm import SplitKPartials, TiledWeight
     cos, sin, qw, kw, t_row, r0, t_start, t_end, s0, e0, max_rows, scale = _qkv_arguments(
         qkv, q_norm_weight, k_norm_weight, cos, sin, kcache, vcache, Hq, row, start, end, scale)
@@ -278,6 +279,9 @@ def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tens
     L = _lib.lib()
     ptr = lambda t: None if t is None else t.data_ptr()
     with _lib.on_device(dev):
+        if nsplit is None and wide:
+            nsplit = L.ksa_decode_qkv_o_wide_splits(b, Hq, Hkv, D, N, max_rows) or None
+            wide = nsplit is not None
         if nsplit is None:
             nsplit = L.ksa_decode_qkv_o_splits(b, Hq, Hkv, D, max_rows)
         ws_bytes = L.ksa_decode_qkv_o_workspace_bytes(b, Hq, Hkv, D, nsplit)
@@ -285,7 +289,7 @@ def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tens
         ks = Hq * D // 512
         part = torch.empty(ks * 16 * N, dtype=torch.float32, device=dev)
         dims = (0, 1, 2)
-        rc = L.ksa_decode_qkv_o_fwd(
+        rc = (L.ksa_decode_qkv_o_wide_fwd if wide else L.ksa_decode_qkv_o_fwd)(
             qkv.workspace.data_ptr(), qkv.ksplit, qw.data_ptr(), kw.data_ptr(), cos.data_ptr(), sin.data_ptr(),
             D if cos.shape[0] > 1 else 0, float(eps), kcache.data_ptr(), vcache.data_ptr(), ptr(t_row), r0,
             ptr(t_start), ptr(t_end), s0, e0, b, Hq, Hkv, D, _DTYPES[dt], _lib.strides3(kcache, dims),

@@ -251,7 +251,7 @@ class HipOps:
         if not isinstance(tiled, self._gemm.TiledWeight):
             return None
         return self._decode_mod.ksa_decode_qkv_o(qkv, q_norm, k_norm, cos, sin, eps, kbuf, vbuf, Hq, row, start, end,
-                                                 tiled, ws, scale=scale)
+                                                 tiled, ws, scale=scale, wide=True)
 
     def argmax(self, logits):
         """Greedy token choice over the last dimension (lowest index among equal values)."""

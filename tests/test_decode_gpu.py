@@ -538,3 +538,75 @@ def test_decode_wide_workgroups_refuse_what_they_do_not_take():
         assert _lib.lib().ksa_decode_wide_splits(1, Hq, 1, 1, D, 40) == 0
         with pytest.raises(_lib.KsaError):
             torch.ops.ksa_amd.wide_decode_fwd(q, k, k, None, None, 0, 40, 0.1, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,Hq,Hkv,D,N,nsplit", [
+    (1, 32, 8, 128, 2560, None), (1, 32, 8, 128, 256, 1), (1, 16, 2, 128, 144, 39), (1, 8, 4, 64, 16, 64), (1, 64, 4, 64, 272, 2),
+    (2, 32, 8, 128, 272, 32), (3, 8, 8, 64, 128, 21), (5, 4, 2, 128, 512, 7), (7, 16, 1, 128, 528, 3), (16, 32, 8, 128, 1024, 4),
+    (16, 32, 8, 128, 2560, None),
+])
+def test_decode_qkv_o_wide_equals_separate_launches(dtype, b, Hq, Hkv, D, N, nsplit):
+    """The wide form of a step's attention, alone and with the o projection in the launch, with ranges from one row to all (later
+    slices empty) and new rows at every place of a tile, several launches on one workspace.  Attention: against the decode call on
+    the rows of the pre-attention step, both in wide workgroups and bit for bit; with the o projection: the splits are merged in
+    another order, bounds as for the four-wave form."""
+    from ksa_amd import decode, gemm, pre
+    import ksa_amd._lib as _lib
+    rows = 4100 if nsplit is None or nsplit > 16 else 1100
+    n = nsplit or _lib.lib().ksa_decode_qkv_o_wide_splits(b, Hq, Hkv, D, N, rows)
+    assert n > 0
+    g = torch.Generator(device="cuda").manual_seed(b * 10 + N)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    H, width, K = 1536, (Hq + 2 * Hkv) * D, Hq * D
+    wo = (rnd(N, K) * K ** -0.5).to(dtype)
+    tiled, ws = gemm.TiledWeight(wo), gemm.MlpRowsWorkspace(N, 64, torch.device("cuda"))
+    qw, kw = (1 + 0.1 * rnd(D)).to(dtype), (1 + 0.1 * rnd(D)).to(dtype)
+    ang = rnd(b, 1, D // 2)
+    ang = torch.cat((ang, ang), -1)
+    cos, sin = ang.cos().to(dtype), ang.sin().to(dtype)
+    w = (rnd(width, H) * H ** -0.5).to(dtype)
+    forms = [(0, rows, rows - 1), (7, 1031, 7), (128, 129, 128), (3, 40, 20), (0, 300, 127), (1, 1000, 64 * 9 + 1)]
+    dev = lambda v: torch.as_tensor(v, device="cuda", dtype=torch.int32)
+    for rep in range(3):
+        lo, hi, row = (dev([forms[(i + 2 * rep) % len(forms)][j] for i in range(b)]) for j in range(3))
+        qkv = gemm.linear_rows(rnd(b, 1, H).to(dtype), w, defer=True)
+        kc, vc = (rnd(b, Hkv, rows, D).to(dtype) for _ in range(2))
+        for i in range(b):                             # what the new rows overwrite must not be read
+            kc[i, :, row[i]] = vc[i, :, row[i]] = float("nan")
+        kr, vr = kc.clone(), vc.clone()
+        ko, vo = kc.clone(), vc.clone()
+        q, _, _ = pre.pre_attention_partials(qkv, Hq, Hkv, D, qw, kw, cos, sin, 1e-6, k_out=kr[:, :, :1].transpose(1, 2),
+                                             v_out=vr[:, :, :1].transpose(1, 2), kv_out_row=row)
+        want = torch.ops.ksa_amd.wide_decode_fwd(q.transpose(1, 2), kr, vr, lo, hi, 0, 0, D ** -0.5, n)
+        attn = decode.ksa_decode_qkv(qkv, qw, kw, cos, sin, 1e-6, kc, vc, Hq, row, lo, hi, nsplit=n, wide=True)
+        assert torch.equal(attn, want.reshape(b, 1, K)) and torch.equal(kc, kr) and torch.equal(vc, vr)
+        got = decode.ksa_decode_qkv_o(qkv, qw, kw, cos, sin, 1e-6, ko, vo, Hq, row, lo, hi, tiled, ws, nsplit=nsplit, wide=True)
+        torch.cuda.synchronize()
+        assert not ws.failed() and int(ws.step.view(torch.int64).abs().sum().item()) == 0
+        assert torch.equal(ko, kr) and torch.equal(vo, vr)
+        got = got.workspace.view(torch.float32).view(K // 512, 16, N)[:, :b].sum(0)
+        want = attn.view(b, K).double() @ wo.double().t()
+        ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+        term = (attn.view(b, K).double().square() @ wo.double().t().square() / K).sqrt()
+        assert ((got - want).abs() <= 2 * ulp * K ** 0.5 * term + 1e-5 * want.abs().max()).all()
+        assert (got - want).square().mean() <= (0.25 * ulp) ** 2 * (K * term.square()).mean()
+
+
+def test_decode_qkv_o_wide_bounded_wait_gives_up_and_recovers():
+    """As for the four-wave form: counts set far off from the host, every wait ends, the cleared words serve the next launch."""
+    from ksa_amd import decode, gemm
+    g = torch.Generator(device="cuda").manual_seed(9)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").bfloat16()
+    qkv = gemm.linear_rows(rnd(2, 1, 1024), rnd(8 * 128, 1024), defer=True)
+    kc, vc, tiled = rnd(2, 2, 300, 128), rnd(2, 2, 300, 128), gemm.TiledWeight(rnd(256, 512))
+    one, ws = torch.ones(128, device="cuda").bfloat16(), gemm.MlpRowsWorkspace(256, 64, torch.device("cuda"))
+    call = lambda w: decode.ksa_decode_qkv_o(qkv, one, one, one, one, 1e-6, kc, vc, 4, 5, 0, 300, tiled, w, nsplit=2, wide=True)
+    ws.step.view(torch.int64)[4 * 64::64] = -(1 << 40)
+    torch.cuda.synchronize()
+    call(ws)
+    assert ws.failed() and not ws.failed()
+    assert int(ws.step.view(torch.int64).abs().sum().item()) == 0
+    a, b = call(ws), call(gemm.MlpRowsWorkspace(256, 64, torch.device("cuda")))
+    assert not ws.failed()
+    assert torch.equal(*(t.workspace.view(torch.float32).view(1, 16, 256)[:, :2] for t in (a, b)))
