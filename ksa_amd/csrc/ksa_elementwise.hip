@@ -43,6 +43,10 @@ struct EmbedParams : NormParams {
 // One wave per row; the row (after the residual add) stays in registers between the
 // sum-of-squares pass and the scaling pass.  NI = 16-byte items per lane.  Inputs are read once:
 // non-temporal loads.
+// What bounds it is HBM for many rows, the one trip to memory for few; all items of a row and its residual are on their way
+// before the first is used.  (One item after the other, each under its own condition, made a chain of NI trips of it: 2560 x
+// 100 / 740 / 6368 / 34816 rows behind one another in a graph 7.3 / 10.0 / 30.0 / 140 -> 4.7 / 6.8 / 26.7 / 136 us, 5.3 TB/s; 5120 x 100 /
+// 6368 16.2 / 59.3 -> 7.1 / 48.2, 8192 24.6 / 91.5 -> 9.9 / 74.7.)
 // kEmbed: the head of a decode step - embedding rows, their norm for the first layer, the step's rotary row - whose
 // cost is its launches (4.5 us each behind one another, for some 10 KB): as one, and with the ids read where the
 // caller has them, a decode step of 8 layers went from 649 to 643 us (batch 1) and from 759 to 754 (batch 8).
@@ -60,7 +64,7 @@ __global__ __launch_bounds__(256) void ksa_add_rmsnorm_kernel(const std::conditi
         }
     }
     for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < p.rows; row += (int64_t)gridDim.x * 4) {
-        u32x4 r[NI];
+        u32x4 r[NI], q[kEmbed ? 1 : NI];
         float ss = 0.f;
         int64_t src = row;
         bool inside = true;
@@ -71,18 +75,29 @@ __global__ __launch_bounds__(256) void ksa_add_rmsnorm_kernel(const std::conditi
             if (!inside) src = 0;
         }
 #pragma unroll
+        for (int j = 0; j < NI; ++j) {  // (lanes past the row's end repeat its last item)
+            const int idx = min(lane + 64 * j, items - 1);
+            r[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.x + src * p.xs + 8 * idx));
+        }
+        if constexpr (!kEmbed) {
+            if (p.res) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j)
+                    q[j] = __builtin_nontemporal_load(
+                        reinterpret_cast<const u32x4*>(p.res + row * p.rs + 8 * min(lane + 64 * j, items - 1)));
+            }
+        }
+#pragma unroll
         for (int j = 0; j < NI; ++j) {
             const int idx = lane + 64 * j;
             if (idx < items) {
-                r[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.x + src * p.xs + 8 * idx));
                 if constexpr (kEmbed) {
                     if (!inside) r[j] = u32x4{0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};
                     *reinterpret_cast<u32x4*>(p.out_sum + row * p.ss + 8 * idx) = r[j];
                 } else if (p.res) {
-                    const u32x4 q = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.res + row * p.rs + 8 * idx));
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        r[j][i] = C::down2(C::lo(r[j][i]) + C::lo(q[i]), C::hi(r[j][i]) + C::hi(q[i]));
+                        r[j][i] = C::down2(C::lo(r[j][i]) + C::lo(q[j][i]), C::hi(r[j][i]) + C::hi(q[j][i]));
                     *reinterpret_cast<u32x4*>(p.out_sum + row * p.ss + 8 * idx) = r[j];
                 }
 #pragma unroll
@@ -214,6 +229,7 @@ int dispatch_norm(const P& p, hipStream_t st) {
     if (need <= 1) return launch_norm<T, 1>(p, st);
     if (need <= 2) return launch_norm<T, 2>(p, st);
     if (need <= 4) return launch_norm<T, 4>(p, st);
+    if (need <= 5) return launch_norm<T, 5>(p, st);
     if (need <= 8) return launch_norm<T, 8>(p, st);
     if (need <= 16) return launch_norm<T, 16>(p, st);
     return KSA_ERR_UNSUPPORTED;

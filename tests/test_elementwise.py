@@ -71,6 +71,30 @@ def test_gpu_add_rmsnorm(dtype, rows, H, with_res):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H", [8, 512, 520, 2048, 2056, 2552, 2560, 2568, 4104, 8192])
+def test_gpu_add_rmsnorm_row_lengths_in_place(dtype, H):
+    """The items of a row are requested together, lanes past its end its last one: lengths around every count of items per
+    lane, the sum written over the residual."""
+    from ksa_amd import _lib
+    rows = 5
+    g = torch.Generator().manual_seed(H)
+    x = (torch.randn(rows, H, generator=g) * 1.5).to(dtype)
+    r = torch.randn(rows, H, generator=g).to(dtype)
+    w = (1 + 0.1 * torch.randn(H, generator=g)).to(dtype)
+    s_exp, y_exp = cpu_path.add_rmsnorm(x, r, w, 1e-6)
+    buf = torch.full((rows + 1, H), 3.0, dtype=dtype, device="cuda")
+    buf[:rows] = r
+    y = torch.full((rows + 1, H), 3.0, dtype=dtype, device="cuda")
+    xd, wd = x.cuda(), w.cuda()
+    _lib.check(_lib.lib().ksa_add_rmsnorm(xd.data_ptr(), buf.data_ptr(), wd.data_ptr(), y.data_ptr(), buf.data_ptr(), rows, H, H, H,
+                                          H, H, 0 if dtype == torch.bfloat16 else 1, 1e-6, _lib.stream_ptr(xd.device)), "add_rmsnorm")
+    assert torch.equal(buf[:rows].cpu(), s_exp)
+    assert bool((buf[rows] == 3.0).all()) and bool((y[rows] == 3.0).all())
+    _ulp_check(y[:rows], y_exp, 5e-3)
+
+
+@pytest.mark.gpu
 def test_gpu_add_rmsnorm_strided_rows_and_errors():
     from ksa_amd import KsaError
     from ksa_amd.elementwise import add_rmsnorm
