@@ -285,48 +285,48 @@ __device__ __forceinline__ u32x4 ksa_decode_new_row(const DecodeParams& p, int b
     using C = KsaCvt<T>;
     constexpr int LPR = D / 8;
     const int width = (p.Hq + 2 * p.Hkv) * D;
-                const int hrow = it < p.g ? kvh * p.g + it : p.Hq + (it - p.g) * p.Hkv + kvh;
-                const float* src = p.qkv + (int64_t)bz * width + (int64_t)hrow * D + 8 * t;
-                const int64_t pitch = (int64_t)p.qkv_prows * width;
-                f32x4 lo[8], hi[8];
-    #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const float* sp = src + pitch * min(u, p.qkv_ksplit - 1);
-                    lo[u] = *reinterpret_cast<const f32x4*>(sp);
-                    hi[u] = *reinterpret_cast<const f32x4*>(sp + 4);
-                }
-                const u32x4 w = *reinterpret_cast<const u32x4*>((it < p.g ? p.wq : p.wk) + 8 * t);
-                const u32x4 cr = *reinterpret_cast<const u32x4*>(p.cos + bz * p.c_bs + 8 * t);
-                const u32x4 sr = *reinterpret_cast<const u32x4*>(p.sin + bz * p.c_bs + 8 * t);
-                then();
-                float ac[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // summed and rounded as ksa_sum_partials8
-    #pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    if (u < p.qkv_ksplit) {
-    #pragma unroll
-                        for (int i = 0; i < 4; ++i) ac[i] += lo[u][i], ac[4 + i] += hi[u][i];
-                    }
-                }
-                for (int u = 8; u < p.qkv_ksplit; ++u) {
-                    const f32x4 l4 = *reinterpret_cast<const f32x4*>(src + pitch * u);
-                    const f32x4 h4 = *reinterpret_cast<const f32x4*>(src + pitch * u + 4);
-    #pragma unroll
-                    for (int i = 0; i < 4; ++i) ac[i] += l4[i], ac[4 + i] += h4[i];
-                }
-                u32x4 raw;
-    #pragma unroll
-                for (int i = 0; i < 4; ++i) raw[i] = C::down2(ac[2 * i], ac[2 * i + 1]);
-                const uint32_t sgn = t < LPR / 2 ? 0x80008000u : 0u;
-                uint32_t wl[4], wh[4], cl[4], ch[4], sl[4], sh[4];
-    #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    wl[i] = w[i] & 0xffffu, wh[i] = w[i] & 0xffff0000u;
-                    cl[i] = cr[i] & 0xffffu, ch[i] = cr[i] & 0xffff0000u;
-                    sl[i] = (sr[i] ^ sgn) & 0xffffu, sh[i] = (sr[i] ^ sgn) & 0xffff0000u;
-                }
-                const u32x4 z = ksa_row_scale<T>(raw, ksa_row_inv_rms<T, LPR>(raw, p.eps), wl, wh);
-                const u32x4 rot = ksa_row_rope<T, LPR>(z, cl, ch, sl, sh);
-                const u32x4 val = it == p.g + 1 ? raw : rot;  // (the value row changes its place only)
+    const int hrow = it < p.g ? kvh * p.g + it : p.Hq + (it - p.g) * p.Hkv + kvh;
+    const float* src = p.qkv + (int64_t)bz * width + (int64_t)hrow * D + 8 * t;
+    const int64_t pitch = (int64_t)p.qkv_prows * width;
+    f32x4 lo[8], hi[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        const float* sp = src + pitch * min(u, p.qkv_ksplit - 1);
+        lo[u] = *reinterpret_cast<const f32x4*>(sp);
+        hi[u] = *reinterpret_cast<const f32x4*>(sp + 4);
+    }
+    const u32x4 w = *reinterpret_cast<const u32x4*>((it < p.g ? p.wq : p.wk) + 8 * t);
+    const u32x4 cr = *reinterpret_cast<const u32x4*>(p.cos + bz * p.c_bs + 8 * t);
+    const u32x4 sr = *reinterpret_cast<const u32x4*>(p.sin + bz * p.c_bs + 8 * t);
+    then();
+    float ac[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // summed and rounded as ksa_sum_partials8
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        if (u < p.qkv_ksplit) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ac[i] += lo[u][i], ac[4 + i] += hi[u][i];
+        }
+    }
+    for (int u = 8; u < p.qkv_ksplit; ++u) {
+        const f32x4 l4 = *reinterpret_cast<const f32x4*>(src + pitch * u);
+        const f32x4 h4 = *reinterpret_cast<const f32x4*>(src + pitch * u + 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ac[i] += l4[i], ac[4 + i] += h4[i];
+    }
+    u32x4 raw;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) raw[i] = C::down2(ac[2 * i], ac[2 * i + 1]);
+    const uint32_t sgn = t < LPR / 2 ? 0x80008000u : 0u;
+    uint32_t wl[4], wh[4], cl[4], ch[4], sl[4], sh[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        wl[i] = w[i] & 0xffffu, wh[i] = w[i] & 0xffff0000u;
+        cl[i] = cr[i] & 0xffffu, ch[i] = cr[i] & 0xffff0000u;
+        sl[i] = (sr[i] ^ sgn) & 0xffffu, sh[i] = (sr[i] ^ sgn) & 0xffff0000u;
+    }
+    const u32x4 z = ksa_row_scale<T>(raw, ksa_row_inv_rms<T, LPR>(raw, p.eps), wl, wh);
+    const u32x4 rot = ksa_row_rope<T, LPR>(z, cl, ch, sl, sh);
+    const u32x4 val = it == p.g + 1 ? raw : rot;  // (the value row changes its place only)
     if (it >= p.g) {
         uint16_t* dst = it == p.g ? p.kw + bz * p.k_bs + kvh * p.k_hs + (int64_t)new_row * p.k_rs
                                   : p.vw + bz * p.v_bs + kvh * p.v_hs + (int64_t)new_row * p.v_rs;
@@ -1332,11 +1332,11 @@ int decode_qkv_params(DecodeParams& p, const float* qkv_partials, int qkv_ksplit
 
 namespace {
 int decode_qkv_impl(bool wide, const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
-                                  const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
-                                  void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
-                                  const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
-                                  const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
-                                  float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
+                    const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                    void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                    const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                    const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                    float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
     if (!out || !out_strides) return KSA_ERR_NULL;
     DecodeParams p{};
     const int rc = decode_qkv_params(p, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache,
@@ -1370,11 +1370,11 @@ extern "C" int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, con
 
 // ... in workgroups of eight waves
 extern "C" int ksa_decode_qkv_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
-                                  const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
-                                  void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
-                                  const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
-                                  const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
-                                  float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
+                                       const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                       void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
+                                       const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                       const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
+                                       float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream) {
     return decode_qkv_impl(true, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache, vcache, out, row,
                            row0, start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides, v_strides, out_strides, scale,
                            nsplit, workspace, workspace_bytes, stream);
@@ -1432,12 +1432,12 @@ namespace {
 int o_workgroups(int N, int chunks, int waves) { return (N / 16 + 2 * waves - 1) / (2 * waves) * chunks; }
 
 int decode_qkv_o_impl(bool wide, const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
-                                    const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
-                                    void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
-                                    int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
-                                    const int64_t* k_strides, const int64_t* v_strides, float scale, int nsplit,
-                                    const void* o_weight, float* o_partials, int N, void* workspace, size_t workspace_bytes,
-                                    void* step_workspace, size_t step_workspace_bytes, void* stream) {
+                      const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                      void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
+                      int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                      const int64_t* k_strides, const int64_t* v_strides, float scale, int nsplit,
+                      const void* o_weight, float* o_partials, int N, void* workspace, size_t workspace_bytes,
+                      void* step_workspace, size_t step_workspace_bytes, void* stream) {
     if (!o_weight || !o_partials || !workspace || !step_workspace) return KSA_ERR_NULL;
     if (N <= 0) return KSA_ERR_INVALID;
     DecodeOParams p{};
@@ -1492,12 +1492,12 @@ extern "C" int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, c
 
 // ... in workgroups of eight waves
 extern "C" int ksa_decode_qkv_o_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
-                                    const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
-                                    void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
-                                    int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
-                                    const int64_t* k_strides, const int64_t* v_strides, float scale, int nsplit,
-                                    const void* o_weight, float* o_partials, int N, void* workspace, size_t workspace_bytes,
-                                    void* step_workspace, size_t step_workspace_bytes, void* stream) {
+                                         const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
+                                         void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,
+                                         int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
+                                         const int64_t* k_strides, const int64_t* v_strides, float scale, int nsplit,
+                                         const void* o_weight, float* o_partials, int N, void* workspace, size_t workspace_bytes,
+                                         void* step_workspace, size_t step_workspace_bytes, void* stream) {
     return decode_qkv_o_impl(true, qkv_partials, qkv_ksplit, q_weight, k_weight, cos, sin, cos_batch_stride, eps, kcache, vcache, row, row0,
                              start, end, start0, end0, batch, Hq, Hkv, D, dtype, k_strides, v_strides, scale, nsplit, o_weight,
                              o_partials, N, workspace, workspace_bytes, step_workspace, step_workspace_bytes, stream);
