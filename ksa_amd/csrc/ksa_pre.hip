@@ -18,6 +18,8 @@
 // rotate_half partner (element j +- D/2) are lane exchanges inside that group of lanes.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "ksa_api_internal.h"
 #include "ksa_tile.h"
 #include "ksa_cvt.h"
@@ -240,14 +242,20 @@ int launch_pre(PreParams p, hipStream_t stream) {
     // Short-lived workgroups over consecutive tokens, in launch order, keep the window of
     // addresses in flight narrow: measured 5 % faster than a grid-stride loop of long-lived
     // workgroups over the same accesses (a plain copy shows the same preference, 6.2 against
-    // 4.9 TB/s).  Four passes amortise a workgroup's set-up; 2 .. 8 measure alike.
-    // (a handful of tokens - a decode step - get one pass per workgroup: all the parallelism there is)
-    p.passes_per_wg = (int64_t)p.batch * p.S / p.tok_per_pass >= 4 * 1024 ? 4 : 1;
+    // 4.9 TB/s).  As many passes as give a wave four to six row groups, from 4096 passes on: fewer groups pay a workgroup's
+    // set-up too often, more widen the window.  34816 tokens, keys and values to cache rows, 1 / 2 / 4 passes, in groups a
+    // wave and us: 32 / 8 heads of 128 3 / 6 / 12 162 / 157 / 166, 16 / 8 2 / 4 / 8 128 / 110 / 114, 8 / 8 3 / 6 / 12 91 / 86 / 91, 32 / 4 5 / 10 /
+    // 20 134 / 139 / 147, 32 / 8 of 64 3 / 6 / 12 93 / 86 / 93; 32 / 8 heads of 128, 4500 / 6368 / 9000 / 14000 tokens 2 passes 26.7 / 34.8 /
+    // 46.2 / 68.9, 4 passes 28.2 / 37.1 / 50.4 / 72.2.  Below, one pass: 2000 / 3200 tokens 14.7 / 20.4 against 15.1 / 20.9 of two.
+    const int groups = p.tok_per_pass * G / 4;  // of a wave and pass
+    p.passes_per_wg = (int64_t)p.batch * p.S / p.tok_per_pass >= 4 * 1024 ? std::max(1, (5 + (groups - 1) / 2) / groups) : 1;
     const int64_t span = (int64_t)p.passes_per_wg * p.tok_per_pass;
     const int64_t blocks = ((int64_t)p.batch * p.S + span - 1) / span;
-    // a decode step (one pass of one token per workgroup): one workgroup per four row groups of a
-    // token instead of one per token - the groups of a wave are a chain of dependent loads
-    const int parts = (p.passes_per_wg == 1 && p.tok_per_pass == 1 && blocks <= kMaxPartialRows) ? G / 4 : 1;
+    // a decode step, a short prompt (one pass of one token per workgroup): one workgroup per four row groups of a
+    // token instead of one per token - the groups of a wave are a chain of dependent loads.  Up to four workgroups per CU: 32 / 8
+    // heads of 128, 300 tokens 6.8 -> 6.05 us, 16 / 8 5.5 -> 5.2; 800 tokens 9.2 -> 9.6, 2000 14.7 -> 18.0.
+    const bool few = blocks <= kMaxPartialRows || blocks * (G / 4) <= 4ll * ksa_cu_count_or(256);
+    const int parts = (p.passes_per_wg == 1 && p.tok_per_pass == 1 && few) ? G / 4 : 1;
     const dim3 grid((unsigned)blocks, (unsigned)parts);
     if (p.part)
         hipLaunchKernelGGL((ksa_pre_attention_kernel<T, D, true>), grid, dim3(256), 0, stream, p);

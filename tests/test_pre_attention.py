@@ -311,3 +311,26 @@ def test_pre_attention_gpu_row_table_at_the_end_of_its_allocation(b, S):
     want = ksa_amd.pre_attention(*args, eps=1e-6)
     ksa_amd.pre_attention(*args, eps=1e-6, k_out=kc.transpose(1, 2), v_out=vc.transpose(1, 2), kv_out_row=table)
     assert torch.equal(kc.transpose(1, 2).flip(1), want[1]) and torch.equal(vc.transpose(1, 2).flip(1), want[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (16, 8, 128), (8, 8, 128), (32, 4, 128), (32, 8, 64), (4, 4, 128), (3, 1, 128)])
+@pytest.mark.parametrize("S", [129, 342, 511, 513, 4095, 4097, 8191, 8195, 16387])
+def test_pre_attention_gpu_equals_its_pieces(Hq, Hkv, D, S):
+    """How many tokens a workgroup takes and how many workgroups share one does not show: a call equals the same tokens 97
+    at a time, bit for bit, also where it ends inside a pass."""
+    import ksa_amd
+    g = torch.Generator(device="cuda").manual_seed(S)
+    x = lambda *shape: torch.randn(shape, dtype=torch.bfloat16, device="cuda", generator=g)
+    qkv, qw, kw, cos, sin = x(1, S, Hq + 2 * Hkv, D), x(D), x(D), x(1, S, D), x(1, S, D)
+    q, k, v = qkv[:, :, :Hq], qkv[:, :, Hq:Hq + Hkv], qkv[:, :, Hq + Hkv:]
+    kc, vc = (torch.zeros(1, Hkv, S + 3, D, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    got, _, _ = ksa_amd.pre_attention(q, k, v, qw, kw, cos, sin, 1e-6, k_out=kc[:, :, :S].transpose(1, 2),
+                                      v_out=vc[:, :, :S].transpose(1, 2))
+    for i in range(0, S, 97):
+        at = slice(i, i + 97)
+        c, s = cos[:, at].contiguous(), sin[:, at].contiguous()
+        want = ksa_amd.pre_attention(q[:, at], k[:, at], v[:, at], qw, kw, c, s, 1e-6)
+        for a, b in zip((got[:, at], kc[:, :, :S].transpose(1, 2)[:, at], vc[:, :, :S].transpose(1, 2)[:, at]), want):
+            assert torch.equal(a, b)
+    assert not kc[:, :, S:].any() and not vc[:, :, S:].any()
