@@ -474,20 +474,69 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
         }
         if (row0 < s1) load_tile(row0);
     } else {
+        // (ksa_decode_new_row written out: called here, the compiler keeps 66 scalar registers more and spills 16 others to memory)
+        using C = KsaCvt<T>;
         constexpr int LPR = D / 8;      // lanes per head row
         constexpr int RPW = 64 / LPR;   // head rows per wave
         const int t = lane % LPR;
         new_row = p.row_seq ? p.row_seq[bz] : p.row0;
         if (new_row < s0 || new_row >= s1) new_row = -1;
         const int rows_here = p.g + (new_row >= 0 ? 2 : 0);  // query rows, then the key and the value row
+        const int width = (p.Hq + 2 * p.Hkv) * D;
         bool loaded = false;
         for (int i0 = wave * RPW; i0 < rows_here; i0 += kWaves * RPW) {  // (at most once for up to 14 query rows of 128)
             const int it = min(i0 + lane / LPR, rows_here - 1);          // (lanes past the last row repeat it)
-            const u32x4 val = ksa_decode_new_row<T, D>(p, bz, kvh, it, new_row, t, [&]() {
-                if (!loaded && row0 < s1) load_tile(row0);
-                loaded = true;
-            });
+            const int hrow = it < p.g ? kvh * p.g + it : p.Hq + (it - p.g) * p.Hkv + kvh;
+            // requested in this order: the partial sums (first eight slices), the rotary row and the weight, the
+            // first K / V tile - the sums are then worked on while the tile is on its way
+            const float* src = p.qkv + (int64_t)bz * width + (int64_t)hrow * D + 8 * t;
+            const int64_t pitch = (int64_t)p.qkv_prows * width;
+            f32x4 lo[8], hi[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float* sp = src + pitch * min(u, p.qkv_ksplit - 1);
+                lo[u] = *reinterpret_cast<const f32x4*>(sp);
+                hi[u] = *reinterpret_cast<const f32x4*>(sp + 4);
+            }
+            const u32x4 w = *reinterpret_cast<const u32x4*>((it < p.g ? p.wq : p.wk) + 8 * t);
+            const u32x4 cr = *reinterpret_cast<const u32x4*>(p.cos + bz * p.c_bs + 8 * t);
+            const u32x4 sr = *reinterpret_cast<const u32x4*>(p.sin + bz * p.c_bs + 8 * t);
+            if (!loaded && row0 < s1) load_tile(row0);
+            loaded = true;
+            float ac[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // summed and rounded as ksa_sum_partials8
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (u < p.qkv_ksplit) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) ac[i] += lo[u][i], ac[4 + i] += hi[u][i];
+                }
+            }
+            for (int u = 8; u < p.qkv_ksplit; ++u) {
+                const f32x4 l4 = *reinterpret_cast<const f32x4*>(src + pitch * u);
+                const f32x4 h4 = *reinterpret_cast<const f32x4*>(src + pitch * u + 4);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ac[i] += l4[i], ac[4 + i] += h4[i];
+            }
+            u32x4 raw;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) raw[i] = C::down2(ac[2 * i], ac[2 * i + 1]);
+            const uint32_t sgn = t < LPR / 2 ? 0x80008000u : 0u;
+            uint32_t wl[4], wh[4], cl[4], ch[4], sl[4], sh[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                wl[i] = w[i] & 0xffffu, wh[i] = w[i] & 0xffff0000u;
+                cl[i] = cr[i] & 0xffffu, ch[i] = cr[i] & 0xffff0000u;
+                sl[i] = (sr[i] ^ sgn) & 0xffffu, sh[i] = (sr[i] ^ sgn) & 0xffff0000u;
+            }
+            const u32x4 z = ksa_row_scale<T>(raw, ksa_row_inv_rms<T, LPR>(raw, p.eps), wl, wh);
+            const u32x4 rot = ksa_row_rope<T, LPR>(z, cl, ch, sl, sh);
+            const u32x4 val = it == p.g + 1 ? raw : rot;  // (the value row changes its place only)
             *reinterpret_cast<u32x4*>(s_new + (it < p.g ? it : 32 + it - p.g) * D + 8 * t) = val;
+            if (it >= p.g) {
+                uint16_t* dst = it == p.g ? p.kw + bz * p.k_bs + kvh * p.k_hs + (int64_t)new_row * p.k_rs
+                                          : p.vw + bz * p.v_bs + kvh * p.v_hs + (int64_t)new_row * p.v_rs;
+                __builtin_nontemporal_store(val, reinterpret_cast<u32x4*>(dst + 8 * t));
+            }
         }
         if (!loaded && row0 < s1) load_tile(row0);
         __syncthreads();
