@@ -351,10 +351,11 @@ def main():
         end = torch.full((Bz,), S + C + ws + n_sum - min(W * S, n_sum), dtype=torch.int32, device=dev)
         L = (end - start).to(torch.int64)
         bytes_step = int((2 * L * Hkv * D * 2 + 2 * Hq * D * 2).sum())
-        nsplit = args.decode_splits or _lib.lib().ksa_decode_splits(Bz, Hq, Hkv, 1, D, cap)
+        wide = 0 if args.decode_splits else _lib.lib().ksa_decode_wide_splits(Bz, Hq, Hkv, 1, D, cap)
+        nsplit = args.decode_splits or wide or _lib.lib().ksa_decode_splits(Bz, Hq, Hkv, 1, D, cap)  # (what the call below takes)
 
         def dstep():
-            ksa_amd.ksa_decode(qd, kc, vc, start, end, nsplit=nsplit)
+            ksa_amd.ksa_decode(qd, kc, vc, start, end, nsplit=args.decode_splits or None)
 
         wall, dev_ms = time_region(dstep, args.steps, args.warmup)
         us = dev_ms * 1e3 / args.steps
@@ -366,7 +367,7 @@ def main():
             "roofline": {"bound": "hbm", "achieved": bytes_step / (us * 1e-6) / 1e9,
                          "peak": PEAK_HBM_GBPS, "unit": "GB/s",
                          "frac": bytes_step / (us * 1e-6) / 1e9 / PEAK_HBM_GBPS, "traffic": None,
-                         "kernel": "ksa_decode_kernel<bf16,128> (+ merge when nsplit > 1)"},
+                         "kernel": f"ksa_decode_{'wide_' if wide else ''}kernel<bf16,128> (+ merge when nsplit > 1)"},
         }
         if args.skip_prefill:
             result.update({"value": result["decode"]["hbm_gbps"], "unit": "GB/s",
