@@ -179,18 +179,21 @@ class HipOps:
             hit = self._tiled[key] = (weight, self._gemm.TiledWeight(weight))
         return hit[1]
 
-    # Chunk tiles at every length that they take.  4 layers of the 4B shape, 700 / 2 x 3000 tokens, on the grid of the block
-    # index up to 4608 rows -> here 1178 / 5289 -> 1152 / 5232 us; one layer in a graph, 32 / 8 heads of 128, grid
-    # of the block index / chunk tiles, 100 / 300 / 700 / 1500 / 3000 / 4300 tokens: window of 4 chunks 10.4 / 15.9 / 23.7 / 31.3 / 56.7 /
-    # 83.2 against 7.6 / 10.1 / 16.0 / 25.0 / 42.1 / 60.4 us, unbounded 10.1 / 15.6 / 22.7 / 39.4 / 98.8 / 186 against 7.6 / 10.0 / 15.9 / 32.9 / 83.7 /
-    # 151.  Neither rounds the logits more accurately than the other: behind 4 layers, 15 prompts of 150 to 1500 tokens, they lie 1.720 %
-    # (grid) and 1.725 % from fp32, keys and values 1.517 and 1.515 %.
+    # Up to this many rows a prompt's attention stays on the grid of the block index, and its logits what they are there bit for
+    # bit: chunk tiles round them differently by about a unit in their last place, which can tip the greedy token where the two
+    # best logits lie that close (5 of 108 prompts of random weights).  Neither form is the more accurate one - distance of the
+    # logits from fp32 behind 4 layers, 15 prompts of 150 to 1500 tokens, 1.720 % on the grid and 1.725 % on chunk tiles, of keys and
+    # values 1.517 and 1.515 % - so this is a choice for unchanged results where they cost little, not a line that the kernels draw:
+    # prefill of 4 layers of the 4B shape, 700 / 2 x 3000 tokens, grid 1178 / 5289 us, chunk tiles 1152 / 5232; one layer in a graph, 32 / 8
+    # heads of 128, 300 / 1500 / 4300 tokens, window of 4 chunks 15.9 / 31.3 / 83.2 and 10.1 / 25.0 / 60.4 us.
+    GRID_ROWS = 4608
+
     def summary_attn_func(self, q, k, v, *args, **kwargs):
-        return self._summary_attn(q, k, v, *args, **kwargs)
+        return self._summary_attn(q, k, v, *args, chunk_tiles=q.shape[1] > self.GRID_ROWS, **kwargs)
 
     def summary_attn_in_line(self, q, k, v, C, S, W):
         """`summary_attn_func` with the mask of `expand_prompt`."""
-        return self._summary_attn_in_line(q, k, v, C, S, W)
+        return self._summary_attn_in_line(q, k, v, C, S, W, chunk_tiles=q.shape[1] > self.GRID_ROWS)
 
     def expand_prompt(self, input_ids, config, inv_freq, dtype):
         """`expand_with_summary_tokens` and the rotary rows of its positions in one launch (`ksa_expand_prompt`): (ids

@@ -326,14 +326,14 @@ def summary_attn_func(q, k, v, chunk_size, summary_num, sliding_chunk_num,
                     softmax_scale, workgroup_shape, chunk_tiles)
 
 
-def summary_attn_in_line(q, k, v, chunk_size, summary_num, sliding_chunk_num):
+def summary_attn_in_line(q, k, v, chunk_size, summary_num, sliding_chunk_num, *, chunk_tiles: bool = True):
     """`summary_attn_func` for a prompt whose summary rows the caller itself has put behind every whole chunk: with the
     `summary_pos` of that layout, without the host waiting for an analysis of it."""
     def layout(Sq, C, S, k, v):
         assert k.shape[1] == Sq and Sq % (C + S) <= C, "k/v have the rows of q, summary rows stand behind whole chunks"
         return Sq // (C + S) * S, False, k, v
 
-    return _forward(q, k, v, chunk_size, summary_num, sliding_chunk_num, layout, False, False, None, None, True)
+    return _forward(q, k, v, chunk_size, summary_num, sliding_chunk_num, layout, False, False, None, None, chunk_tiles)
 
 
 def _forward(q, k, v, chunk_size, summary_num, sliding_chunk_num, layout, skip_old_summary, return_lse, softmax_scale,

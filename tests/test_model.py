@@ -88,6 +88,33 @@ def test_gpu_expand_prompt_equals_host_form(text, C, S, D, kind, dtype):
             torch.testing.assert_close(got[0], want.to(dtype), rtol=2.0 ** (-7 if dtype == torch.bfloat16 else -10), atol=1e-6)
 
 
+@pytest.mark.gpu
+def test_gpu_prefill_of_short_prompts_keeps_its_results():
+    """The head of a prefill in one launch, closed-form cache rows and the attention without a mask change no bit of a prompt up to
+    `GRID_ROWS`: logits and cache rows are those of the torch head, the mask and the grid of the block index."""
+    from ksa_amd import prefill
+    from ksa_amd.model import HipOps
+
+    class Plain(HipOps):
+        expand_prompt = lambda self, *a: None
+
+        def summary_attn_func(self, *args, **kwargs):
+            return prefill.summary_attn_func(*args, chunk_tiles=False, **kwargs)
+    cfg = tiny_config(hidden_size=256, num_hidden_layers=2, num_attention_heads=8, num_key_value_heads=2, head_dim=128,
+                      intermediate_size=512, vocab_size=4000, summary_token_begin=4000, summary_chunk_size=128, summary_token_num=8,
+                      summary_sliding_chunk_num=[4, 1 << 20])
+    w = init_weights(cfg, "cuda", torch.bfloat16, 3)
+    model, plain = KsaQwen3ForCausalLM(cfg, w), KsaQwen3ForCausalLM(cfg, w, Plain())
+    last = 4608 // 136 * 128 + 4608 % 136     # as many rows as the grid keeps
+    for b, n in ((1, 1), (2, 127), (1, 128), (3, 300), (1, 1000), (8, 2049), (1, 4096), (1, last)):
+        ids = torch.randint(0, cfg.vocab_size, (b, n), generator=torch.Generator().manual_seed(n)).cuda()
+        (got, cache), (want, ref) = model.prefill(ids), plain.prefill(ids)
+        assert torch.equal(got, want), (b, n)
+        for layer in range(2):
+            for x, y in zip(cache.get_attention_kv(layer), ref.get_attention_kv(layer)):
+                assert torch.equal(x, y), (b, n, layer)
+
+
 def test_expand_known_values():
     cfg = tiny_config(summary_token_num=2)
     ids, pos, is_sum = expand_with_summary_tokens(torch.arange(17)[None], cfg)
