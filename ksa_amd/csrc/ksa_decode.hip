@@ -760,10 +760,15 @@ __global__ __launch_bounds__(kThreads) void ksa_decode_merge_kernel(const Decode
 // The probabilities enter the second product as two 16-bit parts, value and remainder: a wave's first tile of 64 rows fixes its
 // reference, where the kernel above has more of them, and a row at its reference has no rounding; with one part the output lay 1.3 %
 // further from 64 bits than the kernel above (60 shapes, up to 5 %), with two 12 % nearer (0.76 to 1.0 times), for 0.2 us a launch.
+// An infinite value has no product with a remainder of 0 or below, nor with the probability 0 of its repetitions past the end: an
+// element that comes out as NaN is made once more by the thread that has it, behind everything else.  (Looked for in the sums of each
+// wave, with a second walk of its tiles, it cost every launch 0.17 us.)
 // kPre as above; the new key goes to the operand registers, the new value to the tile.  kO as above; a decode step's attention and o
 // projection, 32 / 8 heads of 128, N 2560, in the kernel above -> here: 1 sequence of 737 / 4097 rows 15.8 / 18.2 -> 11.7 / 14.6 us, 8
 // of 737 / 4097 21.3 / 38.6 -> 16.2 / 34.9, 16 of 737 / 4097 26.4 / 61.7 -> 22.2 / 54.6.
 constexpr int kWideWaves = 8, kWideRows = 64, kWideColumns = 16;
+// (as an integer: the compiler takes floats for numbers)
+__device__ __forceinline__ bool ksa_is_nan(float x) { return __builtin_bit_cast(uint32_t, x) << 1 > 0xff000000u; }
 template <typename T, int D, bool kPre, bool kO = false>
 __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const std::conditional_t<kO, DecodeOParams, DecodeParams> p) {
     using Ops = KsaOps<T>;
@@ -978,10 +983,10 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const 
         if (kq == 0) row[D] = m_run * c2, row[D + 1] = l_run;  // (log2 units; -inf of a wave without rows)
     }
     __syncthreads();
-    for (int e = tid; e < p.ncols * D; e += 64 * kWideWaves) {
-        const int c = e / D, d = e % D;
+    auto merged = [&](int c, int d, float& mx, float& l) {
         const float* row = mg + c * (D + 2);
-        float mx = -INFINITY, acc = 0.f, l = 0.f;
+        float acc = 0.f;
+        mx = -INFINITY, l = 0.f;
 #pragma unroll
         for (int w = 0; w < kWideWaves; ++w) mx = fmaxf(mx, row[w * 16 * (D + 2) + D]);
 #pragma unroll
@@ -991,14 +996,53 @@ __global__ __launch_bounds__(64 * kWideWaves) void ksa_decode_wide_kernel(const 
             acc += row[w * 16 * (D + 2) + d] * f;
             l += row[w * 16 * (D + 2) + D + 1] * f;
         }
+        return acc;
+    };
+    auto leave = [&](int c, int d, float mx, float acc, float l) {
         if (kO || p.nsplit > 1) {
             put(p.ws_o + (slot0 + c) * D + d, acc);
             if (d == 0) put(p.ws_ml + (slot0 + c) * 2, mx), put(p.ws_ml + (slot0 + c) * 2 + 1, l);
-            continue;
+            return;
         }
         int oq, og;
         ksa_decode_column(p, 0, c, oq, og);
         p.out[bz * p.o_bs + oq * p.o_qs + (kvh * p.g + og) * p.o_hs + d] = (uint16_t)(Ops::pack2(l > 0.f ? acc / l : 0.f, 0.f) & 0xffffu);
+    };
+    bool nan = false;
+    for (int e = tid; e < p.ncols * D; e += 64 * kWideWaves) {
+        float mx, l;
+        const float acc = merged(e / D, e % D, mx, l);
+        nan |= ksa_is_nan(acc);
+        leave(e / D, e % D, mx, acc, l);
+    }
+    if (__builtin_expect(__any(nan), 0)) {
+        // the sum of column c and element d from its definition, at reference mx
+        auto element = [&](int c, int d, float mx) {
+            int oq, og;
+            ksa_decode_column(p, 0, c, oq, og);
+            const uint16_t* qp = kPre ? s_new + og * D : p.q + bz * p.q_bs + (kvh * p.g + og) * p.q_hs + oq * p.q_qs;
+            float acc = 0.f;
+#pragma unroll 1
+            for (int row = r_begin; row < r_end; ++row) {
+                const bool fresh = kPre && row == new_row;
+                const uint16_t* kp = fresh ? s_new + 16 * D : p.k + bz * p.k_bs + kvh * p.k_hs + (int64_t)row * p.k_rs;
+                const uint16_t v = fresh ? s_new[17 * D + d] : p.v[bz * p.v_bs + kvh * p.v_hs + (int64_t)row * p.v_rs + d];
+                float score = 0.f;
+#pragma unroll 1
+                for (int i = 0; i < D; i += 8) {
+                    const u32x4 a = *reinterpret_cast<const u32x4*>(kp + i), b = *reinterpret_cast<const u32x4*>(qp + i);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) score = C::dot2(a[j], b[j], score);
+                }
+                acc = fmaf(ksa_exp2(fmaf(score, c2, -mx)), C::up(v), acc);
+            }
+            return acc;
+        };
+        for (int e = tid; e < p.ncols * D; e += 64 * kWideWaves) {
+            float mx, l;
+            const float acc = merged(e / D, e % D, mx, l);
+            if (ksa_is_nan(acc) && !ksa_is_nan(l)) leave(e / D, e % D, mx, element(e / D, e % D, mx), l);
+        }
     }
     arrive();
 }

@@ -529,6 +529,53 @@ def test_decode_wide_workgroups(dtype, D, b, Hq, Hkv, Q, rows, nsplit):
     assert np.abs(to_np(got).reshape(want.shape) - want).max() <= ATOL * max(1.0, np.abs(want).max())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("b,Hq,Hkv,D,Q,rows,nsplit", [(1, 4, 1, 128, 1, 1, 1), (2, 32, 8, 128, 1, 300, None), (1, 16, 1, 128, 1, 1100, 2),
+                                                      (2, 10, 2, 64, 3, 512, 1), (1, 8, 2, 64, 1, 4500, 7), (1, 32, 8, 128, 1, 577, 1)])
+def test_decode_wide_infinite_values(dtype, b, Hq, Hkv, D, Q, rows, nsplit):
+    """An infinite value of an attended row is the outcome in its column, whatever its row - the first, the last, one in the
+    middle of a cut tile - and of no other column; both signs in a column have no sum.  From the projection's sums as well."""
+    import ksa_amd
+    from ksa_amd import decode, gemm, pre
+    g = torch.Generator().manual_seed(rows + D)
+    rnd = lambda *s: torch.randn(*s, generator=g)
+    q, k, v = rnd(b, Hq, Q, D).to(dtype), rnd(b, Hkv, rows, D).to(dtype), rnd(b, Hkv, rows, D).to(dtype)
+    lo, hi = rows // 7, rows - rows // 9
+    inf = float("inf")
+    for col, row in ((0, lo), (5, hi - 1), (17, (lo + hi) // 2), (D - 1, lo)):
+        v[:, :, row, col] = inf
+    v[:, -1, hi - 1, 9] = v[:, 0, lo, 33] = -inf
+    if hi - lo > 2:
+        v[:, :, lo, 40], v[:, :, hi - 1, 40] = inf, -inf
+    if rows > 9:
+        v[:, :, lo - 1], v[:, :, hi] = inf, float("nan")     # outside of the range
+    args = (q.cuda(), k.cuda(), v.cuda())
+    got = ksa_amd.ksa_decode(*args, lo, hi) if nsplit is None else \
+        torch.ops.ksa_amd.wide_decode_fwd(*args, None, None, lo, hi, D ** -0.5, nsplit)
+    rep = lambda t: t[:, :, lo:hi].double().repeat_interleave(Hq // Hkv, 1)
+    want = ((q.double() @ rep(k).transpose(-1, -2)) * D ** -0.5).softmax(-1) @ rep(v)
+    want = want.transpose(1, 2)
+    assert want.isinf().any() and (hi - lo <= 2 or want.isnan().any())
+    torch.testing.assert_close(got.double().cpu(), want, rtol=0, atol=ATOL, equal_nan=True)
+    if Q > 1:
+        return
+    # the new row somewhere in the range, its cache row holding what must not be read
+    x, w = rnd(b, 1, 1536).to(dtype).cuda(), rnd((Hq + 2 * Hkv) * D, 1536).to(dtype).cuda()
+    qkv, one = gemm.linear_rows(x, w, defer=True), torch.ones(D, dtype=dtype, device="cuda")
+    cos, sin = (torch.full((1, 1, D), c, dtype=dtype, device="cuda") for c in (0.6, 0.8))
+    kc, vc = args[1].clone(), args[2].clone()
+    at = (lo + hi) // 2
+    kc[:, :, at] = vc[:, :, at] = float("nan")
+    kr, vr = kc.clone(), vc.clone()
+    qr, _, _ = pre.pre_attention_partials(qkv, Hq, Hkv, D, one, one, cos, sin, 1e-6, k_out=kr[:, :, at:at + 1].transpose(1, 2),
+                                          v_out=vr[:, :, at:at + 1].transpose(1, 2))
+    n = nsplit or 1
+    want = torch.ops.ksa_amd.wide_decode_fwd(qr.transpose(1, 2), kr, vr, None, None, lo, hi, D ** -0.5, n)
+    got = decode.ksa_decode_qkv(qkv, one, one, cos, sin, 1e-6, kc, vc, Hq, at, lo, hi, nsplit=n, wide=True)
+    torch.testing.assert_close(got.view(want.shape), want, rtol=0, atol=0, equal_nan=True)
+    assert rows == 1 or want.isinf().any()
+
+
 def test_decode_wide_workgroups_refuse_what_they_do_not_take():
     import ksa_amd  # noqa: F401
     from ksa_amd import _lib
