@@ -18,8 +18,9 @@
  *   - dtype: 0 = bf16, 1 = fp16; head_dim 64, 128 or 256 for the two attention entry points
  *     (any other multiple of 8 up to 256, which the reference also takes, is zero-padded to the
  *     next of these by the caller: the Python mirrors do), 64 or 128 for ksa_pre_attention;
- *   - return value 0 = launched, negative = rejected before any launch
- *     (see ksa_error_string).
+ *   - return value 0 = launched, negative = rejected before any launch (see ksa_error_string); only
+ *     KSA_ERR_LAUNCH comes from behind a launch: the HIP runtime reports an error, this launch's or one
+ *     that an earlier HIP call left pending, and the kernel may have run.
  */
 #ifndef KSA_HIP_H
 #define KSA_HIP_H

@@ -127,7 +127,7 @@ def lib():
         except ImportError as e:
             raise KsaError(f"ksa_amd/_fast.so is missing or was built for another PyTorch: build it with `python "
                            f"ksa_amd/build.py` ({e})") from e
-        _fast.bind(*[ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _FAST])
+        _fast.bind(check, *[ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _FAST])
         fast = _fast
         _lib = L
     return _lib

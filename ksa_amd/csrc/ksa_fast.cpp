@@ -39,6 +39,23 @@ struct Library {
     decltype(&ksa_decode_wide_splits) decode_wide_splits;
     decltype(&ksa_decode_wide_fwd) decode_wide_fwd;
 } lib{};
+PyObject* lib_check = nullptr;  // `_lib.check`, which raises
+
+// Whether a library call has launched.  If not, it was refused in front of its launch, and the general way says why; but
+// an error behind a launch is raised here (an exception is set): the kernel may have run, on outputs that may be inputs.
+bool launched(int rc, const char* what) {
+    if (rc == KSA_ERR_LAUNCH) {
+        PyObject* r = PyObject_CallFunction(lib_check, "is", rc, what);
+        Py_XDECREF(r);
+        if (r) PyErr_SetString(PyExc_RuntimeError, what);
+    }
+    return rc == KSA_OK;
+}
+#define KSA_UNLESS_LAUNCHED(rc, what)           \
+    if (!launched(rc, what)) {                  \
+        if (PyErr_Occurred()) return nullptr;   \
+        Py_RETURN_NONE;                         \
+    }
 
 // Nobody records, traces, transforms or profiles (`_lib.direct`, which says why for each).  Whoever steps in front of the
 // dispatcher (a mode, a torch.func transform, a tracer) includes a key of its own in this thread.
@@ -138,14 +155,15 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!get_scale(a[5], D, scale) || (a[6] != Py_None && !get_int(a[6], nsplit))) Py_RETURN_NONE;
     at::Tensor out;
     int rc;
+    bool wide = false;
     {
         Unlocked u;
-        auto forward = lib.decode_fwd;
         if (a[6] == Py_None) {
             nsplit = lib.decode_wide_splits((int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, most);
-            if (nsplit > 0) forward = lib.decode_wide_fwd;
-            else nsplit = lib.decode_splits((int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, most);
+            wide = nsplit > 0;
+            if (!wide) nsplit = lib.decode_splits((int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, most);
         }
+        const auto forward = wide ? lib.decode_wide_fwd : lib.decode_fwd;
         out = at::empty({b, Q, Hq, D}, q->options());
         at::Tensor ws;
         size_t ws_bytes = 0;
@@ -158,7 +176,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
                      (int)b, (int)Hq, (int)Hkv, (int)Q, (int)D, dt, qs.data(), ks.data(), vs.data(), os.data(), scale, nsplit,
                      ws_bytes ? ws.mutable_data_ptr() : nullptr, ws_bytes, stream_of(dev));
     }
-    if (rc != 0) Py_RETURN_NONE;  // rejected in front of the launch: the general way says why
+    KSA_UNLESS_LAUNCHED(rc, wide ? "ksa_decode_wide_fwd" : "ksa_decode_fwd")
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }
@@ -210,7 +228,7 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                     (int)D, dt, qs.data(), ks.data(), os.data(), C, S, W, a[6] == Py_True, scale, 0,
                                     sched.defined() ? sched.mutable_data_ptr<int32_t>() : nullptr, stream_of(dev));
     }
-    if (rc != 0) Py_RETURN_NONE;
+    KSA_UNLESS_LAUNCHED(rc, "ksa_prefill_chunks_fwd")
     PyObject* o = THPVariable_Wrap(out);
     PyObject* l = lse.defined() ? THPVariable_Wrap(lse) : Py_NewRef(Py_None);
     PyObject* r = o && l ? PyTuple_Pack(2, o, l) : nullptr;
@@ -275,7 +293,7 @@ PyObject* pre_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                (int)b, (int)S, (int)Hq, (int)Hkv, (int)D, dt, qs.data(), ks.data(), vs.data(), qo.data(),
                                ko.data(), vo.data(), cs.data(), kv_row, per_token, (float)PyFloat_AS_DOUBLE(a[7]), stream_of(dev));
     }
-    if (rc != 0) Py_RETURN_NONE;
+    KSA_UNLESS_LAUNCHED(rc, "ksa_pre_attention")
     PyObject* r = PyTuple_New(3);
     for (int i = 0; r && i < 3; ++i) {
         PyObject* t = given[i] ? Py_NewRef(a[8 + i]) : THPVariable_Wrap(o[i]);
@@ -306,7 +324,7 @@ PyObject* block_index(PyObject*, PyObject* const* a, Py_ssize_t n) {
         for (int i = 0; i < 4; ++i) p[i] = t[i].mutable_data_ptr<int32_t>();
         rc = lib.block_index(Sq, Sk, C, S, W, Sk - Sq, a[5] == Py_True, tm, tn, p[0], p[1], p[2], p[3], stream_of(dev));
     }
-    if (rc != 0) Py_RETURN_NONE;
+    KSA_UNLESS_LAUNCHED(rc, "ksa_block_index")
     PyObject* r = PyTuple_New(4);
     for (int i = 0; r && i < 4; ++i) {
         PyObject* o = THPVariable_Wrap(t[i]);
@@ -317,16 +335,18 @@ PyObject* block_index(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(addresses of ksa_block_index, ksa_decode_splits, ksa_decode_workspace_bytes, ksa_decode_fwd, ksa_prefill_chunks_fwd,
+// bind(_lib.check, addresses of ksa_block_index, ksa_decode_splits, ksa_decode_workspace_bytes, ksa_decode_fwd, ksa_prefill_chunks_fwd,
 // ksa_pre_attention, ksa_decode_wide_splits, ksa_decode_wide_fwd)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     void** slots[] = {(void**)&lib.block_index, (void**)&lib.decode_splits, (void**)&lib.decode_workspace_bytes,
                       (void**)&lib.decode_fwd, (void**)&lib.prefill_chunks_fwd, (void**)&lib.pre_attention,
                       (void**)&lib.decode_wide_splits, (void**)&lib.decode_wide_fwd};
     constexpr Py_ssize_t kSlots = sizeof(slots) / sizeof(slots[0]);
-    if (n != kSlots) return PyErr_Format(PyExc_TypeError, "bind takes %zd addresses", kSlots);
+    if (n != 1 + kSlots) return PyErr_Format(PyExc_TypeError, "bind takes a function and %zd addresses", kSlots);
+    Py_INCREF(a[0]);
+    Py_XSETREF(lib_check, a[0]);
     for (Py_ssize_t i = 0; i < kSlots; ++i) {
-        *slots[i] = PyLong_AsVoidPtr(a[i]);
+        *slots[i] = PyLong_AsVoidPtr(a[1 + i]);
         if (PyErr_Occurred()) return nullptr;
     }
     Py_RETURN_NONE;

@@ -468,3 +468,49 @@ def test_native_front_steps_aside():
     note(torch._efficientzerotensor((2, 4, 1, 64), dtype=q.dtype, device="cuda"))
     assert len(seen) == 11 and not any(seen), seen
     assert ask()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("code", [-5, -1])
+def test_native_front_never_launches_twice(code):
+    """An error that the library reports behind a launch (-5) is raised: the kernel may have run, on outputs that may be the
+    inputs, so the general way must not run it again.  What the library refuses in front of its launch goes that way."""
+    import ctypes
+
+    import ksa_amd
+    from ksa_amd import _lib
+    L = _lib.lib()
+    rnd = lambda *s: torch.randn(*s, device="cuda").bfloat16()
+    q, kc, vc = rnd(2, 8, 1, 64), rnd(2, 2, 300, 64), rnd(2, 2, 300, 64)
+    p, k, v, w, rope = rnd(1, 200, 8, 128), rnd(1, 200, 2, 128), rnd(1, 200, 2, 128), rnd(128), rnd(1, 200, 128)
+    qo, ko, vo = (torch.zeros_like(t) for t in (p, k, v))
+    calls = {
+        "ksa_decode_wide_fwd": lambda: ksa_amd.ksa_decode(q, kc, vc),
+        "ksa_decode_fwd": lambda: ksa_amd.ksa_decode(q, kc, vc, nsplit=2),
+        "ksa_prefill_chunks_fwd": lambda: ksa_amd.summary_attn_func(p, k, v, 128, 8, 1)[0],
+        "ksa_pre_attention": lambda: ksa_amd.pre_attention(p, k, v, w, w, rope, rope, q_out=qo, k_out=ko, v_out=vo)[0],
+        "ksa_block_index": lambda: ksa_amd.compute_block_sparsity(400, 400, 128, 8, 2)[1],
+    }
+    address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+    seen = []
+
+    @ctypes.CFUNCTYPE(ctypes.c_int)
+    def stub():                       # (launches nothing; its arguments are the caller's to clear)
+        seen.append(code)
+        return code
+    for name, call in calls.items():
+        want = call().clone()
+        qo.zero_()
+        seen.clear()
+        _lib.fast.bind(_lib.check, *(address(stub if n == name else getattr(L, n)) for n in _lib._FAST))
+        try:
+            if code == -5:
+                with pytest.raises(_lib.KsaError, match=name):
+                    call()
+                assert not qo.any()
+            else:
+                assert torch.equal(call(), want)
+        finally:
+            _lib.fast.bind(_lib.check, *(address(getattr(L, n)) for n in _lib._FAST))
+        assert seen == [code], name
+        assert torch.equal(call(), want)
