@@ -6,6 +6,7 @@ import contextlib
 import ctypes
 import functools
 import os
+import warnings
 
 import torch  # noqa: F401  (must be imported first so that its HIP runtime is the one in the process)
 
@@ -13,7 +14,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # KSA_AMD_LIB selects another build of the same library (e.g. a profiling variant)
 LIB_PATH = os.environ.get("KSA_AMD_LIB") or os.path.join(_HERE, "libksa_hip.so")
 _lib = None
-# the native front of the hottest calls (csrc/ksa_fast.cpp); what it calls, in the order of its `bind`
+# the native front of the hottest calls (csrc/ksa_fast.cpp; `_GeneralWay` where it does not load); what it calls, in the order
+# of its `bind`
 fast = None
 _FAST = ("ksa_block_index", "ksa_decode_splits", "ksa_decode_workspace_bytes", "ksa_decode_fwd", "ksa_prefill_chunks_fwd",
          "ksa_pre_attention", "ksa_decode_wide_splits", "ksa_decode_wide_fwd")
@@ -110,6 +112,12 @@ class KsaError(RuntimeError):
     pass
 
 
+class _GeneralWay:
+    """In place of the native front, whose parts of PyTorch are not all public: takes no call, so that every one goes the
+    Python way to the same entry points of the library."""
+    decode = prefill = pre_attention = block_index = staticmethod(lambda *args: None)
+
+
 def lib():
     global _lib, fast
     if _lib is None:
@@ -124,11 +132,12 @@ def lib():
             fn.argtypes = args
         try:
             from . import _fast
-        except ImportError as e:
-            raise KsaError(f"ksa_amd/_fast.so is missing or was built for another PyTorch: build it with `python "
-                           f"ksa_amd/build.py` ({e})") from e
-        _fast.bind(check, *[ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _FAST])
-        fast = _fast
+            _fast.bind(check, *[ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _FAST])
+            fast = _fast
+        except (ImportError, TypeError) as e:   # (TypeError: a build with other entry points)
+            warnings.warn(f"ksa_amd/_fast.so is missing or was built for another PyTorch: the same kernels are called from Python, "
+                          f"small calls take some 10 us longer.  Build it with `python ksa_amd/build.py` ({e})", RuntimeWarning)
+            fast = _GeneralWay
         _lib = L
     return _lib
 

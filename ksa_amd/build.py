@@ -48,14 +48,24 @@ def _run(cmd, verbose):
     # the host pass warns that it does not know the packed-fp32 feature; that is expected
     err = "\n".join(l for l in res.stderr.splitlines() if "packed-fp32-ops" not in l)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{err}")
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed ({res.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
 
 
+def _build_fast(verbose):
+    try:
+        _run(_fast_command(), verbose)
+    except (RuntimeError, OSError) as e:
+        if os.path.exists(FAST):   # of another build
+            os.remove(FAST)
+        print(f"_fast.so was not built, calls go through Python: {e}", file=sys.stderr)
+
+
 def build(verbose: bool = False, extra_flags=(), out: str = LIB, csrc: str = CSRC, jobs: int = 8) -> str:
     """Compiles every source of `csrc` (one hipcc process each, `jobs` at a time) and links them
-    into `out`.  Objects go to a `build/` folder next to `out`, named after it."""
+    into `out`.  Objects go to a `build/` folder next to `out`, named after it.  With the package's own library
+    comes the native front; where that does not compile, the package does without it."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     objdir = os.path.join(os.path.dirname(os.path.abspath(out)), "build",
                           os.path.splitext(os.path.basename(out))[0])
@@ -63,10 +73,11 @@ def build(verbose: bool = False, extra_flags=(), out: str = LIB, csrc: str = CSR
     objs = [os.path.join(objdir, os.path.splitext(s)[0] + ".o") for s in SOURCES]
     cmds = [[hipcc, *FLAGS, *extra_flags, "-I", csrc, "-c", os.path.join(csrc, s), "-o", o]
             for s, o in zip(SOURCES, objs)]
-    if out == LIB:
-        cmds.append(_fast_command())
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
+        front = pool.submit(_build_fast, verbose) if out == LIB else None
         list(pool.map(lambda c: _run(c, verbose), cmds))
+        if front is not None:
+            front.result()
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", out, *objs], verbose)
     return out
 

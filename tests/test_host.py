@@ -332,6 +332,30 @@ def test_decode_splits_rule(b, hq, hkv, q):
     assert L.ksa_decode_splits(1, 32, 7, 1, 128, 1000) == 1 and L.ksa_decode_splits(0, 32, 8, 1, 128, 1000) == 1
 
 
+@pytest.mark.parametrize("broken", ["missing", "other"])
+def test_package_without_its_native_front(broken):
+    """A native front that does not load (it is built against one PyTorch) or that is another build's leaves the Python way,
+    with a warning; the library itself stays indispensable."""
+    import subprocess
+    import sys
+    module = "None" if broken == "missing" else "types.SimpleNamespace(bind=lambda *a: (_ for _ in ()).throw(TypeError('entry points')))"
+    code = f"""
+import sys, types, warnings, importlib
+front = {module}
+sys.modules['ksa_amd._fast'] = front
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter('always')
+    import ksa_amd
+from ksa_amd import _lib
+assert any('_fast.so' in str(w.message) for w in seen), seen
+assert _lib.lib().ksa_version() > 0
+assert _lib.fast.decode(1, 2, 3, None, None, None, None) is None and _lib.fast.block_index(*range(8)) is None
+assert _lib.fast.prefill(*range(11)) is None and _lib.fast.pre_attention(*range(12)) is None
+"""
+    res = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+
+
 def test_decode_qkv_argument_checks():
     """Shapes the fused decode call does not take are refused on the host."""
     from ksa_amd import _lib, decode
