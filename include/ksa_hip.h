@@ -290,6 +290,12 @@ int ksa_copy_rows_runs(int n_moves, const void* const* src, void* const* dst, co
 int ksa_expand_prompt(const long long* ids, long long ids_row_stride, int batch, int n, int C, int S,
                       long long summary_begin, int inner_chunk, int summary_kind, const float* inv_freq, int D,
                       long long* out_ids, void* cos, void* sin, void* is_summary, int dtype, void* stream);
+/* Slots [slot0, slot0 + slots) of the same, for the decode steps (HF:1497-1531): one text row, at the end of a chunk that row and
+ * the chunk's summary rows, or a stretch of rotary rows (C larger than any position).  ids int64 [batch, text tokens among the
+ * slots]; out_ids int64 [batch, slots] or null; rows of cos / sin rope_row_stride elements apart (a multiple of 8). */
+int ksa_expand_slots(const long long* ids, long long ids_row_stride, int batch, int slot0, int slots, int C, int S,
+                     long long summary_begin, int inner_chunk, int summary_kind, const float* inv_freq, int D,
+                     long long* out_ids, void* cos, void* sin, long long rope_row_stride, int dtype, void* stream);
 
 /* Pre-attention step: per-head RMSNorm of q and k, rotary embedding, layout write of q, k, v.
  * Replaces HF:660-666 (q_norm / k_norm = Qwen3RMSNorm HF:64-79 on head_dim, the three

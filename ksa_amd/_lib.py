@@ -57,6 +57,8 @@ _SIGNATURES = {
     "ksa_copy_rows_runs": (_int, [_int] + [_vp] * 5 + [_int] + [_vp] * 2 + [_int] * 3 + [_vp] * 3),
     "ksa_expand_prompt": (_int, [_vp, ctypes.c_longlong] + [_int] * 4 + [ctypes.c_longlong, _int, _int, _vp, _int]
                           + [_vp] * 4 + [_int, _vp]),
+    "ksa_expand_slots": (_int, [_vp, ctypes.c_longlong] + [_int] * 5 + [ctypes.c_longlong, _int, _int, _vp, _int]
+                         + [_vp] * 3 + [ctypes.c_longlong, _int, _vp]),
     "ksa_copy_rows": (_int, [_vp] * 4 + [_int] * 6 + [_i64p] * 2 + [_vp]),
     "ksa_pre_attention": (_int, [_vp] * 10 + [_int] * 6 + [_i64p] * 7 + [_vp, _int, ctypes.c_float, _vp]),
     "ksa_pre_attention_partials": (_int, [_vp, _int] + [_vp] * 7 + [_int] * 6 + [_i64p] * 4

@@ -195,18 +195,25 @@ class HipOps:
         """`summary_attn_func` with the mask of `expand_prompt`."""
         return self._summary_attn_in_line(q, k, v, C, S, W, chunk_tiles=q.shape[1] > self.GRID_ROWS)
 
-    def expand_prompt(self, input_ids, config, inv_freq, dtype):
-        """`expand_with_summary_tokens` and the rotary rows of its positions in one launch (`ksa_expand_prompt`): (ids
-        [b, L], cos, sin [1, L, D], mask [L]); None where those have to do it."""
+    @staticmethod
+    def _expand_kinds(config, inv_freq, dtype):
+        """(text positions, summary positions) as the kernel names them; None where it does not know them or the types."""
         text = {"origin": 0, "inner_chunk": 1}.get(config.summary_chunk_position_ids_type)
         summary = {"zeros": 0, "last_chunk_slice_left": 1, "last_chunk_slice_right": 2}.get(
             config.summary_token_position_ids_type)
         D = config.head_dim
-        if (text is None or summary is None or dtype not in (torch.bfloat16, torch.float16) or D % 16
-                or input_ids.dtype != torch.long or input_ids.dim() != 2 or not input_ids.is_cuda or input_ids.numel() == 0
+        if (text is None or summary is None or dtype not in (torch.bfloat16, torch.float16) or D % 16 or not inv_freq.is_cuda
                 or inv_freq.dtype != torch.float32 or inv_freq.shape != (D // 2,) or not inv_freq.is_contiguous()):
             return None
-        C, S, dev = config.summary_chunk_size, config.summary_token_num, input_ids.device
+        return text, summary
+
+    def expand_prompt(self, input_ids, config, inv_freq, dtype):
+        """`expand_with_summary_tokens` and the rotary rows of its positions in one launch (`ksa_expand_prompt`): (ids
+        [b, L], cos, sin [1, L, D], mask [L]); None where those have to do it."""
+        kinds = self._expand_kinds(config, inv_freq, dtype)
+        if kinds is None or input_ids.dtype != torch.long or input_ids.dim() != 2 or not input_ids.is_cuda or input_ids.numel() == 0:
+            return None
+        C, S, D, dev = config.summary_chunk_size, config.summary_token_num, config.head_dim, input_ids.device
         if input_ids.stride(1) != 1:
             input_ids = input_ids.contiguous()
         b, n = input_ids.shape
@@ -216,11 +223,49 @@ class HipOps:
         mask = torch.empty(L, dtype=torch.bool, device=dev)
         with self._lib.on_device(dev):
             rc = self._lib.lib().ksa_expand_prompt(
-                input_ids.data_ptr(), input_ids.stride(0), b, n, C, S, config.summary_token_begin, text, summary,
+                input_ids.data_ptr(), input_ids.stride(0), b, n, C, S, config.summary_token_begin, *kinds,
                 inv_freq.data_ptr(), D, ids.data_ptr(), rope[0].data_ptr(), rope[1].data_ptr(), mask.data_ptr(),
                 0 if dtype == torch.bfloat16 else 1, self._lib.stream_ptr(dev))
         self._lib.check(rc, "ksa_expand_prompt")
         return ids, rope[0], rope[1], mask
+
+    def _expand_slots(self, ids, slot, C, S, begin, kinds, inv_freq, out_ids, cos, sin, row_stride):
+        dev = cos.device
+        with self._lib.on_device(dev):
+            rc = self._lib.lib().ksa_expand_slots(
+                None if ids is None else ids.data_ptr(), 0 if ids is None else ids.stride(0), 1 if ids is None else ids.shape[0],
+                slot, cos.shape[-2], C, S, begin, *kinds, inv_freq.data_ptr(), cos.shape[-1],
+                None if out_ids is None else out_ids.data_ptr(), cos.data_ptr(), sin.data_ptr(), row_stride,
+                0 if cos.dtype == torch.bfloat16 else 1, self._lib.stream_ptr(dev))
+        self._lib.check(rc, "ksa_expand_slots")
+
+    def expand_step(self, token_ids, index, boundary, config, inv_freq, dtype, out=None):
+        """Ids [b, rows] and rotary rows cos, sin [1, rows, D] of a decode step whose token is number `index` of the text (from
+        0): its row, at a chunk's end (`boundary`) also those of the summary tokens, in one launch (`ksa_expand_slots`).
+        `out`: the three to write to.  None where `boundary_position_ids` and torch have to do it."""
+        kinds = self._expand_kinds(config, inv_freq, dtype)
+        C, S, D = config.summary_chunk_size, config.summary_token_num, config.head_dim
+        if (kinds is None or token_ids.dtype != torch.long or token_ids.dim() != 2 or token_ids.shape[1] != 1
+                or token_ids.device != inv_freq.device or token_ids.shape[0] == 0 or C <= 0 or S <= 0
+                or index // C * (C + S) + index % C >= 1 << 30 or (boundary and index % C != C - 1)):
+            return None
+        b, rows = token_ids.shape[0], 1 + S if boundary else 1
+        if out is None:
+            rope = torch.empty(2, 1, rows, D, dtype=dtype, device=token_ids.device)
+            out = (torch.empty(b, rows, dtype=torch.long, device=token_ids.device) if boundary else token_ids, rope[0], rope[1])
+        self._expand_slots(token_ids, index // C * (C + S) + index % C, C, S, config.summary_token_begin, kinds, inv_freq,
+                           out[0] if boundary else None, out[1], out[2], D)
+        return out
+
+    def rope_rows(self, first, n, config, inv_freq, dtype, out=None):
+        """Rotary rows [n, 2, D] (cos, sin) of the positions first .. first + n - 1 in one launch; None where torch has to
+        make them."""
+        if self._expand_kinds(config, inv_freq, dtype) is None or not 0 <= first <= (1 << 30) - n:
+            return None
+        if out is None:
+            out = torch.empty(n, 2, config.head_dim, dtype=dtype, device=inv_freq.device)
+        self._expand_slots(None, first, 1 << 30, 1, 0, (0, 0), inv_freq, None, out[:, 0], out[:, 1], out.stride(0))
+        return out
 
     def decode(self, q, kbuf, vbuf, start, end, scale):
         return self._decode(q, kbuf, vbuf, start, end, scale=scale)
@@ -441,24 +486,16 @@ class KsaQwen3ForCausalLM:
         return (hasattr(self.ops, "decode_boundary") and hasattr(self.ops, "pre_attention_partials")
                 and not self.config.summary_independent_parameters)
 
-    def _boundary_row_table(self, text, base, b):
-        """int32 [b, 1 + S] on the device: the cache row of every token of a boundary step - the text token's
-        row `text`, summary token i at `base + i`; `text` / `base` ints or int32 device tensors [b]."""
-        S = self.config.summary_token_num
-        if not torch.is_tensor(text) and not torch.is_tensor(base):
-            row = [int(text)] + [int(base) + i for i in range(S)]
-            return torch.tensor([row] * b, dtype=torch.int32).to(self.device)
-        # (no host-to-device copies: this runs inside a recording)
-        some = text if torch.is_tensor(text) else base
-        as_rows = lambda v: v.to(torch.int32).expand(b) if torch.is_tensor(v) else torch.full_like(some, int(v), dtype=torch.int32).expand(b)
-        ar = torch.arange(S, dtype=torch.int32, device=self.device)
-        return torch.cat([as_rows(text)[:, None], as_rows(base)[:, None] + ar[None]], dim=1).contiguous()
+    def _boundary_rows(self, text, base):
+        """The cache row of every token of a boundary step, 1 + S of them: the text token's row `text`, summary token i
+        at `base + i`."""
+        return [int(text)] + [int(base) + i for i in range(self.config.summary_token_num)]
 
     def _boundary_qkv(self, lw, h, sum_rows, cos, sin, slots=None):
         """q, k, v [b, 1 + S, H, D] (normalised, rotated) of a chunk-boundary step's rows.  With one
         set of projection weights the product may stay the K-split partial sums of the few-rows GEMM,
         which the pre-attention kernel adds itself (one launch less).  `slots` = (key cache, value cache,
-        row table of `_boundary_row_table`): k and v go straight to those cache rows and are not returned."""
+        `_boundary_rows` of every sequence, int32 [b, 1 + S]): k and v go straight to those cache rows and are not returned."""
         cfg, ops = self.config, self.ops
         out = {}
         if slots is not None:
@@ -719,16 +756,22 @@ class KsaQwen3ForCausalLM:
         if boundary:
             self.check_steps(cache)   # before the step that cannot be undone (it flushes the chunk)
         ids = token_ids.to(self.device)
-        if boundary:
-            sids = torch.arange(S, device=self.device, dtype=ids.dtype) + cfg.summary_token_begin
-            ids = torch.cat([ids, sids[None].expand(b, -1)], dim=1)
-            pos = boundary_position_ids(true_tokens, cfg, self.device)
-            sum_rows = torch.arange(1, 1 + S, device=self.device)
+        # (where the row stands by the count of the text, which the cache's own place in the chunk has to agree with)
+        head = None
+        if hasattr(ops, "expand_step") and true_tokens % C == cache.get_cur_chunk_size():
+            head = ops.expand_step(ids, true_tokens, boundary, cfg, self.inv_freq_dev, self.dtype)
+        if head is not None:
+            ids, cos, sin = head
         else:
-            p = true_tokens if cfg.summary_chunk_position_ids_type == "origin" else cache.get_cur_chunk_size()
-            pos = torch.tensor([[p]], dtype=torch.long, device=self.device)
-            sum_rows = None
-        cos, sin = self._rope_tables(pos)
+            if boundary:
+                sids = torch.arange(S, device=self.device, dtype=ids.dtype) + cfg.summary_token_begin
+                ids = torch.cat([ids, sids[None].expand(b, -1)], dim=1)
+                pos = boundary_position_ids(true_tokens, cfg, self.device)
+            else:
+                p = true_tokens if cfg.summary_chunk_position_ids_type == "origin" else cache.get_cur_chunk_size()
+                pos = torch.tensor([[p]], dtype=torch.long, device=self.device)
+            cos, sin = self._rope_tables(pos)
+        sum_rows = torch.arange(1, 1 + S, device=self.device) if boundary and cfg.summary_independent_parameters else None
         x = self.w["embed_tokens"][ids]
         delta = None
         tables = {}   # boundary step: (text row, first summary row) -> row table on the device
@@ -758,7 +801,7 @@ class KsaQwen3ForCausalLM:
                 if fused and self._boundary_rows_in_cache():
                     key = (rows["text"], rows["spare"] if cache.is_large_window[li] else 0)
                     if key not in tables:  # the same for every layer of a kind: two small copies per step
-                        tables[key] = self._boundary_row_table(key[0], key[1], b)
+                        tables[key] = torch.tensor([self._boundary_rows(*key)] * b, dtype=torch.int32).to(self.device)
                     slots = (cache.key_cache[li], cache.value_cache[li], tables[key])
                 q, k, v = self._boundary_qkv(lw, h, sum_rows, cos, sin, slots)
                 qh = q.transpose(1, 2)
@@ -831,12 +874,10 @@ class KsaQwen3ForCausalLM:
         ids, bc = st["btok"], st["bcur"]
         b = ids.shape[0]
         sum_rows = st["bsum_rows"]
-        cos, sin = self._rope_tables(st["bpos"])
+        cos, sin = st["brope"]   # filled in front of the replay, as the ids, see `decode_step_graph`
         x = self.w["embed_tokens"][ids]
         delta = None
-        tables = None
-        if self._boundary_rows_in_cache():  # where the step's K/V rows go: small window, large window
-            tables = (self._boundary_row_table(bc[0, 0], 0, b), self._boundary_row_table(bc[1, 0], bc[1, 3], b))
+        tables = st["btab"] if self._boundary_rows_in_cache() else None
         for li, lw in enumerate(self.w["layers"]):
             kind = 1 if cache.is_large_window[li] else 0
             kc, vc, mv = cache.key_cache[li], cache.value_cache[li], cache._move_rows
@@ -936,19 +977,21 @@ class KsaQwen3ForCausalLM:
         nl = cfg.num_hidden_layers
         st = getattr(cache, "_ksa_graph_state", None)
         if st is None or st["batch"] != b or st["owner"] is not self:
-            sids = torch.arange(S, device=self.device, dtype=torch.long) + cfg.summary_token_begin
+            # (made on the host: no kernel of torch's is loaded for them)
+            on_dev = lambda rows: torch.tensor(rows, dtype=torch.long).to(self.device)
             st = {"batch": b, "owner": self, "graphs": {}, "rings": {},
                   "tok": torch.zeros(b, 1, dtype=torch.long, device=self.device),
                   # a step inside a chunk: [kind: small / large window][destination row, range start, range end]
                   # [sequence], and behind it the step's row of the rotary table
                   "step": torch.zeros(6 * b + 1, dtype=torch.int32, device=self.device),
-                  # the same for a boundary step (see `_boundary_step_body`), its ids and positions
-                  "bcur": torch.zeros(2, 6, b, dtype=torch.int32, device=self.device),
-                  "btok": torch.cat([torch.zeros(b, 1, dtype=torch.long, device=self.device),
-                                     sids[None].expand(b, -1)], dim=1).contiguous(),
-                  "bpos": torch.zeros(1, 1 + S, dtype=torch.int32, device=self.device),
-                  "bsum_rows": torch.arange(1, 1 + S, device=self.device),
+                  # the same for a boundary step (see `_boundary_step_body`), and behind it, for either kind of layer, where
+                  # its K/V rows go [sequence][token]; its ids and rotary rows
+                  "bstep": torch.zeros(2 * b * (7 + S), dtype=torch.int32, device=self.device),
+                  "btok": on_dev([[0] + [cfg.summary_token_begin + i for i in range(S)]] * b),
+                  "brope": tuple(torch.empty(1, 1 + S, D, dtype=self.dtype, device=self.device) for _ in range(2)),
+                  "bsum_rows": on_dev(list(range(1, 1 + S))),
                   "head": None}
+            st["bcur"], st["btab"] = st["bstep"][:12 * b].view(2, 6, b), st["bstep"][12 * b:].view(2, b, 1 + S)
             st["cur"], st["rope_rel"] = st["step"][:6 * b].view(2, 3, b), st["step"][6 * b:]
             emb, norm = self.w["embed_tokens"], self.w["layers"][0]["input_layernorm"]
             if getattr(self.ops, "embed_rmsnorm_supported", lambda *a: False)(emb, norm):
@@ -966,7 +1009,7 @@ class KsaQwen3ForCausalLM:
                     cache.boundary_fits_one_piece(li) and (kinds[li] or cache._chunk_buf_len[li] == C - 1)
                     for li in range(nl)):
                 return self.decode_step(token_ids, cache)
-            pos = boundary_position_ids(cache.get_true_token_num(), cfg, "cpu")[0].tolist()
+            n = cache.get_true_token_num()   # (`boundary_slots` counts the step)
             vals = [[0, 0, 1, 0, 0, 0], [0, 0, 1, 0, 0, 1]]
             seen = [None, None]
             for li in range(nl):
@@ -979,16 +1022,21 @@ class KsaQwen3ForCausalLM:
                     row = [sl["text"], a, e, sl["flush_dst"], sl["append"], 0]
                 assert seen[kinds[li]] in (None, row), "layers of one kind must move in step"
                 seen[kinds[li]] = vals[kinds[li]] = row
-            self._stage_ints(st, "bpos", pos)
-            st["btok"][:, :1].copy_(token_ids.to(self.device))
+            ids = token_ids.to(self.device)
+            if not hasattr(self.ops, "expand_step") or self.ops.expand_step(
+                    ids, n, True, cfg, self.inv_freq_dev, self.dtype, out=(st["btok"], *st["brope"])) is None:
+                st["btok"][:, :1].copy_(ids)
+                for dst, src in zip(st["brope"], self._rope_tables(boundary_position_ids(n, cfg, "cpu"))):
+                    dst.copy_(src)
+            table = self._boundary_rows(vals[0][0], 0) * b + self._boundary_rows(vals[1][0], vals[1][3]) * b
             # A boundary step is not idempotent (its flush overwrites ring rows that its text query
             # still attends), so the warm-up run flushes the chunk onto itself and appends the
             # summaries onto the scratch rows that already hold them.
             if ("boundary", b) not in getattr(self, "_graph_warm", ()):
                 harmless = [vals[0][:3] + [S, 0, 0], vals[1]]
-                self._stage_ints(st, "bcur", [v for kind in harmless for x in kind for v in [x] * b])
+                self._stage_ints(st, "bstep", [v for kind in harmless for x in kind for v in [x] * b] + table)
                 self._warm_up(st, "boundary", self._boundary_step_body, cache)
-            self._stage_ints(st, "bcur", [v for kind in vals for x in kind for v in [x] * b])
+            self._stage_ints(st, "bstep", [v for kind in vals for x in kind for v in [x] * b] + table)
             logits = self._replay(st, "boundary", self._boundary_step_body, cache)
             cache.reset_chunk_counter()
             return logits
@@ -1006,17 +1054,20 @@ class KsaQwen3ForCausalLM:
                 a, e = cache.attention_range(li)
                 vals[kinds[li]] = [rows[kinds[li]], a, e]
                 rows[kinds[li]] = None
-        # rotary rows of a window of positions, made with the prefill's own tensor ops (so a step's
-        # cos / sin are the values `_rope_tables` gives) and refilled in place when p leaves it; the
-        # recorded step only picks a row
+        # rotary rows of a window of positions (the values that `_rope_tables` gives), refilled in place when p leaves
+        # it; the recorded step only picks a row
         if st.get("rope_p0") is None or not (st["rope_p0"] <= p < st["rope_p0"] + st["rope_tab"].shape[0]):
             n = 1024
-            c, s_ = self._rope_tables(torch.arange(p, p + n, device=self.device)[None])
-            tab = torch.stack((c[0], s_[0]), dim=1)
-            if "rope_tab" in st:
-                st["rope_tab"].copy_(tab)
-            else:
+            tab = None
+            if hasattr(self.ops, "rope_rows"):
+                tab = self.ops.rope_rows(p, n, cfg, self.inv_freq_dev, self.dtype, out=st.get("rope_tab"))
+            if tab is None:
+                c, s_ = self._rope_tables(torch.arange(p, p + n, device=self.device)[None])
+                tab = torch.stack((c[0], s_[0]), dim=1)
+            if "rope_tab" not in st:
                 st["rope_tab"] = tab.contiguous()
+            elif tab is not st["rope_tab"]:
+                st["rope_tab"].copy_(tab)
             st["rope_p0"] = p
         self._stage_ints(st, "step", [v for kind in vals for x in kind for v in [x] * b] + [p - st["rope_p0"]])
         ids = token_ids

@@ -89,6 +89,69 @@ def test_gpu_expand_prompt_equals_host_form(text, C, S, D, kind, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["last_chunk_slice_right", "last_chunk_slice_left", "zeros"])
+@pytest.mark.parametrize("text,C,S,D", [("origin", 128, 8, 128), ("inner_chunk", 100, 7, 64), ("origin", 5, 3, 16)])
+def test_gpu_step_rows_equal_host_form(text, C, S, D, kind, dtype):
+    """Ids and rotary rows of a decode step at every kind of place, and stretches of the rotary table, bit for bit."""
+    from ksa_amd.model import HipOps
+    cfg = tiny_config(head_dim=D, summary_chunk_size=C, summary_token_num=S, summary_token_position_ids_type=kind,
+                      summary_chunk_position_ids_type=text, num_hidden_layers=1, summary_sliding_chunk_num=[2])
+    ops, model = HipOps(), KsaQwen3ForCausalLM(cfg, init_weights(cfg, "cuda", dtype, 0))
+    inv = model.inv_freq_dev
+    for b, index in ((1, 0), (3, C - 2), (2, C - 1), (1, C), (9, 7 * C - 1), (1, 20001 * C - 1), (1, 100003)):
+        tok = torch.randint(0, 200, (b, 2), device="cuda")[:, 1:]
+        boundary = index % C == C - 1
+        ids, cos, sin = ops.expand_step(tok, index, boundary, cfg, inv, dtype)
+        p = index if text == "origin" else index % C
+        pos = boundary_position_ids(index, cfg, "cpu") if boundary else torch.tensor([[p]])
+        want = model._rope_tables(pos)
+        assert torch.equal(cos, want[0]) and torch.equal(sin, want[1]), index
+        new = torch.arange(S)[None].expand(b, -1) + cfg.summary_token_begin
+        assert torch.equal(ids.cpu(), torch.cat([tok.cpu(), new], 1) if boundary else tok.cpu()), index
+    assert ops.expand_step(tok, C - 2, True, cfg, inv, dtype) is None and ops.expand_step(tok.int(), 3, False, cfg, inv, dtype) is None
+    for first in (0, 1000, 130000):
+        tab = ops.rope_rows(first, 33, cfg, inv, dtype)
+        want = model._rope_tables(torch.arange(first, first + 33)[None])
+        assert torch.equal(tab[:, 0], want[0][0]) and torch.equal(tab[:, 1], want[1][0])
+    buf = torch.full((35, 2, D), 7.0, dtype=dtype, device="cuda")
+    assert ops.rope_rows(5, 33, cfg, inv, dtype, out=buf[1:34]).data_ptr() == buf[1].data_ptr()
+    assert torch.equal(buf[1:34], ops.rope_rows(5, 33, cfg, inv, dtype)) and (buf[0] == 7).all() and (buf[34] == 7).all()
+    L = ops._lib.lib()
+    call = lambda **kw: L.ksa_expand_slots(*{**dict(ids=tok.data_ptr(), rs=1, b=1, slot0=0, n=1, C=C, S=S, beg=0, inner=0, kind=0,
+                                                    inv=inv.data_ptr(), D=D, out=None, cos=buf.data_ptr(), sin=buf.data_ptr(), rr=D,
+                                                    dt=0, st=None), **kw}.values())
+    for bad in (dict(b=0), dict(slot0=-1), dict(n=0), dict(slot0=2 ** 31 - 1), dict(C=0), dict(S=0), dict(C=2 ** 31 - 1), dict(D=24),
+                dict(inv=None), dict(cos=None), dict(sin=buf.data_ptr() + 2), dict(rr=D + 4), dict(ids=None, out=tok.data_ptr()), dict(kind=3), dict(dt=2)):
+        assert call(**bad) != 0, bad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("graph", [False, True])
+def test_gpu_steps_make_their_rows_without_torch(graph, monkeypatch):
+    """No step of a generation - the first one, the first at a chunk's end, the first recorded one - leaves its positions or rotary rows to
+    torch, whose kernels would have to be loaded in the middle of it; its logits are those of the torch form bit for bit."""
+    import ksa_amd.model as M
+    cfg = tiny_config(hidden_size=128, num_hidden_layers=2, summary_token_num=2, summary_sliding_chunk_num=[2, 1 << 20])
+    w = init_weights(cfg, "cuda", torch.bfloat16, 1)
+
+    class Plain(M.HipOps):
+        expand_step = rope_rows = lambda self, *a, **k: None
+    ids = torch.randint(0, 200, (2, 13), generator=torch.Generator().manual_seed(0)).cuda()
+    runs = []
+    for ops in (Plain(), M.HipOps()):
+        model = KsaQwen3ForCausalLM(cfg, w, ops)
+        model.BOUNDARY_GRAPH_AFTER = 2
+        if runs:
+            def refuse(*a, **k):
+                raise AssertionError("left to torch")
+            monkeypatch.setattr(model, "_rope_tables", refuse)
+            monkeypatch.setattr(M, "boundary_position_ids", refuse)
+        runs.append(model.generate(ids, 40, return_logits=True, use_graph=graph))
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])
+
+
+@pytest.mark.gpu
 def test_gpu_prefill_of_short_prompts_keeps_its_results():
     """The head of a prefill in one launch, closed-form cache rows and the attention without a mask change no bit of a prompt up to
     `GRID_ROWS`: logits and cache rows are those of the torch head, the mask and the grid of the block index."""
