@@ -112,6 +112,11 @@ bool fits(const at::Tensor& t) {
         if (s <= 0 || s > INT32_MAX) return false;
     return true;
 }
+// 16-byte items: what the library would refuse, behind the allocations
+bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+bool aligned(const at::Tensor& t) {
+    return aligned(t.const_data_ptr()) && ((t.stride(0) | t.stride(1) | t.stride(2)) & 7) == 0;
+}
 using Strides = std::array<int64_t, 3>;
 Strides first3(const at::Tensor& t) { return {t.stride(0), t.stride(1), t.stride(2)}; }
 
@@ -132,7 +137,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t b = q->size(0), Hq = q->size(1), Q = q->size(2), D = q->size(3), Hkv = k->size(1), rows = k->size(2);
     if (dt < 0 || k->scalar_type() != q->scalar_type() || v->scalar_type() != q->scalar_type() || k->get_device() != dev ||
         v->get_device() != dev || dev != c10::hip::current_device() || k->size(0) != b || k->size(3) != D || Hq % Hkv != 0 ||
-        !kernel_dim(D) || q->stride(3) != 1 || k->stride(3) != 1 || v->stride(3) != 1)
+        !kernel_dim(D) || q->stride(3) != 1 || k->stride(3) != 1 || v->stride(3) != 1 || !aligned(*q) || !aligned(*k) || !aligned(*v))
         Py_RETURN_NONE;
     const int32_t *start = nullptr, *end = nullptr;
     int s0 = 0, e0 = (int)rows, most = (int)rows;
@@ -152,7 +157,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     }
     float scale;
     int nsplit = 0;
-    if (!get_scale(a[5], D, scale) || (a[6] != Py_None && !get_int(a[6], nsplit))) Py_RETURN_NONE;
+    if (!get_scale(a[5], D, scale) || (a[6] != Py_None && (!get_int(a[6], nsplit) || nsplit < 1))) Py_RETURN_NONE;
     at::Tensor out;
     int rc;
     bool wide = false;
@@ -192,7 +197,8 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int64_t b = q->size(0), Sq = q->size(1), Hq = q->size(2), D = q->size(3), Hkv = k->size(2);
     if (dt < 0 || k->scalar_type() != q->scalar_type() || v->scalar_type() != q->scalar_type() || k->get_device() != dev ||
         v->get_device() != dev || dev != c10::hip::current_device() || k->size(0) != b || k->size(1) != Sq || k->size(3) != D ||
-        Hq % Hkv != 0 || !kernel_dim(D) || q->stride(3) != 1 || k->stride(3) != 1 || k->strides() != v->strides())
+        Hq % Hkv != 0 || !kernel_dim(D) || q->stride(3) != 1 || k->stride(3) != 1 || k->strides() != v->strides() ||
+        !aligned(*q) || !aligned(*k) || !aligned(*v) || Sq * k->stride(1) * 2 >= 1ll << 32)
         Py_RETURN_NONE;
     int C, S, W;
     float scale;
@@ -247,17 +253,20 @@ PyObject* pre_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     const int dt = dtype_of(*q), dev = q->get_device();
     const int64_t b = q->size(0), S = q->size(1), Hq = q->size(2), D = q->size(3), Hkv = k->size(2);
     auto same = [&](const at::Tensor* t) { return t && t->scalar_type() == q->scalar_type() && t->get_device() == dev; };
+    auto rows = [](const at::Tensor& t) { return aligned(t) && t.stride(2) >= 0 && t.stride(2) * 8 + 128 < 1ll << 32; };
     if (dt < 0 || !same(k) || !same(v) || dev != c10::hip::current_device() || k->size(0) != b || k->size(1) != S ||
-        k->size(3) != D || q->stride(3) != 1 || k->stride(3) != 1 || v->stride(3) != 1)
+        k->size(3) != D || (D != 64 && D != 128) || b * S >= (1ll << 31) - 64 || q->stride(3) != 1 || k->stride(3) != 1 ||
+        v->stride(3) != 1 || !rows(*q) || !rows(*k) || !rows(*v) || !(PyFloat_AS_DOUBLE(a[7]) >= 0))
         Py_RETURN_NONE;
     const at::Tensor* w[2];
     const at::Tensor* rope[2];
     for (int i = 0; i < 2; ++i) {
         w[i] = plain(a[3 + i], true);
         rope[i] = plain(a[5 + i], true);
-        if (!same(w[i]) || w[i]->dim() != 1 || w[i]->size(0) != D || !w[i]->is_contiguous()) Py_RETURN_NONE;
+        if (!same(w[i]) || w[i]->dim() != 1 || w[i]->size(0) != D || !w[i]->is_contiguous() || !aligned(w[i]->const_data_ptr()))
+            Py_RETURN_NONE;
         if (!same(rope[i]) || rope[i]->dim() != 3 || (rope[i]->size(0) != 1 && rope[i]->size(0) != b) || rope[i]->size(1) != S ||
-            rope[i]->size(2) != D || !rope[i]->is_contiguous())
+            rope[i]->size(2) != D || !rope[i]->is_contiguous() || !aligned(rope[i]->const_data_ptr()))
             Py_RETURN_NONE;
     }
     if (rope[0]->size(0) != rope[1]->size(0)) Py_RETURN_NONE;
@@ -266,7 +275,7 @@ PyObject* pre_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     for (int i = 0; i < 3; ++i) {
         given[i] = a[8 + i] == Py_None ? nullptr : plain(a[8 + i], true);
         if (a[8 + i] != Py_None &&
-            (!same(given[i]) || given[i]->sizes() != like[i]->sizes() || given[i]->stride(3) != 1))
+            (!same(given[i]) || given[i]->sizes() != like[i]->sizes() || given[i]->stride(3) != 1 || !rows(*given[i])))
             Py_RETURN_NONE;
     }
     const int32_t* kv_row = nullptr;
@@ -310,7 +319,7 @@ PyObject* block_index(PyObject*, PyObject* const* a, Py_ssize_t n) {
     int Sq, Sk, C, S, W, tm, tn;
     if (n != 8 || !quiet() || !get_int(a[0], Sq) || !get_int(a[1], Sk) || !get_int(a[2], C) || !get_int(a[3], S) ||
         !get_int(a[4], W) || !PyBool_Check(a[5]) || !get_int(a[6], tm) || !get_int(a[7], tn) || Sq <= 0 || Sk < Sq || tm <= 0 ||
-        tn <= 0)
+        tn <= 0 || C <= 0 || S <= 0 || W < 0)
         Py_RETURN_NONE;
     const int64_t M = ((int64_t)Sq + tm - 1) / tm, N = ((int64_t)Sk + tn - 1) / tn;
     const int dev = c10::hip::current_device();

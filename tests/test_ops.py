@@ -514,3 +514,35 @@ def test_native_front_never_launches_twice(code):
             _lib.fast.bind(_lib.check, *(address(getattr(L, n)) for n in _lib._FAST))
         assert seen == [code], name
         assert torch.equal(call(), want)
+
+
+@pytest.mark.gpu
+def test_native_front_allocates_nothing_for_what_it_leaves():
+    """Calls that the library refuses - addresses and strides off the 16-byte grid, head dimensions, arguments out
+    of range - are left to the general way in front of the first allocation."""
+    from ksa_amd import _lib
+    rnd = lambda *s: torch.randn(*s, device="cuda").bfloat16()
+    shifted = lambda *s: rnd(torch.Size(s).numel() + 4)[4:].view(s)          # 8 bytes off
+    odd = lambda *s: rnd(*s[:-1], s[-1] + 4)[..., :s[-1]]                    # rows 8 bytes off each other
+    q, kc, vc = rnd(2, 4, 1, 64), rnd(2, 2, 40, 64), rnd(2, 2, 40, 64)
+    f = _lib.fast
+    dec = lambda a=q, k=kc, v=vc, n=None: f.decode(a, k, v, None, None, None, n)
+    p, k, v = rnd(1, 200, 4, 64), rnd(1, 200, 2, 64), rnd(1, 200, 2, 64)
+    pre_ = lambda a=p, k=k, v=v, w=rnd(64), c=rnd(1, 200, 64), e=1e-6, o=None: f.pre_attention(a, k, v, w, w, c, c, e, o, None, None, None)
+    sa = lambda a=p, k=k, v=v: f.prefill(a, k, v, 128, 8, 1, False, None, False, None, None)
+    p256 = [rnd(1, 200, n, 256) for n in (4, 2, 2)]
+    w256, c256 = rnd(256), rnd(1, 200, 256)
+    args = [shifted(2, 4, 1, 64), odd(2, 4, 1, 64), shifted(2, 2, 40, 64), odd(2, 2, 40, 64), shifted(1, 200, 4, 64), odd(1, 200, 4, 64),
+            shifted(1, 200, 2, 64), odd(1, 200, 2, 64), shifted(64), shifted(1, 200, 64)]
+    for call in (dec, pre_, sa, lambda: f.block_index(400, 400, 128, 8, 2, False, 128, 64)):
+        assert call() is not None
+    left = [lambda: dec(args[0]), lambda: dec(args[1]), lambda: dec(k=args[2]), lambda: dec(v=args[3]), lambda: dec(n=0),
+            lambda: sa(args[4]), lambda: sa(args[5]), lambda: sa(k=args[6], v=args[6]), lambda: sa(k=args[7], v=args[7]),
+            lambda: pre_(args[4]), lambda: pre_(args[5]), lambda: pre_(k=args[6]), lambda: pre_(v=args[7]), lambda: pre_(w=args[8]),
+            lambda: pre_(c=args[9]), lambda: pre_(e=-1.0), lambda: pre_(e=float("nan")), lambda: pre_(o=args[4]),
+            lambda: pre_(*p256, w=w256, c=c256), lambda: f.block_index(400, 400, 0, 8, 2, False, 128, 64),
+            lambda: f.block_index(400, 400, 128, 8, -1, False, 128, 64)]
+    count = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    for i, call in enumerate(left):
+        before = count()
+        assert call() is None and count() == before, i
