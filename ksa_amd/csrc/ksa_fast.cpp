@@ -186,6 +186,22 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// `_chunk_tiles` of prefill.py for summary rows in line, and its `_QUEUE_ROWS`: written twice because compiled programs trace through
+// the Python ones; tests/test_host.py holds them together
+bool chunk_tiles(int64_t Sq, int64_t D, int64_t C, int64_t S) {
+    return C > 0 && C <= 512 && C % 128 == 0 && S > 0 && (8 % S == 0 || (S == 16 && D <= 128)) && Sq >= 64 && Sq < 1 << 29 &&
+           Sq % (C + S) <= C;
+}
+constexpr int64_t kQueueRows = 1 << 19;
+
+// layout_rules(Sq, D, C, S) -> (whether chunk tiles take it, kQueueRows)
+PyObject* layout_rules(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    int v[4];
+    for (int i = 0; i < 4; ++i)
+        if (n != 4 || !get_int(a[i], v[i])) return PyErr_Format(PyExc_TypeError, "layout_rules takes four ints");
+    return Py_BuildValue("Oi", chunk_tiles(v[0], v[1], v[2], v[3]) ? Py_True : Py_False, (int)kQueueRows);
+}
+
 // prefill(q, k, v, C, S, W, skip_old_summary, scale, return_lse, summary_pos, analyse): chunk tiles only.
 // analyse(summary_pos, Sq, C, S) -> (prefix rows, whether they lie in line, ...)
 PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -205,10 +221,7 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!get_int(a[3], C) || !get_int(a[4], S) || !get_int(a[5], W) || !PyBool_Check(a[6]) || !get_scale(a[7], D, scale) ||
         !PyBool_Check(a[8]))
         Py_RETURN_NONE;
-    // the layouts of `_chunk_tiles`
-    if (C <= 0 || C > 512 || C % 128 != 0 || S <= 0 || !(8 % S == 0 || (S == 16 && D <= 128)) || W < 0 || Sq < 64 ||
-        Sq >= 1 << 29 || Sq % (C + S) > C)
-        Py_RETURN_NONE;
+    if (!chunk_tiles(Sq, D, C, S) || W < 0) Py_RETURN_NONE;
     if (a[9] != Py_None) {
         if (!plain(a[9])) Py_RETURN_NONE;
         PyObject* r = PyObject_CallFunction(a[10], "OLii", a[9], (long long)Sq, C, S);
@@ -227,7 +240,7 @@ PyObject* prefill(PyObject*, PyObject* const* a, Py_ssize_t n) {
         out = at::empty_like(*q);
         if (a[8] == Py_True) lse = at::empty({b, Hq, Sq}, q->options().dtype(at::kFloat));
         at::Tensor sched;  // as in `_launch_chunks`
-        if (b * Hq * Sq >= 1 << 19) sched = at::empty({8}, q->options().dtype(at::kInt));
+        if (b * Hq * Sq >= kQueueRows) sched = at::empty({8}, q->options().dtype(at::kInt));
         const Strides qs = first3(*q), ks = first3(*k), os = first3(out);
         rc = lib.prefill_chunks_fwd(q->const_data_ptr(), k->const_data_ptr(), v->const_data_ptr(), out.mutable_data_ptr(),
                                     lse.defined() ? lse.mutable_data_ptr<float>() : nullptr, (int)b, (int)Sq, (int)Hq, (int)Hkv,
@@ -364,6 +377,7 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyMethodDef methods[] = {
 #define KSA_METHOD(name) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(name)), METH_FASTCALL, nullptr}
     KSA_METHOD(bind), KSA_METHOD(decode), KSA_METHOD(prefill), KSA_METHOD(pre_attention), KSA_METHOD(block_index),
+    KSA_METHOD(layout_rules),
 #undef KSA_METHOD
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_fast", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -184,6 +184,9 @@ def fold_scale(q: torch.Tensor, scale: float):
 
 
 _CHUNK_MAX = 512   # the largest chunk that takes tiles laid along the chunks (ksa_prefill_chunks_fwd)
+# From so many rows of all heads on a launch is long enough to use work queues (the library's own bound is 32 workgroups
+# per CU; a workgroup takes 128 rows of one or two heads).  This and `_chunk_tiles` stand in csrc/ksa_fast.cpp as well.
+_QUEUE_ROWS = 1 << 19
 
 
 def _chunk_tiles(Sq: int, D: int, C: int, S: int, P: int, phys: bool) -> bool:
@@ -200,9 +203,7 @@ def _launch_chunks(q, k, v, C, S, W, skip_old, scale, want_lse):
     dev = q.device
     out = torch.empty_like(q)
     lse = torch.empty((b, Hq, Sq), dtype=torch.float32, device=dev) if want_lse else None
-    # work queues of this call alone, for a launch long enough to use them (the library's own bound is 32
-    # workgroups per CU; a workgroup takes 128 rows of one or two heads)
-    sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= 1 << 19 else None
+    sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= _QUEUE_ROWS else None  # of this call alone
     dims = (0, 1, 2)
     with _lib.on_device(dev):
         rc = _lib.lib().ksa_prefill_chunks_fwd(
@@ -221,7 +222,7 @@ def _launch_prefill(q, k, v, mask_cnt, mask_idx, full_cnt, full_idx, C, S, W, P,
     dev = q.device
     out = torch.empty_like(q)
     lse = torch.empty((b, Hq, Sq), dtype=torch.float32, device=dev) if want_lse else None
-    sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= 1 << 19 else None  # as in _launch_chunks
+    sched = torch.empty(8, dtype=torch.int32, device=dev) if b * Hq * Sq >= _QUEUE_ROWS else None  # as in _launch_chunks
     dims = (0, 1, 2)
     with _lib.on_device(dev):
         rc = _lib.lib().ksa_prefill_fwd(

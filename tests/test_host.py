@@ -332,6 +332,25 @@ def test_decode_splits_rule(b, hq, hkv, q):
     assert L.ksa_decode_splits(1, 32, 7, 1, 128, 1000) == 1 and L.ksa_decode_splits(0, 32, 8, 1, 128, 1000) == 1
 
 
+def test_rules_of_the_native_front_are_those_of_the_general_way():
+    """Which prompts take chunk tiles and which launches get work queues, over chunks, summaries, head dimensions and lengths on
+    both sides of every line: the same in the native front and in Python."""
+    from ksa_amd import _lib, prefill
+    if _lib.fast is _lib._GeneralWay:
+        pytest.skip("no native front")
+    for C in (0, 1, 64, 100, 127, 128, 129, 256, 384, 500, 512, 513, 640, 1024):
+        for S in (0, 1, 2, 3, 4, 5, 7, 8, 9, 12, 15, 16, 17, 32, 64):
+            for D in (64, 128, 256):
+                B = C + S
+                for Sq in {1, 63, 64, 65, 127, 128, B - 1, B, B + 1, C, C + 1, 3 * B, 3 * B + C - 1, 3 * B + C, 3 * B + C + 1, 4 * B - 1,
+                           9001, 139264, (1 << 29) - 1, 1 << 29, (1 << 31) - 1}:
+                    if Sq <= 0:
+                        continue
+                    got, queue = _lib.fast.layout_rules(Sq, D, C, S)
+                    want = C > 0 and S > 0 and prefill._chunk_tiles(Sq, D, C, S, Sq // B * S, False)
+                    assert got == want and queue == prefill._QUEUE_ROWS, (C, S, D, Sq)
+
+
 @pytest.mark.parametrize("broken", ["missing", "other"])
 def test_package_without_its_native_front(broken):
     """A native front that does not load (it is built against one PyTorch) or that is another build's leaves the Python way,
