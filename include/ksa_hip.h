@@ -168,13 +168,15 @@ int ksa_decode_qkv_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_
                        const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
                        const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
                        float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
-/* ... in workgroups of eight waves, as ksa_decode_wide_fwd (Hq / Hkv <= 16) */
+/* ... in workgroups of eight waves, as ksa_decode_wide_fwd (Hq / Hkv <= 16).  ksa_decode_qkv_wide_splits: the count to call it with,
+ * all workgroups at once, or 0 where it is not the faster form. */
 int ksa_decode_qkv_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
                        const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
                        void* vcache, void* out, const int32_t* row, int row0, const int32_t* start,
                        const int32_t* end, int start0, int end0, int batch, int Hq, int Hkv, int D, int dtype,
                        const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides,
                        float scale, int nsplit, void* workspace, size_t workspace_bytes, void* stream);
+int ksa_decode_qkv_wide_splits(int batch, int Hq, int Hkv, int D, int max_rows);
 
 /* ksa_decode_qkv_fwd and the o projection behind it (HF:879) in one launch, for at most 16 sequences: the workgroups of the
  * product request their weights and wait for the attention of their heads.  Instead of out:
@@ -204,7 +206,7 @@ int ksa_decode_qkv_o_fwd(const float* qkv_partials, int qkv_ksplit, const void* 
                          size_t step_workspace_bytes, void* stream);
 
 /* ... in workgroups of eight waves, as ksa_decode_wide_fwd (Hq / Hkv <= 16).  _splits: the count to call it with, 0 where it does
- * not take the sizes; _pays: whether it is faster than ksa_decode_qkv_wide_fwd and ksa_gemm_rows behind it. */
+ * not take the sizes or ksa_decode_qkv_o_fwd is the faster form; _pays: whether it is faster than the two launches. */
 int ksa_decode_qkv_o_wide_fwd(const float* qkv_partials, int qkv_ksplit, const void* q_weight, const void* k_weight,
                          const void* cos, const void* sin, long long cos_batch_stride, float eps, void* kcache,
                          void* vcache, const int32_t* row, int row0, const int32_t* start, const int32_t* end,

@@ -82,6 +82,7 @@ _SIGNATURES = {
     "ksa_gemm_rows_gate_up_silu": (_int, [_vp] * 3 + [_int] * 3 + [ctypes.c_longlong] * 3 + [_int, _vp]),
     "ksa_mlp_rows_down_splits": (_int, [_int, _int]),
     "ksa_mlp_rows_workspace_bytes": (ctypes.c_size_t, [_int, _int]),
+    "ksa_decode_qkv_wide_splits": (_int, [_int] * 5),
     "ksa_mlp_rows_status_offset": (ctypes.c_size_t, []),
     "ksa_mlp_rows": (_int, [_vp] * 4 + [_int] * 3 + [ctypes.c_longlong] * 3 + [_int, _vp, ctypes.c_size_t, _vp]),
     "ksa_add_rmsnorm_mlp_rows": (_int, [_vp, _int] + [_vp] * 6 + [_int] * 3 + [ctypes.c_longlong] * 4

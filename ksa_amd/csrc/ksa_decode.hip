@@ -1202,20 +1202,12 @@ extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int m
     return n < 1 ? 1 : (int)n;
 }
 
-// Number of splits for ksa_decode_wide_fwd, or 0 where ksa_decode_fwd is the one to call: more than 16 columns, head_dim 256, and
-// more pairs of sequence and kv head than CUs over few rows, where two of its workgroups share a CU (48 / 64 sequences of
-// 8 kv heads, 150 / 300 / 500 rows 11.3 / 16.6 / 21.5 against 12.3 / 17.0 / 24.0 us, 12.3 / 19.0 / 25.3 against 13.2 / 19.2 / 25.8;
-// 737 rows 33.6 against 30.9, 35.2 against 34.2).
-// The count is the one with the least time by what was measured of one workgroup to a CU, for 1 to 64 sequences of 150 to 9000 rows:
-// 3 us for the start of each round of workgroups, 10.2 ns a row of head_dim 128 and CU when the other CUs are idle and 9.4 more when all
-// are at work, 2.4 to 4 us for the merge.  Of those shapes the count is within 4 % of the best of twelve counts but for 16
-// sequences of 1100 rows and 2 of 500.
-extern "C" int ksa_decode_wide_splits(int batch, int Hq, int Hkv, int Q, int D, int max_rows) {
-    if (batch <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || Q <= 0 || max_rows <= 0 || (D != 64 && D != 128)) return 0;
-    const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
-    if ((int64_t)Q * (Hq / Hkv) > kWideColumns || (units > cus && max_rows <= 600)) return 0;
-    const int64_t tiles = ((int64_t)max_rows + kWideRows - 1) / kWideRows;
-    int64_t most = 4 * cus / units;
+// Split count of the wide kernel, at most `most`: the one with the least time by what was measured of one workgroup to a CU, 3 us for the
+// start of the first round of workgroups and 5 of each one behind it, 10.2 ns a row of head_dim 128 and CU when the other CUs are idle and
+// 9.4 more when all are at work (half of that at head_dim 64), 2.2 to 3.8 us for the merge.  Against the best of nine counts around it
+// (2081 calls): within 5 % but for 18.
+static int wide_count(int64_t units, int D, int64_t max_rows, int64_t cus, int64_t most) {
+    const int64_t tiles = (max_rows + kWideRows - 1) / kWideRows;
     most = most < tiles ? most : tiles;
     most = most < 1 ? 1 : most < 64 ? most : 64;
     const double row = D / 128.0 * 0.0102, load = D / 128.0 * 0.0094;
@@ -1227,12 +1219,48 @@ extern "C" int ksa_decode_wide_splits(int batch, int Hq, int Hkv, int Q, int D, 
         if (used == before) continue;
         before = used;
         const int64_t wgs = units * used, full = wgs / cus, rest = wgs % cus;
-        double us = full * (3.0 + per * kWideRows * (row + load));
-        if (rest) us += 3.0 + per * kWideRows * (row + load * rest / cus);
-        if (used > 1) us += 2.4 + (full ? 1.6 : 1.6 * rest / cus);
+        double us = full * (5.0 + per * kWideRows * (row + load));
+        if (rest) us += 5.0 + per * kWideRows * (row + load * rest / cus);
+        if (used > 1) us += 2.2 + (full ? 1.6 : 1.6 * rest / cus);
         if (us < least) least = us, best = used;
     }
     return best;
+}
+
+// Number of splits for ksa_decode_wide_fwd, or 0 where ksa_decode_fwd is the one to call: more than 16 columns, head_dim 256, and
+// where it measured faster.  Both were timed in graphs over 1 to 64 sequences, eight forms of heads, 150 to 131000 rows: of 3848 calls
+// 3636 taken, 0.91 times the time of the other on average, more than 1.04 times in 33 (profiles/decode_wide_vs_four_waves.md).
+//  - More pairs of sequence and kv head than CUs (units) over few rows: two of its workgroups share a CU.  Up to 600 rows: 48 / 64
+//    sequences of 8 kv heads, 150 / 300 / 500 rows 11.3 / 16.6 / 21.5 against 12.3 / 17.0 / 24.0 us, 12.3 / 19.0 / 25.3 against
+//    13.2 / 19.2 / 25.8.  Up to 2500 rows from one and a half rounds of units on, and below that from 1200 rows on: 512 units of 737 /
+//    2000 rows 1.04 to 1.07 (head_dim 64: 1.03 to 1.10) times its time, 1536 and 2048 of 737 1.08 (1.13), 384 of 2000 1.02 to 1.05; but 384
+//    of 1100 rows 0.89 to 0.97.
+//  - head_dim 128, its workgroups are one to a CU at the most and walk their rows in one round (128 rows), and slices here are longer than
+//    a wave's 64 rows: 2 to 4 of the eight waves then have rows, 64 of them each where its four have 32.  8 units of 2000 rows 1.04 to
+//    1.08 times its time, 24 of 737 1.04 to 1.09, 32 of 900 1.05 to 1.07; in slices of 64 rows 0.93 to 1.03.  (Head_dim 64: 0.93 to 1.10,
+//    as fast on average.)
+extern "C" int ksa_decode_wide_splits(int batch, int Hq, int Hkv, int Q, int D, int max_rows) {
+    if (batch <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0 || Q <= 0 || max_rows <= 0 || (D != 64 && D != 128)) return 0;
+    const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
+    if ((int64_t)Q * (Hq / Hkv) > kWideColumns) return 0;
+    if (units > cus && max_rows <= 2500 && (max_rows <= 600 || max_rows > 1200 || 2 * units > 3 * cus)) return 0;
+    const int best = wide_count(units, D, max_rows, cus, 4 * cus / units), four = ksa_decode_splits(batch, Hq, Hkv, Q, D, max_rows);
+    if (D == 128 && (int64_t)best * kWideRows < max_rows && four > 1 && units * four <= cus && four * 128 >= max_rows) return 0;
+    return best;
+}
+
+// The same for ksa_decode_qkv_wide_fwd, where all workgroups run at once: so the outputs are bit for bit those of ksa_decode_wide_fwd behind
+// the pre-attention step wherever that runs in one round.  Of 32 / 8 heads, 1 to 32 sequences of 737 to 24000 rows 0.64 to 1.03 times the
+// time of what took its place before.  Not taken for long ranges where one round of slices leaves CUs idle, and their share of the memory's
+// rate: 11 / 12 sequences of 8 kv heads, 176 / 192 workgroups, 6000 to 24000 rows 1.04 to 1.10; at head_dim 64 17 to 21 sequences of
+// 12000 and 24000 rows 1.02 to 1.16.
+extern "C" int ksa_decode_qkv_wide_splits(int batch, int Hq, int Hkv, int D, int max_rows) {
+    const int n = ksa_decode_wide_splits(batch, Hq, Hkv, 1, D, max_rows);
+    const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
+    if (n == 0 || units > cus) return 0;
+    const int64_t most = cus / units, round = most * units;
+    if (D == 128 ? 5 * round < 4 * cus && max_rows > 5000 : 3 * round < 2 * cus && max_rows > 10000) return 0;
+    return n < most ? n : (int)most;
 }
 
 namespace {
@@ -1599,12 +1627,15 @@ extern "C" int ksa_decode_qkv_o_wide_fwd(const float* qkv_partials, int qkv_kspl
 // Splits of ksa_decode_qkv_o_wide_fwd, or 0 where it does not take the call.  The terms of ksa_decode_wide_splits without rounds (one
 // workgroup to a CU), 30 ns for every row and split that a workgroup of the product merges, and 4 us more where the product's
 // workgroups have to wait for a CU: 32 / 8 heads of 128, N 2560, 8 sequences of 737 / 1100 / 4097 rows in 2 / 4 splits 16.2 / 19.2 / 38.7
-// and 19.2 / 20.5 / 34.9 us (176 CUs are left to the attention, 64 slices a split).
+// and 19.2 / 20.5 / 34.9 us (176 CUs are left to the attention, 64 slices a split).  Not taken either where the four-wave form is faster:
+// long ranges at head_dim 128 where a round of slices leaves more than a fifth of the CUs idle, 11 / 12 sequences of 8 kv heads, 9000 to
+// 34816 rows 1.02 to 1.08 times its time.
 extern "C" int ksa_decode_qkv_o_wide_splits(int batch, int Hq, int Hkv, int D, int N, int max_rows) {
     if (batch <= 0 || batch > 16 || Hkv <= 0 || Hkv > kStepMaxHeads || Hq <= 0 || Hq % Hkv != 0 || Hq / Hkv > kWideColumns || N <= 0 ||
         N % 16 != 0 || max_rows <= 0 || (D != 64 && D != 128) || Hq * D % kChunkK != 0 || Hq * D > 64 * kChunkK)
         return 0;
     const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
+    if (units > cus || (D == 128 && 5 * (cus / units * units) < 4 * cus && max_rows > 5000)) return 0;
     const int64_t room = cus - o_workgroups(N, Hq * D / kChunkK, kWideWaves);
     const int64_t tiles = ((int64_t)max_rows + kWideRows - 1) / kWideRows;
     int64_t most = cus / units;
@@ -1625,17 +1656,18 @@ extern "C" int ksa_decode_qkv_o_wide_splits(int batch, int Hq, int Hkv, int D, i
     return best;
 }
 
-// Whether ksa_decode_qkv_o_wide_fwd is faster than ksa_decode_qkv_wide_fwd and ksa_gemm_rows behind it: 499 shapes timed (17 of heads, head_dim
-// and N, 1 to 16 sequences of 300 to 16384 rows; graphs), 360 taken, 0.89 of the two launches on average, 1.05 at the worst.
+// Whether ksa_decode_qkv_o_wide_fwd is faster than ksa_decode_qkv_fwd in its faster form and ksa_gemm_rows behind it
+// (1630 shapes timed - 17 of heads, head_dim and N, 1 to 16 sequences of 300 to 34816 rows; graphs -, 1024 taken, 0.91 of the two on average,
+// more than 1.03 in 15; profiles/decode_wide_vs_four_waves.md).
 // Left to the two: a product of more workgroups than CUs (64 heads, N 5120 up to 1.20); few kv heads over long ranges (16 / 2
-// heads, 4097 rows and more up to 1.19), whose count the sums limit; half a CU's worth of slices and more of few heads (16 / 8,
+// heads, 4352 rows and more up to 1.26 times the two), whose count the sums limit; half a CU's worth of slices and more of few heads (16 / 8,
 // 16 x 300 rows 1.06) or of any (32 / 32, 8 x 300 1.15); at head_dim 64 few rows (1.05 to 1.15), many slices (1.1 to 1.46) and
 // long ranges (1.01 to 1.09).
 extern "C" int ksa_decode_qkv_o_wide_pays(int batch, int Hq, int Hkv, int D, int N, int max_rows) {
     if (ksa_decode_qkv_o_wide_splits(batch, Hq, Hkv, D, N, max_rows) == 0) return 0;
     const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
     if (o_workgroups(N, Hq * D / kChunkK, kWideWaves) > cus) return 0;
-    if (Hkv < 4 && (Hq * D < 4096 || max_rows > 2048)) return 0;
+    if (Hkv < 4 && max_rows > (Hq * D < 4096 ? 1100 : 2048)) return 0;
     if (D == 128) return 2 * units < cus || (2 * units == cus && Hq * D >= 4096);
     return 8 * units <= 3 * cus && max_rows >= 600 && max_rows <= 8192;
 }

@@ -154,12 +154,10 @@ def decode_qkv_supported(Hq: int, Hkv: int, D: int) -> bool:
 
 
 def _qkv_splits(b: int, Hq: int, Hkv: int, D: int, max_rows: int) -> Tuple[int, bool]:
-    """(splits, whether in workgroups of eight waves) of a `ksa_decode_qkv` call that names no count, on the current GPU.  Of the
-    wide ones no more than a workgroup per CU, so that all run at once."""
+    """(splits, whether in workgroups of eight waves) of a `ksa_decode_qkv` call that names no count, on the current GPU."""
     L = _lib.lib()
-    cus = max(1, L.ksa_device_cu_count())
-    n = _wide_splits(b, Hq, Hkv, 1, D, max_rows) if b * Hkv <= cus else 0
-    return (min(n, cus // (b * Hkv)), True) if n else (L.ksa_decode_splits(b, Hq, Hkv, 1, D, max_rows), False)
+    n = L.ksa_decode_qkv_wide_splits(b, Hq, Hkv, D, max_rows)
+    return (n, True) if n else (L.ksa_decode_splits(b, Hq, Hkv, 1, D, max_rows), False)
 
 
 def decode_qkv_pays(kcache: torch.Tensor, Hq: int, start, end) -> bool:
@@ -253,14 +251,15 @@ def decode_qkv_o_supported(kcache: torch.Tensor, Hq: int, N: int) -> bool:
 
 
 def decode_qkv_o_pays(kcache: torch.Tensor, Hq: int, N: int, start, end) -> bool:
-    """Whether `ksa_decode_qkv_o` is the faster way (`ksa_decode_qkv_o_wide_pays`, for groups of more than 16 heads, which the wide
-    form does not take, `ksa_decode_qkv_o_pays`; by the longest possible range where the ranges are on the device)."""
+    """Whether `ksa_decode_qkv_o` is the faster way (`ksa_decode_qkv_o_wide_pays`, or `ksa_decode_qkv_o_pays` where the wide form is not
+    taken, as for groups of more than 16 heads; by the longest possible range where the ranges are on the device)."""
     b, Hkv, rows, D = kcache.shape
     if not (isinstance(start, torch.Tensor) or isinstance(end, torch.Tensor)):
         rows = max(1, int(end) - int(start))
     with _lib.on_device(kcache.device):
         L = _lib.lib()
-        return (L.ksa_decode_qkv_o_wide_pays if Hq // Hkv <= 16 else L.ksa_decode_qkv_o_pays)(b, Hq, Hkv, D, N, rows) != 0
+        wide = L.ksa_decode_qkv_o_wide_splits(b, Hq, Hkv, D, N, rows) > 0
+        return (L.ksa_decode_qkv_o_wide_pays if wide else L.ksa_decode_qkv_o_pays)(b, Hq, Hkv, D, N, rows) != 0
 
 
 def ksa_decode_qkv_o(qkv, q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,

@@ -591,7 +591,7 @@ def test_decode_wide_workgroups_refuse_what_they_do_not_take():
 @pytest.mark.parametrize("b,Hq,Hkv,D,N,nsplit", [
     (1, 32, 8, 128, 2560, None), (1, 32, 8, 128, 256, 1), (1, 16, 2, 128, 144, 39), (1, 8, 4, 64, 16, 64), (1, 64, 4, 64, 272, 2),
     (2, 32, 8, 128, 272, 32), (3, 8, 8, 64, 128, 21), (5, 4, 2, 128, 512, 7), (7, 16, 1, 128, 528, 3), (16, 32, 8, 128, 1024, 4),
-    (16, 32, 8, 128, 2560, None),
+    (8, 32, 8, 128, 2560, None), (16, 32, 8, 128, 2560, None),
 ])
 def test_decode_qkv_o_wide_equals_separate_launches(dtype, b, Hq, Hkv, D, N, nsplit):
     """The wide form of a step's attention, alone and with the o projection in the launch, with ranges from one row to all (later

@@ -438,6 +438,69 @@ def test_decode_splits_of_column_blocks(b, hq, hkv, q, D):
             assert n % a == 0 or n < a
 
 
+def _cus_of_the_rules(L):
+    if L.ksa_device_cu_count() not in (0, 256):
+        pytest.skip("the figures are those of 256 CUs")
+
+
+@pytest.mark.parametrize("b,Hq,Hkv,Q,D,rows,n", [
+    (1, 32, 8, 1, 128, 150, 1), (1, 32, 8, 1, 128, 737, 12), (1, 32, 8, 1, 128, 1500, 24),          # slices of one tile
+    (1, 32, 8, 1, 128, 2000, 0), (8, 32, 8, 1, 128, 500, 0), (3, 32, 8, 1, 128, 737, 0),            # of two: four waves of 32 rows
+    (1, 32, 8, 1, 64, 2000, 16), (3, 32, 8, 1, 64, 1100, 6), (1, 32, 8, 1, 128, 4100, 22),          # (not at head_dim 64)
+    (8, 32, 8, 1, 128, 737, 4), (8, 32, 8, 1, 128, 1500, 4), (8, 32, 8, 1, 128, 4352, 4),
+    (1, 32, 8, 1, 128, 9000, 29), (1, 32, 8, 1, 128, 131072, 32), (32, 32, 8, 1, 128, 500, 1),
+    (12, 32, 8, 1, 128, 4100, 2),                                                                   # one round, not two
+    (33, 32, 8, 1, 128, 600, 0), (33, 32, 8, 1, 128, 601, 1), (33, 32, 8, 1, 128, 1200, 1), (33, 32, 8, 1, 128, 1201, 0),
+    (33, 32, 8, 1, 128, 2500, 0), (33, 32, 8, 1, 128, 2501, 2), (48, 32, 8, 1, 128, 1100, 1), (49, 32, 8, 1, 128, 1100, 0),
+    (64, 32, 8, 1, 128, 2500, 0), (64, 32, 8, 1, 128, 2501, 1), (64, 32, 8, 1, 128, 8704, 1),       # more slices than CUs
+    (4, 32, 8, 1, 64, 24000, 8), (31, 8, 1, 1, 64, 131072, 8),
+    (1, 32, 8, 4, 128, 737, 12), (1, 32, 8, 5, 128, 737, 0), (1, 32, 2, 1, 128, 737, 12), (1, 34, 2, 1, 128, 737, 0),   # columns
+    (1, 32, 8, 1, 256, 737, 0), (1, 32, 8, 1, 96, 737, 0), (1, 33, 8, 1, 128, 737, 0), (1, 32, 8, 1, 128, 0, 0),
+])
+def test_decode_wide_splits_on_both_sides_of_each_line(b, Hq, Hkv, Q, D, rows, n):
+    """Which decode calls take workgroups of eight waves, and with how many splits (0: the four-wave kernel is faster)."""
+    from ksa_amd import _lib
+    _cus_of_the_rules(_lib.lib())
+    assert _lib.lib().ksa_decode_wide_splits(b, Hq, Hkv, Q, D, rows) == n
+
+
+@pytest.mark.parametrize("b,Hq,Hkv,D,rows,n", [
+    (1, 32, 8, 128, 737, 12), (1, 32, 8, 128, 2000, 0), (1, 32, 8, 64, 2000, 16), (8, 32, 8, 128, 4352, 4), (32, 32, 8, 128, 131072, 1),
+    (33, 32, 8, 128, 737, 0), (1, 34, 2, 128, 737, 0), (1, 32, 8, 256, 737, 0), (1, 33, 8, 128, 737, 0), (1, 32, 8, 128, 0, 0),
+    (12, 32, 8, 128, 5000, 2), (12, 32, 8, 128, 5001, 0), (13, 32, 8, 128, 5001, 2), (25, 32, 8, 128, 5001, 0), (26, 32, 8, 128, 5001, 1),
+    (21, 32, 8, 64, 10000, 1), (21, 32, 8, 64, 10001, 0), (22, 32, 8, 64, 10001, 1), (12, 32, 8, 64, 10001, 2),
+])
+def test_decode_qkv_wide_splits_on_both_sides_of_each_line(b, Hq, Hkv, D, rows, n):
+    """The same for a step with the pre-attention in it: one round of workgroups, and none that leaves CUs idle over long ranges."""
+    from ksa_amd import _lib
+    _cus_of_the_rules(_lib.lib())
+    assert _lib.lib().ksa_decode_qkv_wide_splits(b, Hq, Hkv, D, rows) == n
+
+
+@pytest.mark.parametrize("b,Hq,Hkv,D,N,rows,n,pays", [
+    (1, 32, 8, 128, 2560, 737, 12, 1), (1, 32, 8, 128, 2560, 4097, 22, 1), (8, 32, 8, 128, 2560, 737, 2, 1),
+    (8, 32, 8, 128, 2560, 4352, 4, 1), (16, 32, 8, 128, 2560, 4097, 2, 1),
+    (17, 32, 8, 128, 2560, 737, 0, 0), (1, 136, 8, 64, 2560, 737, 0, 0), (1, 128, 8, 64, 2560, 737, 12, 1),             # batch, columns
+    (1, 32, 8, 256, 2560, 737, 0, 0), (1, 32, 8, 128, 2568, 737, 0, 0), (1, 32, 8, 128, 2560, 0, 0, 0),
+    (1, 64, 8, 128, 4096, 737, 12, 1), (1, 64, 8, 128, 4112, 737, 12, 0), (1, 64, 8, 128, 5120, 400, 7, 0),             # product > CUs
+    (1, 16, 2, 128, 2048, 1100, 18, 1), (1, 16, 2, 128, 2048, 1101, 18, 0), (1, 32, 2, 128, 2048, 2048, 32, 1),         # few kv heads
+    (1, 32, 2, 128, 2048, 2049, 33, 0), (1, 32, 4, 128, 2048, 2049, 33, 1),
+    (12, 32, 8, 128, 2560, 5000, 2, 1), (12, 32, 8, 128, 2560, 5001, 0, 0), (13, 32, 8, 128, 2560, 5001, 2, 1),         # idle CUs
+    (12, 32, 8, 64, 2048, 5001, 2, 1), (5, 32, 8, 128, 2560, 131072, 6, 1),
+    (16, 16, 8, 128, 2048, 300, 1, 0), (15, 16, 8, 128, 2048, 300, 1, 1), (16, 32, 8, 128, 2048, 300, 1, 1),            # half the CUs
+    (8, 32, 32, 128, 4096, 300, 1, 0), (4, 32, 32, 128, 4096, 300, 1, 1),
+    (1, 32, 8, 64, 2048, 599, 10, 0), (1, 32, 8, 64, 2048, 600, 10, 1), (1, 32, 8, 64, 2048, 8192, 26, 1),              # head_dim 64
+    (1, 32, 8, 64, 2048, 8193, 26, 0), (12, 32, 8, 64, 2048, 1000, 2, 1), (13, 32, 8, 64, 2048, 1000, 2, 0),
+])
+def test_wide_attention_and_o_projection_on_both_sides_of_each_line(b, Hq, Hkv, D, N, rows, n, pays):
+    """The split count of the one launch in workgroups of eight waves (0: not taken), and whether it is faster than the two."""
+    from ksa_amd import _lib
+    L = _lib.lib()
+    _cus_of_the_rules(L)
+    assert L.ksa_decode_qkv_o_wide_splits(b, Hq, Hkv, D, N, rows) == n
+    assert L.ksa_decode_qkv_o_wide_pays(b, Hq, Hkv, D, N, rows) == pays
+
+
 def test_attention_and_o_projection_in_one_launch_where_it_is_faster():
     """The rule for the one launch at 256 CUs, both sides of each of its lines, and the split counts that it rests on (the
     counts of the attention alone beside them): what measured slower goes to the separate launches."""
