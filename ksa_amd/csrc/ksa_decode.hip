@@ -474,7 +474,8 @@ __global__ __launch_bounds__(kThreads, (D <= 128 ? 2 : 1)) void ksa_decode_kerne
         }
         if (row0 < s1) load_tile(row0);
     } else {
-        // (ksa_decode_new_row written out: called here, the compiler keeps 66 scalar registers more and spills 16 others to memory)
+        // (ksa_decode_new_row written out: called here, the compiler keeps 66 scalar registers more and spills 16 others to memory; the
+        // tests hold both, bit for bit, against ksa_pre_attention_partials)
         using C = KsaCvt<T>;
         constexpr int LPR = D / 8;      // lanes per head row
         constexpr int RPW = 64 / LPR;   // head rows per wave
@@ -751,12 +752,14 @@ __global__ __launch_bounds__(kThreads) void ksa_decode_merge_kernel(const Decode
 // trips - a tile's loads, LDS, scores, sums - with 64 KB on its way, and a launch of few sequences is some of them and a merge.
 // Here a wave takes 64 rows at once on 16x16x32 products: with 16 columns instead of 32 the sums take half the registers, K goes
 // from memory straight to the operand registers (64 bytes of 16 rows an instruction), V through LDS, and a round's 256 KB are
-// requested before the round in front is worked on.  What bounds it is what one CU fetches, 50 GB/s of its own and
-// 27 when all do, and the chain once per launch; the split counts follow that (ksa_decode_wide_splits).
+// requested before the round in front is worked on.  What bounds it: with many sequences the memory (64 of 9000 rows 6.8 TB/s, its waves 61 % of
+// the time waiting to issue the next loads, every byte read once), with few the chain of trips, once per launch (1 of 1500 rows: 71 % in
+// waits for what is requested), and what one CU fetches, 50 GB/s of its own and 27 when all do; the split counts follow that
+// (ksa_decode_wide_splits).
 // Attention and merge of calls behind one another in a graph, 32 / 8 heads of 128, in the kernel above -> here, us: 1 sequence of 150 / 300 /
-// 1500 / 9000 rows 6.4 / 7.7 / 8.7 / 15.3 -> 5.6 / 7.0 / 8.7 / 13.0; 4 of 300 / 3000 9.9 / 16.7 -> 7.5 / 14.6; 8 of 1500 18.0 ->
-// 14.6; 16 of 737 / 3000 15.9 / 39.9 -> 13.3 / 35.2; 24 of 737 / 1500 / 9000 20.5 / 37.5 / 178 -> 15.7 / 26.8 / 138; 32 of 737 / 9000
-// 23.8 / 188 -> 18.4 / 179; 48 of 1100 / 9000 46.8 / 301 -> 39.6 / 264; 64 of 1100 / 9000 49.7 / 359 -> 46.7 / 348.
+// 1500 / 9000 rows 6.2 / 8.1 / 8.7 / 15.4 -> 5.7 / 7.1 / 8.4 / 13.5; 4 of 300 / 3000 9.8 / 16.7 -> 7.8 / 14.9; 8 of 1500 18.1 ->
+// 15.0; 16 of 737 / 3000 16.0 / 38.7 -> 13.6 / 37.7; 24 of 737 / 1500 / 9000 20.6 / 37.3 / 172 -> 15.4 / 27.3 / 139; 32 of 737 / 9000
+// 23.4 / 180 -> 19.0 / 175; 48 of 1100 / 9000 45.1 / 286 -> 43.3 / 264; 64 of 9000 340 -> 341.
 // The probabilities enter the second product as two 16-bit parts, value and remainder: a wave's first tile of 64 rows fixes its
 // reference, where the kernel above has more of them, and a row at its reference has no rounding; with one part the output lay 1.3 %
 // further from 64 bits than the kernel above (60 shapes, up to 5 %), with two 12 % nearer (0.76 to 1.0 times), for 0.2 us a launch.
@@ -1202,10 +1205,10 @@ extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int m
     return n < 1 ? 1 : (int)n;
 }
 
-// Split count of the wide kernel, at most `most`: the one with the least time by what was measured of one workgroup to a CU, 3 us for the
-// start of the first round of workgroups and 5 of each one behind it, 10.2 ns a row of head_dim 128 and CU when the other CUs are idle and
-// 9.4 more when all are at work (half of that at head_dim 64), 2.2 to 3.8 us for the merge.  Against the best of nine counts around it
-// (2081 calls): within 5 % but for 18.
+// Split count of the wide kernel, at most `most`: the one with the least time by what was measured of one workgroup to a CU, 5 us for the
+// start of a round of workgroups (the first one takes 3, for every count alike), 10.2 ns a row of head_dim 128 and CU when the other CUs are
+// idle and 9.4 more when all are at work (half of that at head_dim 64), 2.2 to 3.8 us for the merge.  Against the best of nine counts around
+// it (2081 calls): within 5 % but for 18.
 static int wide_count(int64_t units, int D, int64_t max_rows, int64_t cus, int64_t most) {
     const int64_t tiles = (max_rows + kWideRows - 1) / kWideRows;
     most = most < tiles ? most : tiles;
