@@ -1210,18 +1210,18 @@ extern "C" int ksa_decode_splits(int batch, int Hq, int Hkv, int Q, int D, int m
 // idle and 9.4 more when all are at work (half of that at head_dim 64), 2.2 to 3.8 us for the merge.  Against the best of nine counts around
 // it (2081 calls): within 5 % but for 18.
 static int wide_count(int64_t units, int D, int64_t max_rows, int64_t cus, int64_t most) {
-    const int64_t tiles = (max_rows + kWideRows - 1) / kWideRows;
+    const unsigned tiles = (unsigned)((max_rows + kWideRows - 1) / kWideRows);
     most = most < tiles ? most : tiles;
     most = most < 1 ? 1 : most < 64 ? most : 64;
     const double row = D / 128.0 * 0.0102, load = D / 128.0 * 0.0094;
     int best = 1, before = 0;
     double least = 1e30;
-    for (int64_t n = 1; n <= most; ++n) {
-        const int64_t per = (tiles + n - 1) / n;
-        const int used = (int)((tiles + per - 1) / per);  // slices that have rows
+    for (unsigned n = 1; n <= (unsigned)most; ++n) {  // (every call walks this: no 64-bit divisions but for more than a round)
+        const unsigned per_tiles = (tiles + n - 1) / n;
+        const int used = (int)((tiles + per_tiles - 1) / per_tiles);  // slices that have rows
         if (used == before) continue;
         before = used;
-        const int64_t wgs = units * used, full = wgs / cus, rest = wgs % cus;
+        const int64_t per = per_tiles, wgs = units * used, full = wgs < cus ? 0 : wgs / cus, rest = wgs - full * cus;
         double us = full * (5.0 + per * kWideRows * (row + load));
         if (rest) us += 5.0 + per * kWideRows * (row + load * rest / cus);
         if (used > 1) us += 2.2 + (full ? 1.6 : 1.6 * rest / cus);
@@ -1247,8 +1247,11 @@ extern "C" int ksa_decode_wide_splits(int batch, int Hq, int Hkv, int Q, int D, 
     const int64_t units = (int64_t)batch * Hkv, cus = ksa_cu_count_or(256);
     if ((int64_t)Q * (Hq / Hkv) > kWideColumns) return 0;
     if (units > cus && max_rows <= 2500 && (max_rows <= 600 || max_rows > 1200 || 2 * units > 3 * cus)) return 0;
-    const int best = wide_count(units, D, max_rows, cus, 4 * cus / units), four = ksa_decode_splits(batch, Hq, Hkv, Q, D, max_rows);
-    if (D == 128 && (int64_t)best * kWideRows < max_rows && four > 1 && units * four <= cus && four * 128 >= max_rows) return 0;
+    const int best = wide_count(units, D, max_rows, cus, 4 * cus / units);
+    if (D == 128 && (int64_t)best * kWideRows < max_rows && units <= cus && units * max_rows <= 128 * cus) {  // (may be one round)
+        const int four = ksa_decode_splits(batch, Hq, Hkv, Q, D, max_rows);
+        if (four > 1 && units * four <= cus && four * 128 >= max_rows) return 0;
+    }
     return best;
 }
 

@@ -115,7 +115,8 @@ bool fits(const at::Tensor& t) {
 // 16-byte items: what the library would refuse, behind the allocations
 bool aligned(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 bool aligned(const at::Tensor& t) {
-    return aligned(t.const_data_ptr()) && ((t.stride(0) | t.stride(1) | t.stride(2)) & 7) == 0;
+    const auto s = t.strides();
+    return aligned(t.const_data_ptr()) && ((s[0] | s[1] | s[2]) & 7) == 0;
 }
 using Strides = std::array<int64_t, 3>;
 Strides first3(const at::Tensor& t) { return {t.stride(0), t.stride(1), t.stride(2)}; }
