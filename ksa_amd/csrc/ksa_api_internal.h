@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 // status codes returned by every extern "C" entry point (0 = success)
 enum {
     KSA_OK = 0,
@@ -30,10 +32,15 @@ static inline int ksa_check_launch() {
 }
 
 // Compute units of the current device, or `fallback` when no device can be asked (host-only use
-// of the heuristics).
+// of the heuristics).  A call's rules ask up to three times: the runtime is asked once for each device.
 static inline int ksa_cu_count_or(int fallback) {
+    constexpr int kDevices = 64;
+    static std::atomic<int> known[kDevices];  // 0: not asked yet
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess) return fallback;
+    const bool slot = dev >= 0 && dev < kDevices;
+    if (slot && (n = known[dev].load(std::memory_order_relaxed)) > 0) return n;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) return fallback;
+    if (slot) known[dev].store(n, std::memory_order_relaxed);
     return n;
 }
